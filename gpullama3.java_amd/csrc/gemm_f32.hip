@@ -1,0 +1,347 @@
+// C[M,N] = A[M,K] . W[N,K]^T with all operands, products and sums in true 32-bit on the matrix cores: the products of a
+// float32 engine (a wave's v_mfma_f32_16x16x4_f32 multiplies and adds IEEE floats; nothing is rounded to fewer bits on
+// the way). gl3_gemm_generic sends products here whose operands and output are float, K and W's rows in whole 16-byte
+// pieces; everything else stays with its own kernel.
+//
+// A token's result does not depend on how many tokens share the step, nor on the kernel below that works it out: both
+// add up an output element in the same order. K is cut into chunks of 256; inside a chunk k advances in blocks of 16,
+// a block being four instructions of which the j-th takes k = 4q + j, q = 0..3; each chunk's sum starts from zero, and
+// the chunks' sums are added in order. (Short chains of sums are also closer to the 64-bit result than one chain of K.)
+//
+// Two kernels, by the number of rows of A:
+// * up to 64 rows (gated 32): bound by the weights' way from memory. A block takes 16 rows of W (gated: 16 gate rows and
+//   their 16 up rows) and its sixteen waves a chunk of K each (16 KB of weights); the chunks' sums meet in shared memory.
+//   One row, weights from memory, 1B layers: gate/up 513 -> 29 us (134 MB: 4.6 TB/s), down projection 950 -> 26 us (67 MB:
+//   2.6 TB/s; 128 blocks), the head 179 us (5.9 TB/s), against the kernel for any sizes, whose 64 x 64 tiles leave a
+//   product of 2,048 columns 32 blocks that walk K in steps of 16 behind two barriers each. Eight waves a block were 1.0
+//   to 1.3 times as long.
+// * more: bound by the matrix cores (256 flops a clock and CU). Tiles through shared memory in steps of 32 k, two
+//   buffers, one barrier a step; rows in shared memory are 36 floats apart, so that the sixteen lanes that read 16 bytes of
+//   sixteen rows meet all 64 banks once. 4,096 x 4,096 x 4,096: 1.15 ms, 119 TFLOP/s (157 is the unit's peak); 513 rows of
+//   the 1B layers: 57 to 92 TFLOP/s against about 20.
+#include "common.h"
+#include <type_traits>
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+enum { F3_STORE = 0, F3_ADD = 1, F3_GATED = 2 };
+
+#define F3_CHUNK 256
+
+struct F3Out {     // what the epilogues need besides the sums
+  const float* bias;
+  const float* col_scale;
+  int act;
+  float act_limit, act_shift;
+};
+
+template <int EPI>
+__device__ __forceinline__ void f3_finish(float* c, float s, float up, int n, int N, const F3Out& o) {
+  if (o.bias) s += o.bias[n];
+  if (EPI == F3_GATED) {
+    if (o.bias) up += o.bias[N + n];
+    *c = gl3_gated<false>(s, up, o.act, o.act_limit, o.act_shift);
+    return;
+  }
+  if (o.col_scale) s *= o.col_scale[n];
+  if (EPI == F3_ADD) *c += s;
+  else *c = s;
+}
+
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));     // rows of A may begin at any float
+
+// loads of A for few rows go through a descriptor that ends where A ends: a lane without a token row of its own gives an
+// offset beyond it, asks memory for nothing and gets zeros, without a branch around the load
+#define F3_NOWHERE 0x80000000u
+__device__ __forceinline__ f32x4 f3_load_a(__amdgpu_buffer_rsrc_t buf, unsigned row, unsigned byte) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, row == F3_NOWHERE ? F3_NOWHERE : row + byte, 0, 0));
+}
+
+// ---- few rows
+#define F3_WAVES 16
+
+template <int EPI, int TM>
+__global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                      float* __restrict__ C, int M, int N, int K, long lda,
+                                                                      long ldw, long ldc, F3Out o) {
+  constexpr int NW = F3_WAVES;
+  constexpr int G = EPI == F3_GATED ? 2 : 1;
+  constexpr int NE = (256 * TM + 64 * NW - 1) / (64 * NW);     // output elements a thread adds up
+  constexpr int SLOTS = 32 / (G * TM) > NW ? 32 / (G * TM) : NW;   // chunks whose sums lie in shared memory at a time
+  __shared__ __attribute__((aligned(16))) f32x4 sums[SLOTS][G][TM][64];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int r = lane & 15, q = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  const int wrow = min(n0 + r, N - 1);
+  const float* wp[G];
+  wp[0] = W + (long)wrow * ldw + q * 4;
+  if (G == 2) wp[G - 1] = W + ((long)N + wrow) * ldw + q * 4;
+  const __amdgpu_buffer_rsrc_t a_buf = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)(((long)(M - 1) * lda + K) * 4), 0x00020000);
+  unsigned ao[TM];
+#pragma unroll
+  for (int t = 0; t < TM; ++t) ao[t] = t * 16 + r < M ? (unsigned)(((long)(t * 16 + r) * lda + q * 4) * 4) : F3_NOWHERE;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  float total[G][NE] = {};
+  const int chunks = (K + F3_CHUNK - 1) / F3_CHUNK;
+  for (int first = 0; first < chunks; first += SLOTS) {
+    const int n_here = min(SLOTS, chunks - first);
+    if (first) __syncthreads();
+    for (int slot = wave; slot < n_here; slot += NW) {
+      const int k0 = (first + slot) * F3_CHUNK;
+      f32x4 acc[G][TM];
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int t = 0; t < TM; ++t) acc[g][t] = zero;
+      if (k0 + F3_CHUNK <= K) {
+        // a whole chunk: sixteen loads of each operand, unrolled, for the scheduler to send ahead (all of them in front of the
+        // first product was slower: 23.8 -> 27.0 us)
+        constexpr int PART = 16 / G;
+#pragma unroll
+        for (int p = 0; p < 16; p += PART) {
+          f32x4 w[G][PART];
+#pragma unroll
+          for (int b = 0; b < PART; ++b)
+#pragma unroll
+            for (int g = 0; g < G; ++g) w[g][b] = *(const f32x4*)(wp[g] + k0 + (p + b) * 16);
+#pragma unroll
+          for (int b = 0; b < PART; ++b) {
+#pragma unroll
+            for (int t = 0; t < TM; ++t) {
+              const f32x4 a = f3_load_a(a_buf, ao[t], (unsigned)(k0 + (p + b) * 16) * 4);
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int g = 0; g < G; ++g) acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[g][b][j], a[j], acc[g][t], 0, 0, 0);
+            }
+          }
+        }
+      } else {
+        for (int k = k0; k < K; k += 16) {     // (K is a multiple of 4: a lane's four k lie inside it or beyond it)
+          const bool in = k + q * 4 < K;
+#pragma unroll
+          for (int t = 0; t < TM; ++t) {
+            const f32x4 a = f3_load_a(a_buf, in ? ao[t] : F3_NOWHERE, (unsigned)k * 4);
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+              const f32x4 w = in ? *(const f32x4*)(wp[g] + k) : zero;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], a[j], acc[g][t], 0, 0, 0);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int t = 0; t < TM; ++t) sums[slot][g][t][lane] = acc[g][t];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      const int e = tid + 64 * NW * i;
+      if (e < 256 * TM) {
+        for (int s = 0; s < n_here; ++s)
+#pragma unroll
+          for (int g = 0; g < G; ++g) total[g][i] += ((const float*)&sums[s][g][0][0])[e];
+      }
+    }
+  }
+  // element e: token tile e / 256, lane (e / 4) % 64, v = e % 4: token lane % 16, column 4 * (lane / 16) + v
+#pragma unroll
+  for (int i = 0; i < NE; ++i) {
+    const int e = tid + 64 * NW * i;
+    const int l = (e >> 2) & 63, m = (e >> 8) * 16 + (l & 15), n = n0 + 4 * (l >> 4) + (e & 3);
+    if (e < 256 * TM && m < M && n < N) f3_finish<EPI>(C + (long)m * ldc + n, total[0][i], total[G - 1][i], n, N, o);
+  }
+}
+
+// ---- many rows: four waves, 2 x 2, a wave owns 16 * TW rows of W by 16 * TT tokens
+#define F3_BK 32
+#define F3_LD (F3_BK + 4)
+
+template <int EPI, int TW, int TT>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                               float* __restrict__ C, int M, int N, int K, long lda,
+                                                               long ldw, long ldc, int tiles_m, int tiles_n, F3Out o) {
+  constexpr int BN = 32 * TW, BM = 32 * TT;
+  constexpr int NCOLS = EPI == F3_GATED ? BN / 2 : BN;
+  static_assert(EPI != F3_GATED || TW % 2 == 0, "a wave's tiles are gate rows and their up rows");
+  __shared__ __attribute__((aligned(16))) float Ws[2][BN][F3_LD];
+  __shared__ __attribute__((aligned(16))) float As[2][BM][F3_LD];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int r = lane & 15, q = lane >> 4;
+  const int ww = wave & 1, wt = wave >> 1;
+  // an XCD (consecutive block ids take turns) works on neighbouring tiles: all token tiles of a column, then the next
+  const int n_tiles = tiles_m * tiles_n, per_xcd = (n_tiles + 7) / 8;
+  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (tile >= n_tiles) return;
+  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * NCOLS;
+
+  // memory -> registers -> shared memory in pieces of 16 bytes, eight a row and step; rows beyond the matrix repeat its
+  // last one (their sums are dropped), k beyond K is zero
+  constexpr int NW = BN * 8 / 256, NA = BM * 8 / 256;
+  const float *wp[NW], *ap[NA];
+  const int kc = (tid & 7) * 4;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const int row = (tid >> 3) + 32 * i;
+    int n = n0 + row;
+    if (EPI == F3_GATED) {       // (a wave's rows: TW / 2 tiles of gate rows, then the up rows of the same columns)
+      const int sec = row / (16 * TW), in = row % (16 * TW);
+      n = min(n0 + sec * 8 * TW + in % (8 * TW), N - 1) + (in >= 8 * TW ? N : 0);
+    } else {
+      n = min(n, N - 1);
+    }
+    wp[i] = W + (long)n * ldw;
+  }
+#pragma unroll
+  for (int i = 0; i < NA; ++i) ap[i] = A + (long)min(m0 + (tid >> 3) + 32 * i, M - 1) * lda;
+  f32x4 rw[NW], ra[NA];
+  bool r_ok = false;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  auto fetch = [&](int k0) {      // (loads without a branch: a piece beyond K reads the row's last one and is not kept)
+    r_ok = k0 + kc < K;
+    const int k = min(k0 + kc, K - 4);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) ra[i] = *(const f32x4_any*)(ap[i] + k);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) rw[i] = *(const f32x4*)(wp[i] + k);
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) *(f32x4*)&As[buf][(tid >> 3) + 32 * i][kc] = r_ok ? ra[i] : zero;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) *(f32x4*)&Ws[buf][(tid >> 3) + 32 * i][kc] = r_ok ? rw[i] : zero;
+  };
+
+  f32x4 acc[TW][TT], total[TW][TT];
+#pragma unroll
+  for (int a = 0; a < TW; ++a)
+#pragma unroll
+    for (int b = 0; b < TT; ++b) acc[a][b] = total[a][b] = zero;
+  fetch(0);
+  store(0);
+  fetch(F3_BK);
+  __syncthreads();
+  for (int k0 = 0, buf = 0; k0 < K; k0 += F3_BK, buf ^= 1) {
+    if (k0 + F3_BK < K) {
+      store(buf ^ 1);
+      fetch(k0 + 2 * F3_BK);
+    }
+#pragma unroll
+    for (int kb = 0; kb < F3_BK; kb += 16) {
+      f32x4 w[TW], a[TT];
+#pragma unroll
+      for (int i = 0; i < TW; ++i) w[i] = *(const f32x4*)&Ws[buf][ww * 16 * TW + i * 16 + r][kb + q * 4];
+#pragma unroll
+      for (int i = 0; i < TT; ++i) a[i] = *(const f32x4*)&As[buf][wt * 16 * TT + i * 16 + r][kb + q * 4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < TW; ++x)
+#pragma unroll
+          for (int y = 0; y < TT; ++y)
+            acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[x][j], a[y][j], acc[x][y], 0, 0, 0);
+    }
+    if ((k0 + F3_BK) % F3_CHUNK == 0 || k0 + F3_BK >= K) {
+#pragma unroll
+      for (int x = 0; x < TW; ++x)
+#pragma unroll
+        for (int y = 0; y < TT; ++y) {
+          total[x][y] += acc[x][y];
+          acc[x][y] = zero;
+        }
+    }
+    __syncthreads();
+  }
+  // a lane holds four consecutive columns of one token per tile
+#pragma unroll
+  for (int y = 0; y < TT; ++y) {
+    const int m = m0 + wt * 16 * TT + y * 16 + r;
+    if (m >= M) continue;
+    float* c = C + (long)m * ldc;
+#pragma unroll
+    for (int x = 0; x < (EPI == F3_GATED ? TW / 2 : TW); ++x) {
+      const int n = n0 + ww * (EPI == F3_GATED ? 8 : 16) * TW + x * 16 + q * 4;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (n + v < N)
+          f3_finish<EPI>(c + n + v, total[x][y][v], total[EPI == F3_GATED ? TW / 2 + x : x][y][v], n + v, N, o);
+    }
+  }
+}
+
+template <int EPI, int TM>
+static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
+                       const F3Out& o, hipStream_t stream) {
+  gemm_f32_rows_kernel<EPI, TM><<<dim3((N + 15) / 16), dim3(64 * F3_WAVES), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, o);
+  GL3_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int EPI, int TW, int TT>
+static int launch_tile(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
+                       const F3Out& o, hipStream_t stream) {
+  const int ncols = EPI == F3_GATED ? 16 * TW : 32 * TW;
+  const int tiles_m = (M + 32 * TT - 1) / (32 * TT), tiles_n = (N + ncols - 1) / ncols;
+  const long blocks = ((long)tiles_m * tiles_n + 7) / 8 * 8;
+  GL3_REQUIRE(blocks < (1L << 31), "gl3_gemm_generic: too many tiles");
+  gemm_f32_tile_kernel<EPI, TW, TT><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, tiles_m,
+                                                                                    tiles_n, o);
+  GL3_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int EPI>
+static int launch_f32(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
+                      const F3Out& o, int shape, hipStream_t stream) {
+#define F3_ARGS A, W, C, M, N, K, lda, ldw, ldc, o, stream
+  if (shape == 0) shape = gl3_f32_shape(M, N, EPI == F3_GATED);
+  if (shape == 1 && ((long)(M - 1) * lda + K) * 4 >= (1L << 31)) shape = 5;      // (a descriptor's 31 bits)
+  switch (shape) {
+    case 1:
+      if (M <= 16) return launch_rows<EPI, 1>(F3_ARGS);
+      if (M <= 32) return launch_rows<EPI, 2>(F3_ARGS);
+      if constexpr (EPI != F3_GATED) return launch_rows<EPI, 4>(F3_ARGS);
+    case 2: return launch_tile<EPI, 4, 4>(F3_ARGS);
+    case 3: return launch_tile<EPI, 4, 2>(F3_ARGS);
+    case 4: return launch_tile<EPI, 2, 2>(F3_ARGS);
+    default: return launch_tile<EPI, 2, 1>(F3_ARGS);
+  }
+#undef F3_ARGS
+}
+
+// 1: the kernel for few rows; 2 to 5: tiles of 128 x 128, 128 x 64, 64 x 64 and 64 rows of W x 32 tokens. Of the tiles the
+// one that takes the least time: one tile alone on a CU takes `alone`, a CU with several of them `each` a tile (us for
+// K = 2,048, both measured; the sum of a CU's tiles was within 4% of the measured time at 513 to 4,096 rows). Few rows: 48
+// rows of the down projection of the 1B layers 136 us in the smallest tile; gated products of more than 32 rows fill the
+// chip with those (48 rows: 55 us) where the other kernel would hold 128 KB of sums a block.
+int gl3_f32_shape(int M, int N, bool gated) {
+  if (M <= (gated ? 32 : 64)) return 1;
+  static const int bn[4] = {128, 128, 64, 64}, bm[4] = {128, 64, 64, 32}, alone[4] = {154, 89, 53, 34}, each[4] = {144, 76, 41, 23};
+  int best = 5;
+  long least = -1;
+  for (int i = 0; i < 4; ++i) {
+    const long tiles = (long)((M + bm[i] - 1) / bm[i]) * (((gated ? 2L : 1L) * N + bn[i] - 1) / bn[i]);
+    const long cu = (tiles + 255) / 256 * each[i], cost = cu < alone[i] ? alone[i] : cu;
+    if (least < 0 || cost < least) {
+      least = cost;
+      best = i + 2;
+    }
+  }
+  return best;
+}
+
+bool gl3_f32_takes(const void* W, int K, long ldw) { return K % 4 == 0 && ldw % 4 == 0 && (uintptr_t)W % 16 == 0; }
+
+int gl3_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc, int epi,
+                 const float* bias, int act, float act_limit, float act_shift, const float* col_scale, int shape,
+                 hipStream_t stream) {
+  const F3Out o{bias, col_scale, act, act_limit, act_shift};
+#define F3_ARGS (const float*)A, (const float*)W, (float*)C, M, N, K, lda, ldw, ldc, o, shape, stream
+  if (epi == F3_STORE) return launch_f32<F3_STORE>(F3_ARGS);
+  if (epi == F3_ADD) return launch_f32<F3_ADD>(F3_ARGS);
+  return launch_f32<F3_GATED>(F3_ARGS);
+#undef F3_ARGS
+}

@@ -1,7 +1,8 @@
 // C[M,N] = A[M,K] . W[N,K]^T for any sizes and any mix of float / bfloat16
 // operands, with 32-bit multiply-adds only (no matrix-core, no reduced-precision
 // mode): the true 32-bit path of the model and the fallback for shapes that the
-// matrix-core kernels refuse. W is row-major [out, in] as the reference's matmul
+// matrix-core kernels refuse. (Products whose operands and output are all float go on to gemm_f32.hip where K and W
+// come in whole 16-byte pieces.) W is row-major [out, in] as the reference's matmul
 // reads it (J/core/model/tensor/FloatTensor.java:98-100).
 //
 // Every output element is the sum over k = 0..K-1 in ascending order, one
@@ -141,6 +142,8 @@ extern "C" int gl3_gemm_generic(const void* A, int a_dtype, const void* W, int w
                   (w_order == 1 || !w_pos),
               "gl3_gemm_generic: W in order %d with N=%d, epilogue %d", w_order, N, epilogue);
   const int w_steps = w_order == 1 ? (K + 31) / 32 : (K + 63) / 64;
+  if (a_dtype == GL3_F32 && w_dtype == GL3_F32 && c_dtype == GL3_F32 && w_order == 0 && gl3_f32_takes(W, K, ldw))
+    return gl3_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, epilogue, bias, act, act_limit, act_shift, col_scale, 0, stream);
   const int key = a_dtype * 4 + w_dtype * 2 + c_dtype;
   switch (key) {
     case 0: return launch_generic<float, float, float>(A, W, C, M, N, K, lda, ldw, ldc, epilogue, bias, act, w_order, w_steps, w_pos, act_limit, act_shift, col_scale, stream);

@@ -1,0 +1,75 @@
+"""The 32-bit products on the matrix cores at the edges of their tiles: against 64 bits, against the kernel for any sizes,
+and a row alone against the same row in company."""
+import numpy as np
+import pytest
+import torch
+
+import plain_llama as P
+from test_gpu_kernels import K, dev
+
+pytestmark = pytest.mark.gpu
+
+
+def bound(a, w, K_):
+    """What 32-bit sums may be off by: each sum is a chain of at most 256 products behind one of K / 256 partial sums, and
+    every link rounds to 2^-24 of at most the sum of magnitudes."""
+    return (256 + K_ / 256 + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64).T)
+
+
+# rows of one tile and one more (16, 32, 64, 128), columns likewise, K in one piece of 4, up to a chunk of 256 and beyond it
+@pytest.mark.parametrize("M, N, Kd", [(1, 16, 4), (3, 130, 72), (16, 33, 256), (17, 48, 260), (32, 257, 1028), (33, 77, 96), (48, 2048, 8192),
+                                      (64, 129, 516), (65, 200, 300), (130, 513, 2052), (513, 1024, 1024), (1030, 2500, 64)])
+def test_float32_products(M, N, Kd):
+    lib = K()
+    rng = np.random.default_rng(M * N + Kd)
+    a, w = rng.standard_normal((M, Kd)).astype(np.float32), rng.standard_normal((2 * N, Kd)).astype(np.float32)
+    bias, factor = rng.standard_normal(2 * N).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    A, W, B, F = dev(a), dev(w), dev(bias), dev(factor)
+    both = a.astype(np.float64) @ w.astype(np.float64).T
+    off = bound(a, w, Kd)
+    out = torch.full((M, N + 3), -7.0, device=A.device)
+    lib.gemm_generic(A, W[:N], out[:, 1:N + 1])                                    # rows of the output apart
+    assert (np.abs(out[:, 1:N + 1].double().cpu().numpy() - both[:, :N]) <= off[:, :N]).all()
+    assert torch.all(out[:, 0] == -7.0) and torch.all(out[:, N + 1:] == -7.0)
+    res = rng.standard_normal((M, N)).astype(np.float32)
+    x = dev(res)
+    lib.gemm_generic(A, W[:N], x, lib.EPI_ADD, bias=B[:N], col_scale=F)
+    want = res + (both[:, :N] + bias[:N]) * factor.astype(np.float64)
+    slack = 4 * 2.0 ** -24 * (np.abs(res) + (np.abs(both[:, :N]) + np.abs(bias[:N])) * np.abs(factor))
+    assert (np.abs(x.double().cpu().numpy() - want) <= off[:, :N] * np.abs(factor) + slack).all()
+    gated = torch.empty(M, N, device=A.device)
+    lib.gemm_generic(A, W, gated, lib.EPI_GATED, bias=B)
+    gate, up = both[:, :N] + bias[:N], both[:, N:] + bias[N:]
+    sig = 1.0 / (1.0 + np.exp(-gate))
+    # (|silu'| <= 1.1; the exponential and the division are within 4 units of the last place)
+    slack = (1.1 * (off[:, :N] + 2.0 ** -23 * np.abs(gate)) * (np.abs(up) + off[:, N:])
+             + np.abs(gate * sig) * (off[:, N:] + 2.0 ** -23 * np.abs(up)) + 8 * 2.0 ** -24 * np.abs(gate * sig * up))
+    assert (np.abs(gated.double().cpu().numpy() - gate * sig * up) <= slack + 1e-30).all()
+    # a row alone, and rows that begin at any float, give the same bits
+    one, shifted = torch.empty(1, N, device=A.device), torch.empty(M, Kd + 1, device=A.device)[:, 1:]
+    shifted.copy_(A)
+    for r in {0, M // 2, M - 1}:
+        lib.gemm_generic(A[r:r + 1], W[:N], one)
+        assert torch.equal(one[0], out[r, 1:N + 1])
+        lib.gemm_generic(shifted[r:r + 1], W, one, lib.EPI_GATED, bias=B)
+        assert torch.equal(one[0], gated[r])
+    # W at an odd float: the kernel for any sizes
+    odd = torch.empty(N * Kd + 1, device=A.device)[1:].view(N, Kd)
+    odd.copy_(W[:N])
+    general = torch.empty(M, N, device=A.device)
+    lib.gemm_generic(A, odd, general)
+    one_chain = (Kd + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w[:N]).astype(np.float64).T)
+    assert (np.abs((general - out[:, 1:N + 1]).double().cpu().numpy()) <= off[:, :N] + one_chain).all()
+
+
+def test_float32_products_keep_small_numbers_and_infinities():
+    lib = K()
+    a, w = np.zeros((20, 64), np.float32), np.zeros((32, 64), np.float32)
+    a[0, 3], w[5, 3] = 2e-39, 0.5                        # below the smallest normal number
+    a[1, 7], w[6, 7] = 1e-20, 3e-20
+    a[2, 9], w[:, 9] = np.inf, 1.0
+    out = torch.empty(20, 32, device="cuda:0")
+    lib.gemm_generic(dev(a), dev(w), out)
+    out = out.cpu().numpy()
+    assert out[0, 5] == np.float32(1e-39) and out[1, 6] == np.float32(np.float32(1e-20) * np.float32(3e-20))
+    assert np.isinf(out[2]).all() and np.isfinite(np.delete(out, 2, 0)).all()
