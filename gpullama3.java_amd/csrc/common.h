@@ -39,6 +39,13 @@ int gl3_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, lon
                  const float* bias, int act, float act_limit, float act_shift, const float* col_scale, int shape,
                  hipStream_t stream);
 
+// attention_f32.hip: the plain causal rule in true 32-bit on the matrix cores, which gl3_attention_generic hands on where the
+// layer's sizes allow (a rule on the layer alone, as above)
+bool gl3_attention_f32_takes(int head_dim, int page_size);
+int gl3_attention_f32(const float* q, long q_stride, const float* k_cache, const float* v_cache, const int* positions,
+                      const int* table_rows, const int* block_table, int table_stride, float* out, long out_stride, int n_tokens,
+                      int n_heads, int n_kv, int head_dim, int page_size, float scale, hipStream_t stream);
+
 // dtype codes shared with the Python side
 enum { GL3_F32 = 0, GL3_BF16 = 1 };
 

@@ -1,11 +1,10 @@
-"""The 32-bit products on the matrix cores at the edges of their tiles: against 64 bits, against the kernel for any sizes,
+"""The 32-bit products and attention on the matrix cores at the edges of their tiles: against a plain reference, against the kernels for any sizes,
 and a row alone against the same row in company."""
 import numpy as np
 import pytest
 import torch
 
-import plain_llama as P
-from test_gpu_kernels import K, dev
+from test_gpu_kernels import K, attention_case, dev, run_attention
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +72,43 @@ def test_float32_products_keep_small_numbers_and_infinities():
     out = out.cpu().numpy()
     assert out[0, 5] == np.float32(1e-39) and out[1, 6] == np.float32(np.float32(1e-20) * np.float32(3e-20))
     assert np.isinf(out[2]).all() and np.isfinite(np.delete(out, 2, 0)).all()
+
+
+# ------------------------------------------------------------------ attention
+# heads alone and in groups (3: rows of a tile that are no whole tokens; 17: a group in two tiles), contexts of one key, of the
+# edges of a step of 64 and of a wave's turn (8 steps), several sequences in a tile's tokens; enough tokens for whole tiles in the last
+@pytest.mark.parametrize("H, Kh, hs, before, new", [(4, 2, 32, [0, 70, 130, 5], [33, 1, 2, 1]), (8, 2, 64, [0, 511, 0], [1, 2, 130]),
+                                                    (3, 1, 96, [62, 0], [4, 63]), (2, 2, 128, [0, 600], [65, 1]), (17, 1, 64, [0, 9], [20, 3]),
+                                                    (32, 8, 64, [100, 0], [200, 150])])
+def test_float32_attention(H, Kh, hs, before, new):
+    lib = K()
+    rng = np.random.default_rng(H * hs)
+    sk, sv, qs = attention_case(rng, H, Kh, hs, before, new, "float32")
+    got, ref = run_attention(lib.attention_generic, sk, sv, qs, before, new, H, Kh, hs, "float32", np.random.default_rng(5))
+    np.testing.assert_allclose(got, ref, atol=2e-5 * np.abs(ref).max())
+    # a window that hides nothing takes the kernel for any rule
+    general, _ = run_attention(lib.attention_generic, sk, sv, qs, before, new, H, Kh, hs, "float32", np.random.default_rng(5), window=1 << 20)
+    np.testing.assert_allclose(got, general, atol=4e-6 * np.abs(ref).max())
+    # every token alone: the same bits
+    first = 0
+    for b, (n0, n) in enumerate(zip(before, new)):
+        for p in sorted({0, 1, n // 2, n - 1} & set(range(n))):
+            cut = [[s[b][:n0 + p + 1]] for s in (sk, sv, qs)]
+            one, _ = run_attention(lib.attention_generic, *cut, [n0 + p], [1], H, Kh, hs, "float32", rng)
+            np.testing.assert_array_equal(one[0], got[first + p])
+        first += n
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_float32_attention_leaves_values_out_that_a_row_does_not_see(bad):
+    lib = K()
+    rng = np.random.default_rng(2)
+    H, Kh, hs, n, at = 4, 2, 64, 150, 101
+    sk, sv, qs = attention_case(rng, H, Kh, hs, [0], [n], "float32")
+    clean, _ = run_attention(lib.attention_generic, sk, sv, qs, [0], [n], H, Kh, hs, "float32", np.random.default_rng(5))
+    sv[0][at, 1, 7] = bad
+    got, _ = run_attention(lib.attention_generic, sk, sv, qs, [0], [n], H, Kh, hs, "float32", np.random.default_rng(5))
+    np.testing.assert_array_equal(got[:at], clean[:at])
+    assert not np.isfinite(got[at:, 2:, 7]).any()
+    got[at:, 2:, 7] = clean[at:, 2:, 7] = 0
+    np.testing.assert_array_equal(got, clean)
