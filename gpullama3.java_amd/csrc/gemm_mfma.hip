@@ -14,12 +14,16 @@
 // contiguous range of tiles, ordered so that the tiles it holds at one time form a rectangle
 // and share their panels of A and of W.
 //
+// Tiles of 256 x 256 over whole steps of 64 k have a kernel of their own (gemm_mfma_turns_kernel, below).
+//
 // Epilogues as in gemm_generic.hip: store, add into a float matrix, gated.
 #include "common.h"
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 enum { MF_STORE = 0, MF_ADD = 1, MF_GATED = 2 };
 
@@ -263,6 +267,274 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
   else finish(std::true_type{});
 }
 
+// ---- 256 x 256 tiles over whole steps of 64 k: operands straight from memory into shared memory, waves in two groups
+// that take turns.
+//
+// Eight waves; wave w's rows of A are 64 of each half of the tile's (group w / 4), its rows of W 32 of each half (gated:
+// half 0 holds gate rows, half 1 the up rows of the same columns). A step of 64 k is four phases, one pair of halves
+// each: (A0, W0), (A0, W1), (A1, W1), (A1, W0). A phase is a memory part (operands from shared memory to registers, a half
+// tile of a later step from memory to shared memory) and sixteen 16x16x32 matrix instructions, with a barrier after each
+// part; the second group runs one part behind the first, so on every SIMD one wave's matrix instructions run while the
+// other wave's memory part does. Without that lag the same loop is 19% slower (1.24 against 1.50 PFLOP/s at 8,192 x 8,192 x
+// 4,096). What bounds it now is the power budget: the matrix cores are busy 82% of the cycles at 1.5 to 1.6 GHz, and with
+// the 32x32x16 instruction, whose accumulators pass through the registers twice as often per flop, the same loop lost 11%.
+// (8,192 x 28,672 x 4,096: the kernel above 1,680 us, this one 1,312.)
+//
+// Registers are read a part or two before they are used: in the memory part of phase 0 W0 and half of A1, of phase 1 the
+// rest of A1, of phases 2 and 3 the next step's A0 and W1. A half tile's place in shared memory is written for the step after
+// next as soon as both groups have read it (their reads have returned: lgkmcnt before the barrier in front of the part
+// that asks), and the loads are only waited for where the next barrier hands them out, so six to eight are on their way
+// through a whole step:
+//   part of phase 0:                          reads of this step's A0, W1 are behind every wave after it
+//   part of phase 1: load A0, W1 of step + 2; wait until 8 are out: A0, W1 of step + 1 have come (read from phase 2 on)
+//   part of phase 2: load W0 of step + 2;     reads of this step's A1 are behind every wave after it
+//   part of phase 3: load A1 of step + 2;     wait until 8 are out: W0, A1 of step + 1 have come (read from phase 0 on)
+// Steps beyond the last read the last again, so that the counts hold; nothing is in flight when a block ends.
+//
+// In shared memory rows of A (and of W as stored) are 128 bytes in eight pieces of 16, piece c of row r at place
+// c ^ (r / 2 % 8): the sixteen rows that sixteen lanes read at one piece meet all banks once. W in a copy's order lies as
+// the operands want it, [strip of 16][k-step of 32][lane][16 bytes].
+__device__ __forceinline__ void mf_dma16(unsigned lds, unsigned offset, i32x4 rsrc, unsigned step_offset) {
+  // (by hand: behind the builtin the compiler waits for every load in front of every read of shared memory. The
+  // instruction has no destination register; its data lands at m0 + 16 * lane)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(offset), "s"(rsrc), "s"(step_offset)
+               : "memory", "m0");
+}
+template <int N>
+__device__ __forceinline__ void mf_wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void mf_wait_reads() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void mf_barrier() {      // no wait of its own, and nothing moves across it
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ i32x4 mf_rsrc(const void* p) {
+  const unsigned long a = (unsigned long)p;
+  return i32x4{__builtin_amdgcn_readfirstlane((int)a), __builtin_amdgcn_readfirstlane((int)(a >> 32)), 0x7fffffff, 0x00020000};
+}
+// Byte offset, from the address that mf_w_base gives, of the 16 bytes of W at row `row`, piece k .. k + 7 of the first step,
+// and how far a step of 64 k lies behind the one before it.
+template <int WT>
+__device__ __forceinline__ unsigned mf_w_offset(int row, int k, long ldw, int w_steps, const int* w_pos, int n0) {
+  return WT == 1   ? (unsigned)gl3_operand_offset(w_pos ? w_pos[row] : row, k, w_steps) * 2
+         : WT == 2 ? (unsigned)gl3_packed_offset(row, k, w_steps) * 2
+                   : (unsigned)((long)(row - n0) * ldw + k) * 2;
+}
+
+// Four consecutive columns n .. n + 3 of an output row (`vec`: they may go at once).
+template <int EPI, typename TC>
+__device__ __forceinline__ void mf_finish4(TC* c, f32x4 s, f32x4 up, int n, int N, bool vec, const float* bias, int act, const MfExtras& ex) {
+  typedef TC tc4 __attribute__((ext_vector_type(4)));
+  const int left = N - n;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int at = min(n + j, N - 1);
+    if (bias) {
+      s[j] += bias[at];
+      if (EPI == MF_GATED) up[j] += bias[N + at];
+    }
+    if (EPI == MF_GATED) s[j] = gl3_gated<true>(s[j], up[j], act, ex.act_limit, ex.act_shift);
+    else if (ex.col_scale) s[j] *= ex.col_scale[at];
+  }
+  if (vec && left >= 4) {
+    if (EPI == MF_ADD) {
+      const tc4 old = *(const tc4*)c;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[j] += to_f32<TC>(old[j]);
+    }
+    tc4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = from_f32<TC>(s[j]);
+    *(tc4*)c = o;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j < left) c[j] = from_f32<TC>(EPI == MF_ADD ? to_f32<TC>(c[j]) + s[j] : s[j]);
+  }
+}
+
+template <int EPI, typename TC, int WT>
+__global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                  TC* __restrict__ C, int M, int N, int K, long lda, long ldw,
+                                                                  long ldc, int tiles_m, int tiles_n, int group_m,
+                                                                  int k_per_slice, float* __restrict__ P, long p_stride, long ldp,
+                                                                  const float* __restrict__ bias, int act, int w_steps,
+                                                                  const int* __restrict__ w_pos, MfExtras ex) {
+  constexpr int NCOLS = EPI == MF_GATED ? 128 : 256;
+  __shared__ __attribute__((aligned(1024))) char lds[131072];       // A: two steps of 32 KB, then W: two steps of 32 KB
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave >> 2, wn = wave & 3;
+  const int lr = lane & 15, lq = lane >> 4;
+  const int n_tiles = tiles_m * tiles_n, per_xcd = (n_tiles + 7) / 8;
+  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;       // (block -> tile as above)
+  if (tile >= n_tiles) return;
+  const int band = tile / (group_m * tiles_n), in_band = tile % (group_m * tiles_n);
+  const int band_rows = min(group_m, tiles_m - band * group_m);
+  const int m0 = (band * group_m + in_band % band_rows) * 256;
+  const int n0 = (in_band / band_rows) * NCOLS;
+  const int slice = blockIdx.y;
+  // (the last of many slices may have no step left: it stores zeros)
+  const int k_begin = min(slice * k_per_slice, K - 64), steps = max(0, (min(K, (slice + 1) * k_per_slice) - slice * k_per_slice) >> 6);
+
+  // who brings what: a half tile is 16 pieces of 1 KB, two a wave
+  const i32x4 a_buf = mf_rsrc(A + (long)m0 * lda + k_begin);
+  const i32x4 w_buf = mf_rsrc(WT ? W + (long)(k_begin >> 6) * (WT == 1 ? 1024 : 512) : W + (long)n0 * ldw + k_begin);
+  constexpr unsigned W_STEP = WT == 1 ? 2048 : WT == 2 ? 1024 : 128;
+  unsigned ao[2][2], wo[2][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int piece = wave * 2 + i;
+      const int row = piece * 8 + (lane >> 3), at = ((lane & 7) ^ ((row >> 1) & 7)) * 8;      // (rows of 128 bytes)
+      ao[h][i] = (unsigned)((long)(min(m0 + h * 128 + row, M - 1) - m0) * lda + at) * 2;
+      const int w_row = WT ? (piece >> 1) * 16 + lr : row, w_k = WT ? (piece & 1) * 32 + lq * 8 : at;
+      const int n = min(n0 + (EPI == MF_GATED ? 0 : h * 128) + w_row, N - 1) + (EPI == MF_GATED && h ? N : 0);
+      wo[h][i] = mf_w_offset<WT>(n, w_k, ldw, w_steps, w_pos, n0);
+    }
+  const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)lds + wave * 2048;
+  auto load_a = [&](int h, int t) {
+    const unsigned s = (unsigned)max(0, min(t, steps - 1)) * 128;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) mf_dma16(lds0 + (t & 1) * 32768 + h * 16384 + i * 1024, ao[h][i], a_buf, s);
+  };
+  auto load_w = [&](int h, int t) {
+    const unsigned s = (unsigned)max(0, min(t, steps - 1)) * W_STEP;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) mf_dma16(lds0 + 65536 + (t & 1) * 32768 + h * 16384 + i * 1024, wo[h][i], w_buf, s);
+  };
+
+  f32x4 acc[2][4][2][2];      // [half of A][16 rows][half of W][16 rows]
+#pragma unroll
+  for (int i = 0; i < 32; ++i) (&acc[0][0][0][0])[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 af[2][4][2], wf[2][2][2];      // [half][16 rows][k-step of 32]
+  const char* a_at = lds + (wm * 64 + lr) * 128;
+  const char* w_at = lds + 65536 + (WT ? wn * 4096 + lane * 16 : (wn * 32 + lr) * 128);
+  const int twist = (lr >> 1) & 7;
+  auto read_a = [&](int h, int buf, int ks) {
+#pragma unroll
+    for (int tm = 0; tm < 4; ++tm)
+      af[h][tm][ks] = *(const bf16x8*)(a_at + buf * 32768 + h * 16384 + tm * 2048 + (((ks * 4 + lq) ^ twist) << 4));
+  };
+  auto read_w = [&](int h, int buf) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int tn = 0; tn < 2; ++tn)
+        wf[h][tn][ks] = *(const bf16x8*)(w_at + buf * 32768 + h * 16384 + tn * 2048 + (WT ? ks * 1024 : ((ks * 4 + lq) ^ twist) << 4));
+  };
+  auto products = [&](int ah, int wh) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+        for (int tm = 0; tm < 4; ++tm)
+          acc[ah][tm][wh][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[wh][tn][ks], af[ah][tm][ks], acc[ah][tm][wh][tn], 0, 0, 0);
+  };
+
+  load_a(0, 0);
+  load_w(1, 0);
+  load_w(0, 0);
+  load_a(1, 0);
+  load_a(0, 1);
+  load_w(1, 1);
+  load_w(0, 1);
+  load_a(1, 1);
+  mf_wait_loads<8>();
+  mf_barrier();
+  if (wm == 1) mf_barrier();          // the second group runs a part behind
+  read_a(0, 0, 0);
+  read_a(0, 0, 1);
+  read_w(1, 0);
+  for (int t = 0; t < steps; ++t) {
+    const int buf = t & 1;
+    read_w(0, buf);
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(1, buf, 0);
+    mf_wait_reads<4>();
+    mf_barrier();
+    products(0, 0);
+    mf_barrier();
+    read_a(1, buf, 1);
+    load_a(0, t + 2);
+    load_w(1, t + 2);
+    mf_wait_loads<8>();
+    mf_barrier();
+    products(0, 1);
+    mf_barrier();
+    read_a(0, buf ^ 1, 0);
+    load_w(0, t + 2);
+    mf_wait_reads<4>();
+    mf_barrier();
+    products(1, 1);
+    mf_barrier();
+    read_a(0, buf ^ 1, 1);
+    read_w(1, buf ^ 1);
+    load_a(1, t + 2);
+    mf_wait_loads<8>();
+    mf_barrier();
+    products(1, 0);
+    mf_barrier();
+  }
+  if (wm == 0) mf_barrier();
+  mf_wait_loads<0>();                 // (what was asked for beyond the last step has landed)
+
+  // A lane holds four consecutive columns of a row (column 4 * (lane / 16), row lane % 16 of a 16 x 16 tile). The sums
+  // go through shared memory, half the tile's rows at a time, so that a wave then works on whole rows: 1 KB of a row of
+  // floats an instruction. Row r's sixteen bytes c lie at place c ^ (r % 16): no two lanes of a write meet in a bank.
+  const bool vec = slice ? ldp % 4 == 0 && p_stride % 4 == 0 && (uintptr_t)P % 16 == 0
+                         : ldc % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;
+#pragma unroll
+  for (int ah = 0; ah < 2; ++ah) {
+    mf_barrier();                     // (both groups have read what lay here)
+#pragma unroll
+    for (int tm = 0; tm < 4; ++tm)
+#pragma unroll
+      for (int wh = 0; wh < 2; ++wh)
+#pragma unroll
+        for (int tn = 0; tn < 2; ++tn)
+          *(f32x4*)(lds + (wm * 64 + tm * 16 + lr) * 1024 + (((wh * 32 + wn * 8 + tn * 4 + lq) ^ lr) << 4)) = acc[ah][tm][wh][tn];
+    mf_wait_reads<0>();
+    mf_barrier();
+    const int rows = min(128, M - m0 - ah * 128);
+    if (EPI == MF_GATED) {            // two rows a wave: 128 columns
+#pragma unroll 2
+      for (int r = wave * 2 + (lane >> 5); r < rows; r += 16) {
+        const int c4 = lane & 31, n = n0 + c4 * 4;
+        const f32x4 g = *(const f32x4*)(lds + r * 1024 + ((c4 ^ (r & 15)) << 4));
+        const f32x4 u = *(const f32x4*)(lds + r * 1024 + (((32 + c4) ^ (r & 15)) << 4));
+        if (n < N) mf_finish4<EPI, TC>(C + (long)(m0 + ah * 128 + r) * ldc + n, g, u, n, N, vec, bias, act, ex);
+      }
+    } else {
+#pragma unroll 4
+      for (int r = wave; r < rows; r += 8) {
+        const int n = n0 + lane * 4;
+        const f32x4 v = *(const f32x4*)(lds + r * 1024 + ((lane ^ (r & 15)) << 4));
+        if (n >= N) continue;
+        const long m = m0 + ah * 128 + r;
+        if (slice > 0) mf_finish4<MF_STORE, float>(P + (long)(slice - 1) * p_stride + m * ldp + n, v, v, n, N, vec, nullptr, act, ex);
+        else mf_finish4<EPI, TC>(C + m * ldc + n, v, v, n, N, vec, bias, act, ex);
+      }
+    }
+  }
+}
+
+// What gemm_mfma_turns_kernel is built for: whole steps of 64 k, and byte offsets of 31 bits inside a tile's rows of A and
+// inside W (or, as stored, from the tile's first row of W to its last).
+static bool turns_takes(int N, int K, long lda, long ldw, bool gated, int w_order) {
+  const long rows = gated ? 2L * N : (long)N;
+  return K % 64 == 0 && (255 * lda + K) * 2 < (1L << 31) &&
+         (w_order ? rows * K * 2 : ((gated ? (long)N : 0) + 255) * ldw * 2 + 2L * K) < (1L << 31);
+}
+
 template <int EPI, typename TC, int TM, int WM, int WN, int WT = 0>
 static int launch_shape(const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc,
                         int slices, float* P, long p_stride, long ldp, const float* bias, int act, int w_steps,
@@ -279,6 +551,15 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
   // them a rectangle of 4 x 8 (8 x 8), which asks memory for a third of the bytes that one column of
   // 32 row tiles does (3 to 5% of the time of the large products)
   const int group_m = tiles_m < (bm == 256 ? 4 : 8) ? tiles_m : (bm == 256 ? 4 : 8);
+  if constexpr (TM == 2 && WM == 4 && WN == 4) {
+    if (turns_takes(N, K, lda, ldw, EPI == MF_GATED, WT)) {
+      gemm_mfma_turns_kernel<EPI, TC, WT><<<dim3((unsigned)blocks, slices), dim3(512), 0, stream>>>(
+          (const bf16_t*)A, (const bf16_t*)W, (TC*)C, M, N, K, lda, ldw, ldc, tiles_m, tiles_n, group_m, k_per_slice, P, p_stride,
+          ldp, bias, act, w_steps, w_pos, ex);
+      GL3_LAUNCH_CHECK();
+      return 0;
+    }
+  }
   gemm_mfma_kernel<EPI, TC, TM, WM, WN, WT><<<dim3((unsigned)blocks, slices), dim3(64 * WM * WN), 0, stream>>>(
       (const bf16_t*)A, (const bf16_t*)W, (TC*)C, M, N, K, lda, ldw, ldc, tiles_m, tiles_n, group_m, k_per_slice, P,
       p_stride, ldp, bias, act, w_steps, w_pos, ex);

@@ -1,0 +1,78 @@
+"""The tiled products at the edges of their tiles and of their pipelines, over every order that a weight may lie in."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_kernels import DEV, K, dev, rounded
+
+pytestmark = pytest.mark.gpu
+
+
+def held(lib, w, order):
+    if order == "stored":
+        return w
+    v = w.clone()
+    if order == "strips of 16":
+        v.tiled = lib.tile_weight(v)
+    else:
+        v.tiled8 = lib.tile_weight8(v)
+    return lib.hold_once(v)
+
+
+def off_by(a, w, out_bits):
+    """32-bit sums of K products: at most K roundings of the sum of magnitudes; the output rounded to ``out_bits``."""
+    s = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    return a.shape[1] * 2.0 ** -24 * s, 2.0 ** -out_bits
+
+
+# (rows and columns of one tile of 128 or 256, one more, one less and many; K of one, two, three and an odd number of steps;
+# 2,304 columns are nine tiles of 256 over the XCDs)
+@pytest.mark.parametrize("shape", [1, 2, 5])
+@pytest.mark.parametrize("order", ["stored", "strips of 16", "strips of 8"])
+@pytest.mark.parametrize("M, N, Kd", [(1, 16, 64), (255, 256, 128), (257, 272, 192), (300, 2304, 320), (513, 128, 1088), (1100, 528, 2048)])
+def test_tiled_products(shape, order, M, N, Kd):
+    lib = K()
+    rng = np.random.default_rng(M + N + Kd)
+    a, w = rounded(rng.standard_normal((M, Kd)), "bfloat16"), rounded(rng.standard_normal((N, Kd)) / np.sqrt(Kd), "bfloat16")
+    A = torch.zeros(M, Kd + 8, device=DEV, dtype=torch.bfloat16)[:, :Kd]              # (rows apart)
+    A.copy_(dev(a))
+    W = held(lib, dev(w, torch.bfloat16), order)
+    ref = a.astype(np.float64) @ w.astype(np.float64).T
+    sums, _ = off_by(a, w, 24)
+    factor, bias = rng.standard_normal(N).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    for pad in (0, 3):                                                                # (3: no four columns of a row at once)
+        out = torch.full((M, N + pad), -7.0, device=DEV)
+        for again in range(2):
+            lib.gemm_mfma(A, W, out[:, :N], shape=shape)
+            assert (np.abs(out[:, :N].double().cpu().numpy() - ref) <= sums + 1e-30).all(), again
+        assert torch.all(out[:, N:] == -7.0)
+    half = torch.zeros(M, N, device=DEV, dtype=torch.bfloat16)
+    lib.gemm_mfma(A, W, half, shape=shape, bias=dev(bias))
+    want = ref + bias
+    assert (np.abs(half.double().cpu().numpy() - want) <= 2.0 ** -8 * np.abs(want) + 2 * sums + 1e-6).all()
+    res = rng.standard_normal((M, N)).astype(np.float32)
+    for more in (0, 1, 3):
+        if (more + 1) * 64 > Kd or (more and shape == 5):
+            continue
+        x = dev(res)
+        part = torch.full((more, M, N), -7.0, device=DEV) if more else None
+        lib.gemm_mfma(A, W, x, lib.EPI_ADD, more_slices=part, shape=shape, col_scale=dev(factor))
+        got = x.double().cpu().numpy() + (part.double().sum(0).cpu().numpy() if more else 0.0)
+        assert (np.abs(got - (res + ref * factor)) <= sums * np.abs(factor) + 2.0 ** -21 * (np.abs(res) + np.abs(ref * factor)) + 1e-6).all(), more
+
+
+@pytest.mark.parametrize("shape", [1, 2, 5])
+@pytest.mark.parametrize("order", ["stored", "strips of 16"])
+@pytest.mark.parametrize("M, N, Kd", [(3, 16, 64), (256, 128, 192), (258, 144, 128), (700, 1040, 576)])
+def test_tiled_gated_products(shape, order, M, N, Kd):
+    lib = K()
+    rng = np.random.default_rng(M * 3 + N)
+    a, w = rounded(rng.standard_normal((M, Kd)), "bfloat16"), rounded(rng.standard_normal((2 * N, Kd)) / np.sqrt(Kd), "bfloat16")
+    W = held(lib, dev(w, torch.bfloat16), order)
+    ref = a.astype(np.float64) @ w.astype(np.float64).T
+    want = ref[:, :N] / (1 + np.exp(-ref[:, :N])) * ref[:, N:]
+    out, wide = torch.zeros(M, N, device=DEV), torch.full((M, N + 1), -7.0, device=DEV, dtype=torch.bfloat16)
+    lib.gemm_mfma(dev(a, torch.bfloat16), W, out, lib.EPI_GATED, shape=shape)
+    assert np.abs(out.cpu().numpy() - want).max() <= 2e-5 * np.abs(want).max()         # (the fast exponential: 2^-20)
+    lib.gemm_mfma(dev(a, torch.bfloat16), W, wide[:, :N], lib.EPI_GATED, shape=shape)
+    assert torch.equal(wide[:, :N], out.to(torch.bfloat16)) and torch.all(wide[:, N:] == -7.0)
