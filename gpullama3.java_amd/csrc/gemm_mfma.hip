@@ -14,7 +14,7 @@
 // contiguous range of tiles, ordered so that the tiles it holds at one time form a rectangle
 // and share their panels of A and of W.
 //
-// Tiles of 256 x 256 over whole steps of 64 k have a kernel of their own (gemm_mfma_turns_kernel, below).
+// Tiles of 256 x 256 and of 128 rows x 256 over whole steps of 64 k have a kernel of their own (gemm_mfma_turns_kernel, below).
 //
 // Epilogues as in gemm_generic.hip: store, add into a float matrix, gated.
 #include "common.h"
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
   else finish(std::true_type{});
 }
 
-// ---- 256 x 256 tiles over whole steps of 64 k: operands straight from memory into shared memory, waves in two groups
+// ---- tiles of 256 x 256 and of 128 rows x 256 over whole steps of 64 k: operands straight from memory into shared memory, waves in two groups
 // that take turns.
 //
 // Eight waves; wave w's rows of A are 64 of each half of the tile's (group w / 4), its rows of W 32 of each half (gated:
@@ -280,7 +280,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 // the 32x32x16 instruction, whose accumulators pass through the registers twice as often per flop, the same loop lost 11%.
 // (8,192 x 28,672 x 4,096: the kernel above 1,680 us, this one 1,312.)
 //
-// Registers are read a part or two before they are used: in the memory part of phase 0 W0 and half of A1, of phase 1 the
+// AH = 1 is the tile of 128 rows x 256: two phases a step, a third step in shared memory instead of registers read ahead.
+// (2,048 rows, 3,072 columns, K = 2,048: 42 -> 31 us; 512 rows of the 3B layers' gate/up product: 59 -> 50 us.)
+//
+// AH = 2: registers are read a part or two before they are used: in the memory part of phase 0 W0 and half of A1, of phase 1 the
 // rest of A1, of phases 2 and 3 the next step's A0 and W1. A half tile's place in shared memory is written for the step after
 // next as soon as both groups have read it (their reads have returned: lgkmcnt before the barrier in front of the part
 // that asks), and the loads are only waited for where the next barrier hands them out, so six to eight are on their way
@@ -296,9 +299,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 // the operands want it, [strip of 16][k-step of 32][lane][16 bytes].
 __device__ __forceinline__ void mf_dma16(unsigned lds, unsigned offset, i32x4 rsrc, unsigned step_offset) {
   // (by hand: behind the builtin the compiler waits for every load in front of every read of shared memory. The
-  // instruction has no destination register; its data lands at m0 + 16 * lane)
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(offset), "s"(rsrc), "s"(step_offset)
-               : "memory", "m0");
+  // instruction has no destination register; its data lands at m0 + 16 * lane. Nothing else in these kernels uses m0)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(offset), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(step_offset))
+               : "memory");
 }
 template <int N>
 __device__ __forceinline__ void mf_wait_loads() {
@@ -360,7 +363,7 @@ __device__ __forceinline__ void mf_finish4(TC* c, f32x4 s, f32x4 up, int n, int 
   }
 }
 
-template <int EPI, typename TC, int WT>
+template <int EPI, typename TC, int WT, int AH>
 __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                                   TC* __restrict__ C, int M, int N, int K, long lda, long ldw,
                                                                   long ldc, int tiles_m, int tiles_n, int group_m,
@@ -368,7 +371,8 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
                                                                   const float* __restrict__ bias, int act, int w_steps,
                                                                   const int* __restrict__ w_pos, MfExtras ex) {
   constexpr int NCOLS = EPI == MF_GATED ? 128 : 256;
-  __shared__ __attribute__((aligned(1024))) char lds[131072];       // A: two steps of 32 KB, then W: two steps of 32 KB
+  constexpr int STAGES = AH == 2 ? 2 : 3, STAGE = AH * 16384 + 32768;      // a step: A's halves, then W's
+  __shared__ __attribute__((aligned(1024))) char lds[STAGES * STAGE];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wm = wave >> 2, wn = wave & 3;
   const int lr = lane & 15, lq = lane >> 4;
@@ -377,7 +381,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   if (tile >= n_tiles) return;
   const int band = tile / (group_m * tiles_n), in_band = tile % (group_m * tiles_n);
   const int band_rows = min(group_m, tiles_m - band * group_m);
-  const int m0 = (band * group_m + in_band % band_rows) * 256;
+  const int m0 = (band * group_m + in_band % band_rows) * (128 * AH);
   const int n0 = (in_band / band_rows) * NCOLS;
   const int slice = blockIdx.y;
   // (the last of many slices may have no step left: it stores zeros)
@@ -387,7 +391,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   const i32x4 a_buf = mf_rsrc(A + (long)m0 * lda + k_begin);
   const i32x4 w_buf = mf_rsrc(WT ? W + (long)(k_begin >> 6) * (WT == 1 ? 1024 : 512) : W + (long)n0 * ldw + k_begin);
   constexpr unsigned W_STEP = WT == 1 ? 2048 : WT == 2 ? 1024 : 128;
-  unsigned ao[2][2], wo[2][2];
+  unsigned ao[2][2], wo[2][2];      // (AH 1: the first half of A alone)
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -400,35 +404,36 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
       wo[h][i] = mf_w_offset<WT>(n, w_k, ldw, w_steps, w_pos, n0);
     }
   const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)lds + wave * 2048;
-  auto load_a = [&](int h, int t) {
+  // (`place`: the byte where the step lies in shared memory)
+  auto load_a = [&](int h, int t, int place) {
     const unsigned s = (unsigned)max(0, min(t, steps - 1)) * 128;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) mf_dma16(lds0 + (t & 1) * 32768 + h * 16384 + i * 1024, ao[h][i], a_buf, s);
+    for (int i = 0; i < 2; ++i) mf_dma16(lds0 + place + h * 16384 + i * 1024, ao[h][i], a_buf, s);
   };
-  auto load_w = [&](int h, int t) {
+  auto load_w = [&](int h, int t, int place) {
     const unsigned s = (unsigned)max(0, min(t, steps - 1)) * W_STEP;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) mf_dma16(lds0 + 65536 + (t & 1) * 32768 + h * 16384 + i * 1024, wo[h][i], w_buf, s);
+    for (int i = 0; i < 2; ++i) mf_dma16(lds0 + place + AH * 16384 + h * 16384 + i * 1024, wo[h][i], w_buf, s);
   };
 
-  f32x4 acc[2][4][2][2];      // [half of A][16 rows][half of W][16 rows]
+  f32x4 acc[AH][4][2][2];     // [half of A][16 rows][half of W][16 rows]
 #pragma unroll
-  for (int i = 0; i < 32; ++i) (&acc[0][0][0][0])[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 af[2][4][2], wf[2][2][2];      // [half][16 rows][k-step of 32]
+  for (int i = 0; i < 16 * AH; ++i) (&acc[0][0][0][0])[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 af[AH][4][2], wf[2][2][2];      // [half][16 rows][k-step of 32]
   const char* a_at = lds + (wm * 64 + lr) * 128;
-  const char* w_at = lds + 65536 + (WT ? wn * 4096 + lane * 16 : (wn * 32 + lr) * 128);
+  const char* w_at = lds + AH * 16384 + (WT ? wn * 4096 + lane * 16 : (wn * 32 + lr) * 128);
   const int twist = (lr >> 1) & 7;
-  auto read_a = [&](int h, int buf, int ks) {
+  auto read_a = [&](int h, int place, int ks) {
 #pragma unroll
     for (int tm = 0; tm < 4; ++tm)
-      af[h][tm][ks] = *(const bf16x8*)(a_at + buf * 32768 + h * 16384 + tm * 2048 + (((ks * 4 + lq) ^ twist) << 4));
+      af[h][tm][ks] = *(const bf16x8*)(a_at + place + h * 16384 + tm * 2048 + (((ks * 4 + lq) ^ twist) << 4));
   };
-  auto read_w = [&](int h, int buf) {
+  auto read_w = [&](int h, int place) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
       for (int tn = 0; tn < 2; ++tn)
-        wf[h][tn][ks] = *(const bf16x8*)(w_at + buf * 32768 + h * 16384 + tn * 2048 + (WT ? ks * 1024 : ((ks * 4 + lq) ^ twist) << 4));
+        wf[h][tn][ks] = *(const bf16x8*)(w_at + place + h * 16384 + tn * 2048 + (WT ? ks * 1024 : ((ks * 4 + lq) ^ twist) << 4));
   };
   auto products = [&](int ah, int wh) {
 #pragma unroll
@@ -440,49 +445,86 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
           acc[ah][tm][wh][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[wh][tn][ks], af[ah][tm][ks], acc[ah][tm][wh][tn], 0, 0, 0);
   };
 
-  load_a(0, 0);
-  load_w(1, 0);
-  load_w(0, 0);
-  load_a(1, 0);
-  load_a(0, 1);
-  load_w(1, 1);
-  load_w(0, 1);
-  load_a(1, 1);
-  mf_wait_loads<8>();
-  mf_barrier();
-  if (wm == 1) mf_barrier();          // the second group runs a part behind
-  read_a(0, 0, 0);
-  read_a(0, 0, 1);
-  read_w(1, 0);
-  for (int t = 0; t < steps; ++t) {
-    const int buf = t & 1;
-    read_w(0, buf);
-    __builtin_amdgcn_sched_barrier(0);
-    read_a(1, buf, 0);
-    mf_wait_reads<4>();
-    mf_barrier();
-    products(0, 0);
-    mf_barrier();
-    read_a(1, buf, 1);
-    load_a(0, t + 2);
-    load_w(1, t + 2);
+  if constexpr (AH == 2) {
+    load_a(0, 0, 0);
+    load_w(1, 0, 0);
+    load_w(0, 0, 0);
+    load_a(1, 0, 0);
+    load_a(0, 1, STAGE);
+    load_w(1, 1, STAGE);
+    load_w(0, 1, STAGE);
+    load_a(1, 1, STAGE);
     mf_wait_loads<8>();
     mf_barrier();
-    products(0, 1);
+    if (wm == 1) mf_barrier();          // the second group runs a part behind
+    read_a(0, 0, 0);
+    read_a(0, 0, 1);
+    read_w(1, 0);
+    for (int t = 0, here = 0; t < steps; ++t, here = STAGE - here) {
+      const int there = STAGE - here;
+      read_w(0, here);
+      __builtin_amdgcn_sched_barrier(0);
+      read_a(1, here, 0);
+      mf_wait_reads<4>();
+      mf_barrier();
+      products(0, 0);
+      mf_barrier();
+      read_a(1, here, 1);
+      load_a(0, t + 2, here);
+      load_w(1, t + 2, here);
+      mf_wait_loads<8>();
+      mf_barrier();
+      products(0, 1);
+      mf_barrier();
+      read_a(0, there, 0);
+      load_w(0, t + 2, here);
+      mf_wait_reads<4>();
+      mf_barrier();
+      products(1, 1);
+      mf_barrier();
+      read_a(0, there, 1);
+      read_w(1, there);
+      load_a(1, t + 2, here);
+      mf_wait_loads<8>();
+      mf_barrier();
+      products(1, 0);
+      mf_barrier();
+    }
+  } else {
+    // 128 rows of A: two phases a step, (A, W0) and (A, W1), three steps in shared memory. What a part reads it uses at
+    // once; a place is written again, for the step three further, in the part after both groups have read it.
+    load_a(0, 0, 0);
+    load_w(0, 0, 0);
+    load_w(1, 0, 0);
+    load_a(0, 1, STAGE);
+    load_w(0, 1, STAGE);
+    load_w(1, 1, STAGE);
+    load_a(0, 2, 2 * STAGE);
+    load_w(0, 2, 2 * STAGE);
+    mf_wait_loads<12>();
     mf_barrier();
-    read_a(0, buf ^ 1, 0);
-    load_w(0, t + 2);
-    mf_wait_reads<4>();
-    mf_barrier();
-    products(1, 1);
-    mf_barrier();
-    read_a(0, buf ^ 1, 1);
-    read_w(1, buf ^ 1);
-    load_a(1, t + 2);
-    mf_wait_loads<8>();
-    mf_barrier();
-    products(1, 0);
-    mf_barrier();
+    if (wm == 1) mf_barrier();
+    for (int t = 0, here = 0, before = 2 * STAGE; t < steps; ++t) {
+      read_a(0, here, 0);
+      read_a(0, here, 1);
+      read_w(0, here);
+      load_w(1, t + 2, before);
+      mf_wait_loads<12>();              // this step's W1 has come
+      mf_wait_reads<0>();
+      mf_barrier();
+      products(0, 0);
+      mf_barrier();
+      read_w(1, here);
+      load_a(0, t + 3, here);
+      load_w(0, t + 3, here);
+      mf_wait_loads<12>();              // the next step's A and W0 have
+      mf_wait_reads<0>();
+      mf_barrier();
+      products(0, 1);
+      mf_barrier();
+      before = here;
+      here = here == 2 * STAGE ? 0 : here + STAGE;
+    }
   }
   if (wm == 0) mf_barrier();
   mf_wait_loads<0>();                 // (what was asked for beyond the last step has landed)
@@ -493,7 +535,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   const bool vec = slice ? ldp % 4 == 0 && p_stride % 4 == 0 && (uintptr_t)P % 16 == 0
                          : ldc % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;
 #pragma unroll
-  for (int ah = 0; ah < 2; ++ah) {
+  for (int ah = 0; ah < AH; ++ah) {
     mf_barrier();                     // (both groups have read what lay here)
 #pragma unroll
     for (int tm = 0; tm < 4; ++tm)
@@ -551,9 +593,9 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
   // them a rectangle of 4 x 8 (8 x 8), which asks memory for a third of the bytes that one column of
   // 32 row tiles does (3 to 5% of the time of the large products)
   const int group_m = tiles_m < (bm == 256 ? 4 : 8) ? tiles_m : (bm == 256 ? 4 : 8);
-  if constexpr (TM == 2 && WM == 4 && WN == 4) {
+  if constexpr (WM == 4 && WN == 4) {
     if (turns_takes(N, K, lda, ldw, EPI == MF_GATED, WT)) {
-      gemm_mfma_turns_kernel<EPI, TC, WT><<<dim3((unsigned)blocks, slices), dim3(512), 0, stream>>>(
+      gemm_mfma_turns_kernel<EPI, TC, WT, TM><<<dim3((unsigned)blocks, slices), dim3(512), 0, stream>>>(
           (const bf16_t*)A, (const bf16_t*)W, (TC*)C, M, N, K, lda, ldw, ldc, tiles_m, tiles_n, group_m, k_per_slice, P, p_stride,
           ldp, bias, act, w_steps, w_pos, ex);
       GL3_LAUNCH_CHECK();
@@ -567,7 +609,22 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
   return 0;
 }
 
-// The tile the library takes where the caller names none: 1 (128 x 128), 2 (256 x 256) or 5 (128 rows x 256).
+// The tile the library takes where the caller names none. Where gemm_mfma_turns_kernel takes the product the time (us) of
+// each tile over its rounds on the chip, steps of 64 k and what a round costs beside them, as measured: 256 x 256 1.06 a step
+// and 3.3 a round, 128 rows x 256 0.67 and 0.9 (one block a CU, the last round as long as a full one); tiles of 128 x 128,
+// which have the kernel above, are ahead by a tenth where they are at most one a CU and the larger ones leave more than half of
+// the chip idle (512 rows, 5,120 columns, K = 3,072: 33 us against 37; 2,048 rows, 3,072 columns, K = 2,048: 41 against 31).
+static int choose_turns_shape(int M, int N, int K, bool gated) {
+  const long small_n = gated ? (N + 63) / 64 : (N + 127) / 128, big_n = gated ? (N + 127) / 128 : (N + 255) / 256;
+  const long small_tiles = (long)((M + 127) / 128) * small_n, wide_tiles = (long)((M + 127) / 128) * big_n,
+             big_tiles = (long)((M + 255) / 256) * big_n;
+  const double steps = K / 64;
+  const double small = small_tiles <= 256 ? 5 + 0.62 * steps : (small_tiles + 511) / 512 * (2 + 1.05 * steps);
+  const double wide = 4 + (wide_tiles + 255) / 256 * (0.9 + 0.671 * steps), big = 4 + (big_tiles + 255) / 256 * (3.3 + 1.063 * steps);
+  return small < wide && small < big ? 1 : wide < big ? 5 : 2;
+}
+
+// The same where it does not (K in no whole steps of 64, or K in slices): 1 (128 x 128), 2 (256 x 256) or 5 (128 rows x 256).
 // 256 x 256 tiles of sixteen waves, one block a CU, have half the operand traffic per product, and
 // that traffic is what bounds the large products; of the 128 x 128 tiles of eight waves two fit a CU and
 // overlap each other's waits. A step of 64 columns takes a chip full of the large tiles 1.7 us and a chip
@@ -597,7 +654,9 @@ static int launch_mfma(const void* A, const void* W, void* C, int M, int N, int 
                        int slices, float* P, long p_stride, long ldp, const float* bias, int act, int shape, int w_order,
                        const int* w_pos, MfExtras ex, hipStream_t stream) {
   const int w_steps = w_order == 1 ? (K + 31) / 32 : w_order == 2 ? (K + 63) / 64 : 0;
-  if (shape == 0) shape = choose_shape(M, N, slices, EPI == MF_GATED);
+  if (shape == 0)
+    shape = slices == 1 && turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order) ? choose_turns_shape(M, N, K, EPI == MF_GATED)
+                                                                                 : choose_shape(M, N, slices, EPI == MF_GATED);
 #define MF_ARGS A, W, C, M, N, K, lda, ldw, ldc, slices, P, p_stride, ldp, bias, act, w_steps, w_pos, ex, stream
   if (w_order) {
     // W is one of its copies in the matrix cores' order (a weight that is held once): the three tiles that the library

@@ -1993,6 +1993,34 @@ def mfma_plan(M, N, K):
     return best[1], best[2]
 
 
+def turns_planned(N, K):
+    """Whether ``turns_plan`` rather than ``mfma_plan`` plans a product into the residual stream: whole steps of 64 columns, and
+    rows of 2,048 columns or more, the narrowest that it was fitted to."""
+    return K % 64 == 0 and N >= 2048
+
+
+def turns_plan(M, N, K):
+    """``mfma_plan`` for K in whole steps of 64, where tiles of 256 x 256 and of 128 rows x 256 run on the kernel whose waves
+    take turns (``gemm_mfma_turns_kernel``): the plan with the least estimated time among those two with one to eight
+    slices of at least 512 columns. The estimate: rounds of 256 blocks (one a CU), each of 1.06 us a step of 64 columns and 3.3 us
+    beside them (128 rows: 0.67 and 0.9), and for every slice beyond the first 0.41 us a MB of the output, which is
+    written, read by the norm that follows, and added. Fitted to 21 sizes (150 to 8,192 rows, the output and down
+    projections of three models) times up to twelve plans, product and norm together: the plan chosen is within 6% of the best
+    of them and of the tiles of 128 x 128 everywhere but at 150 rows over K = 14,336 (52 against 45 us). Against the
+    plan before it: 2,048 rows of the 1B layers' down projection 98 -> 81 us, 512 rows of the 3B layers' 51 -> 45 us, 300 rows
+    over K = 8,192 38 -> 33 us."""
+    best = None
+    for shape, rows, step_us, round_us in ((5, 128, 0.671, 0.9), (2, 256, 1.063, 3.3)):
+        for slices in range(1, 9):
+            if slices > 1 and K // slices < 512:
+                break
+            blocks = -(-M // rows) * -(-N // 256) * slices
+            estimate = -(-blocks // 256) * (-(-K // (64 * slices)) * step_us + round_us) + 0.413e-6 * (slices - 1) * M * N * 4
+            if best is None or estimate < best[0]:
+                best = (estimate, shape, slices)
+    return best[1], best[2]
+
+
 # ------------------------------------------------------------------ bfloat16 attention of a prefill step
 def attention_prefill_fits(head_dim, n_heads, n_kv, page_size):
     return bool(library().gl3_attention_prefill_supports(head_dim, page_size)) and n_heads % n_kv == 0
