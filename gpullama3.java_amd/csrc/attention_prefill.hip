@@ -313,13 +313,22 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(
 // its 16 keys a step.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-template <int HS, int CK, int AHEAD, int OCC, bool BIAS = false, bool RULE = false>
+// SPLIT: the chunks of a block's keys are shared out over `splits` blocks; each leaves its sums as they are, with their
+// maximum and weight, for attention_prefill_merge_kernel.
+#define PF_SPLITS 8      // at most
+struct PfSplit {
+  int splits;
+  int n_tokens;
+  float* o;      // [split][token][head][head_dim]
+  float* ml;     // [split][token][head][2]: maximum in units of log2, sum
+};
+template <int HS, int CK, int AHEAD, int OCC, bool BIAS = false, bool RULE = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
     const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ cu_seqlens, const int* __restrict__ kv_before, const int* __restrict__ block_table,
     const int* __restrict__ seq_rows, int table_stride, bf16_t* __restrict__ out, long out_stride, int n_heads, int n_kv, int page_size, int window,
     float scale, int q_blocks, const float* __restrict__ slopes, int has_sink, float sink, int keep_first, int mask_chunk, int maps,
-    const float* __restrict__ sinks, Gl3ScoreRule rule) {
+    const float* __restrict__ sinks, Gl3ScoreRule rule, PfSplit sp) {
   constexpr int KS = HS / 16;             // steps of the score product
   constexpr int DT = HS / 32;             // tiles of 32 dims of the output
   constexpr int NT = CK / 32;             // score tiles of a chunk of CK keys
@@ -334,7 +343,7 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
   const int g = n_heads / n_kv;
   const int qb = q_blocks - 1 - blockIdx.z;      // the longest query blocks of all heads and sequences first
   const int b = blockIdx.y;
-  const int head = blockIdx.x;                 // one query head to a block
+  const int head = SPLIT ? blockIdx.x % n_heads : blockIdx.x;                 // one query head to a block
   const int c = maps > 1 ? ((head / maps) / g) * maps + head % maps : head / g;      // (its key head: map head % maps of its group)
   const int n_v = n_kv / maps, cv = c / maps;
   const int tid = threadIdx.x;
@@ -351,8 +360,14 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
   auto low_of = [&](int p) { return mask_chunk > 0 ? p - p % mask_chunk : (window > 0 && p + 1 > window) ? p + 1 - window : 0; };
   const int blk_lo = low_of(blk_first);
   // (kept first keys: as in the kernel above, their chunks before the window's first chunk are numbered in front of it)
-  const int ckw = blk_lo / CK, ck1 = blk_last / CK;
-  const int ck0 = ckw - (BIAS ? min((keep_first + CK - 1) / CK, ckw) : 0);
+  const int ckw = blk_lo / CK;
+  int ck1 = blk_last / CK, ck0 = ckw - (BIAS ? min((keep_first + CK - 1) / CK, ckw) : 0);
+  const int split = SPLIT ? blockIdx.x / n_heads : 0;
+  if (SPLIT) {
+    const int chunks = ck1 - ck0 + 1, lo = ck0;
+    ck0 = lo + chunks * split / sp.splits;
+    ck1 = lo + chunks * (split + 1) / sp.splits - 1;      // (no chunk: the block leaves a weight of nothing)
+  }
   auto real = [&](int ck) { return (BIAS && ck < ckw) ? ck - ck0 : ck; };
   const int qi0 = qb * QB + wave * 32;
   const bool active = qi0 < q_len;
@@ -518,7 +533,7 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
   };
 
 #pragma unroll
-  for (int r = 0; r < AHEAD; ++r) fetch(real(min(ck0 + r, ck1)), rk[r], rv[r]);
+  for (int r = 0; r < AHEAD; ++r) fetch(real(SPLIT ? max(ck0, min(ck0 + r, ck1)) : min(ck0 + r, ck1)), rk[r], rv[r]);
   stage(0, rk[0], rv[0]);
   __syncthreads();
   int buf = 0;
@@ -545,6 +560,19 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
   float l = l_run;
   l += __shfl_xor(l, 32, 64);
   if (!q_ok) return;
+  if (SPLIT) {
+    const long row = ((long)split * sp.n_tokens + tok0 + qi0 + n) * n_heads + head;
+    float* po = sp.o + row * HS + 4 * h;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) *(f32x4*)(po + dt * 32 + 8 * a) = f32x4{o[dt][4 * a], o[dt][4 * a + 1], o[dt][4 * a + 2], o[dt][4 * a + 3]};
+    if (h == 0) {
+      sp.ml[row * 2] = m_run;
+      sp.ml[row * 2 + 1] = l;
+    }
+    return;
+  }
   const float inv = 1.0f / l;
   bf16_t* op = out + (long)(tok0 + qi0 + n) * out_stride + (long)head * HS + 4 * h;
 #pragma unroll
@@ -562,6 +590,41 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
       for (int v = 0; v < 4; ++v) r[v] = static_cast<bf16_t>(o[dt][4 * a + v] * inv);
       *(bf16x4*)(op + dt * 32 + 8 * a) = r;
     }
+}
+
+// The splits' sums of a row (token, head) brought to the greatest of their maxima, added in the order of the splits, and divided
+// by the weight: a thread four dims of a row, its splits' loads all on their way at once.
+template <int HS>
+__global__ __launch_bounds__(256) void attention_prefill_merge_kernel(PfSplit sp, bf16_t* __restrict__ out, long out_stride, int n_heads) {
+  constexpr int TPR = HS / 4;      // threads a row
+  const long at = (long)blockIdx.x * 256 + threadIdx.x, rows = (long)sp.n_tokens * n_heads;
+  const long row = at / TPR;
+  const int d = (int)(at % TPR) * 4;
+  if (row >= rows) return;
+  f32x4 v[PF_SPLITS];
+  float m[PF_SPLITS], l[PF_SPLITS], top = -INFINITY;
+#pragma unroll
+  for (int s = 0; s < PF_SPLITS; ++s) {
+    const long r = min(s, sp.splits - 1) * rows + row;
+    v[s] = *(const f32x4*)(sp.o + r * HS + d);
+    m[s] = s < sp.splits ? sp.ml[r * 2] : -INFINITY;
+    l[s] = sp.ml[r * 2 + 1];
+  }
+#pragma unroll
+  for (int s = 0; s < PF_SPLITS; ++s) top = fmaxf(top, m[s]);
+  float weight = 0.f;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < PF_SPLITS; ++s) {
+    if (m[s] == -INFINITY && top != -INFINITY) continue;      // (a split whose keys the row does not see)
+    const float f = __builtin_amdgcn_exp2f(m[s] - top);
+    weight += f * l[s];
+    sum += f * v[s];
+  }
+  bf16x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o[j] = static_cast<bf16_t>(sum[j] / weight);
+  *(bf16x4*)(out + row / n_heads * out_stride + row % n_heads * HS + d) = o;
 }
 
 // Which of the two kernels a step takes, unless the caller says otherwise. Heads of 32 and 64: the one
@@ -588,7 +651,8 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
                                      int max_q_len, int n_heads, int n_kv, int head_dim, int page_size, int window,
                                      float scale, int wide_from, const float* slopes, int has_sink, float sink,
                                      int keep_first, int mask_chunk, int maps, const float* sinks, float softcap,
-                                     float temp_coef, int temp_every, const void* gate, long gate_ld, hipStream_t stream) {
+                                     float temp_coef, int temp_every, const void* gate, long gate_ld, int splits,
+                                     int n_tokens, float* part_o, float* part_ml, hipStream_t stream) {
   if (n_seqs == 0 || max_q_len == 0) return 0;
   GL3_REQUIRE(q && k_cache && v_cache && cu_seqlens && kv_before && block_table && out,
               "gl3_attention_prefill: null argument");
@@ -605,29 +669,37 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
               "gl3_attention_prefill: queries must be 16-byte aligned, outputs 8-byte aligned");
   const int g = n_heads / n_kv;
   // query heads per wave: as many as the registers hold with two blocks on a CU
-  const bool wide = wide_from > 0 ? max_q_len >= wide_from : prefill_wide(head_dim, n_heads, n_seqs, max_q_len);
+  const bool wide = splits > 1 ? true : wide_from > 0 ? max_q_len >= wide_from : prefill_wide(head_dim, n_heads, n_seqs, max_q_len);
   // query heads per wave: as many as the registers hold with two blocks on a CU; one with 32 queries a wave
   const int gh = wide ? 1 : head_dim <= 32 ? 4 : head_dim <= 64 ? 2 : 1;
   const long z = (long)n_kv * ((g + gh - 1) / gh);
   const int q_blocks = wide ? (max_q_len + 127) / 128 : (max_q_len + 63) / 64;
   GL3_REQUIRE(n_seqs <= 65535 && q_blocks <= 65535, "gl3_attention_prefill: %d sequences / %d blocks of queries exceed the grid",
               n_seqs, q_blocks);
-  dim3 grid((unsigned)z, n_seqs, q_blocks), block(256);
+  dim3 grid((unsigned)z * (splits > 1 ? splits : 1), n_seqs, q_blocks), block(256);
   GL3_REQUIRE(keep_first >= 0 && (keep_first == 0 || window > 0), "gl3_attention_prefill: %d kept first keys without a window", keep_first);
   const Gl3ScoreRule rule{softcap, temp_coef, temp_every, gate, gate_ld};
   GL3_CHECK_RULE(rule, "gl3_attention_prefill");
   GL3_REQUIRE(!gate || (gate_ld % 4 == 0 && (uintptr_t)gate % 8 == 0), "gl3_attention_prefill: gate rows must be 8-byte aligned");
   const bool ruled = rule.any();
   const bool biased = slopes != nullptr || has_sink || sinks != nullptr || keep_first > 0;    // (the kernels that know of kept first keys)
+  const PfSplit sp{splits, n_tokens, part_o, part_ml};
+  GL3_REQUIRE(splits >= 1 && splits <= PF_SPLITS, "gl3_attention_prefill: %d splits (1 to %d)", splits, PF_SPLITS);
+  GL3_REQUIRE(splits == 1 || (part_o && part_ml && n_tokens > 0 && !ruled && !biased && maps == 1 && (uintptr_t)part_o % 16 == 0),
+              "gl3_attention_prefill: splits need buffers for their sums and the plain rule (one score map, no bias, sink, kept keys, cap, temperature or gate)");
   if (wide) {
 #define PF_ARGS                                                                                                     \
   (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu_seqlens, kv_before, block_table,     \
       seq_rows, table_stride, (bf16_t*)out, out_stride, n_heads, n_kv, page_size, window, scale, q_blocks, slopes, has_sink, sink, keep_first, mask_chunk, maps, sinks, rule
 #define GOW(HS, CK, AH, OCC)                                                                                        \
   do {                                                                                                              \
-    if (ruled) attention_prefill_wide_kernel<HS, CK, AH, OCC, true, true><<<grid, block, 0, stream>>>(PF_ARGS);     \
-    else if (biased) attention_prefill_wide_kernel<HS, CK, AH, OCC, true><<<grid, block, 0, stream>>>(PF_ARGS);     \
-    else attention_prefill_wide_kernel<HS, CK, AH, OCC, false><<<grid, block, 0, stream>>>(PF_ARGS);                \
+    if (ruled) attention_prefill_wide_kernel<HS, CK, AH, OCC, true, true><<<grid, block, 0, stream>>>(PF_ARGS, sp);     \
+    else if (biased) attention_prefill_wide_kernel<HS, CK, AH, OCC, true><<<grid, block, 0, stream>>>(PF_ARGS, sp);     \
+    else if (splits > 1) {                                                                                          \
+      attention_prefill_wide_kernel<HS, CK, AH, OCC, false, false, true><<<grid, block, 0, stream>>>(PF_ARGS, sp);  \
+      const long n = (long)n_tokens * n_heads * (HS / 4);                                                          \
+      attention_prefill_merge_kernel<HS><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(sp, (bf16_t*)out, out_stride, n_heads); \
+    } else attention_prefill_wide_kernel<HS, CK, AH, OCC, false><<<grid, block, 0, stream>>>(PF_ARGS, sp);          \
   } while (0)
     // chunks of 64 keys (one barrier for twice the work, two score tiles whose sums do not wait for
     // each other) where the registers hold them and a page holds whole chunks

@@ -109,7 +109,7 @@ def _declare(lib):
         "gl3_gemm_mfma": [P, P, P, I, I, I, I, L, L, L, I, I, P, L, L, P, I, I, I, P, F, F, P, P],
         "gl3_attention_decode_supports": [I, I],
         "gl3_attention_prefill_supports": [I, I],
-        "gl3_attention_prefill": [P, L, P, P, P, P, P, P, I, P, L, I, I, I, I, I, I, I, F, I, P, I, F, I, I, I, P, F, F, I, P, L, P],
+        "gl3_attention_prefill": [P, L, P, P, P, P, P, P, I, P, L, I, I, I, I, I, I, I, F, I, P, I, F, I, I, I, P, F, F, I, P, L, I, I, P, P, P],
         "gl3_scatter_i32": [P, L, P, P, I, P],
         "gl3_upload": [P, P, L, P],
         "gl3_stage_decode": [P, I, I, P, P, P, I, P, P],
@@ -2026,15 +2026,34 @@ def attention_prefill_fits(head_dim, n_heads, n_kv, page_size):
     return bool(library().gl3_attention_prefill_supports(head_dim, page_size)) and n_heads % n_kv == 0
 
 
+PREFILL_SPLIT_ROWS = 1024 * 128      # (token, head, split) rows that a step's splits never exceed
+
+
+def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len):
+    """Blocks of 128 queries that share their keys out (``attention_prefill``'s ``splits``): for steps that bring few tokens behind
+    a long context (a prompt in portions, the next turn of a dialogue), whose blocks are fewer than two for every CU and walk
+    the context one chunk after another. Only where every sequence held at least as many tokens as the longest one
+    brings (``kv_before``: their counts) and the longest reaches 1,024 keys; 256 keys a split at least, 8 splits at most. 512 tokens behind
+    4,000: 32 heads of 64 79 -> 39 us, 24 heads of 128 109 -> 61; 64 tokens behind 4,000 69 -> 17 and 98 -> 25; 2,048 behind 12,000,
+    24 heads of 128 692 -> 391. Prompts without a context lose: 1,024 tokens, 24 heads of 128 31 -> 36 us (their blocks' keys are
+    few, and the merge costs 5 to 10 us)."""
+    blocks = n_heads * n_seqs * -(-max_q_len // 128)
+    if blocks >= 512 or max_kv_len < 1024 or not kv_before or min(kv_before) < max_q_len:
+        return 1
+    return max(1, min(8, -(-512 // blocks), max_kv_len // 256))
+
+
 def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, out, max_q_len, n_heads, n_kv,
                       head_dim, page_size, window, scale, seq_rows=None, wide_from=0, slopes=None, sink=None, keep_first=0,
-                      chunk=0, n_v_heads=None, rule=None):
+                      chunk=0, n_v_heads=None, rule=None, splits=1, part_o=None, part_ml=None):
     """``rule``: a ``ScoreRule``; ``slopes`` (float32 [H]): score - slopes[h] * distance; ``sink``: the score of a key without a value that every
     query sees (None: none); ``chunk`` and ``n_v_heads`` as in ``attention_generic``. Any number of tokens per sequence; ``cu_seqlens`` [B+1] and ``kv_before`` [B] say which tokens
     of the packed ``q`` belong to which sequence and where they sit in it. ``seq_rows`` [B] (optional)
     names each sequence's row of ``block_table``; without it sequence b reads row b. ``wide_from``: from
     how many tokens of the step's longest sequence on the kernel with 128 queries a block runs
-    (0: the library's choice; tests run both kernels on the same inputs)."""
+    (0: the library's choice; tests run both kernels on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
+    128 queries are shared out over that many blocks of the same kernel, whose sums lie in ``part_o`` (float32, at least
+    splits * T * H * hs) and ``part_ml`` (2 * splits * T * H) until a second kernel merges them; the plain rule only."""
     _dev(q, "q", torch.bfloat16, contiguous=False); _dev(out, "out", torch.bfloat16, contiguous=False)
     _dev(k_cache, "k_cache", torch.bfloat16); _dev(v_cache, "v_cache", torch.bfloat16)
     _dev(cu_seqlens, "cu_seqlens", torch.int32); _dev(kv_before, "kv_before", torch.int32)
@@ -2058,12 +2077,17 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
     elif block_table.shape[0] < B:
         raise KernelError("attention: the block table has fewer rows than there are sequences")
     has_sink, sink_value, sinks = _sink(sink, n_heads, "attention_prefill")
+    if splits > 1:
+        _dev(part_o, "part_o", torch.float32); _dev(part_ml, "part_ml", torch.float32)
+        if part_o.numel() < splits * T * n_heads * head_dim or part_ml.numel() < 2 * splits * T * n_heads:
+            raise KernelError(f"attention: buffers of {part_o.numel()} and {part_ml.numel()} floats for {splits} splits of {T} tokens")
     _check(library().gl3_attention_prefill(
         _ptr(q), q.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(cu_seqlens), _ptr(kv_before), _ptr(block_table),
         _ptr(seq_rows), block_table.shape[1], _ptr(out), out.stride(0), B, int(max_q_len), n_heads, n_kv, head_dim,
         page_size, int(window or 0), float(scale), int(wide_from), _slopes(slopes, n_heads, "attention_prefill"),
         has_sink, sink_value, int(keep_first or 0) if window else 0, int(chunk or 0), n_kv // n_v, sinks,
-        *_rule(rule, T, n_heads * head_dim, q.dtype, "attention_prefill"), _stream()), "attention_prefill")
+        *_rule(rule, T, n_heads * head_dim, q.dtype, "attention_prefill"), int(splits), T, _ptr(part_o), _ptr(part_ml),
+        _stream()), "attention_prefill")
 
 
 # ------------------------------------------------------------------ host to device without tensor objects

@@ -1,0 +1,69 @@
+"""The prefill attention with a block's keys shared out over several blocks: against the plain reference and the unsplit kernel."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_kernels import DEV, K, attention_case, dev, run_attention
+
+pytestmark = pytest.mark.gpu
+
+
+def fn(lens_before, new, splits):
+    lib = K()
+
+    def call(q, kc, vc, positions, seq_of, table, out, H, Kh, hs, page, window, scale):
+        cu = dev(np.concatenate([[0], np.cumsum(new)]), torch.int32)
+        n = splits * len(positions) * H
+        part_o, part_ml = torch.full((n * hs,), float("nan"), device=DEV), torch.full((2 * n,), float("nan"), device=DEV)
+        lib.attention_prefill(q, kc, vc, cu, dev(lens_before, torch.int32), table, out, max(new), H, Kh, hs, page, window, scale,
+                              wide_from=1, **(dict(splits=splits, part_o=part_o, part_ml=part_ml) if splits > 1 else {}))
+    return call
+
+
+# contexts of fewer chunks than splits, of one page, long ones; last blocks of one query and of 128
+@pytest.mark.parametrize("splits", [2, 3, 8])
+@pytest.mark.parametrize("H, Kh, hs, page", [(4, 2, 32, 64), (6, 2, 64, 64), (2, 1, 64, 96), (5, 5, 96, 32), (3, 1, 128, 64)])
+def test_split_prefill_attention(H, Kh, hs, page, splits):
+    rng = np.random.default_rng(H * hs + splits)
+    before, new = [700, 0, 129, 1300, 31], [40, 3, 129, 1, 256]
+    sk, sv, qs = attention_case(rng, H, Kh, hs, before, new, "bfloat16")
+    got, ref = run_attention(fn(before, new, splits), sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1), page=page)
+    np.testing.assert_allclose(got, ref, atol=1e-2 * np.abs(ref).max())
+    whole, _ = run_attention(fn(before, new, 1), sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1), page=page)
+    np.testing.assert_allclose(got, whole, atol=2.0 ** -7 * np.abs(ref).max())       # (weights are rounded to 16 bits around another maximum)
+
+
+def test_split_prefill_attention_with_one_key_that_counts_and_a_window():
+    rng = np.random.default_rng(3)
+    H, Kh, hs, before, new = 4, 2, 64, [1500], [70]
+    sk, sv, qs = attention_case(rng, H, Kh, hs, before, new, "bfloat16")
+    for at in (3, 777, 1499):                        # in the first, a middle and the last split
+        k = [s.copy() for s in sk]
+        k[0][at] = 0
+        k[0][at, :, 5] = 40.0
+        q = [s.copy() for s in qs]
+        q[0][1500:, :, 5] = 8.0
+        got, ref = run_attention(fn(before, new, 4), k, sv, q, before, new, H, Kh, hs, "bfloat16", rng)
+        np.testing.assert_allclose(got, ref, atol=1e-2 * np.abs(ref).max())
+        np.testing.assert_allclose(got[:, 0], np.broadcast_to(sv[0][at, 0], got[:, 0].shape), atol=0.05)
+    got, ref = run_attention(fn(before, new, 4), sk, sv, qs, before, new, H, Kh, hs, "bfloat16", rng, window=100)
+    np.testing.assert_allclose(got, ref, atol=1e-2 * np.abs(ref).max())
+
+
+def test_split_prefill_attention_refuses_what_it_is_not_built_for():
+    lib = K()
+    rng = np.random.default_rng(4)
+    H, Kh, hs, before, new = 4, 2, 64, [300], [70]
+    sk, sv, qs = attention_case(rng, H, Kh, hs, before, new, "bfloat16")
+
+    def bad(**kw):
+        def call(q, kc, vc, positions, seq_of, table, out, *rest):
+            cu = dev([0, 70], torch.int32)
+            n = 70 * H
+            arguments = dict(splits=2, part_o=torch.zeros(2 * n * hs, device=DEV), part_ml=torch.zeros(4 * n, device=DEV))
+            arguments.update(kw)
+            lib.attention_prefill(q, kc, vc, cu, dev(before, torch.int32), table, out, 70, *rest, **arguments)
+        return call
+    for kw in (dict(sink=0.5), dict(slopes=torch.zeros(H, device=DEV)), dict(splits=9), dict(part_o=torch.zeros(8, device=DEV)), dict(part_ml=None)):
+        with pytest.raises((lib.KernelError, AttributeError)):
+            run_attention(bad(**kw), sk, sv, qs, before, new, H, Kh, hs, "bfloat16", rng)
