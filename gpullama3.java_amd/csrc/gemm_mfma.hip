@@ -14,7 +14,7 @@
 // contiguous range of tiles, ordered so that the tiles it holds at one time form a rectangle
 // and share their panels of A and of W.
 //
-// Tiles of 256 x 256 and of 128 rows x 256 over whole steps of 64 k have a kernel of their own (gemm_mfma_turns_kernel, below).
+// Tiles of 256 x 256, 128 rows x 256 and 128 x 128 over whole steps of 64 k have a kernel of their own (gemm_mfma_turns_kernel, below).
 //
 // Epilogues as in gemm_generic.hip: store, add into a float matrix, gated.
 #include "common.h"
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
   else finish(std::true_type{});
 }
 
-// ---- tiles of 256 x 256 and of 128 rows x 256 over whole steps of 64 k: operands straight from memory into shared memory, waves in two groups
+// ---- tiles of 256 x 256, 128 rows x 256 and 128 x 128 over whole steps of 64 k: operands straight from memory into shared memory, waves in two groups
 // that take turns.
 //
 // Eight waves; wave w's rows of A are 64 of each half of the tile's (group w / 4), its rows of W 32 of each half (gated:
@@ -280,8 +280,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 // the 32x32x16 instruction, whose accumulators pass through the registers twice as often per flop, the same loop lost 11%.
 // (8,192 x 28,672 x 4,096: the kernel above 1,680 us, this one 1,312.)
 //
-// AH = 1 is the tile of 128 rows x 256: two phases a step, a third step in shared memory instead of registers read ahead.
-// (2,048 rows, 3,072 columns, K = 2,048: 42 -> 31 us; 512 rows of the 3B layers' gate/up product: 59 -> 50 us.)
+// Halves of A and of W: AH = WH = 2 is the tile of 256 x 256. AH = 1: 128 rows x 256, two phases a step, a third step in shared
+// memory instead of registers read ahead (2,048 rows, 3,072 columns, K = 2,048: 42 -> 30 us; 512 rows of the 3B layers' gate/up
+// product: 59 -> 48 us). AH = WH = 1: 128 x 128, one phase a step, four steps in shared memory (2,048 rows of the 1B layers' down
+// projection in one piece of K 111 -> 79 us with its norm, where two pieces took 98; 512 rows, 5,120 columns, K = 3,072 33 -> 25 us).
+// The smaller tiles ask the second-level caches for up to twice the bytes per flop: 128 x 128 on every CU for 16 KB a clock, all
+// that they give.
 //
 // AH = 2: registers are read a part or two before they are used: in the memory part of phase 0 W0 and half of A1, of phase 1 the
 // rest of A1, of phases 2 and 3 the next step's A0 and W1. A half tile's place in shared memory is written for the step after
@@ -363,15 +367,15 @@ __device__ __forceinline__ void mf_finish4(TC* c, f32x4 s, f32x4 up, int n, int 
   }
 }
 
-template <int EPI, typename TC, int WT, int AH>
+template <int EPI, typename TC, int WT, int AH, int WH>
 __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                                   TC* __restrict__ C, int M, int N, int K, long lda, long ldw,
                                                                   long ldc, int tiles_m, int tiles_n, int group_m,
                                                                   int k_per_slice, float* __restrict__ P, long p_stride, long ldp,
                                                                   const float* __restrict__ bias, int act, int w_steps,
                                                                   const int* __restrict__ w_pos, MfExtras ex) {
-  constexpr int NCOLS = EPI == MF_GATED ? 128 : 256;
-  constexpr int STAGES = AH == 2 ? 2 : 3, STAGE = AH * 16384 + 32768;      // a step: A's halves, then W's
+  constexpr int NCOLS = (EPI == MF_GATED ? 64 : 128) * WH;
+  constexpr int STAGES = AH == 2 ? 2 : WH == 2 ? 3 : 4, STAGE = (AH + WH) * 16384;      // a step: A's halves, then W's
   __shared__ __attribute__((aligned(1024))) char lds[STAGES * STAGE];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wm = wave >> 2, wn = wave & 3;
@@ -400,7 +404,10 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
       const int row = piece * 8 + (lane >> 3), at = ((lane & 7) ^ ((row >> 1) & 7)) * 8;      // (rows of 128 bytes)
       ao[h][i] = (unsigned)((long)(min(m0 + h * 128 + row, M - 1) - m0) * lda + at) * 2;
       const int w_row = WT ? (piece >> 1) * 16 + lr : row, w_k = WT ? (piece & 1) * 32 + lq * 8 : at;
-      const int n = min(n0 + (EPI == MF_GATED ? 0 : h * 128) + w_row, N - 1) + (EPI == MF_GATED && h ? N : 0);
+      // (gated: half 1 are the up rows; with one half every other strip of 16 is, behind the gate rows of its columns)
+      const bool up = EPI == MF_GATED && (WH == 2 ? h == 1 : (w_row >> 4) & 1);
+      const int col = EPI != MF_GATED ? h * 128 + w_row : WH == 2 ? w_row : (w_row >> 5) * 16 + (w_row & 15);
+      const int n = min(n0 + col, N - 1) + (up ? N : 0);
       wo[h][i] = mf_w_offset<WT>(n, w_k, ldw, w_steps, w_pos, n0);
     }
   const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)lds + wave * 2048;
@@ -416,10 +423,10 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
     for (int i = 0; i < 2; ++i) mf_dma16(lds0 + place + AH * 16384 + h * 16384 + i * 1024, wo[h][i], w_buf, s);
   };
 
-  f32x4 acc[AH][4][2][2];     // [half of A][16 rows][half of W][16 rows]
+  f32x4 acc[AH][4][WH][2];    // [half of A][16 rows][half of W][16 rows]
 #pragma unroll
-  for (int i = 0; i < 16 * AH; ++i) (&acc[0][0][0][0])[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 af[AH][4][2], wf[2][2][2];      // [half][16 rows][k-step of 32]
+  for (int i = 0; i < 8 * AH * WH; ++i) (&acc[0][0][0][0])[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 af[AH][4][2], wf[WH][2][2];      // [half][16 rows][k-step of 32]
   const char* a_at = lds + (wm * 64 + lr) * 128;
   const char* w_at = lds + AH * 16384 + (WT ? wn * 4096 + lane * 16 : (wn * 32 + lr) * 128);
   const int twist = (lr >> 1) & 7;
@@ -490,7 +497,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
       products(1, 0);
       mf_barrier();
     }
-  } else {
+  } else if constexpr (WH == 2) {
     // 128 rows of A: two phases a step, (A, W0) and (A, W1), three steps in shared memory. What a part reads it uses at
     // once; a place is written again, for the step three further, in the part after both groups have read it.
     load_a(0, 0, 0);
@@ -525,6 +532,31 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
       before = here;
       here = here == 2 * STAGE ? 0 : here + STAGE;
     }
+  } else {
+    // 128 x 128: one phase a step, four steps in shared memory.
+    load_a(0, 0, 0);
+    load_w(0, 0, 0);
+    load_a(0, 1, STAGE);
+    load_w(0, 1, STAGE);
+    load_a(0, 2, 2 * STAGE);
+    load_w(0, 2, 2 * STAGE);
+    mf_wait_loads<8>();
+    mf_barrier();
+    if (wm == 1) mf_barrier();
+    for (int t = 0, here = 0, before = 3 * STAGE; t < steps; ++t) {
+      read_a(0, here, 0);
+      read_w(0, here);
+      read_a(0, here, 1);
+      load_a(0, t + 3, before);         // (where the step before lay, which both groups have read)
+      load_w(0, t + 3, before);
+      mf_wait_loads<8>();               // the next step has come
+      mf_wait_reads<0>();
+      mf_barrier();
+      products(0, 0);
+      mf_barrier();
+      before = here;
+      here = here == 3 * STAGE ? 0 : here + STAGE;
+    }
   }
   if (wm == 0) mf_barrier();
   mf_wait_loads<0>();                 // (what was asked for beyond the last step has landed)
@@ -534,37 +566,30 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   // floats an instruction. Row r's sixteen bytes c lie at place c ^ (r % 16): no two lanes of a write meet in a bank.
   const bool vec = slice ? ldp % 4 == 0 && p_stride % 4 == 0 && (uintptr_t)P % 16 == 0
                          : ldc % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;
+  constexpr int LPR = NCOLS / 4, RPW = 64 / LPR, ROW = 512 * WH;      // lanes of an output row, such rows a wave, bytes of a row of sums
 #pragma unroll
   for (int ah = 0; ah < AH; ++ah) {
     mf_barrier();                     // (both groups have read what lay here)
 #pragma unroll
     for (int tm = 0; tm < 4; ++tm)
 #pragma unroll
-      for (int wh = 0; wh < 2; ++wh)
+      for (int wh = 0; wh < WH; ++wh)
 #pragma unroll
         for (int tn = 0; tn < 2; ++tn)
-          *(f32x4*)(lds + (wm * 64 + tm * 16 + lr) * 1024 + (((wh * 32 + wn * 8 + tn * 4 + lq) ^ lr) << 4)) = acc[ah][tm][wh][tn];
+          *(f32x4*)(lds + (wm * 64 + tm * 16 + lr) * ROW + (((wh * 32 + wn * 8 + tn * 4 + lq) ^ lr) << 4)) = acc[ah][tm][wh][tn];
     mf_wait_reads<0>();
     mf_barrier();
-    const int rows = min(128, M - m0 - ah * 128);
-    if (EPI == MF_GATED) {            // two rows a wave: 128 columns
-#pragma unroll 2
-      for (int r = wave * 2 + (lane >> 5); r < rows; r += 16) {
-        const int c4 = lane & 31, n = n0 + c4 * 4;
-        const f32x4 g = *(const f32x4*)(lds + r * 1024 + ((c4 ^ (r & 15)) << 4));
-        const f32x4 u = *(const f32x4*)(lds + r * 1024 + (((32 + c4) ^ (r & 15)) << 4));
-        if (n < N) mf_finish4<EPI, TC>(C + (long)(m0 + ah * 128 + r) * ldc + n, g, u, n, N, vec, bias, act, ex);
-      }
-    } else {
+    const int rows = min(128, M - m0 - ah * 128), c4 = lane % LPR, n = n0 + c4 * 4;
+    const int gate = EPI == MF_GATED && WH == 1 ? (c4 >> 2) * 8 + (c4 & 3) : c4, up = WH == 1 ? gate + 4 : gate + 32;
 #pragma unroll 4
-      for (int r = wave; r < rows; r += 8) {
-        const int n = n0 + lane * 4;
-        const f32x4 v = *(const f32x4*)(lds + r * 1024 + ((lane ^ (r & 15)) << 4));
-        if (n >= N) continue;
-        const long m = m0 + ah * 128 + r;
-        if (slice > 0) mf_finish4<MF_STORE, float>(P + (long)(slice - 1) * p_stride + m * ldp + n, v, v, n, N, vec, nullptr, act, ex);
-        else mf_finish4<EPI, TC>(C + m * ldc + n, v, v, n, N, vec, bias, act, ex);
-      }
+    for (int r = wave * RPW + lane / LPR; r < rows; r += 8 * RPW) {
+      const f32x4 v = *(const f32x4*)(lds + r * ROW + ((gate ^ (r & 15)) << 4));
+      f32x4 u = v;
+      if (EPI == MF_GATED) u = *(const f32x4*)(lds + r * ROW + ((up ^ (r & 15)) << 4));
+      if (n >= N) continue;
+      const long m = m0 + ah * 128 + r;
+      if (EPI != MF_GATED && slice > 0) mf_finish4<MF_STORE, float>(P + (long)(slice - 1) * p_stride + m * ldp + n, v, u, n, N, vec, nullptr, act, ex);
+      else mf_finish4<EPI, TC>(C + m * ldc + n, v, u, n, N, vec, bias, act, ex);
     }
   }
 }
@@ -593,9 +618,9 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
   // them a rectangle of 4 x 8 (8 x 8), which asks memory for a third of the bytes that one column of
   // 32 row tiles does (3 to 5% of the time of the large products)
   const int group_m = tiles_m < (bm == 256 ? 4 : 8) ? tiles_m : (bm == 256 ? 4 : 8);
-  if constexpr (WM == 4 && WN == 4) {
+  if constexpr (WM == 4 && (WN == 4 || TM == 1)) {
     if (turns_takes(N, K, lda, ldw, EPI == MF_GATED, WT)) {
-      gemm_mfma_turns_kernel<EPI, TC, WT, TM><<<dim3((unsigned)blocks, slices), dim3(512), 0, stream>>>(
+      gemm_mfma_turns_kernel<EPI, TC, WT, TM, WN / 2><<<dim3((unsigned)blocks, slices), dim3(512), 0, stream>>>(
           (const bf16_t*)A, (const bf16_t*)W, (TC*)C, M, N, K, lda, ldw, ldc, tiles_m, tiles_n, group_m, k_per_slice, P, p_stride,
           ldp, bias, act, w_steps, w_pos, ex);
       GL3_LAUNCH_CHECK();
@@ -609,19 +634,25 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
   return 0;
 }
 
-// The tile the library takes where the caller names none. Where gemm_mfma_turns_kernel takes the product the time (us) of
-// each tile over its rounds on the chip, steps of 64 k and what a round costs beside them, as measured: 256 x 256 1.06 a step
-// and 3.3 a round, 128 rows x 256 0.67 and 0.9 (one block a CU, the last round as long as a full one); tiles of 128 x 128,
-// which have the kernel above, are ahead by a tenth where they are at most one a CU and the larger ones leave more than half of
-// the chip idle (512 rows, 5,120 columns, K = 3,072: 33 us against 37; 2,048 rows, 3,072 columns, K = 2,048: 41 against 31).
+// The tile the library takes where the caller names none. Where gemm_mfma_turns_kernel takes the product: the tile whose rounds on
+// the chip (256 blocks, one a CU) take the least time, a round being 0.41 us a step of 64 k and 1.6 us beside them for 128 x 128,
+// 0.64 and 2.8 for 128 rows x 256, 1.0 and 6.0 for 256 x 256 (fitted to 29 products into the residual rows of 70 to 8,192 rows, see
+// lib.turns_plan; at 31 sizes of other products, 70 to 8,192 rows, it takes the fastest of the three every time).
 static int choose_turns_shape(int M, int N, int K, bool gated) {
-  const long small_n = gated ? (N + 63) / 64 : (N + 127) / 128, big_n = gated ? (N + 127) / 128 : (N + 255) / 256;
-  const long small_tiles = (long)((M + 127) / 128) * small_n, wide_tiles = (long)((M + 127) / 128) * big_n,
-             big_tiles = (long)((M + 255) / 256) * big_n;
-  const double steps = K / 64;
-  const double small = small_tiles <= 256 ? 5 + 0.62 * steps : (small_tiles + 511) / 512 * (2 + 1.05 * steps);
-  const double wide = 4 + (wide_tiles + 255) / 256 * (0.9 + 0.671 * steps), big = 4 + (big_tiles + 255) / 256 * (3.3 + 1.063 * steps);
-  return small < wide && small < big ? 1 : wide < big ? 5 : 2;
+  static const int rows[3] = {128, 128, 256}, cols[3] = {128, 256, 256}, shape[3] = {1, 5, 2};
+  static const double step_us[3] = {0.41, 0.64, 1.0}, round_us[3] = {1.6, 2.8, 6.0};
+  int best = 0;
+  double least = 0;
+  for (int i = 0; i < 3; ++i) {
+    const int columns = gated ? cols[i] / 2 : cols[i];
+    const long blocks = (long)((M + rows[i] - 1) / rows[i]) * ((N + columns - 1) / columns);
+    const double time = (blocks + 255) / 256 * (K / 64 * step_us[i] + round_us[i]);
+    if (!best || time < least) {
+      best = shape[i];
+      least = time;
+    }
+  }
+  return best;
 }
 
 // The same where it does not (K in no whole steps of 64, or K in slices): 1 (128 x 128), 2 (256 x 256) or 5 (128 rows x 256).

@@ -2000,22 +2000,21 @@ def turns_planned(N, K):
 
 
 def turns_plan(M, N, K):
-    """``mfma_plan`` for K in whole steps of 64, where tiles of 256 x 256 and of 128 rows x 256 run on the kernel whose waves
-    take turns (``gemm_mfma_turns_kernel``): the plan with the least estimated time among those two with one to eight
-    slices of at least 512 columns. The estimate: rounds of 256 blocks (one a CU), each of 1.06 us a step of 64 columns and 3.3 us
-    beside them (128 rows: 0.67 and 0.9), and for every slice beyond the first 0.41 us a MB of the output, which is
-    written, read by the norm that follows, and added. Fitted to 21 sizes (150 to 8,192 rows, the output and down
-    projections of three models) times up to twelve plans, product and norm together: the plan chosen is within 6% of the best
-    of them and of the tiles of 128 x 128 everywhere but at 150 rows over K = 14,336 (52 against 45 us). Against the
-    plan before it: 2,048 rows of the 1B layers' down projection 98 -> 81 us, 512 rows of the 3B layers' 51 -> 45 us, 300 rows
-    over K = 8,192 38 -> 33 us."""
+    """``mfma_plan`` for K in whole steps of 64, where the tiles run on the kernel whose waves take turns
+    (``gemm_mfma_turns_kernel``): the plan with the least estimated time among its three tiles with one to eight slices of
+    at least 512 columns. The estimate: rounds of 256 blocks (one a CU), each of so many us a step of 64 columns and beside the steps,
+    and for every slice beyond the first 0.8 us and 0.376 us a MB of the output, which is written, read by the norm that follows,
+    and added. Fitted to 29 sizes (70 to 8,192 rows, the output and down projections of three models) times up to
+    eighteen plans, product and norm together: the plan chosen is the fastest of them or within 4% of it everywhere but at 1,000 rows
+    over 2,048 x 2,048 (28 against 25 us). Against the plans before it: 2,048 rows of the 1B layers' output projection 45 -> 32 us,
+    down projection 98 -> 79; 512 rows of the 3B layers' 36 -> 27 and 51 -> 44; 150 rows over 4,096 x 14,336 51 -> 43."""
     best = None
-    for shape, rows, step_us, round_us in ((5, 128, 0.671, 0.9), (2, 256, 1.063, 3.3)):
+    for shape, rows, cols, step_us, round_us in ((1, 128, 128, 0.41, 1.6), (5, 128, 256, 0.64, 2.8), (2, 256, 256, 1.0, 6.0)):
         for slices in range(1, 9):
             if slices > 1 and K // slices < 512:
                 break
-            blocks = -(-M // rows) * -(-N // 256) * slices
-            estimate = -(-blocks // 256) * (-(-K // (64 * slices)) * step_us + round_us) + 0.413e-6 * (slices - 1) * M * N * 4
+            blocks = -(-M // rows) * -(-N // cols) * slices
+            estimate = -(-blocks // 256) * (-(-K // (64 * slices)) * step_us + round_us) + (slices - 1) * (0.8 + 0.376e-6 * M * N * 4)
             if best is None or estimate < best[0]:
                 best = (estimate, shape, slices)
     return best[1], best[2]
