@@ -11,8 +11,8 @@
 // Two kernels, by the number of rows of A:
 // * up to 64 rows (gated 32): bound by the weights' way from memory. A block takes 16 rows of W (gated: 16 gate rows and
 //   their 16 up rows) and its sixteen waves a chunk of K each (16 KB of weights); the chunks' sums meet in shared memory.
-//   One row, weights from memory, 1B layers: gate/up 513 -> 29 us (134 MB: 4.6 TB/s), down projection 950 -> 26 us (67 MB:
-//   2.6 TB/s; 128 blocks), the head 179 us (5.9 TB/s), against the kernel for any sizes, whose 64 x 64 tiles leave a
+//   One row, weights from memory, 1B layers: gate/up 513 -> 29 us (134 MB: 4.6 TB/s), down projection 950 -> 17 us (67 MB:
+//   4.0 TB/s), the head 179 us (5.9 TB/s), against the kernel for any sizes, whose 64 x 64 tiles leave a
 //   product of 2,048 columns 32 blocks that walk K in steps of 16 behind two barriers each. Eight waves a block were 1.0
 //   to 1.3 times as long.
 // * more: bound by the matrix cores (256 flops a clock and CU). Tiles through shared memory in steps of 32 k, two
@@ -60,7 +60,10 @@ __device__ __forceinline__ f32x4 f3_load_a(__amdgpu_buffer_rsrc_t buf, unsigned 
 // ---- few rows
 #define F3_WAVES 16
 
-template <int EPI, int TM>
+// PAIRS (at most 8 rows of A, one tile): strips of 8 rows of W. A tile's rows 8..15 are the same rows of W one chunk of K further and
+// its token columns 8..15 the same tokens there, so that a product of the two works out two chunks at once, in its two diagonal
+// quarters; every element's sum is the same sum.
+template <int EPI, int TM, bool PAIRS = false>
 __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                                       float* __restrict__ C, int M, int N, int K, long lda,
                                                                       long ldw, long ldc, F3Out o) {
@@ -71,29 +74,35 @@ __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const floa
   __shared__ __attribute__((aligned(16))) f32x4 sums[SLOTS][G][TM][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int r = lane & 15, q = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  const int wrow = min(n0 + r, N - 1);
+  static_assert(!PAIRS || (TM == 1 && EPI != F3_GATED), "strips of 8: one tile of tokens");
+  const int n0 = blockIdx.x * (PAIRS ? 8 : 16);
+  const int wrow = min(n0 + (PAIRS ? r & 7 : r), N - 1);
   const float* wp[G];
   wp[0] = W + (long)wrow * ldw + q * 4;
   if (G == 2) wp[G - 1] = W + ((long)N + wrow) * ldw + q * 4;
   const __amdgpu_buffer_rsrc_t a_buf = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)(((long)(M - 1) * lda + K) * 4), 0x00020000);
   unsigned ao[TM];
 #pragma unroll
-  for (int t = 0; t < TM; ++t) ao[t] = t * 16 + r < M ? (unsigned)(((long)(t * 16 + r) * lda + q * 4) * 4) : F3_NOWHERE;
+  for (int t = 0; t < TM; ++t) {
+    const int row = PAIRS ? r & 7 : t * 16 + r;
+    ao[t] = row < M ? (unsigned)(((long)row * lda + q * 4) * 4) : F3_NOWHERE;
+  }
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   float total[G][NE] = {};
+  constexpr int CPS = PAIRS ? 2 : 1;                             // chunks a slot
   const int chunks = (K + F3_CHUNK - 1) / F3_CHUNK;
-  for (int first = 0; first < chunks; first += SLOTS) {
-    const int n_here = min(SLOTS, chunks - first);
+  for (int first = 0; first < chunks; first += SLOTS * CPS) {
+    const int n_here = min(SLOTS * CPS, chunks - first);
     if (first) __syncthreads();
-    for (int slot = wave; slot < n_here; slot += NW) {
-      const int k0 = (first + slot) * F3_CHUNK;
+    for (int slot = wave; slot * CPS < n_here; slot += NW) {
+      const int k0 = (first + slot * CPS + (PAIRS ? r >> 3 : 0)) * F3_CHUNK;      // (PAIRS: a lane's own chunk)
+      const bool whole = (first + (slot + 1) * CPS) * F3_CHUNK <= K;
       f32x4 acc[G][TM];
 #pragma unroll
       for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int t = 0; t < TM; ++t) acc[g][t] = zero;
-      if (k0 + F3_CHUNK <= K) {
+      if (whole) {
         // a whole chunk: sixteen loads of each operand, unrolled, for the scheduler to send ahead (all of them in front of the
         // first product was slower: 23.8 -> 27.0 us)
         constexpr int PART = 16 / G;
@@ -117,7 +126,8 @@ __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const floa
           }
         }
       } else {
-        for (int k = k0; k < K; k += 16) {     // (K is a multiple of 4: a lane's four k lie inside it or beyond it)
+        // (K is a multiple of 4: a lane's four k lie inside it or beyond it; blocks of 16 beyond K add nothing)
+        for (int k = k0, b = 0; b < F3_CHUNK / 16; k += 16, ++b) {
           const bool in = k + q * 4 < K;
 #pragma unroll
           for (int t = 0; t < TM; ++t) {
@@ -140,12 +150,26 @@ __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const floa
 #pragma unroll
     for (int i = 0; i < NE; ++i) {
       const int e = tid + 64 * NW * i;
-      if (e < 256 * TM) {
+      if (PAIRS) {
+        // element e < 64 (a quarter of a tile): token e / 8, column e % 8; in the other quarter 8 rows and 8 columns further
+        if (e < 64) {
+          const int m = e >> 3, n = e & 7;
+          for (int s = 0; s < n_here; ++s) {
+            const int row = n + 8 * (s & 1), col = m + 8 * (s & 1);
+            total[0][i] += ((const float*)&sums[s >> 1][0][0][(row >> 2) * 16 + col])[row & 3];
+          }
+        }
+      } else if (e < 256 * TM) {
         for (int s = 0; s < n_here; ++s)
 #pragma unroll
           for (int g = 0; g < G; ++g) total[g][i] += ((const float*)&sums[s][g][0][0])[e];
       }
     }
+  }
+  if (PAIRS) {
+    const int m = tid >> 3, n = n0 + (tid & 7);
+    if (tid < 64 && m < M && n < N) f3_finish<EPI>(C + (long)m * ldc + n, total[0][0], 0.f, n, N, o);
+    return;
   }
   // element e: token tile e / 256, lane (e / 4) % 64, v = e % 4: token lane % 16, column 4 * (lane / 16) + v
 #pragma unroll
@@ -272,10 +296,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
   }
 }
 
-template <int EPI, int TM>
+template <int EPI, int TM, bool PAIRS = false>
 static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
                        const F3Out& o, hipStream_t stream) {
-  gemm_f32_rows_kernel<EPI, TM><<<dim3((N + 15) / 16), dim3(64 * F3_WAVES), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, o);
+  gemm_f32_rows_kernel<EPI, TM, PAIRS><<<dim3(PAIRS ? (N + 7) / 8 : (N + 15) / 16), dim3(64 * F3_WAVES), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, o);
   GL3_LAUNCH_CHECK();
   return 0;
 }
@@ -293,6 +317,11 @@ static int launch_tile(const float* A, const float* W, float* C, int M, int N, i
   return 0;
 }
 
+// Strips of 8 rows of W for at most 8 rows of A: where strips of 16 leave half of the CUs without a block (a block's loads, 16 rows
+// of 64 bytes an instruction, come at 16 bytes a clock and CU) and K has more chunks than a block has waves. 2,048 columns, K =
+// 8,192: 25.7 -> 16.7 us; K = 2,048: 8.1 -> 9.3 us (half of the waves find no pair of chunks); 3,072 columns, K = 8,192: 28.6 and 29.1.
+static bool f32_pairs(int M, int N, int K) { return M <= 8 && N <= 2048 && K > F3_CHUNK * F3_WAVES; }
+
 template <int EPI>
 static int launch_f32(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
                       const F3Out& o, int shape, hipStream_t stream) {
@@ -301,6 +330,8 @@ static int launch_f32(const float* A, const float* W, float* C, int M, int N, in
   if (shape == 1 && ((long)(M - 1) * lda + K) * 4 >= (1L << 31)) shape = 5;      // (a descriptor's 31 bits)
   switch (shape) {
     case 1:
+      if constexpr (EPI != F3_GATED)
+        if (f32_pairs(M, N, K)) return launch_rows<EPI, 1, true>(F3_ARGS);
       if (M <= 16) return launch_rows<EPI, 1>(F3_ARGS);
       if (M <= 32) return launch_rows<EPI, 2>(F3_ARGS);
       if constexpr (EPI != F3_GATED) return launch_rows<EPI, 4>(F3_ARGS);

@@ -15,8 +15,9 @@ def bound(a, w, K_):
     return (256 + K_ / 256 + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64).T)
 
 
-# rows of one tile and one more (16, 32, 64, 128), columns likewise, K in one piece of 4, up to a chunk of 256 and beyond it
-@pytest.mark.parametrize("M, N, Kd", [(1, 16, 4), (3, 130, 72), (16, 33, 256), (17, 48, 260), (32, 257, 1028), (33, 77, 96), (48, 2048, 8192),
+# rows of one tile and one more (16, 32, 64, 128), columns likewise, K in one piece of 4, up to a chunk of 256 and beyond it, pairs
+# of chunks with and without a last one of its own
+@pytest.mark.parametrize("M, N, Kd", [(1, 16, 4), (1, 2048, 8192), (8, 44, 4100), (7, 33, 4608), (3, 130, 72), (16, 33, 256), (17, 48, 260), (32, 257, 1028), (33, 77, 96), (48, 2048, 8192),
                                       (64, 129, 516), (65, 200, 300), (130, 513, 2052), (513, 1024, 1024), (1030, 2500, 64)])
 def test_float32_products(M, N, Kd):
     lib = K()
