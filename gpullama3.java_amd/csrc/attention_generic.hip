@@ -154,7 +154,8 @@ extern "C" int gl3_attention_generic(const void* q, long q_stride, const void* k
   const Gl3ScoreRule rule{softcap, temp_coef, temp_every, gate, gate_ld};
   GL3_CHECK_RULE(rule, "gl3_attention_generic");
   if (dtype == GL3_F32 && out_dtype == GL3_F32 && window == 0 && chunk == 0 && !slopes && !has_sink && !sinks && v_in_k < 0 &&
-      n_v == n_kv && v_head_dim == head_dim && !rule.any() && n_kv <= 65535 && gl3_attention_f32_takes(head_dim, page_size))
+      n_v == n_kv && v_head_dim == head_dim && !rule.any() && n_kv <= 65535 && (uintptr_t)k_cache % 16 == 0 &&
+      (uintptr_t)v_cache % 16 == 0 && gl3_attention_f32_takes(head_dim, page_size))
     return gl3_attention_f32((const float*)q, q_stride, (const float*)k_cache, (const float*)v_cache, positions, seq_of_token,
                              block_table, table_stride, (float*)out, out_stride, n_tokens, n_heads, n_kv, head_dim, page_size, scale, stream);
   dim3 grid(n_tokens, n_heads), block(64);

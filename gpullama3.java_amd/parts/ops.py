@@ -1,7 +1,7 @@
 """Which kernel runs an operation: chosen by dtype and shape, never silently wrong.
 
-float32 activations always take the 32-bit kernels (plain multiply-adds, accurate
-exp and sqrt). bfloat16 activations take the matrix-core kernels where the shape
+float32 activations always take the 32-bit kernels (IEEE multiplies and adds, on the matrix cores' 32-bit instruction
+where the sizes allow, accurate exp and sqrt). bfloat16 activations take the matrix-core kernels where the shape
 fits what they are written for and the generic kernels otherwise.
 """
 from __future__ import annotations

@@ -90,6 +90,12 @@ def test_float32_attention(H, Kh, hs, before, new):
     # a window that hides nothing takes the kernel for any rule
     general, _ = run_attention(lib.attention_generic, sk, sv, qs, before, new, H, Kh, hs, "float32", np.random.default_rng(5), window=1 << 20)
     np.testing.assert_allclose(got, general, atol=4e-6 * np.abs(ref).max())
+    # so does a cache that does not begin at 16 bytes: the same numbers as that kernel's, bit for bit
+    def shifted(q, kc, vc, *rest, **more):
+        caches = [torch.empty(c.numel() + 1, device=c.device)[1:].view(c.shape).copy_(c) for c in (kc, vc)]
+        lib.attention_generic(q, *caches, *rest, **more)
+    apart, _ = run_attention(shifted, sk, sv, qs, before, new, H, Kh, hs, "float32", np.random.default_rng(5))
+    np.testing.assert_array_equal(apart, general)
     # every token alone: the same bits
     first = 0
     for b, (n0, n) in enumerate(zip(before, new)):
