@@ -636,17 +636,18 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
 
 // The tile the library takes where the caller names none. Where gemm_mfma_turns_kernel takes the product: the tile whose rounds on
 // the chip (256 blocks, one a CU) take the least time, a round being 0.41 us a step of 64 k and 1.6 us beside them for 128 x 128,
-// 0.64 and 2.8 for 128 rows x 256, 1.0 and 6.0 for 256 x 256 (fitted to 29 products into the residual rows of 70 to 8,192 rows, see
-// lib.turns_plan; at 31 sizes of other products, 70 to 8,192 rows, it takes the fastest of the three every time).
-static int choose_turns_shape(int M, int N, int K, bool gated) {
+// 0.64 and 2.8 for 128 rows x 256, 1.0 and 6.0 for 256 x 256 (at 31 sizes of products beside those into the residual rows, 70 to 8,192
+// rows, it takes the fastest of the three every time).
+static int choose_turns_shape(int M, int N, int K, int slices, bool gated) {
   static const int rows[3] = {128, 128, 256}, cols[3] = {128, 256, 256}, shape[3] = {1, 5, 2};
   static const double step_us[3] = {0.41, 0.64, 1.0}, round_us[3] = {1.6, 2.8, 6.0};
+  const int steps = (K / 64 + slices - 1) / slices;
   int best = 0;
   double least = 0;
   for (int i = 0; i < 3; ++i) {
     const int columns = gated ? cols[i] / 2 : cols[i];
-    const long blocks = (long)((M + rows[i] - 1) / rows[i]) * ((N + columns - 1) / columns);
-    const double time = (blocks + 255) / 256 * (K / 64 * step_us[i] + round_us[i]);
+    const long tiles = (long)((M + rows[i] - 1) / rows[i]) * ((N + columns - 1) / columns);
+    const double time = (tiles * slices + 255) / 256 * (steps * step_us[i] + round_us[i]);
     if (!best || time < least) {
       best = shape[i];
       least = time;
@@ -655,7 +656,7 @@ static int choose_turns_shape(int M, int N, int K, bool gated) {
   return best;
 }
 
-// The same where it does not (K in no whole steps of 64, or K in slices): 1 (128 x 128), 2 (256 x 256) or 5 (128 rows x 256).
+// The same where it does not (K in no whole steps of 64, or offsets beyond its 31 bits): 1 (128 x 128), 2 (256 x 256) or 5 (128 rows x 256).
 // 256 x 256 tiles of sixteen waves, one block a CU, have half the operand traffic per product, and
 // that traffic is what bounds the large products; of the 128 x 128 tiles of eight waves two fit a CU and
 // overlap each other's waits. A step of 64 columns takes a chip full of the large tiles 1.7 us and a chip
@@ -686,8 +687,8 @@ static int launch_mfma(const void* A, const void* W, void* C, int M, int N, int 
                        const int* w_pos, MfExtras ex, hipStream_t stream) {
   const int w_steps = w_order == 1 ? (K + 31) / 32 : w_order == 2 ? (K + 63) / 64 : 0;
   if (shape == 0)
-    shape = slices == 1 && turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order) ? choose_turns_shape(M, N, K, EPI == MF_GATED)
-                                                                                 : choose_shape(M, N, slices, EPI == MF_GATED);
+    shape = turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order) ? choose_turns_shape(M, N, K, slices, EPI == MF_GATED)
+                                                                  : choose_shape(M, N, slices, EPI == MF_GATED);
 #define MF_ARGS A, W, C, M, N, K, lda, ldw, ldc, slices, P, p_stride, ldp, bias, act, w_steps, w_pos, ex, stream
   if (w_order) {
     // W is one of its copies in the matrix cores' order (a weight that is held once): the three tiles that the library
@@ -709,6 +710,11 @@ static int launch_mfma(const void* A, const void* W, void* C, int M, int N, int 
   if (shape == 4) return launch_shape<EPI, TC, 2, 4, 2>(MF_ARGS);
   return launch_shape<EPI, TC, 1, 4, 4>(MF_ARGS);
 #undef MF_ARGS
+}
+
+// Whether tiles of the shapes 1, 2 and 5 of such a product run on gemm_mfma_turns_kernel.
+extern "C" int gl3_gemm_mfma_turns(int N, int K, long lda, long ldw, int gated, int w_order) {
+  return turns_takes(N, K, lda, ldw, gated != 0, w_order);
 }
 
 // N counts output columns: for the gated epilogue W has 2N rows (gate, then up).

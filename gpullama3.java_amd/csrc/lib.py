@@ -107,6 +107,7 @@ def _declare(lib):
         "gl3_qkv_rope_cache": [P, P, I, F, P, P, L, I, I, L, L, P, P, P, I, P, P, P, P, I, I, I, I, I, I, P, P, P, I, P],
         "gl3_token_facts": [P, P, P, I, I, P, P, I, P, P, P, I, P],
         "gl3_gemm_mfma": [P, P, P, I, I, I, I, L, L, L, I, I, P, L, L, P, I, I, I, P, F, F, P, P],
+        "gl3_gemm_mfma_turns": [I, I, L, L, I, I],
         "gl3_attention_decode_supports": [I, I],
         "gl3_attention_prefill_supports": [I, I],
         "gl3_attention_prefill": [P, L, P, P, P, P, P, P, I, P, L, I, I, I, I, I, I, I, F, I, P, I, F, I, I, I, P, F, F, I, P, L, I, I, P, P, P],
@@ -1966,8 +1967,7 @@ def mfma_slices(M, N, K):
 
 def mfma_plan(M, N, K):
     """(tile shape, slices of K) for the tiled product [M, K] x [N, K] into the residual stream, whose
-    slices the norm that follows adds up. For the sizes that ``turns_plan`` does not
-    take, on the kernel without turns: few tiles: tiles of 128 x 128 and ``mfma_slices``. More tiles
+    slices the norm that follows adds up. Few tiles: tiles of 128 x 128 and ``mfma_slices``. More tiles
     than places: the plan with the least estimated time among tiles of 128 (512 places) or 256 (256
     places) with one to four slices and tiles of 128 rows x 256 (256 places) with one, the estimate being (rounds the blocks need on their places) x
     (steps of 64 columns a block walks) x (time of such a step with the chip full: 1.05 us and 1.7 us)
@@ -1975,7 +1975,8 @@ def mfma_plan(M, N, K):
     276 tiles of 256 take two rounds for the work of 1.08, and two slices of them 2.16 of 3. Fitted to
     60 sizes (300 to 8,192 rows, the output and down projections of three models) times ten plans: the
     plan chosen is on average 1.4% slower than the best one measured, 13% at worst; one slice and the
-    tile by the number of tiles alone was 4.1% and 36%."""
+    tile by the number of tiles alone was 4.1% and 36%. (Times of the kernel without turns; the slices
+    hold for both kernels, ``residual_plan``.)"""
     if -(-M // 128) * -(-N // 128) <= 256:
         return 1, mfma_slices(M, N, K)
     best = None
@@ -1994,35 +1995,17 @@ def mfma_plan(M, N, K):
     return best[1], best[2]
 
 
-def turns_planned(N, K):
-    """Whether ``turns_plan`` rather than ``mfma_plan`` plans a product into the residual stream: whole steps of 64 columns, and
-    rows of 2,048 columns or more, the narrowest that it was fitted to."""
-    return K % 64 == 0 and N >= 2048
-
-
-def turns_plan(M, N, K):
-    """``mfma_plan`` for K in whole steps of 64, where the tiles run on the kernel whose waves take turns
-    (``gemm_mfma_turns_kernel``): the plan with the least estimated time among its three tiles with one to eight slices of
-    at least 512 columns. The estimate: rounds of 256 blocks (one a CU), each of so many us a step of 64 columns and beside the steps,
-    and for every slice beyond the first 0.8 us and 0.376 us a MB of the output, which is written, read by the norm that follows,
-    and added. Fitted to 29 sizes (70 to 8,192 rows, the output and down projections of three models) times up to
-    eighteen plans, product and norm together: the plan chosen is the fastest of them or within 4% of it everywhere but at 1,000 rows
-    over 2,048 x 2,048 (28 against 25 us). Against the plans before it: 2,048 rows of the 1B layers' output projection 45 -> 32 us,
-    down projection 98 -> 79; 512 rows of the 3B layers' 36 -> 27 and 51 -> 44; 150 rows over 4,096 x 14,336 51 -> 43.
-    Fewer slices are longer chains of 32-bit sums: a product's own error against 64 bits is 1.4e-7 to 7.6e-7 of its size under this
-    plan as under the one before, at single sizes up to 2.05 times as large (4,096 rows over 3,072 x 8,192: 2.8e-7 -> 5.7e-7). The rows
-    are bfloat16, so the logits don't show it: over 120 prompts of 150, 700 and 2,048 tokens (1B layers, against the 32-bit
-    engine) the error is 0.998 +- 0.002 times what it was, larger in 54 of them."""
-    best = None
-    for shape, rows, cols, step_us, round_us in ((1, 128, 128, 0.41, 1.6), (5, 128, 256, 0.64, 2.8), (2, 256, 256, 1.0, 6.0)):
-        for slices in range(1, 9):
-            if slices > 1 and K // slices < 512:
-                break
-            blocks = -(-M // rows) * -(-N // cols) * slices
-            estimate = -(-blocks // 256) * (-(-K // (64 * slices)) * step_us + round_us) + (slices - 1) * (0.8 + 0.376e-6 * M * N * 4)
-            if best is None or estimate < best[0]:
-                best = (estimate, shape, slices)
-    return best[1], best[2]
+def residual_plan(a, w, N):
+    """(tile shape, slices of K) for the tiled product a @ w.T into N columns of the residual stream: ``mfma_plan``'s slices, which say
+    how long the chains of 32-bit sums are that a result is made of, on every kernel; its tile too, but where the product has 2,048 columns or more and runs on
+    the kernel whose waves take turns (``gemm_mfma_turns_kernel``): 0, the library's choice among that kernel's tiles. A tile has no
+    say in the sums; fewer slices would (one slice of 8,192 for four: a product's error against 64 bits twice as large). Product and norm
+    against the kernel without turns: 2,048 rows of the 1B layers' down projection 100 -> 81 us, 512 rows of the 3B layers' 56 -> 47,
+    150 rows of the 8B layers' 52 -> 46."""
+    shape, slices = mfma_plan(a.shape[0], N, a.shape[1])
+    if N >= 2048 and library().gl3_gemm_mfma_turns(N, a.shape[1], a.stride(0), w.stride(0), 0, _w_order(w)[0]):
+        shape = 0
+    return shape, slices
 
 
 # ------------------------------------------------------------------ bfloat16 attention of a prefill step

@@ -319,7 +319,7 @@ def linear(a, w, out, epilogue=EPI_STORE, ctx=None, bias=None, act="silu", pack_
             shape, slices = 0, 1
             if (epilogue == EPI_ADD and plain_sums and ctx is not None and getattr(ctx, "fuse", False)
                     and "fused" not in disabled):
-                shape, slices = (K.turns_plan if K.turns_planned(out.shape[1], Kd) else K.mfma_plan)(M, out.shape[1], Kd)
+                shape, slices = K.residual_plan(a, w, out.shape[1])
             if slices > 1:
                 # the first slice adds into the rows, the norm that follows adds the others
                 settle_residual(ctx, out)

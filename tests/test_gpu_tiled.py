@@ -76,3 +76,22 @@ def test_tiled_gated_products(shape, order, M, N, Kd):
     assert np.abs(out.cpu().numpy() - want).max() <= 2e-5 * np.abs(want).max()         # (the fast exponential: 2^-20)
     lib.gemm_mfma(dev(a, torch.bfloat16), W, wide[:, :N], lib.EPI_GATED, shape=shape)
     assert torch.equal(wide[:, :N], out.to(torch.bfloat16)) and torch.all(wide[:, N:] == -7.0)
+
+
+# (rows and columns in no whole tiles, slices of unequal length; the plans: 8, 4, 3, 2 and 1 slices)
+@pytest.mark.parametrize("M, N, Kd", [(150, 2064, 4672), (513, 2048, 2048), (1000, 2304, 2240), (2047, 2048, 2112), (2050, 3072, 1024)])
+def test_products_into_the_residual_rows_keep_their_sums(M, N, Kd):
+    """The plan of a product into the residual rows on the kernel whose waves take turns: the same sums, bit for bit, as tiles on the
+    kernel without turns in the slices of ``mfma_plan``."""
+    lib = K()
+    rng = np.random.default_rng(M)
+    A, W = dev(rounded(rng.standard_normal((M, Kd)), "bfloat16"), torch.bfloat16), dev(rounded(rng.standard_normal((N, Kd)), "bfloat16"), torch.bfloat16)
+    res = dev(rng.standard_normal((M, N)))
+
+    def rows(shape, slices):
+        x, part = res.clone(), torch.full((slices - 1, M, N), -7.0, device=DEV) if slices > 1 else None
+        lib.gemm_mfma(A, W, x, lib.EPI_ADD, more_slices=part, shape=shape)
+        if part is not None:
+            lib.add_slices_rmsnorm(x, part)
+        return x
+    assert torch.equal(rows(*lib.residual_plan(A, W, N)), rows(3, lib.mfma_plan(M, N, Kd)[1]))

@@ -1,23 +1,17 @@
-"""Rules that choose a prompt step's kernels (the plan of the tiled products over whole steps of 64 columns, the splits of its attention):
+"""Rules that choose a prompt step's kernels (the plan of the tiled products into the residual rows, the splits of its attention):
 plain arithmetic on the host, at sizes they were measured at."""
+import torch
+
 from gpullama3_java_amd.csrc import lib
 
 
-def test_plans_of_products_into_the_residual_rows():
-    plan = lib.turns_plan
-    # the large tile where its blocks fill the chip; K in slices where they do not
-    assert plan(8192, 4096, 14336) == (2, 1) and plan(8192, 2048, 2048) == (2, 1)
-    assert plan(2048, 4096, 14336) == (2, 2) and plan(2221, 2048, 8192) == (2, 3)
-    # 128 rows x 256: one round where the large tile leaves half of the chip idle
-    assert plan(2048, 3072, 3072) == (5, 1) and plan(4096, 2048, 2048) == (5, 1) and plan(2048, 4096, 4096) == (5, 1)
-    # 128 x 128 where those would, whole or, for few rows, in slices
-    assert plan(2048, 2048, 8192) in ((1, 1), (5, 2)) and plan(2048, 2048, 2048) == (1, 1) and plan(512, 3072, 8192) == (1, 2)
-    assert plan(100, 2048, 8192) == (1, 8) and plan(150, 4096, 14336) == (1, 4)
-    assert lib.turns_planned(2048, 8192) and not lib.turns_planned(2048, 8200) and not lib.turns_planned(1024, 8192)
-    for M in range(65, 9000, 433):
-        for N, K in ((2048, 8192), (3072, 3072), (4096, 14336), (1000, 576), (3072, 256), (16, 64)):
-            shape, slices = plan(M, N, K)
-            assert shape in (1, 2, 5) and 1 <= slices <= 8 and (slices == 1 or K // slices >= 512)
+def test_plans_of_products_into_the_residual_rows_keep_their_slices():
+    """Which kernel a product runs on has no say in its sums: K in the slices of ``mfma_plan``, no chain of 32-bit sums is longer."""
+    for M in (65, 100, 150, 300, 512, 700, 1000, 2048, 3000, 4096, 5886, 8192):
+        for N, Kd in ((2048, 2048), (2048, 8192), (3072, 3072), (3072, 8192), (4096, 4096), (4096, 14336), (2048, 8200)):
+            a, w = (torch.empty((n, Kd), dtype=torch.bfloat16, device="meta") for n in (M, N))
+            shape, slices = lib.mfma_plan(M, N, Kd)
+            assert lib.residual_plan(a, w, N) == (0 if Kd % 64 == 0 else shape, slices)
 
 
 def test_splits_of_a_prompt_step_s_attention():
