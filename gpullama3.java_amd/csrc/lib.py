@@ -1997,13 +1997,13 @@ def mfma_plan(M, N, K):
 
 def residual_plan(a, w, N):
     """(tile shape, slices of K) for the tiled product a @ w.T into N columns of the residual stream: ``mfma_plan``'s slices, which say
-    how long the chains of 32-bit sums are that a result is made of, on every kernel; its tile too, but where the product has 2,048 columns or more and runs on
+    how long the chains of 32-bit sums are that a result is made of, on every kernel; its tile too, but where the product runs on
     the kernel whose waves take turns (``gemm_mfma_turns_kernel``): 0, the library's choice among that kernel's tiles. A tile has no
     say in the sums; fewer slices would (one slice of 8,192 for four: a product's error against 64 bits twice as large). Product and norm
     against the kernel without turns: 2,048 rows of the 1B layers' down projection 100 -> 81 us, 512 rows of the 3B layers' 56 -> 47,
-    150 rows of the 8B layers' 52 -> 46."""
+    150 rows of the 8B layers' 52 -> 46, 4,096 rows over 1,024 x 8,192 97 -> 81."""
     shape, slices = mfma_plan(a.shape[0], N, a.shape[1])
-    if N >= 2048 and library().gl3_gemm_mfma_turns(N, a.shape[1], a.stride(0), w.stride(0), 0, _w_order(w)[0]):
+    if library().gl3_gemm_mfma_turns(N, a.shape[1], a.stride(0), w.stride(0), 0, _w_order(w)[0]):
         shape = 0
     return shape, slices
 

@@ -6,9 +6,10 @@ from gpullama3_java_amd.csrc import lib
 
 
 def test_plans_of_products_into_the_residual_rows_keep_their_slices():
-    """Which kernel a product runs on has no say in its sums: K in the slices of ``mfma_plan``, no chain of 32-bit sums is longer."""
+    """Which kernel a product runs on has no say in its sums: K in the slices of ``mfma_plan``, no chain of 32-bit sums is longer.
+    The tile is that kernel's choice, for narrow products too: ``mfma_plan``'s tile is for two blocks a CU, the other kernel has one."""
     for M in (65, 100, 150, 300, 512, 700, 1000, 2048, 3000, 4096, 5886, 8192):
-        for N, Kd in ((2048, 2048), (2048, 8192), (3072, 3072), (3072, 8192), (4096, 4096), (4096, 14336), (2048, 8200)):
+        for N, Kd in ((2048, 2048), (2048, 8192), (3072, 3072), (3072, 8192), (4096, 4096), (4096, 14336), (2048, 8200), (512, 4096), (1024, 8192), (1536, 8960)):
             a, w = (torch.empty((n, Kd), dtype=torch.bfloat16, device="meta") for n in (M, N))
             shape, slices = lib.mfma_plan(M, N, Kd)
             assert lib.residual_plan(a, w, N) == (0 if Kd % 64 == 0 else shape, slices)
