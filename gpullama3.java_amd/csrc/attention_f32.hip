@@ -188,7 +188,7 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
 #pragma unroll
         for (int w = 0; w < AF_WAVES; ++w) {
           const float mw = part_m[w][rr];
-          if (mw == -INFINITY && top != -INFINITY) continue;     // (a wave whose keys the row does not see)
+          if (mw == -INFINITY && part_l[w][rr] == 0.f) continue;     // (a wave whose keys the row does not see; scores that are all NaN have a weight)
           const float f = expf(mw - top);
           total += part_l[w][rr] * f;
           o += part[w][d][ln] * f;

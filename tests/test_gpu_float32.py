@@ -119,3 +119,21 @@ def test_float32_attention_leaves_values_out_that_a_row_does_not_see(bad):
     assert not np.isfinite(got[at:, 2:, 7]).any()
     got[at:, 2:, 7] = clean[at:, 2:, 7] = 0
     np.testing.assert_array_equal(got, clean)
+
+
+# keys of one wave's whole turn, of part of one, of two turns (a row's other waves have finite scores)
+@pytest.mark.parametrize("lo, hi", [(64, 128), (70, 72), (128, 256)])
+def test_float32_attention_keeps_nan_scores(lo, hi):
+    """Scores that are not numbers are in the result of every row that sees them, also where all of a wave's scores are, and in no other."""
+    lib = K()
+    rng = np.random.default_rng(8)
+    H, Kh, hs, n = 4, 2, 64, 300
+    sk, sv, qs = attention_case(rng, H, Kh, hs, [0], [n], "float32")
+    clean, _ = run_attention(lib.attention_generic, sk, sv, qs, [0], [n], H, Kh, hs, "float32", np.random.default_rng(5))
+    sk[0][lo:hi, 1] = np.nan
+    got, _ = run_attention(lib.attention_generic, sk, sv, qs, [0], [n], H, Kh, hs, "float32", np.random.default_rng(5))
+    assert np.isnan(got[lo:, 2:]).all()
+    np.testing.assert_array_equal(got[:lo], clean[:lo])
+    np.testing.assert_array_equal(got[:, :2], clean[:, :2])
+    general, _ = run_attention(lib.attention_generic, sk, sv, qs, [0], [n], H, Kh, hs, "float32", np.random.default_rng(5), window=1 << 20)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(general))
