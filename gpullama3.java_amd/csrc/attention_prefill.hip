@@ -608,7 +608,7 @@ __global__ __launch_bounds__(256) void attention_prefill_merge_kernel(PfSplit sp
     const long r = min(s, sp.splits - 1) * rows + row;
     v[s] = *(const f32x4*)(sp.o + r * HS + d);
     m[s] = s < sp.splits ? sp.ml[r * 2] : -INFINITY;
-    l[s] = sp.ml[r * 2 + 1];
+    l[s] = s < sp.splits ? sp.ml[r * 2 + 1] : 0.f;
   }
 #pragma unroll
   for (int s = 0; s < PF_SPLITS; ++s) top = fmaxf(top, m[s]);
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(256) void attention_prefill_merge_kernel(PfSplit sp
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < PF_SPLITS; ++s) {
-    if (m[s] == -INFINITY && top != -INFINITY) continue;      // (a split whose keys the row does not see)
+    if (m[s] == -INFINITY && l[s] == 0.f) continue;      // (a split whose keys the row does not see; scores that are all NaN have a weight)
     const float f = __builtin_amdgcn_exp2f(m[s] - top);
     weight += f * l[s];
     sum += f * v[s];

@@ -50,6 +50,20 @@ def test_split_prefill_attention_with_one_key_that_counts_and_a_window():
     np.testing.assert_allclose(got, ref, atol=1e-2 * np.abs(ref).max())
 
 
+# 1,570 keys are 25 chunks of 64 in 4 splits: all of the second split's, part of it, the last two splits' keys that a row sees
+@pytest.mark.parametrize("lo, hi", [(384, 768), (400, 402), (768, 1500)])
+def test_split_prefill_attention_keeps_nan_scores(lo, hi):
+    """Scores that are not numbers are in the result of every row that sees them, also where all of a split's scores are."""
+    rng = np.random.default_rng(6)
+    H, Kh, hs, before, new = 4, 2, 64, [1500], [70]
+    sk, sv, qs = attention_case(rng, H, Kh, hs, before, new, "bfloat16")
+    clean, _ = run_attention(fn(before, new, 4), sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1))
+    sk[0][lo:hi, 1] = np.nan
+    got, _ = run_attention(fn(before, new, 4), sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1))
+    assert np.isnan(got[:, 2:]).all()
+    np.testing.assert_array_equal(got[:, :2], clean[:, :2])
+
+
 def test_split_prefill_attention_refuses_what_it_is_not_built_for():
     lib = K()
     rng = np.random.default_rng(4)
