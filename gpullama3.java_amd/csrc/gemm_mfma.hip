@@ -303,8 +303,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 // the operands want it, [strip of 16][k-step of 32][lane][16 bytes].
 __device__ __forceinline__ void mf_dma16(unsigned lds, unsigned offset, i32x4 rsrc, unsigned step_offset) {
   // (by hand: behind the builtin the compiler waits for every load in front of every read of shared memory. The
-  // instruction has no destination register; its data lands at m0 + 16 * lane. Nothing else in these kernels uses m0)
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(offset), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(step_offset))
+  // instruction has no destination register; its data lands at m0 + 16 * lane. m0 is an operand that the compiler sets, so that it
+  // knows what the register holds; an instruction stands between its setting and the load.)
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(__builtin_amdgcn_readfirstlane(lds)), "v"(offset), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(step_offset))
                : "memory");
 }
 template <int N>
