@@ -23,6 +23,7 @@ class Workspace:
         self._flat = {}
         self.frozen = False
         self.generation = 0        # counts reallocations: captured graphs hold the old addresses
+        self._no_room = set()
 
     def get(self, name, shape, dtype):
         n = 1
@@ -38,6 +39,17 @@ class Workspace:
             flat = torch.empty(max(n, 1), dtype=dtype, device=self.device)
             self._flat[key] = flat
         return flat[:n].view(shape)
+
+    def get_if_room(self, name, shape, dtype):
+        """``get`` for a buffer that a step can do without: None where the device has no room for it. Asked once: every
+        refused request would make the allocator give back what it keeps and wait for the device."""
+        if (name, dtype) in self._no_room:
+            return None
+        try:
+            return self.get(name, shape, dtype)
+        except torch.cuda.OutOfMemoryError:
+            self._no_room.add((name, dtype))
+            return None
 
 
 class StepContext:
@@ -84,6 +96,9 @@ class StepContext:
 
     def buffer(self, name, shape, dtype):
         return self.engine.workspace.get(name, shape, dtype)
+
+    def buffer_if_room(self, name, shape, dtype):
+        return self.engine.workspace.get_if_room(name, shape, dtype)
 
     def ssq_buffer(self, n_partials):
         """[n_partials, 64] partial sums of squares; one buffer, as large as the widest writer needs."""

@@ -27,3 +27,35 @@ def test_splits_of_a_prompt_step_s_attention():
             for T in (1, 128, 129, 1000, 5000):
                 n = s(heads, n_seqs, T, [T] * n_seqs, 100000)
                 assert 1 <= n <= 8 and (n == 1 or n * n_seqs * T * heads <= lib.PREFILL_SPLIT_ROWS)
+
+
+def test_a_prompt_step_runs_without_splits_where_their_buffers_have_no_room(monkeypatch):
+    """A portion behind a long context asks for buffers that it can do without: on a full device it runs as it would without them."""
+    from types import SimpleNamespace
+
+    from gpullama3_java_amd.engine.context import StepContext, Workspace
+    from gpullama3_java_amd.parts import ops
+
+    engine = SimpleNamespace(cache=None, dtype=torch.bfloat16, device=torch.device("cpu"), workspace=Workspace("cpu"))
+    ctx = StepContext(engine, 300, 1, [300], [4000], [0], False, 300, 4300)
+    calls, asked, full = [], [], [True]
+    empty = torch.empty
+
+    def no_room(n, **kw):
+        asked.append(n)
+        if full[0]:
+            raise torch.cuda.OutOfMemoryError("no room")
+        return empty(n, **kw)
+    monkeypatch.setattr(ops, "attention_kernel", lambda *a: "prefill")
+    monkeypatch.setattr(lib, "attention_prefill", lambda *a, **kw: calls.append(kw.get("splits", 1)))
+    q, cache = torch.zeros(300, 64), torch.zeros(1, 1, 64, 16)
+
+    def step():
+        with monkeypatch.context() as m:
+            m.setattr(torch, "empty", no_room)
+            ops.attention(ctx, q, cache, cache, None, q, 32, 8, 16, None, 0.25)
+    step(); step()
+    assert calls == [1, 1] and len(asked) == 2              # (each buffer asked for once)
+    full[0], engine.workspace = False, Workspace("cpu")
+    step()
+    assert calls[2] == lib.prefill_splits(32, 1, 300, [4000], 4300) > 1
