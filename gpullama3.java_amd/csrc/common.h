@@ -31,13 +31,12 @@ void gl3_set_error(const char* fmt, ...);
   } while (0)
 
 // gemm_f32.hip: products in true 32-bit on the matrix cores, which gl3_gemm_generic hands on where gl3_f32_takes says so
-// (a rule on W alone: whether a token's product goes there does not depend on the tokens beside it). shape: gl3_f32_shape
-// (0: as it says; others for measurements).
+// (a rule on W alone: whether a token's product goes there does not depend on the tokens beside it). gl3_f32_shape: the kernel
+// and tile that a product takes there.
 bool gl3_f32_takes(const void* W, int K, long ldw);
-int gl3_f32_shape(int M, int N, bool gated);
+extern "C" int gl3_f32_shape(int M, int N, int gated);
 int gl3_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc, int epi,
-                 const float* bias, int act, float act_limit, float act_shift, const float* col_scale, int shape,
-                 hipStream_t stream);
+                 const float* bias, int act, float act_limit, float act_shift, const float* col_scale, hipStream_t stream);
 
 // attention_f32.hip: the plain causal rule in true 32-bit on the matrix cores, which gl3_attention_generic hands on where the
 // layer's sizes allow (a rule on the layer alone, as above)

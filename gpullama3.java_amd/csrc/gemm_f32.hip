@@ -324,9 +324,9 @@ static bool f32_pairs(int M, int N, int K) { return M <= 8 && N <= 2048 && K > F
 
 template <int EPI>
 static int launch_f32(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
-                      const F3Out& o, int shape, hipStream_t stream) {
+                      const F3Out& o, hipStream_t stream) {
 #define F3_ARGS A, W, C, M, N, K, lda, ldw, ldc, o, stream
-  if (shape == 0) shape = gl3_f32_shape(M, N, EPI == F3_GATED);
+  int shape = gl3_f32_shape(M, N, EPI == F3_GATED);
   if (shape == 1 && ((long)(M - 1) * lda + K) * 4 >= (1L << 31)) shape = 5;      // (a descriptor's 31 bits)
   switch (shape) {
     case 1:
@@ -348,7 +348,7 @@ static int launch_f32(const float* A, const float* W, float* C, int M, int N, in
 // K = 2,048, both measured; the sum of a CU's tiles was within 4% of the measured time at 513 to 4,096 rows). Few rows: 48
 // rows of the down projection of the 1B layers 136 us in the smallest tile; gated products of more than 32 rows fill the
 // chip with those (48 rows: 55 us) where the other kernel would hold 128 KB of sums a block.
-int gl3_f32_shape(int M, int N, bool gated) {
+extern "C" int gl3_f32_shape(int M, int N, int gated) {
   if (M <= (gated ? 32 : 64)) return 1;
   static const int bn[4] = {128, 128, 64, 64}, bm[4] = {128, 64, 64, 32}, alone[4] = {154, 89, 53, 34}, each[4] = {144, 76, 41, 23};
   int best = 5;
@@ -367,10 +367,9 @@ int gl3_f32_shape(int M, int N, bool gated) {
 bool gl3_f32_takes(const void* W, int K, long ldw) { return K % 4 == 0 && ldw % 4 == 0 && (uintptr_t)W % 16 == 0; }
 
 int gl3_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc, int epi,
-                 const float* bias, int act, float act_limit, float act_shift, const float* col_scale, int shape,
-                 hipStream_t stream) {
+                 const float* bias, int act, float act_limit, float act_shift, const float* col_scale, hipStream_t stream) {
   const F3Out o{bias, col_scale, act, act_limit, act_shift};
-#define F3_ARGS (const float*)A, (const float*)W, (float*)C, M, N, K, lda, ldw, ldc, o, shape, stream
+#define F3_ARGS (const float*)A, (const float*)W, (float*)C, M, N, K, lda, ldw, ldc, o, stream
   if (epi == F3_STORE) return launch_f32<F3_STORE>(F3_ARGS);
   if (epi == F3_ADD) return launch_f32<F3_ADD>(F3_ARGS);
   return launch_f32<F3_GATED>(F3_ARGS);

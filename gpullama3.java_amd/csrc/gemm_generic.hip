@@ -143,7 +143,7 @@ extern "C" int gl3_gemm_generic(const void* A, int a_dtype, const void* W, int w
               "gl3_gemm_generic: W in order %d with N=%d, epilogue %d", w_order, N, epilogue);
   const int w_steps = w_order == 1 ? (K + 31) / 32 : (K + 63) / 64;
   if (a_dtype == GL3_F32 && w_dtype == GL3_F32 && c_dtype == GL3_F32 && w_order == 0 && gl3_f32_takes(W, K, ldw))
-    return gl3_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, epilogue, bias, act, act_limit, act_shift, col_scale, 0, stream);
+    return gl3_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, epilogue, bias, act, act_limit, act_shift, col_scale, stream);
   const int key = a_dtype * 4 + w_dtype * 2 + c_dtype;
   switch (key) {
     case 0: return launch_generic<float, float, float>(A, W, C, M, N, K, lda, ldw, ldc, epilogue, bias, act, w_order, w_steps, w_pos, act_limit, act_shift, col_scale, stream);

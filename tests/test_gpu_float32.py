@@ -62,6 +62,41 @@ def test_float32_products(M, N, Kd):
     assert (np.abs((general - out[:, 1:N + 1]).double().cpu().numpy()) <= off[:, :N] + one_chain).all()
 
 
+# every tile that products of many rows take (2: 128 x 128, 3: 128 x 64, 4: 64 x 64, 5: 64 x 32), one row and one column beyond whole
+# tiles; K of a chunk and a tail, of four chunks and a tail, of eight
+@pytest.mark.parametrize("Kd", [260, 1028, 2052])
+@pytest.mark.parametrize("tile, gated, M, N", [(2, False, 2049, 3585), (3, False, 1025, 3073), (4, False, 513, 3073), (5, False, 129, 257),
+                                               (2, True, 1281, 4097), (3, True, 513, 3073), (4, True, 193, 3585), (5, True, 97, 65)])
+def test_float32_products_in_every_tile(tile, gated, M, N, Kd):
+    lib = K()
+    assert lib.library().gl3_f32_shape(M, N, int(gated)) == tile
+    gen = torch.Generator(device="cuda").manual_seed(M + Kd)
+    A, W = (torch.randn(n, Kd, generator=gen, device="cuda") for n in (M, 2 * N if gated else N))
+    res = torch.randn(M, N, generator=gen, device="cuda")
+    both = A.double() @ W.double().T
+    off = (256 + Kd / 256 + 2) * 2.0 ** -24 * (A.double().abs() @ W.double().abs().T)        # (as in ``bound``)
+    one = torch.empty(1, N, device="cuda")
+    if gated:
+        out = torch.full((M, N + 1), -7.0, device="cuda")
+        lib.gemm_generic(A, W, out[:, :N], lib.EPI_GATED)
+        gate, up = both[:, :N], both[:, N:]
+        sig = torch.sigmoid(gate)
+        # (|silu'| <= 1.1; the exponential and the division are within 4 units of the last place)
+        slack = (1.1 * (off[:, :N] + 2.0 ** -23 * gate.abs()) * (up.abs() + off[:, N:]) + (gate * sig).abs() * (off[:, N:] + 2.0 ** -23 * up.abs())
+                 + 8 * 2.0 ** -24 * (gate * sig * up).abs())
+        assert ((out[:, :N] - gate * sig * up).abs() <= slack + 1e-30).all() and torch.all(out[:, N] == -7.0)
+    else:
+        out, x = torch.full((M, N + 1), -7.0, device="cuda"), res.clone()
+        lib.gemm_generic(A, W, out[:, :N])
+        lib.gemm_generic(A, W, x, lib.EPI_ADD)
+        assert ((out[:, :N] - both).abs() <= off).all() and torch.all(out[:, N] == -7.0)
+        assert torch.equal(x, res + out[:, :N])
+    # a row alone gives the same bits (the kernel for few rows: the same order of sums)
+    for r in (0, 63, 64, M // 2, M - 2, M - 1):
+        lib.gemm_generic(A[r:r + 1], W, one, lib.EPI_GATED if gated else lib.EPI_STORE)
+        assert torch.equal(one[0], out[r, :N])
+
+
 def test_float32_products_keep_small_numbers_and_infinities():
     lib = K()
     a, w = np.zeros((20, 64), np.float32), np.zeros((32, 64), np.float32)
