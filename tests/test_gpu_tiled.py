@@ -51,8 +51,8 @@ def test_tiled_products(shape, order, M, N, Kd):
     want = ref + bias
     assert (np.abs(half.double().cpu().numpy() - want) <= 2.0 ** -8 * np.abs(want) + 2 * sums + 1e-6).all()
     res = rng.standard_normal((M, N)).astype(np.float32)
-    for more in (0, 1, 3):
-        if (more + 1) * 64 > Kd or (more and shape == 5):
+    for more in (0, 1, 3, 4, 7):                                                     # (K of five steps: the last of four slices has none)
+        if (more + 1) * 64 > Kd:
             continue
         x = dev(res)
         part = torch.full((more, M, N), -7.0, device=DEV) if more else None
@@ -78,8 +78,8 @@ def test_tiled_gated_products(shape, order, M, N, Kd):
     assert torch.equal(wide[:, :N], out.to(torch.bfloat16)) and torch.all(wide[:, N:] == -7.0)
 
 
-# (rows and columns in no whole tiles, slices of unequal length; the plans: 8, 4, 3, 2 and 1 slices)
-@pytest.mark.parametrize("M, N, Kd", [(150, 2064, 4672), (513, 2048, 2048), (1000, 2304, 2240), (2047, 2048, 2112), (2050, 3072, 1024)])
+# (rows and columns in no whole tiles, slices of unequal length; the plans: 8, 2, 4, 3, 2 and 1 slices)
+@pytest.mark.parametrize("M, N, Kd", [(150, 2064, 4672), (2048, 2048, 8192), (513, 2048, 2048), (1000, 2304, 2240), (2047, 2048, 2112), (2050, 3072, 1024)])
 def test_products_into_the_residual_rows_keep_their_sums(M, N, Kd):
     """The plan of a product into the residual rows on the kernel whose waves take turns: the same sums, bit for bit, as tiles on the
     kernel without turns in the slices of ``mfma_plan``."""
@@ -95,3 +95,19 @@ def test_products_into_the_residual_rows_keep_their_sums(M, N, Kd):
             lib.add_slices_rmsnorm(x, part)
         return x
     assert torch.equal(rows(*lib.residual_plan(A, W, N)), rows(3, lib.mfma_plan(M, N, Kd)[1]))
+
+
+# slices of equal and unequal length, a last one without a step
+@pytest.mark.parametrize("M, N, Kd, slices", [(257, 272, 192, 1), (300, 256, 320, 4), (513, 528, 1088, 3), (130, 1024, 4160, 8), (1100, 2048, 8192, 2)])
+def test_a_tile_and_its_kernel_have_no_say_in_the_sums(M, N, Kd, slices):
+    """Tiles on the kernel whose waves take turns (1, 2, 5) and on the one without (3, 4): bit for bit the same sums for the same slices of K."""
+    lib = K()
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    A, W = (torch.randn(n, Kd, generator=gen, device="cuda").to(torch.bfloat16) for n in (M, N))
+    res = torch.randn(M, N, generator=gen, device="cuda")
+    got = []
+    for shape in (3, 4, 1, 2, 5):
+        x, part = res.clone(), torch.full((slices - 1, M, N), -7.0, device=DEV) if slices > 1 else None
+        lib.gemm_mfma(A, W, x, lib.EPI_ADD, more_slices=part, shape=shape)
+        got.append(torch.cat([x[None], part]) if part is not None else x[None])
+        assert torch.equal(got[-1], got[0]), shape
