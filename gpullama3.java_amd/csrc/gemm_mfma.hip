@@ -282,8 +282,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 //
 // Halves of A and of W: AH = WH = 2 is the tile of 256 x 256. AH = 1: 128 rows x 256, two phases a step, a third step in shared
 // memory instead of registers read ahead (2,048 rows, 3,072 columns, K = 2,048: 42 -> 30 us; 512 rows of the 3B layers' gate/up
-// product: 59 -> 48 us). AH = WH = 1: 128 x 128, one phase a step, four steps in shared memory (2,048 rows of the 1B layers' down
-// projection in one piece of K 111 -> 79 us with its norm, where two pieces took 98; 512 rows, 5,120 columns, K = 3,072 33 -> 25 us).
+// product: 59 -> 48 us). AH = WH = 1: 128 x 128, one phase a step, four steps in shared memory (150 rows of the 1B layers' down
+// projection in eight slices of K 31 -> 24 us with its norm; 512 rows, 5,120 columns, K = 3,072 33 -> 25 us).
 // The smaller tiles ask the second-level caches for up to twice the bytes per flop: 128 x 128 on every CU for 16 KB a clock, all
 // that they give.
 //
@@ -623,8 +623,8 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
   const long blocks = ((n_tiles + 7) / 8) * 8;
   GL3_REQUIRE(blocks < (1L << 31), "gl3_gemm_mfma: too many tiles");
   const int k_per_slice = ((K + MF_BK - 1) / MF_BK + slices - 1) / slices * MF_BK;
-  // 32 tiles of 256 x 256 (64 of 128 x 128) run on an XCD at a time: bands of 4 (8) row tiles make
-  // them a rectangle of 4 x 8 (8 x 8), which asks memory for a third of the bytes that one column of
+  // 32 tiles of 256 x 256 (of 128 x 128 as many on the kernel of turns, 64 on the other) run on an XCD at a time: bands of 4 (8)
+  // row tiles make them a rectangle of 4 x 8 (8 x 4, 8 x 8), which asks memory for a third of the bytes that one column of
   // 32 row tiles does (3 to 5% of the time of the large products)
   const int group_m = tiles_m < (bm == 256 ? 4 : 8) ? tiles_m : (bm == 256 ? 4 : 8);
   if constexpr (WM == 4 && (WN == 4 || TM == 1)) {
@@ -669,7 +669,8 @@ static int choose_turns_shape(int M, int N, int K, int slices, bool gated) {
   return best;
 }
 
-// The same where it does not (K in no whole steps of 64, or offsets beyond its 31 bits): 1 (128 x 128), 2 (256 x 256) or 5 (128 rows x 256).
+// The same where it does not (K in no whole steps of 64, or offsets beyond its 31 bits), on the kernel without turns: 1 (128 x 128),
+// 2 (256 x 256) or 5 (128 rows x 256).
 // 256 x 256 tiles of sixteen waves, one block a CU, have half the operand traffic per product, and
 // that traffic is what bounds the large products; of the 128 x 128 tiles of eight waves two fit a CU and
 // overlap each other's waits. A step of 64 columns takes a chip full of the large tiles 1.7 us and a chip
@@ -737,9 +738,9 @@ extern "C" int gl3_gemm_mfma_turns(int N, int K, long lda, long ldw, int gated, 
 // bias (may be null; not with slices): N floats (gated: 2N). act: the gated epilogue's activation, with its bound
 // and shift (gl3_gated; 0, 0: none). col_scale (may be null; not gated): N floats, a factor per column (every slice's sums
 // are multiplied, so the caller adds up scaled sums).
-// shape: 0 lets the library choose the tile; 1: 128 x 128, eight waves; 2: 256 x 256, sixteen waves of
-// 64 x 64; 3: 256 x 256, eight waves of 128 x 64; 4: 256 rows x 128, eight waves of 64 x 64; 5: 128 rows x 256,
-// sixteen waves of 32 x 64.
+// shape: 0 lets the library choose the tile; 1: 128 x 128; 2: 256 x 256; 5: 128 rows x 256: eight waves in turns where
+// gl3_gemm_mfma_turns says so, else eight waves of 32 x 64, sixteen of 64 x 64 and sixteen of 32 x 64 as the two below; 3: 256 x 256,
+// eight waves of 128 x 64; 4: 256 rows x 128, eight waves of 64 x 64.
 // w_order, w_pos: how W lies (see below): as stored, or one of its copies in the matrix cores' order alone.
 extern "C" int gl3_gemm_mfma(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, long lda, long ldw,
                              long ldc, int epilogue, int slices, float* P, long p_stride, long ldp, const float* bias,
