@@ -700,6 +700,7 @@ static int launch_mfma(const void* A, const void* W, void* C, int M, int N, int 
                        int slices, float* P, long p_stride, long ldp, const float* bias, int act, int shape, int w_order,
                        const int* w_pos, MfExtras ex, hipStream_t stream) {
   const int w_steps = w_order == 1 ? (K + 31) / 32 : w_order == 2 ? (K + 63) / 64 : 0;
+  if (shape < 0) shape = turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order) ? 0 : -shape;
   if (shape == 0)
     shape = turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order) ? choose_turns_shape(M, N, K, slices, EPI == MF_GATED)
                                                                   : choose_shape(M, N, slices, EPI == MF_GATED);
@@ -726,11 +727,6 @@ static int launch_mfma(const void* A, const void* W, void* C, int M, int N, int 
 #undef MF_ARGS
 }
 
-// Whether tiles of the shapes 1, 2 and 5 of such a product run on gemm_mfma_turns_kernel.
-extern "C" int gl3_gemm_mfma_turns(int N, int K, long lda, long ldw, int gated, int w_order) {
-  return turns_takes(N, K, lda, ldw, gated != 0, w_order);
-}
-
 // N counts output columns: for the gated epilogue W has 2N rows (gate, then up).
 // slices > 1 (not with the gated epilogue): K is cut into that many slices; the first ends in the
 // epilogue into C, slice s > 0 stores its sums into P[s - 1] ([slices - 1][M][ldp] floats,
@@ -739,8 +735,9 @@ extern "C" int gl3_gemm_mfma_turns(int N, int K, long lda, long ldw, int gated, 
 // and shift (gl3_gated; 0, 0: none). col_scale (may be null; not gated): N floats, a factor per column (every slice's sums
 // are multiplied, so the caller adds up scaled sums).
 // shape: 0 lets the library choose the tile; 1: 128 x 128; 2: 256 x 256; 5: 128 rows x 256: eight waves in turns where
-// gl3_gemm_mfma_turns says so, else eight waves of 32 x 64, sixteen of 64 x 64 and sixteen of 32 x 64 as the two below; 3: 256 x 256,
-// eight waves of 128 x 64; 4: 256 rows x 128, eight waves of 64 x 64.
+// turns_takes says so, else eight waves of 32 x 64, sixteen of 64 x 64 and sixteen of 32 x 64 as the two below; 3: 256 x 256,
+// eight waves of 128 x 64; 4: 256 rows x 128, eight waves of 64 x 64. -1, -2, -5: such a tile on the kernel without turns, and the
+// library's choice where the product runs on the other (a plan for the former, whose slices hold for both).
 // w_order, w_pos: how W lies (see below): as stored, or one of its copies in the matrix cores' order alone.
 extern "C" int gl3_gemm_mfma(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, long lda, long ldw,
                              long ldc, int epilogue, int slices, float* P, long p_stride, long ldp, const float* bias,
@@ -765,7 +762,7 @@ extern "C" int gl3_gemm_mfma(const void* A, const void* W, void* C, int c_dtype,
   GL3_REQUIRE(GL3_ACT_KNOWN(act), "gl3_gemm_mfma: unknown activation %d", act);
   GL3_REQUIRE(!col_scale || epilogue != MF_GATED, "gl3_gemm_mfma: a factor per column goes with the store and add epilogues");
   const MfExtras ex{col_scale, act_limit, act_shift};
-  GL3_REQUIRE(shape >= 0 && shape <= 5, "gl3_gemm_mfma: unknown tile shape %d", shape);
+  GL3_REQUIRE(shape >= -5 && shape <= 5, "gl3_gemm_mfma: unknown tile shape %d", shape);
   // w_order: 0: W holds the rows as stored. 1: W is the copy in the matrix operands' order (lib.tile_weight), w_pos (may be
   // null) naming each row's place in it. 2: the copy in packed strips of 8 rows (lib.tile_weight8).
   {

@@ -107,7 +107,6 @@ def _declare(lib):
         "gl3_qkv_rope_cache": [P, P, I, F, P, P, L, I, I, L, L, P, P, P, I, P, P, P, P, I, I, I, I, I, I, P, P, P, I, P],
         "gl3_token_facts": [P, P, P, I, I, P, P, I, P, P, P, I, P],
         "gl3_gemm_mfma": [P, P, P, I, I, I, I, L, L, L, I, I, P, L, L, P, I, I, I, P, F, F, P, P],
-        "gl3_gemm_mfma_turns": [I, I, L, L, I, I],
         "gl3_f32_shape": [I, I, I],
         "gl3_attention_decode_supports": [I, I],
         "gl3_attention_prefill_supports": [I, I],
@@ -1932,7 +1931,8 @@ def gemm_mfma(a, w, out, epilogue=EPI_STORE, more_slices=None, bias=None, act="s
               act_shift=0.0, col_scale=None):
     """out (=, +=, gated) a @ w.T on the matrix cores, tiled for many rows of ``a``. With
     ``more_slices`` [S, M, N] float32 K is cut into S + 1 slices: the first goes into ``out``, the
-    others' sums are stored there, for the caller to add to ``out`` in that order."""
+    others' sums are stored there, for the caller to add to ``out`` in that order. ``shape``: the tile, 0 the
+    library's choice, -tile a plan's (``mfma_plan``): the library's choice where the waves take turns."""
     _dev(a, "a", torch.bfloat16, contiguous=False); _dev(w, "w", torch.bfloat16); _dev(out, "out", contiguous=False)
     slices, p_stride, ldp = 1, 0, 0
     if more_slices is not None:
@@ -1976,8 +1976,13 @@ def mfma_plan(M, N, K):
     276 tiles of 256 take two rounds for the work of 1.08, and two slices of them 2.16 of 3. Fitted to
     60 sizes (300 to 8,192 rows, the output and down projections of three models) times ten plans: the
     plan chosen is on average 1.4% slower than the best one measured, 13% at worst; one slice and the
-    tile by the number of tiles alone was 4.1% and 36%. (Times of the kernel without turns; the slices
-    hold for both kernels, ``residual_plan``.)"""
+    tile by the number of tiles alone was 4.1% and 36%. These are times of the kernel without turns. Where
+    the product runs on the one whose waves take turns the tile is that kernel's choice (``gemm_mfma`` is given
+    the plan's as -tile), but the slices hold for both: they say how long the chains of 32-bit sums are that
+    a result is made of, which a tile does not (one slice of 8,192 for four: a product's error against 64
+    bits twice as large). Product and norm against the kernel without turns: 2,048 rows of the 1B layers' down
+    projection 100 -> 81 us, 512 rows of the 3B layers' 56 -> 47, 150 rows of the 8B layers' 52 -> 46, 4,096
+    rows over 1,024 x 8,192 97 -> 81."""
     if -(-M // 128) * -(-N // 128) <= 256:
         return 1, mfma_slices(M, N, K)
     best = None
@@ -1996,24 +2001,12 @@ def mfma_plan(M, N, K):
     return best[1], best[2]
 
 
-def residual_plan(a, w, N):
-    """(tile shape, slices of K) for the tiled product a @ w.T into N columns of the residual stream: ``mfma_plan``'s slices, which say
-    how long the chains of 32-bit sums are that a result is made of, on every kernel; its tile too, but where the product runs on
-    the kernel whose waves take turns (``gemm_mfma_turns_kernel``): 0, the library's choice among that kernel's tiles. A tile has no
-    say in the sums; fewer slices would (one slice of 8,192 for four: a product's error against 64 bits twice as large). Product and norm
-    against the kernel without turns: 2,048 rows of the 1B layers' down projection 100 -> 81 us, 512 rows of the 3B layers' 56 -> 47,
-    150 rows of the 8B layers' 52 -> 46, 4,096 rows over 1,024 x 8,192 97 -> 81."""
-    shape, slices = mfma_plan(a.shape[0], N, a.shape[1])
-    if library().gl3_gemm_mfma_turns(N, a.shape[1], a.stride(0), w.stride(0), 0, _w_order(w)[0]):
-        shape = 0
-    return shape, slices
-
-
 # ------------------------------------------------------------------ bfloat16 attention of a prefill step
 def attention_prefill_fits(head_dim, n_heads, n_kv, page_size):
     return bool(library().gl3_attention_prefill_supports(head_dim, page_size)) and n_heads % n_kv == 0
 
 
+PREFILL_SPLIT_KEYS = 1024            # keys that the longest sequence of a step with splits reaches
 PREFILL_SPLIT_ROWS = 1024 * 128      # (token, head, split) rows that a step's splits never exceed
 
 
@@ -2026,7 +2019,7 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len):
     24 heads of 128 692 -> 391. Prompts without a context lose: 1,024 tokens, 24 heads of 128 31 -> 36 us (their blocks' keys are
     few, and the merge costs 5 to 10 us)."""
     blocks = n_heads * n_seqs * -(-max_q_len // 128)
-    if blocks >= 512 or max_kv_len < 1024 or not kv_before or min(kv_before) < max_q_len:
+    if blocks >= 512 or max_kv_len < PREFILL_SPLIT_KEYS or not kv_before or min(kv_before) < max_q_len:
         return 1
     return max(1, min(8, -(-512 // blocks), max_kv_len // 256))
 
@@ -2074,7 +2067,7 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
         _ptr(seq_rows), block_table.shape[1], _ptr(out), out.stride(0), B, int(max_q_len), n_heads, n_kv, head_dim,
         page_size, int(window or 0), float(scale), int(wide_from), _slopes(slopes, n_heads, "attention_prefill"),
         has_sink, sink_value, int(keep_first or 0) if window else 0, int(chunk or 0), n_kv // n_v, sinks,
-        *_rule(rule, T, n_heads * head_dim, q.dtype, "attention_prefill"), int(splits), T, _ptr(part_o), _ptr(part_ml),
+        *_rule(rule, T, n_heads * head_dim, q.dtype, "attention_prefill"), splits, T, *((_ptr(part_o), _ptr(part_ml)) if splits > 1 else (None, None)),
         _stream()), "attention_prefill")
 
 

@@ -319,7 +319,8 @@ def linear(a, w, out, epilogue=EPI_STORE, ctx=None, bias=None, act="silu", pack_
             shape, slices = 0, 1
             if (epilogue == EPI_ADD and plain_sums and ctx is not None and getattr(ctx, "fuse", False)
                     and "fused" not in disabled):
-                shape, slices = K.residual_plan(a, w, out.shape[1])
+                shape, slices = K.mfma_plan(M, out.shape[1], Kd)
+                shape = -shape
             if slices > 1:
                 # the first slice adds into the rows, the norm that follows adds the others
                 settle_residual(ctx, out)
@@ -523,7 +524,8 @@ def attention(ctx, q, k_cache, v_cache, block_table, out, n_heads, n_kv, head_di
         return K.attention_decode(q, k_cache, v_cache, ctx.positions, _table_rows(ctx), block_table, out, n_heads,
                                   n_kv, head_dim, page, window, scale, splits, part_o, part_ml, **extras)
     if kernel == "prefill":
-        if not window and not chunk and slopes is None and sink is None and n_v_heads is None and rule is None:
+        if (ctx.max_kv_len >= K.PREFILL_SPLIT_KEYS and not window and not chunk and slopes is None and sink is None
+                and n_v_heads is None and rule is None):
             splits = K.prefill_splits(n_heads, ctx.n_seqs, ctx.max_q_len, getattr(ctx, "kv_before_host", None), ctx.max_kv_len)
             if splits > 1:
                 # (of one size, whatever the step brings: a buffer that grew would take the captured decode steps with it. On a

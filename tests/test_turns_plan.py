@@ -5,14 +5,27 @@ import torch
 from gpullama3_java_amd.csrc import lib
 
 
-def test_plans_of_products_into_the_residual_rows_keep_their_slices():
+def test_plans_of_products_into_the_residual_rows_keep_their_slices(monkeypatch):
     """Which kernel a product runs on has no say in its sums: K in the slices of ``mfma_plan``, no chain of 32-bit sums is longer.
-    The tile is that kernel's choice, for narrow products too: ``mfma_plan``'s tile is for two blocks a CU, the other kernel has one."""
+    The tile is that kernel's choice, for narrow products too (-tile: ``mfma_plan``'s, which is for two blocks a CU, on the kernel
+    without turns only)."""
+    from types import SimpleNamespace
+
+    from gpullama3_java_amd.parts import ops
+    got = []
+    monkeypatch.setattr(lib, "gemm_mfma_fits", lambda *a: True)
+    for rule in ("gemm_skinny_wide_fits", "gemm_skinny_fits"):
+        monkeypatch.setattr(lib, rule, lambda *a: False)
+    monkeypatch.setattr(lib, "gemm_mfma", lambda a, w, out, epilogue, more_slices=None, shape=0, **kw:
+                        got.append((shape, 1 if more_slices is None else more_slices.shape[0] + 1)))
     for M in (65, 100, 150, 300, 512, 700, 1000, 2048, 3000, 4096, 5886, 8192):
         for N, Kd in ((2048, 2048), (2048, 8192), (3072, 3072), (3072, 8192), (4096, 4096), (4096, 14336), (2048, 8200), (512, 4096), (1024, 8192), (1536, 8960)):
             a, w = (torch.empty((n, Kd), dtype=torch.bfloat16, device="meta") for n in (M, N))
+            ctx = SimpleNamespace(fuse=True, pending=None, ssq=None, normed=None, replayed=False, disabled=frozenset(),
+                                  buffer=lambda name, shape, dtype: torch.empty(shape, dtype=dtype, device="meta"))
+            ops.linear(a, w, torch.empty((M, N), device="meta"), lib.EPI_ADD, ctx)
             shape, slices = lib.mfma_plan(M, N, Kd)
-            assert lib.residual_plan(a, w, N) == (0 if Kd % 64 == 0 else shape, slices)
+            assert got.pop() == (-shape, slices)
 
 
 def test_splits_of_a_prompt_step_s_attention():
