@@ -529,10 +529,11 @@ def attention(ctx, q, k_cache, v_cache, block_table, out, n_heads, n_kv, head_di
             splits = K.prefill_splits(n_heads, ctx.n_seqs, ctx.max_q_len, getattr(ctx, "kv_before_host", None), ctx.max_kv_len)
             if splits > 1:
                 # (of one size, whatever the step brings: a buffer that grew would take the captured decode steps with it. On a
-                # device without room for them the step runs without splits: it never needed this memory before)
-                part_o = ctx.buffer_if_room("prefill_part_o", (K.PREFILL_SPLIT_ROWS * head_dim,), torch.float32)
+                # device without room for them the step runs without splits: it never needed this memory before. The small one
+                # first: where only the other has no room, little is kept that nothing uses)
                 part_ml = ctx.buffer_if_room("prefill_part_ml", (K.PREFILL_SPLIT_ROWS * 2,), torch.float32)
-                if part_o is not None and part_ml is not None:
+                part_o = ctx.buffer_if_room("prefill_part_o", (K.PREFILL_SPLIT_ROWS * head_dim,), torch.float32) if part_ml is not None else None
+                if part_o is not None:
                     extras.update(splits=splits, part_o=part_o, part_ml=part_ml)
         return K.attention_prefill(q, k_cache, v_cache, ctx.cu_seqlens, ctx.kv_before, block_table, out,
                                    ctx.max_q_len, n_heads, n_kv, head_dim, page, window, scale,

@@ -51,24 +51,31 @@ def test_a_prompt_step_runs_without_splits_where_their_buffers_have_no_room(monk
 
     engine = SimpleNamespace(cache=None, dtype=torch.bfloat16, device=torch.device("cpu"), workspace=Workspace("cpu"))
     ctx = StepContext(engine, 300, 1, [300], [4000], [0], False, 300, 4300)
-    calls, asked, full = [], [], [True]
+    calls, asked, room = [], [], [0]
     empty = torch.empty
 
-    def no_room(n, **kw):
+    def small_device(n, **kw):
         asked.append(n)
-        if full[0]:
+        if n > room[0]:
             raise torch.cuda.OutOfMemoryError("no room")
+        room[0] -= n
         return empty(n, **kw)
     monkeypatch.setattr(ops, "attention_kernel", lambda *a: "prefill")
     monkeypatch.setattr(lib, "attention_prefill", lambda *a, **kw: calls.append(kw.get("splits", 1)))
     q, cache = torch.zeros(300, 64), torch.zeros(1, 1, 64, 16)
 
-    def step():
+    def steps():
         with monkeypatch.context() as m:
-            m.setattr(torch, "empty", no_room)
-            ops.attention(ctx, q, cache, cache, None, q, 32, 8, 16, None, 0.25)
-    step(); step()
-    assert calls == [1, 1] and len(asked) == 2              # (each buffer asked for once)
-    full[0], engine.workspace = False, Workspace("cpu")
-    step()
-    assert calls[2] == lib.prefill_splits(32, 1, 300, [4000], 4300) > 1
+            m.setattr(torch, "empty", small_device)
+            for _ in range(2):
+                ops.attention(ctx, q, cache, cache, None, q, 32, 8, 16, None, 0.25)
+    small, large = lib.PREFILL_SPLIT_ROWS * 2, lib.PREFILL_SPLIT_ROWS * 16
+    for total, held in ((0, 0), (small, small), (large, small), (large + small - 1, small), (large + small, large + small)):
+        room[0] = total
+        engine.workspace = Workspace("cpu")
+        calls.clear(), asked.clear()
+        steps()
+        splits = lib.prefill_splits(32, 1, 300, [4000], 4300) if held > small else 1
+        assert calls == [splits] * 2 and (splits > 1) == (held > small)
+        assert len(asked) == len(set(asked))                                                   # (each buffer asked for once)
+        assert sum(t.numel() for t in engine.workspace._flat.values()) == held                 # (what is of no use is not kept)
