@@ -276,8 +276,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 // tile of a later step from memory to shared memory) and sixteen 16x16x32 matrix instructions, with a barrier after each
 // part; the second group runs one part behind the first, so on every SIMD one wave's matrix instructions run while the
 // other wave's memory part does. Without that lag the same loop is 19% slower (1.24 against 1.50 PFLOP/s at 8,192 x 8,192 x
-// 4,096). What bounds it now is the power budget: the matrix cores are busy 82% of the cycles at 1.5 to 1.6 GHz, and with
-// the 32x32x16 instruction, whose accumulators pass through the registers twice as often per flop, the same loop lost 11%.
+// 4,096). What bounds it now is the power budget: the clock stands at 1.4 to 1.8 GHz of 2.4, the matrix cores are busy 74 to 79% of
+// a CU's cycles (gate/up and plain products of 8,192 rows, K = 4,096), and with the 32x32x16 instruction, whose accumulators pass
+// through the registers twice as often per flop, the same loop lost 11%.
 // (8,192 x 28,672 x 4,096: the kernel above 1,680 us, this one 1,312.)
 //
 // Halves of A and of W: AH = WH = 2 is the tile of 256 x 256. AH = 1: 128 rows x 256, two phases a step, a third step in shared
@@ -647,9 +648,9 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
 // the chip take the least time, a round (a block on every CU: 32 of an XCD, which has an eighth of the tiles of every slice) being
 // 0.42 us a step of 64 k and 0.9 us beside them for 128 x 128, 0.60 and 4.0 for 128 rows x 256, 1.0 and 4.5 for 256 x 256. The
 // constants rank the tiles and are no times of their own (at 8,192 rows of 28,672 x 4,096 they say 959 us and it is 1,312).
-// Measured with the norm behind, 147 products into the residual rows (70 to 5,886 rows, 512 to 4,096 columns, K of 1,024 to 14,336 in
-// mfma_plan's slices): the tile chosen is the fastest of the three or within 5% but at 512 rows of 1,280 x 5,120 (29.3 against
-// 27.4 us) and 1,024 rows of 1,024 x 4,096 (33.9 against 31.1). With rounds of 256 blocks, whatever their XCD, 300 rows of 3,072 x
+// Measured with the norm behind, 143 products into the residual rows (70 to 5,886 rows, 512 to 4,096 columns, K of 1,024 to 14,336 in
+// mfma_plan's slices): the tile chosen is the fastest of the three or within 5% but at 512 rows of 1,280 x 5,120 (29.2 against
+// 27.0 us) and 1,024 rows of 1,024 x 4,096 (34.2 against 31.8). With rounds of 256 blocks, whatever their XCD, 300 rows of 3,072 x
 // 8,192 took 47.3 instead of 40.8 us. At 31 sizes of other products, 70 to 8,192 rows, it takes the fastest of the three every time.
 static int choose_turns_shape(int M, int N, int K, int slices, bool gated) {
   static const int rows[3] = {128, 128, 256}, cols[3] = {128, 256, 256}, shape[3] = {1, 5, 2};

@@ -2017,7 +2017,9 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len):
     brings (``kv_before``: their counts) and the longest reaches 1,024 keys; 256 keys a split at least, 8 splits at most. 512 tokens behind
     4,000: 32 heads of 64 79 -> 39 us, 24 heads of 128 109 -> 61; 64 tokens behind 4,000 69 -> 17 and 98 -> 25; 2,048 behind 12,000,
     24 heads of 128 692 -> 391. Prompts without a context lose: 1,024 tokens, 24 heads of 128 31 -> 36 us (their blocks' keys are
-    few, and the merge costs 5 to 10 us)."""
+    few, and the merge costs 5 to 10 us). A split's sums are 32-bit as the unsplit kernel's and shorter; only the maximum around which
+    weights are rounded is another: the error against 64 bits is 0.967 times that without splits on average, smaller at all of 90
+    sizes (contexts of 700 to 12,000, 37 to 1,100 tokens, heads of 32 to 128)."""
     blocks = n_heads * n_seqs * -(-max_q_len // 128)
     if blocks >= 512 or max_kv_len < PREFILL_SPLIT_KEYS or not kv_before or min(kv_before) < max_q_len:
         return 1
