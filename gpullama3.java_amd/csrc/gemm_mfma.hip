@@ -763,7 +763,7 @@ extern "C" int gl3_gemm_mfma(const void* A, const void* W, void* C, int c_dtype,
   GL3_REQUIRE(GL3_ACT_KNOWN(act), "gl3_gemm_mfma: unknown activation %d", act);
   GL3_REQUIRE(!col_scale || epilogue != MF_GATED, "gl3_gemm_mfma: a factor per column goes with the store and add epilogues");
   const MfExtras ex{col_scale, act_limit, act_shift};
-  GL3_REQUIRE(shape >= -5 && shape <= 5, "gl3_gemm_mfma: unknown tile shape %d", shape);
+  GL3_REQUIRE(shape >= -5 && shape <= 5 && shape != -3 && shape != -4, "gl3_gemm_mfma: unknown tile shape %d", shape);
   // w_order: 0: W holds the rows as stored. 1: W is the copy in the matrix operands' order (lib.tile_weight), w_pos (may be
   // null) naming each row's place in it. 2: the copy in packed strips of 8 rows (lib.tile_weight8).
   {

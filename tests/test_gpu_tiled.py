@@ -112,3 +112,12 @@ def test_a_tile_and_its_kernel_have_no_say_in_the_sums(M, N, Kd, slices):
         lib.gemm_mfma(A, W, x, lib.EPI_ADD, more_slices=part, shape=shape)
         got.append(torch.cat([x[None], part]) if part is not None else x[None])
         assert torch.equal(got[-1], got[0]), shape
+
+
+@pytest.mark.parametrize("shape", [-6, -4, -3, 6])
+def test_unknown_tiles_are_refused(shape):
+    """A plan names one of the library's own tiles (1, 2, 5); nothing is launched for another."""
+    lib = K()
+    a, w, x = (torch.zeros(128, 128, device=DEV, dtype=d) for d in (torch.bfloat16, torch.bfloat16, torch.float32))
+    with pytest.raises(lib.KernelError, match="unknown tile shape"):
+        lib.gemm_mfma(a, w, x, shape=shape)
