@@ -23,6 +23,7 @@
 // rescaled only when some maximum moved. Rows in shared memory are padded by 16 bytes, which
 // spreads the 16 rows that a quarter of the lanes reads over all banks.
 #include "common.h"
+#include "lds_loads.h"
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -592,6 +593,333 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
     }
 }
 
+// Every earlier key (no window, no bias), heads of 128, pages of whole chunks of 64 keys: eight waves in two groups that take turns.
+//
+// In the kernel above a wave's matrix instructions (1,024 cycles a chunk of 64 keys and 32 queries) and its softmax (some 900) add up
+// although two waves share a SIMD: they come to want the same unit at the same time. Here a barrier ends every turn, and in a turn one
+// group has the matrix cores while the other works out its softmax; wave w and wave w + 4, of different groups, share a
+// SIMD. A wave's two turns for chunk i:
+//   matrix turn i:  scores of chunk i, then the values of chunk i - 1 with its weights
+//   vector turn i:  weights of chunk i, the output brought to the new maximum, the first keys of chunk i + 1 read ahead
+// Group 0 has matrix turn i in turn 2 i, group 1 in turn 2 i + 1. What bounds it now: the vector instructions of both waves together with
+// the matrix instructions (a turn takes 1,650 cycles; vector instructions and matrix cores overlap to two thirds at best in a kernel
+// of nothing else). With heads of 64, whose matrix part is half as long, the same loop was no faster than the kernel above
+// (8,192 tokens 345 and 341 us) and is not built.
+// 32 heads, one sequence: 2,048 tokens 78 -> 61 us, 4,096 175 -> 141, 8,192 632 -> 520, 16,384 2,370 -> 1,930 (1.14 PFLOP/s).
+//
+// HEADS = 2: a block is 128 queries of two heads of one kv head, a group of waves to a head; HEADS = 1: 256 queries of one head.
+//
+// Keys and values go from memory straight into shared memory, as they lie in the cache (gl3_k_offset and gl3_v_offset are the
+// operands' order: sixteen lanes read 256 consecutive bytes), four chunks in turn. In matrix turn i a wave asks for its share of the
+// values of chunk i + 2 and of the keys of chunk i + 3; both places were read last in group 1's matrix turn i - 1, a turn that has
+// ended (matrix instructions took what was read before its barrier). Keys of chunk i + 1 are read from turn 2 i + 1 on and values of
+// chunk i from turn 2 i + 2 on: the wait in front of the barrier that ends turn 2 i leaves out only what was asked for after
+// them, two requests of group 0 and one of group 1. Chunks beyond the last repeat it, so that the counts hold; nothing is in flight
+// when a block ends.
+//
+// Score tile: rows 0..15 are the cache's first tile of 32 keys, rows 16..31 the second, so that register 4 a + b of lane (n, h)
+// is key 16 (a % 2) + 8 h + 4 (a / 2) + b: eight consecutive keys of each half, as the second product takes them.
+template <int HEADS, bool SPLIT>
+__global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
+    const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
+    const int* __restrict__ cu_seqlens, const int* __restrict__ kv_before, const int* __restrict__ block_table,
+    const int* __restrict__ seq_rows, int table_stride, bf16_t* __restrict__ out, long out_stride, int n_heads, int n_kv, int page_size,
+    float scale, int q_blocks, int n_seqs, PfSplit sp) {
+  constexpr int HS = 128, CK = 64, KS = HS / 16, DT = HS / 32, QB = 256 / HEADS;
+  constexpr int KB = CK * HS * 2;                  // bytes of a chunk's keys (and of its values)
+  constexpr int STAGE = 2 * KB, STAGES = 4, AHEAD = STAGES - 1;
+  constexpr int PW = KB / 8192;                    // pieces of 1 KB of either that a wave brings
+  constexpr int NK = 2 * KS, NV = 4 * DT;          // matrix instructions of a chunk: scores, values
+  constexpr int RING = 9;                          // operands from shared memory: the next eight, and the one in use
+  __shared__ __attribute__((aligned(1024))) char lds[STAGES * STAGE];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  // the y-th query block of all sequences, those behind the most queries first (a grid over sequences and blocks would start blocks
+  // that have no query, each on a CU of its own: this kernel's shared memory leaves no room beside another block)
+  int b = 0, qb = q_blocks - 1 - blockIdx.y;
+  if (n_seqs > 1) {
+    const int blocks = lane < n_seqs ? (cu_seqlens[lane + 1] - cu_seqlens[lane] + QB - 1) / QB : 0;
+    int left = blockIdx.y;
+    unsigned long here = 0;
+    qb = q_blocks;
+    while (qb > 0) {
+      here = __ballot(blocks > --qb);
+      const int count = __builtin_popcountl(here);
+      if (left < count) break;
+      left -= count;
+      here = 0;
+    }
+    if (here == 0) return;                         // the whole block: no barrier has been passed yet
+    for (; left > 0; --left) here &= here - 1;
+    b = __builtin_ctzl(here);
+  }
+  const int g = n_heads / n_kv, per_split = n_heads / HEADS;
+  const int split = SPLIT ? blockIdx.x / per_split : 0, at = SPLIT ? blockIdx.x % per_split : blockIdx.x;
+  const int c = at % n_kv;                         // (blocks of one kv head are n_kv apart: on one XCD where n_kv is 8)
+  const int group = wave >> 2;
+  const int head = c * g + at / n_kv * HEADS + (HEADS == 2 ? group : 0);
+  const int n = lane & 31, h = lane >> 5;
+  const int tok0 = __builtin_amdgcn_readfirstlane(cu_seqlens[b]);
+  const int q_len = __builtin_amdgcn_readfirstlane(cu_seqlens[b + 1]) - tok0;
+  if (qb * QB >= q_len) return;                    // (and so here)
+  const int before = __builtin_amdgcn_readfirstlane(kv_before[b]);
+  const int* bt = block_table + (long)(seq_rows ? __builtin_amdgcn_readfirstlane(seq_rows[b]) : b) * table_stride;
+  const int blk_last = before + min(qb * QB + QB - 1, q_len - 1);
+  int ck0 = 0, ck1 = blk_last / CK;
+  if (SPLIT) {
+    const int all = ck1 + 1;
+    ck0 = all * split / sp.splits;
+    ck1 = all * (split + 1) / sp.splits - 1;       // (no chunk: the block leaves a weight of nothing)
+  }
+  const int chunks = ck1 - ck0 + 1;
+  const int qi0 = qb * QB + (HEADS == 2 ? (wave & 3) * 32 : wave * 32);
+  const bool active = qi0 < q_len;
+  const bool q_ok = qi0 + n < q_len;
+  const int p_mine = before + qi0 + n;
+  const int p_last = before + min(qi0 + 31, q_len - 1), p_first = before + qi0;
+  // the wave's chunks, counted from the block's first: later ones hold no key that one of its queries sees
+  int my_first = 0, my_last = active ? min(p_last / CK, ck1) - ck0 : -1;
+  if (my_first > my_last) {
+    my_first = chunks;
+    my_last = -1;
+  }
+
+  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  bf16x8 qt[KS];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk)
+    qt[kk] = q_ok ? *(const bf16x8*)(q + (long)(tok0 + qi0 + n) * q_stride + (long)head * HS + kk * 16 + 8 * h) : zero8;
+  float m_run = -INFINITY, l_run = 0.f, alpha = 1.f;      // (alpha: what the output so far is still to be multiplied with)
+  f32x16 o[DT], s[2], w[2];      // (w: the weights of the last chunk, in the order of its keys)
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[dt][v] = 0.f;
+  bf16x8 pb[2][2], f[RING];        // weights as the second product takes them; operands from shared memory
+
+  // where chunks lie, sixty-four of them in a register (a lane one): keys in units of a chunk, values in units of 1,024 elements
+  const int per_page = page_size / CK, v_units = per_page * (HS / 16);
+  auto places = [&](int first, int& k_at, int& v_at) {
+    const int ck = max(ck0, min(ck0 + first + lane, ck1)), entry = ck / per_page, in_page = ck - entry * per_page;
+    const int row = bt[entry] * n_kv + c;
+    k_at = row * per_page + in_page;
+    v_at = row * v_units + in_page;
+  };
+  int k_at, v_at, k_later, v_later;
+  places(0, k_at, v_at);
+  places(64, k_later, v_later);
+  const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)lds + wave * (PW * 1024);
+  unsigned k_off[PW], v_off[PW];
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {
+    const int piece = wave * PW + i;               // (of the values: half of sixteen dims' 64 positions)
+    k_off[i] = piece * 1024 + lane * 16;
+    v_off[i] = (piece >> 1) * (page_size * 32) + (piece & 1) * 1024 + lane * 16;
+  }
+  // chunks are asked for one after the other: values of chunk x, then keys of chunk x + 1
+  i32x4 k_buf, v_buf;
+  auto locate = [&](int x) {                       // where chunk x lies; the keys' place is used first
+    v_buf = mf_rsrc(v_cache + (long)__builtin_amdgcn_readlane(v_at, (x - 1) & 63) * 1024);
+    if (x && (x & 63) == 0) {
+      k_at = k_later;
+      v_at = v_later;
+      places(x + 64, k_later, v_later);
+    }
+    k_buf = mf_rsrc(k_cache + (long)__builtin_amdgcn_readlane(k_at, x & 63) * (CK * HS));
+  };
+  auto load_v = [&](int x) {
+#pragma unroll
+    for (int i = 0; i < PW; ++i) mf_dma16(lds0 + (x % STAGES) * STAGE + KB + i * 1024, v_off[i], v_buf, 0);
+  };
+  auto load_k = [&](int x) {
+#pragma unroll
+    for (int i = 0; i < PW; ++i) mf_dma16(lds0 + (x % STAGES) * STAGE + i * 1024, k_off[i], k_buf, 0);
+  };
+
+  const char* k_lds = lds + (n >> 4) * (32 * HS) + h * 256 + (n & 15) * 16;
+  const char* v_lds = lds + KB + (n >> 4) * 2048 + h * 256 + (n & 15) * 16;
+  auto read_k = [&](int x, int m) {                // operand m of the scores: k-step m / 2 of tile m % 2
+    f[m % RING] = *(const bf16x8*)(k_lds + (x % STAGES) * STAGE + (m & 1) * (64 * HS) + (m >> 1) * 512);
+  };
+  auto read_v = [&](int x, int m, int to) {        // operand m of the values: sixteen keys m / DT, dims 32 (m % DT) ..
+    f[to % RING] = *(const bf16x8*)(v_lds + (x % STAGES) * STAGE + (m % DT) * 4096 + (m / DT) * 512);
+  };
+  // What of the softmax does not need a chunk's scores all at once is done beside the matrix instructions, a few instructions behind
+  // each (it occupies the matrix core for 32 cycles, the wave's issue for 4): the output brought to the new maximum and
+  // the weights rounded beside the scores of the next chunk, the weights added up beside the values; so are the reads of operands
+  // and the requests for later chunks, which cost 300 cycles a turn in front of them.
+  auto matrix_turn = [&](int i, auto with_scores, auto with_values) {
+    constexpr bool QK = decltype(with_scores)::value, PV = decltype(with_values)::value;
+    constexpr int K_COUNT = QK ? NK : 0, COUNT = K_COUNT + (PV ? NV : 0), BEFORE = QK ? NK : 1;
+    f32x16 zero;
+    float sum[4];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) zero[v] = 0.f;
+    auto prepare = [&](int m) {                    // (the m-th of BEFORE parts)
+#pragma unroll
+      for (int e = m * (32 / BEFORE); e < (m + 1) * (32 / BEFORE); ++e) pb[e >> 4][(e >> 3) & 1][e & 7] = static_cast<bf16_t>(w[e >> 4][e & 15]);
+    };
+    if (!QK) {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) read_v(i + STAGES - 1, m, m);
+      prepare(0);
+    }
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int m = 0; m < COUNT; ++m) {
+      const int at = m - K_COUNT;
+      if (m < K_COUNT) s[m & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[m % RING], qt[m >> 1], m < 2 ? zero : s[m & 1], 0, 0, 0);
+      else o[at % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[m % RING], pb[at / DT >> 1][at / DT & 1], o[at % DT], 0, 0, 0);
+      if (m + 8 < K_COUNT) read_k(i, m + 8);
+      else if (m + 8 < COUNT) read_v(i + STAGES - 1, m + 8 - K_COUNT, m + 8);
+      if (m == 1) load_v(i + AHEAD - 1);
+      if (m == 3) load_k(i + AHEAD);
+      if (PV && m < K_COUNT) prepare(m);
+      if (m >= K_COUNT) {
+#pragma unroll
+        for (int e = at * (32 / NV); e < (at + 1) * (32 / NV); ++e)      // (four chains)
+          sum[e & 3] = e < 4 ? w[e >> 4][e & 15] : sum[e & 3] + w[e >> 4][e & 15];
+        if (at * (32 / NV) >= 4) asm volatile("" : "+v"(sum[0]), "+v"(sum[1]), "+v"(sum[2]), "+v"(sum[3]));      // (here, not at the end)
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    if (PV) l_run = l_run * alpha + ((sum[0] + sum[1]) + (sum[2] + sum[3]));
+  };
+
+  const float c2 = scale * 1.4426950408889634f;    // scores in units of log2
+  auto max3 = [](float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+  };
+  auto vector_turn = [&](int key0, bool masked) {
+    // (register of the lane's e-th key of a tile, in the order of the keys; its key)
+    auto reg = [](int e) { return (e & 3) + ((e >> 2) & 1) * 8 + (e >> 3) * 4; };
+    if (masked) {                                  // (the same for the whole wave: a branch around the tests, one body)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int key = key0 + 32 * t + 16 * (e >> 3) + 8 * h + (e & 7);
+          s[t][reg(e)] = key <= p_mine ? s[t][reg(e)] : -INFINITY;
+        }
+    }
+    // (four chains: one would wait for itself, with no other wave of the SIMD at its softmax; the instruction by name, because
+    // fmaxf of a matrix instruction's results costs one more for each pair to quieten NaNs)
+    float top[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int v0 = (u & 1) * 8;
+      top[u] = max3(s[u >> 1][v0], s[u >> 1][v0 + 1], s[u >> 1][v0 + 2]);
+      top[u] = max3(top[u], s[u >> 1][v0 + 3], s[u >> 1][v0 + 4]);
+      top[u] = max3(top[u], s[u >> 1][v0 + 5], s[u >> 1][v0 + 6]);
+    }
+    float mx = max3(max3(top[0], top[1], s[0][7]), max3(top[2], top[3], s[0][15]), max3(s[1][7], s[1][15], s[1][15]));
+    {   // the other half of the keys of this query sits 32 lanes away
+      auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    mx *= c2;                                      // c2 > 0: the greatest score stays the greatest
+    const float m_new = fmaxf(m_run, mx);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) w[t][e] = __builtin_amdgcn_exp2f(fmaf(s[t][reg(e)], c2, -m_use));
+    m_run = m_new;
+    if (!__all(alpha == 1.0f)) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+    }
+    // (the compiler would work the weights out where the next turn first takes them, behind the barrier)
+    asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(alpha), "+v"(m_run));
+  };
+
+#pragma unroll
+  for (int x = 0; x < AHEAD; ++x) {
+    locate(x);
+    if (x) load_v(x - 1);
+    load_k(x);
+  }
+  locate(AHEAD);
+  mf_wait_loads<(2 * AHEAD - 2) * PW>();
+  mf_barrier();
+  // the end of a matrix turn (an even one of group 0) and of a vector turn (an even one of group 1)
+  auto end_matrix = [&]() {
+    if (group == 0) mf_wait_loads<(2 * AHEAD - 2) * PW>();
+    mf_barrier();
+  };
+  auto end_vector = [&]() {
+    if (group == 1) mf_wait_loads<(2 * AHEAD - 4) * PW>();
+    mf_barrier();
+  };
+  if (group == 1) end_vector();                    // the second group runs a turn behind
+  int i = 0;
+  for (; i < my_first; ++i) {
+    load_v(i + AHEAD - 1);
+    load_k(i + AHEAD);
+    end_matrix();
+    locate(i + 1 + AHEAD);
+    end_vector();
+  }
+  if (my_first <= my_last) {                       // (one body for all chunks: where bodies meet the compiler copies the sums)
+#pragma unroll
+    for (int m = 0; m < 8; ++m) read_k(i, m);
+    matrix_turn(i, std::true_type{}, std::false_type{});
+    for (;;) {
+      end_matrix();
+      locate(i + 1 + AHEAD);
+#pragma unroll
+      for (int m = 0; m < 8; ++m) read_k(i + 1, m);
+      const int key0 = (ck0 + i) * CK;
+      vector_turn(key0, key0 + CK - 1 > p_first);
+      end_vector();
+      if (++i > my_last) break;
+      matrix_turn(i, std::true_type{}, std::true_type{});
+    }
+    matrix_turn(i, std::false_type{}, std::true_type{});
+  }
+  for (; i < chunks; ++i) {
+    end_matrix();
+    locate(i + 1 + AHEAD);
+    end_vector();
+    load_v(i + AHEAD);
+    load_k(i + 1 + AHEAD);
+  }
+  if (group == 0) mf_barrier();
+  mf_wait_loads<0>();
+
+  float l = l_run;
+  l += __shfl_xor(l, 32, 64);
+  if (!q_ok) return;
+  if (SPLIT) {
+    const long row = ((long)split * sp.n_tokens + tok0 + qi0 + n) * n_heads + head;
+    float* po = sp.o + row * HS + 4 * h;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) *(f32x4*)(po + dt * 32 + 8 * a) = f32x4{o[dt][4 * a], o[dt][4 * a + 1], o[dt][4 * a + 2], o[dt][4 * a + 3]};
+    if (h == 0) {
+      sp.ml[row * 2] = m_run;
+      sp.ml[row * 2 + 1] = l;
+    }
+    return;
+  }
+  const float inv = 1.0f / l;
+  bf16_t* op = out + (long)(tok0 + qi0 + n) * out_stride + (long)head * HS + 4 * h;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      bf16x4 r;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) r[v] = static_cast<bf16_t>(o[dt][4 * a + v] * inv);
+      *(bf16x4*)(op + dt * 32 + 8 * a) = r;
+    }
+}
+
 // The splits' sums of a row (token, head) brought to the greatest of their maxima, added in the order of the splits, and divided
 // by the weight: a thread four dims of a row, its splits' loads all on their way at once.
 template <int HS>
@@ -638,13 +966,28 @@ static bool prefill_wide(int head_dim, int n_heads, int n_seqs, int max_q_len) {
   return (long)n_heads * n_seqs * ((max_q_len + 127) / 128) >= 512;
 }
 
+// The kernel of turns: what it is built for, and where it is taken unless the caller says otherwise. Its blocks are longer to start
+// (128 KB of shared memory are filled first) and a CU holds one: 1,024 tokens of one sequence, 24 heads of 128, 35 against 33 us for the
+// kernel of 64 queries a block, 32 heads 35 and 34; 1,280 tokens 41 and 40, 41 and 43; 1,536 tokens 47 and 48, 48 and 53; 2,048 61 and 66,
+// 61 and 78. Several sequences, whose blocks fill the chip: two of 1,024 tokens 38 against 45 us (32 heads), 317, 1,203
+// and 701 tokens 37 against 47 (24 heads); eight of 512 40 against 33 (24 heads) and 45 against 47 (32), 32 of 100 30 against 22.
+#define PF_TURNS -1
+static bool turns_takes(int head_dim, int page_size, int group, int n_seqs, int n_tokens) {
+  return head_dim == 128 && page_size % 64 == 0 && (n_seqs == 1 || (n_seqs <= 64 && n_tokens > 0 && n_tokens / (group % 2 ? 256 : 128) + n_seqs <= 65535));
+}
+static bool turns_wanted(int n_heads, int n_seqs, int max_q_len) {
+  const long blocks = (long)n_heads * n_seqs * ((max_q_len + 127) / 128);
+  return max_q_len >= 1280 ? blocks >= 256 : max_q_len >= 1024 && blocks >= 512;
+}
+
 extern "C" int gl3_attention_prefill_supports(int head_dim, int page_size) {
   return (head_dim == 32 || head_dim == 64 || head_dim == 96 || head_dim == 128) && page_size % 32 == 0;
 }
 
 // max_q_len: the most tokens any sequence brings in this step (it sizes the grid).
 // seq_rows (may be null): the row of `block_table` that holds sequence b's pages; null: row b.
-// wide_from: the kernel with 128 queries a block is taken when max_q_len reaches it; <= 0: the library's choice.
+// wide_from: the kernel with 128 queries a block is taken when max_q_len reaches it; 0: the library's choice; PF_TURNS: the kernel
+// of turns.
 extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k_cache, const void* v_cache,
                                      const int* cu_seqlens, const int* kv_before, const int* block_table,
                                      const int* seq_rows, int table_stride, void* out, long out_stride, int n_seqs,
@@ -668,7 +1011,6 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
   GL3_REQUIRE(q_stride % 8 == 0 && (uintptr_t)q % 16 == 0 && out_stride % 4 == 0 && (uintptr_t)out % 8 == 0,
               "gl3_attention_prefill: queries must be 16-byte aligned, outputs 8-byte aligned");
   const int g = n_heads / n_kv;
-  // query heads per wave: as many as the registers hold with two blocks on a CU
   const bool wide = splits > 1 ? true : wide_from > 0 ? max_q_len >= wide_from : prefill_wide(head_dim, n_heads, n_seqs, max_q_len);
   // query heads per wave: as many as the registers hold with two blocks on a CU; one with 32 queries a wave
   const int gh = wide ? 1 : head_dim <= 32 ? 4 : head_dim <= 64 ? 2 : 1;
@@ -687,6 +1029,26 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
   GL3_REQUIRE(splits >= 1 && splits <= PF_SPLITS, "gl3_attention_prefill: %d splits (1 to %d)", splits, PF_SPLITS);
   GL3_REQUIRE(splits == 1 || (part_o && part_ml && n_tokens > 0 && !ruled && !biased && maps == 1 && (uintptr_t)part_o % 16 == 0),
               "gl3_attention_prefill: splits need buffers for their sums and the plain rule (one score map, no bias, sink, kept keys, cap, temperature or gate)");
+  const bool turns_can = turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && !ruled && !biased && maps == 1 && window == 0 && mask_chunk == 0;
+  GL3_REQUIRE(wide_from != PF_TURNS || turns_can, "gl3_attention_prefill: the kernel of turns takes heads of 128, pages of whole 64 keys, at most 64 sequences, the plain rule");
+  if (wide_from == PF_TURNS || (wide_from <= 0 && splits == 1 && turns_can && turns_wanted(n_heads, n_seqs, max_q_len))) {
+    const int heads = g % 2 == 0 ? 2 : 1, queries = 256 / heads, qbs = (max_q_len + queries - 1) / queries;
+    dim3 tgrid((unsigned)(n_heads / heads) * splits, n_seqs == 1 ? qbs : n_tokens / queries + n_seqs);
+#define GOT(HEADS, SP)                                                                                                \
+  attention_prefill_turns_kernel<HEADS, SP><<<tgrid, dim3(512), 0, stream>>>(                                         \
+      (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu_seqlens, kv_before, block_table, \
+      seq_rows, table_stride, (bf16_t*)out, out_stride, n_heads, n_kv, page_size, scale, qbs, n_seqs, sp)
+    if (splits > 1) {
+      if (heads == 2) GOT(2, true);
+      else GOT(1, true);
+      const long n = (long)n_tokens * n_heads * (128 / 4);
+      attention_prefill_merge_kernel<128><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(sp, (bf16_t*)out, out_stride, n_heads);
+    } else if (heads == 2) GOT(2, false);
+    else GOT(1, false);
+#undef GOT
+    GL3_LAUNCH_CHECK();
+    return 0;
+  }
   if (wide) {
 #define PF_ARGS                                                                                                     \
   (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu_seqlens, kv_before, block_table,     \

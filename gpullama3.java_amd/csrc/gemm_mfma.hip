@@ -18,12 +18,12 @@
 //
 // Epilogues as in gemm_generic.hip: store, add into a float matrix, gated.
 #include "common.h"
+#include "lds_loads.h"
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 enum { MF_STORE = 0, MF_ADD = 1, MF_GATED = 2 };
 
@@ -302,40 +302,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 // In shared memory rows of A (and of W as stored) are 128 bytes in eight pieces of 16, piece c of row r at place
 // c ^ (r / 2 % 8): the sixteen rows that sixteen lanes read at one piece meet all banks once. W in a copy's order lies as
 // the operands want it, [strip of 16][k-step of 32][lane][16 bytes].
-__device__ __forceinline__ void mf_dma16(unsigned lds, unsigned offset, i32x4 rsrc, unsigned step_offset) {
-  // (by hand: behind the builtin the compiler waits for every load in front of every read of shared memory. The
-  // instruction has no destination register; its data lands at m0 + 16 * lane. m0 is an operand that the compiler sets, so that it
-  // knows what the register holds. A memory instruction may read a scalar register only five wait states after a vector
-  // instruction wrote it, and the compiler does not look into this block to keep them: 10 of the 806 loads it placed had
-  // readfirstlane of the step's offset three states ahead. A scalar instruction's result may be read at once, so the offset is copied by
-  // one; it is also the instruction that has to stand between m0's setting and the load. Five states of waiting instead: 1% of
-  // 8,192 tokens of the 8B layers.)
-  unsigned s;
-  asm volatile("s_mov_b32 %0, %4\n\tbuffer_load_dwordx4 %2, %3, %0 offen lds" : "=&s"(s) : "{m0}"(__builtin_amdgcn_readfirstlane(lds)), "v"(offset), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(step_offset))
-               : "memory");
-}
-template <int N>
-__device__ __forceinline__ void mf_wait_loads() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void mf_wait_reads() {
-  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void mf_barrier() {      // no wait of its own, and nothing moves across it
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-__device__ __forceinline__ i32x4 mf_rsrc(const void* p) {
-  const unsigned long a = (unsigned long)p;
-  int lo, hi;      // (through scalar instructions, as above)
-  asm("s_mov_b32 %0, %1" : "=s"(lo) : "s"(__builtin_amdgcn_readfirstlane((int)a)));
-  asm("s_mov_b32 %0, %1" : "=s"(hi) : "s"(__builtin_amdgcn_readfirstlane((int)(a >> 32))));
-  return i32x4{lo, hi, 0x7fffffff, 0x00020000};
-}
 // Byte offset, from the address that mf_w_base gives, of the 16 bytes of W at row `row`, piece k .. k + 7 of the first step,
 // and how far a step of 64 k lies behind the one before it.
 template <int WT>

@@ -2026,6 +2026,24 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len):
     return max(1, min(8, -(-512 // blocks), max_kv_len // 256))
 
 
+PREFILL_TURNS = -1                    # ``attention_prefill``'s ``wide_from`` that names the kernel of turns
+PREFILL_TURNS_KEYS = 2048             # splits run on it from this many keys on
+
+
+def prefill_turns_splits(n_heads, n_kv, head_dim, page_size, n_seqs, max_q_len, max_kv_len):
+    """Splits on the kernel of turns (heads of 128) where ``prefill_splits`` shares keys out; 0: the other kernel is taken. A CU holds one
+    of its blocks (256 queries of a head, or 128 of two where the heads of a kv head pair up), so as many splits as keep the
+    blocks within the chip's 256: 512 tokens behind 4,000, 24 heads, 5 splits 49 us, 6 splits (two rounds) 68, the other kernel 64. From
+    2,048 keys on it was the faster one at all of 42 sizes (1.02 to 1.33 times; 200 to 1,100 tokens, 24 and 32 heads), below at 8 of 20.
+    The sums' error against 64 bits is 1.003 times the other kernel's on average (chunks of 64 keys instead of 32 around whose running
+    maximum weights are rounded, and fewer splits; 0.97 times that without splits still)."""
+    if head_dim != 128 or page_size % 64 or n_seqs > 64 or max_kv_len < PREFILL_TURNS_KEYS:
+        return 0
+    heads = 1 if n_heads // n_kv % 2 else 2
+    blocks = n_heads // heads * n_seqs * -(-max_q_len // (256 // heads))
+    return max(1, min(8, 256 // blocks, max_kv_len // 256))
+
+
 def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, out, max_q_len, n_heads, n_kv,
                       head_dim, page_size, window, scale, seq_rows=None, wide_from=0, slopes=None, sink=None, keep_first=0,
                       chunk=0, n_v_heads=None, rule=None, splits=1, part_o=None, part_ml=None):
@@ -2034,7 +2052,8 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
     of the packed ``q`` belong to which sequence and where they sit in it. ``seq_rows`` [B] (optional)
     names each sequence's row of ``block_table``; without it sequence b reads row b. ``wide_from``: from
     how many tokens of the step's longest sequence on the kernel with 128 queries a block runs
-    (0: the library's choice; tests run both kernels on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
+    (0: the library's choice; ``PREFILL_TURNS``: the kernel of turns, which takes heads of 128 and the plain rule; tests run all kernels
+    on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
     128 queries are shared out over that many blocks of the same kernel, whose sums lie in ``part_o`` (float32, at least
     splits * T * H * hs) and ``part_ml`` (2 * splits * T * H) until a second kernel merges them; the plain rule only."""
     _dev(q, "q", torch.bfloat16, contiguous=False); _dev(out, "out", torch.bfloat16, contiguous=False)
