@@ -2,7 +2,7 @@
 // products and sums), for the plain rule: every earlier key, values of the keys' size, heads of 32, 64, 96 or 128.
 // gl3_attention_generic sends such calls here; anything beside the plain rule stays with its own kernel, which visits
 // a key per lane and step and is bound by trips to memory one after the other (two requests of 333 and 180 prompt tokens,
-// then 16 tokens each, 1B layers: 185 us a call on average there, 19 us here).
+// then 16 tokens each, 1B layers: 185 us a call on average there, 13 us here; 19 before the loads of a step went out together).
 //
 // A block works on sixteen rows, a row being one (token, query head) of one sequence and kv head, so that the heads of
 // a group and neighbouring tokens share the keys and values that it reads; its eight waves take the key steps of 64
@@ -22,8 +22,8 @@ typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 #define AF_WAVES 8
 
-template <int HB>
-__global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
+template <int HB, bool AHEAD>
+__global__ __launch_bounds__(64 * AF_WAVES, AHEAD || HB > 4 ? 2 : 4) void attention_f32_kernel(
     const float* __restrict__ Q, long q_stride, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
     const int* __restrict__ positions, const int* __restrict__ table_rows, const int* __restrict__ block_table, int table_stride,
     float* __restrict__ out, long out_stride, int n_tokens, int group, int n_kv, int page_size, float scale, int per_tile) {
@@ -38,10 +38,10 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
   const int t1 = min(t0 + per_tile, n_tokens);
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   while (t0 < t1) {
-    // tokens of one sequence
-    const int row0 = table_rows[t0];
-    int te = t0 + 1;
-    while (te < t1 && table_rows[te] == row0) ++te;
+    // tokens of one sequence (at most sixteen: all their rows of the table in one load)
+    const int rows = t0 + lane < t1 ? table_rows[t0 + lane] : -1;
+    const int row0 = __builtin_amdgcn_readfirstlane(rows);
+    const int te = t0 + __builtin_ctzl(~__ballot(t0 + lane < t1 && rows == row0));
     const int* bt = block_table + (long)row0 * table_stride;
     const int flats = (te - t0) * group;
     for (int base = 0; base < flats; base += 16) {
@@ -49,6 +49,14 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
       const bool have = a < flats;
       const int t = t0 + (have ? a / group : 0), h = c * group + (have ? a % group : 0);
       const int p = have ? positions[t] : -1;
+      // AHEAD: the pages of a step's halves are asked for a step ahead (the first before the positions are there: entries beyond the
+      // sequence's pages are looked up inside the row and not used)
+      int page[2];
+      auto look_up = [&](int first) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) page[b] = bt[min((first + 32 * b) / page_size, table_stride - 1)];
+      };
+      if (AHEAD) look_up(wave * 64);
       int p_max = p, p_min = have ? p : 0x7fffffff;
 #pragma unroll
       for (int o = 8; o > 0; o >>= 1) {
@@ -68,14 +76,40 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
 
       for (int first = wave * 64; first <= p_max; first += 64 * AF_WAVES) {
         const float *kp[2], *vp[2];
+        if (!AHEAD) look_up(first);
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-          const int pos = first + 32 * b <= p_max ? first + 32 * b : first;     // (a second half that no row sees reads the first again)
-          const int pg = bt[pos / page_size], in_page = pos % page_size;
+          const bool seen = first + 32 * b <= p_max;     // (a second half that no row sees reads the first again)
+          const int pg = page[seen ? b : 0], in_page = (seen ? first + 32 * b : first) % page_size;
           const long at = ((long)pg * n_kv + c) * page_size * HS;
           kp[b] = k_cache + at + (long)in_page * HS + ((q >> 1) << 7) + (r << 3) + (q & 1) * 4;
           vp[b] = v_cache + at + (((in_page >> 3) + q) << 7) + (r << 3);
         }
+        // AHEAD (at most one block a CU): all of a step's keys are asked for before the first is waited for, its values in front of the
+        // scores or, where the registers do not hold both, of the softmax. Otherwise the compiler waits for one load after
+        // the other, 32 trips to memory a step, which the other block of a CU hides.
+        constexpr int EARLY = HB > 6 ? HB / 2 : HB;
+        f32x4 vf[AHEAD ? HB : 1][2][2];
+        auto load_values = [&](int d0, int d1) {
+#pragma unroll
+          for (int d = d0; d < d1; ++d)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+              for (int e = 0; e < 2; ++e) vf[AHEAD ? d : 0][b][e] = *(const f32x4*)(vp[b] + (((long)d * (page_size >> 3)) << 7) + e * 4);
+        };
+        f32x4 kf[AHEAD ? HB : 1][2][2];
+        if (AHEAD) {
+#pragma unroll
+          for (int d = 0; d < HB; ++d)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+              for (int e = 0; e < 2; ++e) kf[AHEAD ? d : 0][b][e] = *(const f32x4*)(kp[b] + ((e * (HS >> 3) + d * 2) << 7));
+          if (HB <= 4) load_values(0, HB);
+        }
+        if (AHEAD) look_up(min(first + 64 * AF_WAVES, p_max));
+        if (AHEAD) __builtin_amdgcn_sched_barrier(0);
         f32x4 s[2][2] = {{zero, zero}, {zero, zero}};
 #pragma unroll
         for (int d = 0; d < HB; ++d)
@@ -83,10 +117,15 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
           for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-              const f32x4 k = *(const f32x4*)(kp[b] + ((e * (HS >> 3) + d * 2) << 7));
+              const f32x4 k = AHEAD ? kf[AHEAD ? d : 0][b][e] : *(const f32x4*)(kp[b] + ((e * (HS >> 3) + d * 2) << 7));
 #pragma unroll
               for (int j = 0; j < 4; ++j) s[b][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j], qf[d][j], s[b][e], 0, 0, 0);
             }
+        if (AHEAD && HB > 4) {
+          __builtin_amdgcn_sched_barrier(0);
+          load_values(0, EARLY);
+          __builtin_amdgcn_sched_barrier(0);
+        }
         // a lane's scores: positions first + 32 b + 8 q + 4 e + v of row r
         float most = -INFINITY;
 #pragma unroll
@@ -119,26 +158,46 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
         m = m_new;
         const bool edge = first + 63 > p_min;     // some row does not see some of these keys (or they do not exist)
         bool odd = false;
+        // a weight of zero does not make nothing of an infinite value: such values are left out here
+        auto leave_out = [&](f32x4& val) {
 #pragma unroll
-        for (int d = 0; d < HB; ++d) {
-          acc[d] *= alpha;
+          for (int j = 0; j < 4; ++j) {
+            const bool fine = fabsf(val[j]) < INFINITY;
+            odd |= !fine;
+            val[j] = fine ? val[j] : 0.f;
+          }
+        };
+        if (AHEAD) {
+          if (HB > EARLY) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_values(EARLY, HB);
+          }
+          if (edge) {
 #pragma unroll
-          for (int b = 0; b < 2; ++b)
+            for (int i = 0; i < 4 * HB; ++i) leave_out((&vf[0][0][0])[i]);
+          }
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-              f32x4 val = *(const f32x4*)(vp[b] + (((long)d * (page_size >> 3)) << 7) + e * 4);
-              if (edge) {
-                // a weight of zero does not make nothing of an infinite value: such values are left out here
+          for (int d = 0; d < HB; ++d) acc[d] *= alpha;
+          // (an output tile's products one after the other in the order of the keys; the tiles take turns)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                  const bool fine = fabsf(val[j]) < INFINITY;
-                  odd |= !fine;
-                  val[j] = fine ? val[j] : 0.f;
-                }
+          for (int i = 0; i < 16; ++i)
+#pragma unroll
+            for (int d = 0; d < HB; ++d)
+              acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[AHEAD ? d : 0][i >> 3][(i >> 2) & 1][i & 3], s[i >> 3][(i >> 2) & 1][i & 3], acc[d], 0, 0, 0);
+        } else {
+#pragma unroll
+          for (int d = 0; d < HB; ++d) {
+            acc[d] *= alpha;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+              for (int e = 0; e < 2; ++e) {
+                f32x4 val = *(const f32x4*)(vp[b] + (((long)d * (page_size >> 3)) << 7) + e * 4);
+                if (edge) leave_out(val);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(val[j], s[b][e][j], acc[d], 0, 0, 0);
               }
-#pragma unroll
-              for (int j = 0; j < 4; ++j) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(val[j], s[b][e][j], acc[d], 0, 0, 0);
-            }
+          }
         }
         if (edge && __any(odd)) {
           // and added up apart for the rows that see them (not rescaled later: no factor makes them finite)
@@ -215,14 +274,23 @@ int gl3_attention_f32(const float* q, long q_stride, const float* k_cache, const
   const int most = group >= 16 ? 1 : 16 / group;
   const int per_tile = (long)((n_tokens + most - 1) / most) * n_kv >= 512 ? most : 1;
   const dim3 grid((n_tokens + per_tile - 1) / per_tile, n_kv), block(64 * AF_WAVES);
-#define AF_RUN(HB)                                                                                                        \
-  attention_f32_kernel<HB><<<grid, block, 0, stream>>>(q, q_stride, k_cache, v_cache, positions, table_rows, block_table, \
-                                                      table_stride, out, out_stride, n_tokens, group, n_kv, page_size, scale, per_tile)
+  // (the loads of a step in registers at once take the room of the other block that a CU would hold: 333 and 180 tokens, 32 heads of
+  // 64, 34 us without and 40 with; 2,000 keys for each of four tokens 46 and 35)
+  const bool ahead = (long)grid.x * grid.y <= 256;
+#define AF_GO(HB, AHEAD)                                                                                                        \
+  attention_f32_kernel<HB, AHEAD><<<grid, block, 0, stream>>>(q, q_stride, k_cache, v_cache, positions, table_rows, block_table, \
+                                                             table_stride, out, out_stride, n_tokens, group, n_kv, page_size, scale, per_tile)
+#define AF_RUN(HB)                \
+  do {                            \
+    if (ahead) AF_GO(HB, true);   \
+    else AF_GO(HB, false);        \
+  } while (0)
   if (head_dim == 32) AF_RUN(2);
   else if (head_dim == 64) AF_RUN(4);
   else if (head_dim == 96) AF_RUN(6);
   else AF_RUN(8);
 #undef AF_RUN
+#undef AF_GO
   GL3_LAUNCH_CHECK();
   return 0;
 }

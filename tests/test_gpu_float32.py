@@ -172,3 +172,27 @@ def test_float32_attention_keeps_nan_scores(lo, hi):
     np.testing.assert_array_equal(got[:, :2], clean[:, :2])
     general, _ = run_attention(lib.attention_generic, sk, sv, qs, [0], [n], H, Kh, hs, "float32", np.random.default_rng(5), window=1 << 20)
     np.testing.assert_array_equal(np.isnan(got), np.isnan(general))
+
+
+# one block a CU (the loads of a step in registers at once) and more: contexts of one step and of several rounds of the eight waves, pages
+# of half a step, of a step and of one and a half, tables no wider than the context
+@pytest.mark.parametrize("page", [32, 64, 96])
+@pytest.mark.parametrize("H, Kh, hs", [(8, 8, 32), (16, 8, 64), (8, 8, 96), (16, 8, 128)])
+def test_float32_attention_is_the_same_with_a_step_s_loads_at_once(H, Kh, hs, page):
+    lib, rng = K(), np.random.default_rng(H + hs + page)
+    before, new = [0, 1100, 31, 500], [520, 3, 33, 17]
+    sk, sv, qs = attention_case(rng, H, Kh, hs, before, new, "float32")
+    sv[1][1101, 0, 0] = np.inf                       # a value that the first of its three tokens does not see
+    calls = []
+
+    def call(q, kc, vc, positions, seq_of, table, out, *rest):
+        lib.attention_generic(q, kc, vc, positions, seq_of, table, out, *rest)
+        calls.append(out.clone())
+        for t in (0, 63, 64, 519, 520, 521, 522, 523, 555, 572):      # (eight blocks; all tokens are hundreds)
+            one = torch.empty_like(out[:1])
+            lib.attention_generic(q[t:t + 1], kc, vc, positions[t:t + 1], seq_of[t:t + 1], table, one, *rest)
+            assert torch.equal(one[0].isnan(), out[t].isnan()) and torch.equal(one[0].nan_to_num(), out[t].nan_to_num()), t
+    got, ref = run_attention(call, sk, sv, qs, before, new, H, Kh, hs, "float32", np.random.default_rng(1), page=page)
+    fine = np.isfinite(ref)
+    assert not fine.all() and np.array_equal(np.isfinite(got), fine)
+    np.testing.assert_allclose(got[fine], ref[fine], atol=2e-5 * np.abs(ref[fine]).max())
