@@ -8,18 +8,19 @@
 // a block being four instructions of which the j-th takes k = 4q + j, q = 0..3; each chunk's sum starts from zero, and
 // the chunks' sums are added in order. (Short chains of sums are also closer to the 64-bit result than one chain of K.)
 //
-// Two kernels, by the number of rows of A:
-// * up to 64 rows (gated 32): bound by the weights' way from memory. A block takes 16 rows of W (gated: 16 gate rows and
+// Three kernels, by the number of rows of A:
+// * up to 64 rows (gated 16 or 32): bound by the weights' way from memory. A block takes 16 rows of W (gated: 16 gate rows and
 //   their 16 up rows) and its sixteen waves a chunk of K each (16 KB of weights); the chunks' sums meet in shared memory.
 //   One row, weights from memory, 1B layers: gate/up 513 -> 29 us (134 MB: 4.6 TB/s), down projection 950 -> 17 us (67 MB:
 //   4.0 TB/s), the head 179 us (5.9 TB/s), against the kernel for any sizes, whose 64 x 64 tiles leave a
 //   product of 2,048 columns 32 blocks that walk K in steps of 16 behind two barriers each. Eight waves a block were 1.0
 //   to 1.3 times as long.
-// * more: bound by the matrix cores (256 flops a clock and CU). Tiles through shared memory in steps of 32 k, two
+// * more, K in no whole steps of 32 (for others see gemm_f32_stream_kernel): bound by the matrix cores (256 flops a clock and CU). Tiles through shared memory in steps of 32 k, two
 //   buffers, one barrier a step; rows in shared memory are 36 floats apart, so that the sixteen lanes that read 16 bytes of
 //   sixteen rows meet all 64 banks once. 4,096 x 4,096 x 4,096: 1.15 ms, 119 TFLOP/s (157 is the unit's peak); 513 rows of
 //   the 1B layers: 57 to 92 TFLOP/s against about 20.
 #include "common.h"
+#include "lds_loads.h"
 #include <type_traits>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -180,6 +181,25 @@ __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const floa
   }
 }
 
+// A lane holds four consecutive columns (from n0) of one token (m0) per tile.
+template <int EPI, int TW, int TT>
+__device__ __forceinline__ void f3_finish_tile(float* __restrict__ C, const f32x4 (&total)[TW][TT], int m0, int n0, int M, int N, long ldc, const F3Out& o) {
+#pragma unroll
+  for (int y = 0; y < TT; ++y) {
+    const int m = m0 + y * 16;
+    if (m >= M) continue;
+    float* c = C + (long)m * ldc;
+#pragma unroll
+    for (int x = 0; x < (EPI == F3_GATED ? TW / 2 : TW); ++x) {
+      const int n = n0 + x * 16;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (n + v < N)
+          f3_finish<EPI>(c + n + v, total[x][y][v], total[EPI == F3_GATED ? TW / 2 + x : x][y][v], n + v, N, o);
+    }
+  }
+}
+
 // ---- many rows: four waves, 2 x 2, a wave owns 16 * TW rows of W by 16 * TT tokens
 #define F3_BK 32
 #define F3_LD (F3_BK + 4)
@@ -279,27 +299,128 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
     }
     __syncthreads();
   }
-  // a lane holds four consecutive columns of one token per tile
+  f3_finish_tile<EPI, TW, TT>(C, total, m0 + wt * 16 * TT + r, n0 + ww * (EPI == F3_GATED ? 8 : 16) * TW + q * 4, M, N, ldc, o);
+}
+
+// ---- many rows, K in whole steps of 32: the same products, operands straight from memory into shared memory
+//
+// The kernel above keeps one step of operands in registers on the way to shared memory; behind its barrier every wave then waits for
+// its reads with little else in flight. Here a block asks for steps ahead (STAGES - 1 of them), no wave writes shared memory, and what a
+// tile needs of it is small enough for several blocks a CU, of which one multiplies while another waits. The kernel above and this one at
+// 513 rows of the 1B layers: gate/up 393 -> 292 us (118 TFLOP/s), down 276 -> 212, output 76 -> 58, QKV 91 -> 72; at 4,096 rows gate/up
+// 2,280 -> 1,980 (139 TFLOP/s; the library's own product of 8,192 cubed reaches 153). What bounds the small ones: whole tiles of 32 rows
+// and whole rounds of the chip's 256 CUs. Rows in shared memory are 128
+// bytes in eight pieces of 16, piece c of row r at place c ^ (r / 2 % 8): the sixteen rows that sixteen lanes read at one piece meet all
+// banks once. A step is asked for into the place of the step before, behind the barrier that every wave reaches with that step's
+// products issued (its reads have returned); the wait in front of the barrier leaves out the later steps. Steps beyond the last repeat it,
+// so that the counts hold; nothing is in flight when a block ends. Sums as above: the same bits.
+template <int EPI, int TW, int TT, int STAGES>
+__global__ __launch_bounds__(256, 2) void gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                 float* __restrict__ C, int M, int N, int K, long lda,
+                                                                 long ldw, long ldc, int tiles_m, int tiles_n, F3Out o) {
+  constexpr int BN = 32 * TW, BM = 32 * TT, PW = (BN + BM) / 32;       // PW: pieces of 1 KB (8 rows) of a step that a wave brings
+  constexpr int NCOLS = EPI == F3_GATED ? BN / 2 : BN, STAGE = (BN + BM) * 128;
+  static_assert(EPI != F3_GATED || TW % 2 == 0, "a wave's tiles are gate rows and their up rows");
+  __shared__ __attribute__((aligned(1024))) char lds[STAGES * STAGE];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int r = lane & 15, q = lane >> 4;
+  const int ww = wave & 1, wt = wave >> 1;
+  const int n_tiles = tiles_m * tiles_n, per_xcd = (n_tiles + 7) / 8;          // (block -> tile as above)
+  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (tile >= n_tiles) return;
+  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * NCOLS;
+  const int steps = K / F3_BK;
+
+  const i32x4 a_buf = mf_rsrc(A + (long)m0 * lda), w_buf = mf_rsrc(W + (long)n0 * ldw);
+  unsigned from[PW];
 #pragma unroll
-  for (int y = 0; y < TT; ++y) {
-    const int m = m0 + wt * 16 * TT + y * 16 + r;
-    if (m >= M) continue;
-    float* c = C + (long)m * ldc;
-#pragma unroll
-    for (int x = 0; x < (EPI == F3_GATED ? TW / 2 : TW); ++x) {
-      const int n = n0 + ww * (EPI == F3_GATED ? 8 : 16) * TW + x * 16 + q * 4;
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (n + v < N)
-          f3_finish<EPI>(c + n + v, total[x][y][v], total[EPI == F3_GATED ? TW / 2 + x : x][y][v], n + v, N, o);
+  for (int i = 0; i < PW; ++i) {
+    const int piece = i * 4 + wave, row = piece * 8 + (lane >> 3);             // (rows of W, then rows of A)
+    const int at = ((lane & 7) ^ ((row >> 1) & 7)) * 4;
+    if (i * 4 * 8 < BN) {
+      int n = n0 + row;
+      if (EPI == F3_GATED) {       // (a wave's rows: TW / 2 tiles of gate rows, then the up rows of the same columns)
+        const int sec = row / (16 * TW), in = row % (16 * TW);
+        n = min(n0 + sec * 8 * TW + in % (8 * TW), N - 1) + (in >= 8 * TW ? N : 0);
+      } else {
+        n = min(n, N - 1);
+      }
+      from[i] = (unsigned)((long)(n - n0) * ldw + at) * 4;
+    } else {
+      from[i] = (unsigned)((long)(min(m0 + row - BN, M - 1) - m0) * lda + at) * 4;
     }
   }
+  const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)lds + wave * 1024;
+  auto load = [&](int t, int place) {
+    const unsigned step = (unsigned)min(t, steps - 1) * (F3_BK * 4);
+#pragma unroll
+    for (int i = 0; i < PW; ++i) mf_dma16(lds0 + place * STAGE + i * 4096, from[i], i * 4 * 8 < BN ? w_buf : a_buf, step);
+  };
+
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[TW][TT], total[TW][TT];
+#pragma unroll
+  for (int a = 0; a < TW; ++a)
+#pragma unroll
+    for (int b = 0; b < TT; ++b) acc[a][b] = total[a][b] = zero;
+  const int twist = (r >> 1) & 7;
+  const char* w_at = lds + (ww * 16 * TW + r) * 128;
+  const char* a_at = lds + (BN + wt * 16 * TT + r) * 128;
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t) load(t, t);
+  for (int t = 0, here = 0, there = STAGES - 1; t < steps; ++t) {
+    mf_wait_loads<(STAGES - 2) * PW>();
+    mf_barrier();
+    load(t + STAGES - 1, there);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      f32x4 w[TW], a[TT];
+      const int c = ((kb * 4 + q) ^ twist) << 4;
+#pragma unroll
+      for (int i = 0; i < TW; ++i) w[i] = *(const f32x4*)(w_at + here * STAGE + i * 2048 + c);
+#pragma unroll
+      for (int i = 0; i < TT; ++i) a[i] = *(const f32x4*)(a_at + here * STAGE + i * 2048 + c);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < TW; ++x)
+#pragma unroll
+          for (int y = 0; y < TT; ++y)
+            acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[x][j], a[y][j], acc[x][y], 0, 0, 0);
+    }
+    if ((t + 1) % (F3_CHUNK / F3_BK) == 0 || t + 1 == steps) {
+#pragma unroll
+      for (int x = 0; x < TW; ++x)
+#pragma unroll
+        for (int y = 0; y < TT; ++y) {
+          total[x][y] += acc[x][y];
+          acc[x][y] = zero;
+        }
+    }
+    there = here;
+    here = here + 1 == STAGES ? 0 : here + 1;
+  }
+  mf_wait_loads<0>();
+  f3_finish_tile<EPI, TW, TT>(C, total, m0 + wt * 16 * TT + r, n0 + ww * (EPI == F3_GATED ? 8 : 16) * TW + q * 4, M, N, ldc, o);
 }
 
 template <int EPI, int TM, bool PAIRS = false>
 static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
                        const F3Out& o, hipStream_t stream) {
   gemm_f32_rows_kernel<EPI, TM, PAIRS><<<dim3(PAIRS ? (N + 7) / 8 : (N + 15) / 16), dim3(64 * F3_WAVES), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, o);
+  GL3_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int EPI, int TW, int TT, int STAGES>
+static int launch_stream(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
+                         const F3Out& o, hipStream_t stream) {
+  const int ncols = EPI == F3_GATED ? 16 * TW : 32 * TW;
+  const int tiles_m = (M + 32 * TT - 1) / (32 * TT), tiles_n = (N + ncols - 1) / ncols;
+  const long blocks = ((long)tiles_m * tiles_n + 7) / 8 * 8;
+  GL3_REQUIRE(blocks < (1L << 31), "gl3_gemm_generic: too many tiles");
+  gemm_f32_stream_kernel<EPI, TW, TT, STAGES><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, tiles_m,
+                                                                                               tiles_n, o);
   GL3_LAUNCH_CHECK();
   return 0;
 }
@@ -322,11 +443,46 @@ static int launch_tile(const float* A, const float* W, float* C, int M, int N, i
 // 8,192: 25.7 -> 16.7 us; K = 2,048: 8.1 -> 9.3 us (half of the waves find no pair of chunks); 3,072 columns, K = 8,192: 28.6 and 29.1.
 static bool f32_pairs(int M, int N, int K) { return M <= 8 && N <= 2048 && K > F3_CHUNK * F3_WAVES; }
 
+// What gemm_f32_stream_kernel is built for: whole steps of 32 k, rows of A in whole 16-byte pieces, and byte offsets of 31 bits inside a
+// tile's rows of A (128 at most) and of W (gated: the up rows lie N behind the gate rows).
+static bool f32_streams(const void* A, int N, int K, long lda, long ldw, bool gated) {
+  return K % F3_BK == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 && 128 * lda * 4 < (1L << 31) && ((gated ? (long)N : 0) + 128) * ldw * 4 < (1L << 31);
+}
+// Its tile: 1 to 4: 128 rows of W x 128 tokens, 128 x 64, 64 x 64, 64 x 32; 5: 32 x 32 (not gated). As in gl3_f32_shape: one tile alone
+// on a CU takes `alone`, a CU with several `each` a tile (us for K = 2,048, both measured; of 108 products of 17 to 4,096 rows
+// one was more than 10% from the best of the five tiles).
+extern "C" int gl3_f32_stream_shape(int M, int N, int gated) {
+  static const int bn[5] = {128, 128, 64, 64, 32}, bm[5] = {128, 64, 64, 32, 32};
+  static const float alone[5] = {144, 80, 45.5f, 28.6f, 20.5f}, each[5] = {124.4f, 62.5f, 33.4f, 17.7f, 11.f};
+  int best = 4;
+  float least = 0.f;
+  for (int i = 0; i < (gated ? 4 : 5); ++i) {
+    const long tiles = (long)((M + bm[i] - 1) / bm[i]) * (((gated ? 2L : 1L) * N + bn[i] - 1) / bn[i]);
+    const float cu = (float)((tiles + 255) / 256) * each[i], cost = cu < alone[i] ? alone[i] : cu;
+    if (i == 0 || cost < least) {
+      least = cost;
+      best = i + 1;
+    }
+  }
+  return best;
+}
+
 template <int EPI>
 static int launch_f32(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
                       const F3Out& o, hipStream_t stream) {
 #define F3_ARGS A, W, C, M, N, K, lda, ldw, ldc, o, stream
   int shape = gl3_f32_shape(M, N, EPI == F3_GATED);
+  // (gated products of 17 to 32 rows too: 1B layers' gate/up 35 us with the kernel for few rows, 29 in tiles of 64 x 32)
+  if ((shape != 1 || (EPI == F3_GATED && M > 16)) && f32_streams(A, N, K, lda, ldw, EPI == F3_GATED)) {
+    switch (gl3_f32_stream_shape(M, N, EPI == F3_GATED)) {
+      case 1: return launch_stream<EPI, 4, 4, 2>(F3_ARGS);
+      case 2: return launch_stream<EPI, 4, 2, 2>(F3_ARGS);
+      case 3: return launch_stream<EPI, 2, 2, 3>(F3_ARGS);
+      case 5:
+        if constexpr (EPI != F3_GATED) return launch_stream<EPI, 1, 1, 4>(F3_ARGS);
+      default: return launch_stream<EPI, 2, 1, 3>(F3_ARGS);
+    }
+  }
   if (shape == 1 && ((long)(M - 1) * lda + K) * 4 >= (1L << 31)) shape = 5;      // (a descriptor's 31 bits)
   switch (shape) {
     case 1:

@@ -108,6 +108,7 @@ def _declare(lib):
         "gl3_token_facts": [P, P, P, I, I, P, P, I, P, P, P, I, P],
         "gl3_gemm_mfma": [P, P, P, I, I, I, I, L, L, L, I, I, P, L, L, P, I, I, I, P, F, F, P, P],
         "gl3_f32_shape": [I, I, I],
+        "gl3_f32_stream_shape": [I, I, I],
         "gl3_attention_decode_supports": [I, I],
         "gl3_attention_prefill_supports": [I, I],
         "gl3_attention_prefill": [P, L, P, P, P, P, P, P, I, P, L, I, I, I, I, I, I, I, F, I, P, I, F, I, I, I, P, F, F, I, P, L, I, I, P, P, P],

@@ -97,6 +97,38 @@ def test_float32_products_in_every_tile(tile, gated, M, N, Kd):
         assert torch.equal(one[0], out[r, :N])
 
 
+# every tile over whole steps of 32 k (1: 128 rows of W x 128 tokens, 2: 128 x 64, 3: 64 x 64, 4: 64 x 32, 5: 32 x 32), one row and one column
+# beyond whole tiles; K of a step (fewer than are asked for ahead), of a chunk and a step, of eight chunks
+@pytest.mark.parametrize("Kd", [32, 288, 2048])
+@pytest.mark.parametrize("tile, gated, M, N", [(1, False, 2049, 3585), (2, False, 1025, 3585), (3, False, 513, 3073), (4, False, 513, 2049), (5, False, 65, 257),
+                                               (1, True, 1153, 3073), (2, True, 513, 8193), (3, True, 769, 1025), (4, True, 17, 65), (4, True, 97, 130)])
+def test_float32_products_in_every_tile_of_whole_steps(tile, gated, M, N, Kd):
+    lib = K()
+    assert lib.library().gl3_f32_stream_shape(M, N, int(gated)) == tile
+    gen = torch.Generator(device="cuda").manual_seed(M + Kd)
+    A, W = (torch.randn(n, Kd, generator=gen, device="cuda") for n in (M, 2 * N if gated else N))
+    wide = torch.zeros(M + 1, Kd + 4, device="cuda")           # rows of A apart; the same rows at an odd float: the other kernel
+    wide[:M, :Kd] = A
+    odd = torch.empty(M * (Kd + 1) + 1, device="cuda")[1:].view(M, Kd + 1)[:, :Kd]
+    odd.copy_(A)
+    out, other = torch.full((M, N + 1), -7.0, device="cuda"), torch.empty(M, N, device="cuda")
+    epilogue = lib.EPI_GATED if gated else lib.EPI_STORE
+    lib.gemm_generic(wide[:M, :Kd], W, out[:, :N], epilogue)
+    lib.gemm_generic(odd, W, other, epilogue)
+    assert torch.all(out[:, N] == -7.0) and torch.equal(out[:, :N], other)       # the same sums in the same order
+    if not gated:
+        off = (256 + Kd / 256 + 2) * 2.0 ** -24 * (A.double().abs() @ W.double().abs().T)        # (as in ``bound``)
+        assert ((out[:, :N] - A.double() @ W.double().T).abs() <= off).all()
+        x = torch.randn(M, N, generator=gen, device="cuda")
+        want = x + out[:, :N]
+        lib.gemm_generic(A, W, x, lib.EPI_ADD)
+        assert torch.equal(x, want)
+    one = torch.empty(1, N, device="cuda")
+    for r in (0, 15, M // 2, M - 2, M - 1):
+        lib.gemm_generic(A[r:r + 1], W, one, epilogue)
+        assert torch.equal(one[0], out[r, :N])
+
+
 def test_float32_products_keep_small_numbers_and_infinities():
     lib = K()
     a, w = np.zeros((20, 64), np.float32), np.zeros((32, 64), np.float32)
