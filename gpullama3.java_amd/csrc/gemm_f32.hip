@@ -64,7 +64,13 @@ __device__ __forceinline__ f32x4 f3_load_a(__amdgpu_buffer_rsrc_t buf, unsigned 
 // PAIRS (at most 8 rows of A, one tile): strips of 8 rows of W. A tile's rows 8..15 are the same rows of W one chunk of K further and
 // its token columns 8..15 the same tokens there, so that a product of the two works out two chunks at once, in its two diagonal
 // quarters; every element's sum is the same sum.
-template <int EPI, int TM, bool PAIRS = false>
+//
+// FRONT (one tile of tokens): eight blocks of 16 k are asked for, weights and rows, before the first product. Left to itself the compiler has four
+// to six loads on their way (43 to 58 registers), which suits products of many blocks, whose waves are in different places; where the
+// blocks are at most one a CU all waves start together and the trips to memory add up. One row, weights from memory: 2,048 x 2,048 8.9 ->
+// 8.2 us, 3,072 x 2,048 10.3 -> 8.9, 2,048 x 8,192 17.9 -> 17.1; 128,256 x 2,048 188 -> 224. From 8 rows on it is ahead with more blocks too
+// (the rows' loads are as many as the weights'): gated 14,336 x 4,096, 8 rows 114 -> 105 us, one row 100 -> 103.
+template <int EPI, int TM, bool PAIRS = false, bool FRONT = false>
 __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                                       float* __restrict__ C, int M, int N, int K, long lda,
                                                                       long ldw, long ldc, F3Out o) {
@@ -104,9 +110,8 @@ __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const floa
 #pragma unroll
         for (int t = 0; t < TM; ++t) acc[g][t] = zero;
       if (whole) {
-        // a whole chunk: sixteen loads of each operand, unrolled, for the scheduler to send ahead (all of them in front of the
-        // first product was slower: 23.8 -> 27.0 us)
-        constexpr int PART = 16 / G;
+        // a whole chunk: sixteen loads of each operand, unrolled, for the scheduler to send ahead
+        constexpr int PART = FRONT ? 8 : 16 / G;
 #pragma unroll
         for (int p = 0; p < 16; p += PART) {
           f32x4 w[G][PART];
@@ -114,6 +119,20 @@ __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const floa
           for (int b = 0; b < PART; ++b)
 #pragma unroll
             for (int g = 0; g < G; ++g) w[g][b] = *(const f32x4*)(wp[g] + k0 + (p + b) * 16);
+          if (FRONT) {
+            static_assert(!FRONT || TM == 1, "one tile of tokens");
+            f32x4 a[PART];
+#pragma unroll
+            for (int b = 0; b < PART; ++b) a[b] = f3_load_a(a_buf, ao[0], (unsigned)(k0 + (p + b) * 16) * 4);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int b = 0; b < PART; ++b)
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int g = 0; g < G; ++g) acc[g][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[g][b][j], a[b][j], acc[g][0], 0, 0, 0);
+            continue;
+          }
 #pragma unroll
           for (int b = 0; b < PART; ++b) {
 #pragma unroll
@@ -407,7 +426,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_stream_kernel(const float* __
 template <int EPI, int TM, bool PAIRS = false>
 static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
                        const F3Out& o, hipStream_t stream) {
-  gemm_f32_rows_kernel<EPI, TM, PAIRS><<<dim3(PAIRS ? (N + 7) / 8 : (N + 15) / 16), dim3(64 * F3_WAVES), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, o);
+  const dim3 grid(PAIRS ? (N + 7) / 8 : (N + 15) / 16), block(64 * F3_WAVES);
+  const bool front = TM == 1 && (grid.x <= 256 || (grid.x <= 1024 && M >= 8));
+  if (front) gemm_f32_rows_kernel<EPI, TM, PAIRS, TM == 1><<<grid, block, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, o);
+  else gemm_f32_rows_kernel<EPI, TM, PAIRS><<<grid, block, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, o);
   GL3_LAUNCH_CHECK();
   return 0;
 }
