@@ -97,6 +97,7 @@ def _declare(lib):
         "gl3_norm_add_next": [P, P, P, F, I, I, P, F, P, I, P, P, P],
         "gl3_sample": [P, L, P, P, P, P, P, I, I, P, I, P],
         "gl3_sample_work_floats": [I, I],
+        "gl3_sample_host": [P, L, P, P, P, P, P, I, I, P],
         "gl3_argmax": [P, L, P, P, I, I, P],
         "gl3_argmax_advance": [P, L, P, P, I, I, P, P, P, P, I, P, P],
         "gl3_argmax_static": [P, L, P, I, I, P],
@@ -1462,6 +1463,24 @@ def sample(logits, work, temperature, top_p, uniform, out, step=None, uniform_st
         _dev(step, "step", torch.int32)
     _check(library().gl3_sample(_ptr(logits), logits.stride(0), _ptr(work), _ptr(temperature), _ptr(top_p),
                                 _ptr(uniform), _ptr(out), R, V, _ptr(step), int(uniform_stride), _stream()), "sample")
+
+
+def sample_host(logits, work, parameters, out):
+    """``sample`` (or, with ``parameters`` None, ``argmax``) of every row, waited for: ``parameters``: three lists of one number a row
+    (temperatures, top-p, uniforms) in host memory; ``out``: int32 in pinned host memory, written when the call returns.
+    ``work``: ``sample_work_size`` floats and three a row."""
+    _dev(logits, "logits", torch.float32, contiguous=False); _dev(work, "work", torch.float32)
+    R, V = logits.shape
+    if logits.stride(1) != 1 or work.numel() < sample_work_size(R, V) + 3 * R or out.numel() < R:
+        raise KernelError("sample: argument sizes")
+    if out.dtype != torch.int32 or not out.is_contiguous() or not out.is_pinned():
+        raise KernelError("sample: the tokens go to contiguous int32 in pinned host memory")
+    par = (None, None, None)
+    if parameters is not None:
+        if any(len(p) < R for p in parameters):
+            raise KernelError("sample: argument sizes")
+        par = [(ctypes.c_float * R)(*p[:R]) for p in parameters]
+    _check(library().gl3_sample_host(_ptr(logits), logits.stride(0), _ptr(work), *par, _ptr(out), R, V, _stream()), "sample")
 
 
 # ------------------------------------------------------------------ bfloat16 product for few rows

@@ -92,12 +92,14 @@ class DeviceSampler:
         R, V = logits.shape
         if R == 0:
             return []
-        if self._work is None or self._work.numel() < K.sample_work_size(R, V):
-            self._work = torch.empty(K.sample_work_size(R, V), dtype=torch.float32, device=self.device)
-        out = torch.empty(R, dtype=torch.int32, device=self.device)
-        if all(t == 0 for t in temperatures):           # every row greedy: the rows are read by many blocks at once
-            K.argmax(logits, self._work, out)
-            return out.tolist()
-        par = torch.tensor([list(temperatures), list(top_ps), list(uniforms)], dtype=torch.float32).to(self.device)
-        K.sample(logits, self._work, par[0], par[1], par[2], out)
+        n = K.sample_work_size(R, V) + 3 * R
+        if self._work is None or self._work.numel() < n:
+            self._work = torch.empty(n, dtype=torch.float32, device=self.device)
+        out = torch.empty(R, dtype=torch.int32, pin_memory=True)      # (a call's own: another thread's call may run beside this one)
+        parameters = None
+        if not all(t == 0 for t in temperatures):       # (every row greedy: the rows are read by many blocks at once)
+            parameters = [[float(x) for x in p] for p in (temperatures, top_ps, uniforms)]
+            if len({len(p) for p in parameters}) != 1:
+                raise ValueError("as many temperatures as top-p and uniform numbers")
+        K.sample_host(logits, self._work, parameters, out)
         return out.tolist()
