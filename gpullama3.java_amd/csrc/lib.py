@@ -2054,7 +2054,7 @@ def prefill_turns_splits(n_heads, n_kv, head_dim, page_size, n_seqs, max_q_len, 
     """Splits on the kernel of turns (heads of 128) where ``prefill_splits`` shares keys out; 0: the other kernel is taken. A CU holds one
     of its blocks (256 queries of a head, or 128 of two where the heads of a kv head pair up), so as many splits as keep the
     blocks within the chip's 256: 512 tokens behind 4,000, 24 heads, 5 splits 49 us, 6 splits (two rounds) 68, the other kernel 64. From
-    2,048 keys on it was the faster one at all of 42 sizes (1.02 to 1.33 times; 200 to 1,100 tokens, 24 and 32 heads), below at 8 of 20.
+    2,048 keys on it was the faster one at all of 48 sizes (1.01 to 1.41 times; 64 to 2,048 tokens, 24 and 32 heads), below at 5 of 20.
     The sums' error against 64 bits is 1.003 times the other kernel's on average (chunks of 64 keys instead of 32 around whose running
     maximum weights are rounded, and fewer splits; 0.97 times that without splits still)."""
     if head_dim != 128 or page_size % 64 or n_seqs > 64 or max_kv_len < PREFILL_TURNS_KEYS:
