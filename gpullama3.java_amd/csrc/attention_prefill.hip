@@ -601,11 +601,16 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
 // SIMD. A wave's two turns for chunk i:
 //   matrix turn i:  scores of chunk i, then the values of chunk i - 1 with its weights
 //   vector turn i:  weights of chunk i, the output brought to the new maximum, the first keys of chunk i + 1 read ahead
+// The sums are those of the kernel above (chunks of 32 keys there), the same bits: each half of a chunk has its own running maximum
+// around which its weights are rounded, the output is brought to the second half's between the values of the two (rarely: only where
+// that maximum moved), weights are added up in the order of the keys, and a half that none of a wave's queries sees is left out. One maximum
+// for a whole chunk was 2 to 3% faster and its error against 64 bits up to 1.006 times as large.
 // Group 0 has matrix turn i in turn 2 i, group 1 in turn 2 i + 1. What bounds it now: the vector instructions of both waves together with
-// the matrix instructions (a turn takes 1,650 cycles; vector instructions and matrix cores overlap to two thirds at best in a kernel
-// of nothing else). With heads of 64, whose matrix part is half as long, the same loop was no faster than the kernel above
+// the matrix instructions. With heads of 64, whose matrix part is half as long, such a loop was no faster than the kernel above
 // (8,192 tokens 345 and 341 us) and is not built.
-// 32 heads, one sequence: 2,048 tokens 78 -> 61 us, 4,096 175 -> 141, 8,192 632 -> 520, 16,384 2,370 -> 1,930 (1.14 PFLOP/s).
+// 32 heads, one sequence, the kernel above and this one: 2,048 tokens 75 -> 61 us, 4,096 172 -> 143, 8,192 608 -> 520, 16,384 2,325 -> 1,956
+// (1.12 PFLOP/s). Nor has it splits: one block a CU, so that as many splits as the kernel above has are two rounds of the chip (512 tokens
+// behind 4,000, 24 heads, 6 splits 68 against 64 us), and fewer splits are longer sums.
 //
 // HEADS = 2: a block is 128 queries of two heads of one kv head, a group of waves to a head; HEADS = 1: 256 queries of one head.
 //
@@ -619,12 +624,12 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
 //
 // Score tile: rows 0..15 are the cache's first tile of 32 keys, rows 16..31 the second, so that register 4 a + b of lane (n, h)
 // is key 16 (a % 2) + 8 h + 4 (a / 2) + b: eight consecutive keys of each half, as the second product takes them.
-template <int HEADS, bool SPLIT>
+template <int HEADS>
 __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
     const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ cu_seqlens, const int* __restrict__ kv_before, const int* __restrict__ block_table,
     const int* __restrict__ seq_rows, int table_stride, bf16_t* __restrict__ out, long out_stride, int n_heads, int n_kv, int page_size,
-    float scale, int q_blocks, int n_seqs, PfSplit sp) {
+    float scale, int q_blocks, int n_seqs) {
   constexpr int HS = 128, CK = 64, KS = HS / 16, DT = HS / 32, QB = 256 / HEADS;
   constexpr int KB = CK * HS * 2;                  // bytes of a chunk's keys (and of its values)
   constexpr int STAGE = 2 * KB, STAGES = 4, AHEAD = STAGES - 1;
@@ -653,8 +658,7 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
     for (; left > 0; --left) here &= here - 1;
     b = __builtin_ctzl(here);
   }
-  const int g = n_heads / n_kv, per_split = n_heads / HEADS;
-  const int split = SPLIT ? blockIdx.x / per_split : 0, at = SPLIT ? blockIdx.x % per_split : blockIdx.x;
+  const int g = n_heads / n_kv, at = blockIdx.x;
   const int c = at % n_kv;                         // (blocks of one kv head are n_kv apart: on one XCD where n_kv is 8)
   const int group = wave >> 2;
   const int head = c * g + at / n_kv * HEADS + (HEADS == 2 ? group : 0);
@@ -665,31 +669,25 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
   const int before = __builtin_amdgcn_readfirstlane(kv_before[b]);
   const int* bt = block_table + (long)(seq_rows ? __builtin_amdgcn_readfirstlane(seq_rows[b]) : b) * table_stride;
   const int blk_last = before + min(qb * QB + QB - 1, q_len - 1);
-  int ck0 = 0, ck1 = blk_last / CK;
-  if (SPLIT) {
-    const int all = ck1 + 1;
-    ck0 = all * split / sp.splits;
-    ck1 = all * (split + 1) / sp.splits - 1;       // (no chunk: the block leaves a weight of nothing)
-  }
-  const int chunks = ck1 - ck0 + 1;
+  const int ck1 = blk_last / CK, chunks = ck1 + 1;
   const int qi0 = qb * QB + (HEADS == 2 ? (wave & 3) * 32 : wave * 32);
   const bool active = qi0 < q_len;
   const bool q_ok = qi0 + n < q_len;
   const int p_mine = before + qi0 + n;
   const int p_last = before + min(qi0 + 31, q_len - 1), p_first = before + qi0;
-  // the wave's chunks, counted from the block's first: later ones hold no key that one of its queries sees
-  int my_first = 0, my_last = active ? min(p_last / CK, ck1) - ck0 : -1;
-  if (my_first > my_last) {
-    my_first = chunks;
-    my_last = -1;
-  }
+  // the wave's chunks: later ones hold no key that one of its queries sees, nor does the last one's second half if its queries end in
+  // the first
+  const int my_last = active ? p_last / CK : -1;
+  const bool half = (p_last & 32) == 0;
 
   const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
   bf16x8 qt[KS];
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk)
     qt[kk] = q_ok ? *(const bf16x8*)(q + (long)(tok0 + qi0 + n) * q_stride + (long)head * HS + kk * 16 + 8 * h) : zero8;
-  float m_run = -INFINITY, l_run = 0.f, alpha = 1.f;      // (alpha: what the output so far is still to be multiplied with)
+  // alpha, beta: what the sums so far are multiplied with in front of the last chunk's first and second half
+  float m_run = -INFINITY, l_run = 0.f, alpha = 1.f, beta = 1.f;
+  bool moved = false;              // (some query's maximum in the second half)
   f32x16 o[DT], s[2], w[2];      // (w: the weights of the last chunk, in the order of its keys)
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -700,7 +698,7 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
   // where chunks lie, sixty-four of them in a register (a lane one): keys in units of a chunk, values in units of 1,024 elements
   const int per_page = page_size / CK, v_units = per_page * (HS / 16);
   auto places = [&](int first, int& k_at, int& v_at) {
-    const int ck = max(ck0, min(ck0 + first + lane, ck1)), entry = ck / per_page, in_page = ck - entry * per_page;
+    const int ck = min(first + lane, ck1), entry = ck / per_page, in_page = ck - entry * per_page;
     const int row = bt[entry] * n_kv + c;
     k_at = row * per_page + in_page;
     v_at = row * v_units + in_page;
@@ -751,8 +749,9 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
   auto matrix_turn = [&](int i, auto with_scores, auto with_values) {
     constexpr bool QK = decltype(with_scores)::value, PV = decltype(with_values)::value;
     constexpr int K_COUNT = QK ? NK : 0, COUNT = K_COUNT + (PV ? NV : 0), BEFORE = QK ? NK : 1;
+    static_assert(NV == 16, "beside an instruction of the values a weight of either half");
     f32x16 zero;
-    float sum[4];
+    float sum[2];
 #pragma unroll
     for (int v = 0; v < 16; ++v) zero[v] = 0.f;
     auto prepare = [&](int m) {                    // (the m-th of BEFORE parts)
@@ -768,6 +767,13 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
 #pragma unroll
     for (int m = 0; m < COUNT; ++m) {
       const int at = m - K_COUNT;
+      if (PV && at == NV / 2) {                    // the second half's values: its maximum may be another
+        if (!QK && half) break;
+        if (moved) {
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) o[dt] *= beta;
+        }
+      }
       if (m < K_COUNT) s[m & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[m % RING], qt[m >> 1], m < 2 ? zero : s[m & 1], 0, 0, 0);
       else o[at % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[m % RING], pb[at / DT >> 1][at / DT & 1], o[at % DT], 0, 0, 0);
       if (m + 8 < K_COUNT) read_k(i, m + 8);
@@ -775,16 +781,24 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
       if (m == 1) load_v(i + AHEAD - 1);
       if (m == 3) load_k(i + AHEAD);
       if (PV && m < K_COUNT) prepare(m);
-      if (m >= K_COUNT) {
+      if (m >= K_COUNT && QK) {
 #pragma unroll
-        for (int e = at * (32 / NV); e < (at + 1) * (32 / NV); ++e)      // (four chains)
-          sum[e & 3] = e < 4 ? w[e >> 4][e & 15] : sum[e & 3] + w[e >> 4][e & 15];
-        if (at * (32 / NV) >= 4) asm volatile("" : "+v"(sum[0]), "+v"(sum[1]), "+v"(sum[2]), "+v"(sum[3]));      // (here, not at the end)
+        for (int t = 0; t < 2; ++t) sum[t] = at == 0 ? w[t][0] : sum[t] + w[t][at];
+        if (at) asm volatile("" : "+v"(sum[0]), "+v"(sum[1]));      // (here, not at the end)
       }
       __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_s_setprio(0);
-    if (PV) l_run = l_run * alpha + ((sum[0] + sum[1]) + (sum[2] + sum[3]));
+    if (PV) {
+      if (!QK) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) sum[t] = e == 0 ? w[t][0] : sum[t] + w[t][e];
+      }
+      l_run = l_run * alpha + sum[0];
+      l_run = l_run * beta + sum[1];
+    }
   };
 
   const float c2 = scale * 1.4426950408889634f;    // scores in units of log2
@@ -805,36 +819,43 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
           s[t][reg(e)] = key <= p_mine ? s[t][reg(e)] : -INFINITY;
         }
     }
-    // (four chains: one would wait for itself, with no other wave of the SIMD at its softmax; the instruction by name, because
+    // (two chains a half: one would wait for itself, with no other wave of the SIMD at its softmax; the instruction by name, because
     // fmaxf of a matrix instruction's results costs one more for each pair to quieten NaNs)
-    float top[4];
+    float top[2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int v0 = (u & 1) * 8;
-      top[u] = max3(s[u >> 1][v0], s[u >> 1][v0 + 1], s[u >> 1][v0 + 2]);
-      top[u] = max3(top[u], s[u >> 1][v0 + 3], s[u >> 1][v0 + 4]);
-      top[u] = max3(top[u], s[u >> 1][v0 + 5], s[u >> 1][v0 + 6]);
+    for (int t = 0; t < 2; ++t) {
+      float u[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        u[k] = max3(s[t][8 * k], s[t][8 * k + 1], s[t][8 * k + 2]);
+        u[k] = max3(u[k], s[t][8 * k + 3], s[t][8 * k + 4]);
+        u[k] = max3(u[k], s[t][8 * k + 5], s[t][8 * k + 6]);
+      }
+      top[t] = max3(max3(u[0], u[1], s[t][7]), s[t][15], s[t][15]);
     }
-    float mx = max3(max3(top[0], top[1], s[0][7]), max3(top[2], top[3], s[0][15]), max3(s[1][7], s[1][15], s[1][15]));
-    {   // the other half of the keys of this query sits 32 lanes away
-      auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-      mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    {   // the other half of the keys of this query sits 32 lanes away: the greatest of either half of the chunk
+      auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(top[0]), __float_as_uint(top[1]), false, false);
+      const float mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * c2;      // c2 > 0: the greatest score stays the greatest
+      r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      top[0] = __uint_as_float(r[0]);
+      top[1] = __uint_as_float(r[1]);
     }
-    mx *= c2;                                      // c2 > 0: the greatest score stays the greatest
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    const float m_mid = fmaxf(m_run, top[0]), m_new = fmaxf(m_mid, top[1]);
+    const float use_mid = m_mid == -INFINITY ? 0.f : m_mid, use_new = m_new == -INFINITY ? 0.f : m_new;
+    alpha = __builtin_amdgcn_exp2f(m_run - use_mid);
+    beta = __builtin_amdgcn_exp2f(m_mid - use_new);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) w[t][e] = __builtin_amdgcn_exp2f(fmaf(s[t][reg(e)], c2, -m_use));
+      for (int e = 0; e < 16; ++e) w[t][e] = __builtin_amdgcn_exp2f(fmaf(s[t][reg(e)], c2, t ? -use_new : -use_mid));
     m_run = m_new;
+    moved = !__all(beta == 1.0f);
     if (!__all(alpha == 1.0f)) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
     }
     // (the compiler would work the weights out where the next turn first takes them, behind the barrier)
-    asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(alpha), "+v"(m_run));
+    asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(alpha), "+v"(beta), "+v"(m_run));
   };
 
 #pragma unroll
@@ -857,14 +878,7 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
   };
   if (group == 1) end_vector();                    // the second group runs a turn behind
   int i = 0;
-  for (; i < my_first; ++i) {
-    load_v(i + AHEAD - 1);
-    load_k(i + AHEAD);
-    end_matrix();
-    locate(i + 1 + AHEAD);
-    end_vector();
-  }
-  if (my_first <= my_last) {                       // (one body for all chunks: where bodies meet the compiler copies the sums)
+  if (my_last >= 0) {                              // (one body for all chunks: where bodies meet the compiler copies the sums)
 #pragma unroll
     for (int m = 0; m < 8; ++m) read_k(i, m);
     matrix_turn(i, std::true_type{}, std::false_type{});
@@ -873,13 +887,16 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
       locate(i + 1 + AHEAD);
 #pragma unroll
       for (int m = 0; m < 8; ++m) read_k(i + 1, m);
-      const int key0 = (ck0 + i) * CK;
+      const int key0 = i * CK;
       vector_turn(key0, key0 + CK - 1 > p_first);
       end_vector();
       if (++i > my_last) break;
       matrix_turn(i, std::true_type{}, std::true_type{});
     }
     matrix_turn(i, std::false_type{}, std::true_type{});
+  } else {                                         // (none of the block's rows: its share of the loads, and the barriers)
+    load_v(AHEAD - 1);
+    load_k(AHEAD);
   }
   for (; i < chunks; ++i) {
     end_matrix();
@@ -894,19 +911,6 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
   float l = l_run;
   l += __shfl_xor(l, 32, 64);
   if (!q_ok) return;
-  if (SPLIT) {
-    const long row = ((long)split * sp.n_tokens + tok0 + qi0 + n) * n_heads + head;
-    float* po = sp.o + row * HS + 4 * h;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int a = 0; a < 4; ++a) *(f32x4*)(po + dt * 32 + 8 * a) = f32x4{o[dt][4 * a], o[dt][4 * a + 1], o[dt][4 * a + 2], o[dt][4 * a + 3]};
-    if (h == 0) {
-      sp.ml[row * 2] = m_run;
-      sp.ml[row * 2 + 1] = l;
-    }
-    return;
-  }
   const float inv = 1.0f / l;
   bf16_t* op = out + (long)(tok0 + qi0 + n) * out_stride + (long)head * HS + 4 * h;
 #pragma unroll
@@ -966,19 +970,15 @@ static bool prefill_wide(int head_dim, int n_heads, int n_seqs, int max_q_len) {
   return (long)n_heads * n_seqs * ((max_q_len + 127) / 128) >= 512;
 }
 
-// The kernel of turns: what it is built for, and where it is taken unless the caller says otherwise. Its blocks are longer to start
-// (128 KB of shared memory are filled first) and a CU holds one: 1,024 tokens of one sequence, 24 heads of 128, 35 against 33 us for the
-// kernel of 64 queries a block, 32 heads 35 and 34; 1,280 tokens 41 and 40, 41 and 43; 1,536 tokens 47 and 48, 48 and 53; 2,048 61 and 66,
-// 61 and 78. Several sequences, whose blocks fill the chip: two of 1,024 tokens 38 against 45 us (32 heads), 317, 1,203
-// and 701 tokens 37 against 47 (24 heads); eight of 512 40 against 33 (24 heads) and 45 against 47 (32), 32 of 100 30 against 22.
+// The kernel of turns: what it is built for, and where it is taken instead of the kernel of 128 queries a block (whose bits it gives),
+// unless the caller says otherwise: from 1,024 tokens of the longest sequence on. Its blocks are longer to start (128 KB of shared memory
+// are filled first) and a CU holds one. 32 heads of 128: two sequences of 1,024 tokens 43 -> 36 us, eight of 96 to 1,752 99 -> 89; 24 heads: 317, 1,203 and
+// 701 tokens 46 -> 37, the eight 84 -> 73; but eight of 512 33 -> 39, 32 of 100 21 -> 27.
 #define PF_TURNS -1
 static bool turns_takes(int head_dim, int page_size, int group, int n_seqs, int n_tokens) {
   return head_dim == 128 && page_size % 64 == 0 && (n_seqs == 1 || (n_seqs <= 64 && n_tokens > 0 && n_tokens / (group % 2 ? 256 : 128) + n_seqs <= 65535));
 }
-static bool turns_wanted(int n_heads, int n_seqs, int max_q_len) {
-  const long blocks = (long)n_heads * n_seqs * ((max_q_len + 127) / 128);
-  return max_q_len >= 1280 ? blocks >= 256 : max_q_len >= 1024 && blocks >= 512;
-}
+static bool turns_wanted(int max_q_len) { return max_q_len >= 1024; }
 
 extern "C" int gl3_attention_prefill_supports(int head_dim, int page_size) {
   return (head_dim == 32 || head_dim == 64 || head_dim == 96 || head_dim == 128) && page_size % 32 == 0;
@@ -1029,22 +1029,17 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
   GL3_REQUIRE(splits >= 1 && splits <= PF_SPLITS, "gl3_attention_prefill: %d splits (1 to %d)", splits, PF_SPLITS);
   GL3_REQUIRE(splits == 1 || (part_o && part_ml && n_tokens > 0 && !ruled && !biased && maps == 1 && (uintptr_t)part_o % 16 == 0),
               "gl3_attention_prefill: splits need buffers for their sums and the plain rule (one score map, no bias, sink, kept keys, cap, temperature or gate)");
-  const bool turns_can = turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && !ruled && !biased && maps == 1 && window == 0 && mask_chunk == 0;
-  GL3_REQUIRE(wide_from != PF_TURNS || turns_can, "gl3_attention_prefill: the kernel of turns takes heads of 128, pages of whole 64 keys, at most 64 sequences, the plain rule");
-  if (wide_from == PF_TURNS || (wide_from <= 0 && splits == 1 && turns_can && turns_wanted(n_heads, n_seqs, max_q_len))) {
+  const bool turns_can = turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && splits == 1 && !ruled && !biased && maps == 1 && window == 0 && mask_chunk == 0;
+  GL3_REQUIRE(wide_from != PF_TURNS || turns_can, "gl3_attention_prefill: the kernel of turns takes heads of 128, pages of whole 64 keys, at most 64 sequences, no splits, the plain rule");
+  if (wide_from == PF_TURNS || (wide_from <= 0 && wide && turns_can && turns_wanted(max_q_len))) {
     const int heads = g % 2 == 0 ? 2 : 1, queries = 256 / heads, qbs = (max_q_len + queries - 1) / queries;
-    dim3 tgrid((unsigned)(n_heads / heads) * splits, n_seqs == 1 ? qbs : n_tokens / queries + n_seqs);
-#define GOT(HEADS, SP)                                                                                                \
-  attention_prefill_turns_kernel<HEADS, SP><<<tgrid, dim3(512), 0, stream>>>(                                         \
+    dim3 tgrid((unsigned)(n_heads / heads), n_seqs == 1 ? qbs : n_tokens / queries + n_seqs);
+#define GOT(HEADS)                                                                                                    \
+  attention_prefill_turns_kernel<HEADS><<<tgrid, dim3(512), 0, stream>>>(                                             \
       (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu_seqlens, kv_before, block_table, \
-      seq_rows, table_stride, (bf16_t*)out, out_stride, n_heads, n_kv, page_size, scale, qbs, n_seqs, sp)
-    if (splits > 1) {
-      if (heads == 2) GOT(2, true);
-      else GOT(1, true);
-      const long n = (long)n_tokens * n_heads * (128 / 4);
-      attention_prefill_merge_kernel<128><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(sp, (bf16_t*)out, out_stride, n_heads);
-    } else if (heads == 2) GOT(2, false);
-    else GOT(1, false);
+      seq_rows, table_stride, (bf16_t*)out, out_stride, n_heads, n_kv, page_size, scale, qbs, n_seqs)
+    if (heads == 2) GOT(2);
+    else GOT(1);
 #undef GOT
     GL3_LAUNCH_CHECK();
     return 0;

@@ -2047,21 +2047,6 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len):
 
 
 PREFILL_TURNS = -1                    # ``attention_prefill``'s ``wide_from`` that names the kernel of turns
-PREFILL_TURNS_KEYS = 2048             # splits run on it from this many keys on
-
-
-def prefill_turns_splits(n_heads, n_kv, head_dim, page_size, n_seqs, max_q_len, max_kv_len):
-    """Splits on the kernel of turns (heads of 128) where ``prefill_splits`` shares keys out; 0: the other kernel is taken. A CU holds one
-    of its blocks (256 queries of a head, or 128 of two where the heads of a kv head pair up), so as many splits as keep the
-    blocks within the chip's 256: 512 tokens behind 4,000, 24 heads, 5 splits 49 us, 6 splits (two rounds) 68, the other kernel 64. From
-    2,048 keys on it was the faster one at all of 48 sizes (1.01 to 1.41 times; 64 to 2,048 tokens, 24 and 32 heads), below at 5 of 20.
-    The sums' error against 64 bits is 1.003 times the other kernel's on average (chunks of 64 keys instead of 32 around whose running
-    maximum weights are rounded, and fewer splits; 0.97 times that without splits still)."""
-    if head_dim != 128 or page_size % 64 or n_seqs > 64 or max_kv_len < PREFILL_TURNS_KEYS:
-        return 0
-    heads = 1 if n_heads // n_kv % 2 else 2
-    blocks = n_heads // heads * n_seqs * -(-max_q_len // (256 // heads))
-    return max(1, min(8, 256 // blocks, max_kv_len // 256))
 
 
 def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, out, max_q_len, n_heads, n_kv,
@@ -2072,8 +2057,8 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
     of the packed ``q`` belong to which sequence and where they sit in it. ``seq_rows`` [B] (optional)
     names each sequence's row of ``block_table``; without it sequence b reads row b. ``wide_from``: from
     how many tokens of the step's longest sequence on the kernel with 128 queries a block runs
-    (0: the library's choice; ``PREFILL_TURNS``: the kernel of turns, which takes heads of 128 and the plain rule; tests run all kernels
-    on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
+    (0: the library's choice; ``PREFILL_TURNS``: the kernel of turns, which takes heads of 128 and the plain rule, gives the same bits
+    and has no splits; tests run all kernels on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
     128 queries are shared out over that many blocks of the same kernel, whose sums lie in ``part_o`` (float32, at least
     splits * T * H * hs) and ``part_ml`` (2 * splits * T * H) until a second kernel merges them; the plain rule only."""
     _dev(q, "q", torch.bfloat16, contiguous=False); _dev(out, "out", torch.bfloat16, contiguous=False)

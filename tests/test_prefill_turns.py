@@ -1,5 +1,5 @@
-"""The prefill attention whose two groups of waves take turns (heads of 128): the rule that takes it, and its results against the plain
-reference and the kernels beside it."""
+"""The prefill attention whose two groups of waves take turns (heads of 128): its results against the plain reference and the kernel of
+128 queries a block, whose bits they are."""
 import numpy as np
 import pytest
 import torch
@@ -7,29 +7,13 @@ import torch
 from gpullama3_java_amd.csrc import lib
 
 
-def test_splits_on_the_kernel_of_turns():
-    s = lib.prefill_turns_splits
-    assert s(24, 8, 128, 64, 1, 512, 4512) == 5 and s(32, 8, 128, 64, 1, 512, 4512) == 4          # 48 and 64 blocks
-    assert s(24, 8, 128, 64, 1, 64, 4064) == 8 and s(24, 8, 128, 64, 1, 1100, 7100) == 2 and s(32, 8, 128, 64, 1, 2048, 14048) == 1
-    assert s(24, 8, 128, 64, 1, 300, 2047) == 0 and s(24, 8, 64, 64, 1, 512, 4512) == 0           # few keys; heads of 64
-    assert s(24, 8, 128, 32, 1, 512, 4512) == 0 and s(24, 8, 128, 64, 65, 30, 4512) == 0          # pages of half a chunk; many sequences
-    for heads, kv in ((24, 8), (32, 8), (8, 8), (128, 8), (1, 1)):
-        for n_seqs in (1, 2, 7, 64):
-            for T in (1, 128, 129, 257, 1000, 5000):
-                n = s(heads, kv, 128, 64, n_seqs, T, 100000)
-                assert 1 <= n <= 8 and (n == 1 or n * n_seqs * T * heads <= lib.PREFILL_SPLIT_ROWS)
-
-
-def fn(before, new, wide_from, splits=1):
-    from test_gpu_kernels import DEV, dev
+def fn(before, new, wide_from):
+    from test_gpu_kernels import dev
 
     def call(q, kc, vc, positions, seq_of, table, out, H, Kh, hs, page, window, scale):
         cu = dev(np.concatenate([[0], np.cumsum(new)]), torch.int32)
-        n = splits * len(positions) * H
-        parts = dict(splits=splits, part_o=torch.full((n * hs,), float("nan"), device=DEV),
-                     part_ml=torch.full((2 * n,), float("nan"), device=DEV)) if splits > 1 else {}
         lib.attention_prefill(q, kc, vc, cu, dev(before, torch.int32), table, out, max(new), H, Kh, hs, page, window, scale,
-                              wide_from=wide_from, **parts)
+                              wide_from=wide_from)
     return call
 
 
@@ -40,17 +24,36 @@ CASES = [(4, 2, 64, [0, 70, 0, 130, 5], [33, 1, 200, 17, 64]), (3, 1, 64, [0, 0,
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("splits", [1, 2, 8])
+@pytest.mark.parametrize("sharp", [1, 8])
 @pytest.mark.parametrize("H, Kh, page, before, new", CASES)
-def test_attention_of_turns(H, Kh, page, before, new, splits):
+def test_attention_of_turns(H, Kh, page, before, new, sharp):
     from test_gpu_kernels import attention_case, run_attention
-    sk, sv, qs = attention_case(np.random.default_rng(H * page + splits), H, Kh, 128, before, new, "bfloat16")
+    sk, sv, qs = attention_case(np.random.default_rng(H * page + sharp), H, Kh, 128, before, new, "bfloat16")
+    qs = [q * sharp for q in qs]                     # (8: a few keys have all the weight, and maxima move in all chunks)
     run = lambda f: run_attention(f, sk, sv, qs, before, new, H, Kh, 128, "bfloat16", np.random.default_rng(1), page=page)
-    got, ref = run(fn(before, new, lib.PREFILL_TURNS, splits))
+    got, ref = run(fn(before, new, lib.PREFILL_TURNS))
     np.testing.assert_allclose(got, ref, atol=1e-2 * np.abs(ref).max())
-    other, _ = run(fn(before, new, 1, splits))
-    # (weights are rounded to 16 bits around the running maximum of 64 keys here, of 32 there)
-    np.testing.assert_allclose(got, other, atol=2.0 ** -7 * np.abs(ref).max())
+    other, _ = run(fn(before, new, 1))
+    np.testing.assert_array_equal(got, other)        # (the same sums in the same order as the kernel of 128 queries a block)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at", [0, 31, 32, 63, 64, 95, 1000, 1037, 1038, 1055])
+def test_values_that_are_not_finite_reach_as_far_as_in_the_kernel_beside_it(at):
+    """A weight of zero does not make nothing of an infinite value: it spoils the queries in front of it whose keys share its 32, and
+    what a page still holds behind the sequence's end (here from 1,038 on) likewise; no more than that on either kernel."""
+    from test_gpu_kernels import attention_case, run_attention
+    H, Kh, before, new = 4, 2, [700], [338]
+    sk, sv, qs = attention_case(np.random.default_rng(at), H, Kh, 128, before, [400], "bfloat16")
+    for value in (np.inf, np.nan):
+        sv[0][at, 0, 77] = value
+        run = lambda f: run_attention(f, sk, sv, qs, before, new, H, Kh, 128, "bfloat16", np.random.default_rng(1))[0]
+        got = run(fn(before, new, lib.PREFILL_TURNS))
+        np.testing.assert_array_equal(got, run(fn(before, new, 1)))
+        waves = np.arange(700, 1038) - 700 >> 5      # (32 queries walk their keys together)
+        last = np.minimum(waves * 32 + 731, 1037)
+        assert np.isfinite(got[last // 32 < at // 32]).all() and np.isfinite(got[:, :, :77]).all() and np.isfinite(got[:, 2:]).all()
+        assert not np.isfinite(got[np.arange(700, 1038) >= at, :2, 77]).any()
 
 
 @pytest.mark.gpu
