@@ -802,11 +802,7 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
   };
 
   const float c2 = scale * 1.4426950408889634f;    // scores in units of log2
-  auto max3 = [](float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-  };
+  auto max3 = [](float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); };
   auto vector_turn = [&](int key0, bool masked) {
     // (register of the lane's e-th key of a tile, in the order of the keys; its key)
     auto reg = [](int e) { return (e & 3) + ((e >> 2) & 1) * 8 + (e >> 3) * 4; };
@@ -819,8 +815,8 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
           s[t][reg(e)] = key <= p_mine ? s[t][reg(e)] : -INFINITY;
         }
     }
-    // (two chains a half: one would wait for itself, with no other wave of the SIMD at its softmax; the instruction by name, because
-    // fmaxf of a matrix instruction's results costs one more for each pair to quieten NaNs)
+    // (two chains a half: one would wait for itself, with no other wave of the SIMD at its softmax. v_maximum3, which keeps NaNs: fmaxf of
+    // a matrix instruction's results costs one more for each pair to quieten them. A row with a NaN is NaN by its weights either way)
     float top[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {

@@ -4,7 +4,7 @@ import re
 
 from gpullama3_java_amd.csrc import build
 
-BLOCK = re.compile(r'asm\s+(?:volatile)?\s*\((.*?)\);', re.S)
+BLOCK = re.compile(r'\basm\s*(?:volatile)?\s*\((.*?)\);', re.S)
 
 
 def blocks():
@@ -42,3 +42,10 @@ def test_loads_by_hand_wait_for_their_scalar_operands():
             assert rsrc.count('asm("s_mov_b32 %0, %1"') == rsrc.count("readfirstlane") == 2
             found += 1
     assert found
+
+
+def test_no_vector_instruction_is_written_by_hand():
+    """A vector instruction may read a matrix instruction's result only some wait states after it; the compiler keeps them for its own
+    instructions and does not look into a block."""
+    for where, template, operands in blocks():
+        assert not re.search(r"\bv_\w+", template), (where, template)
