@@ -9,6 +9,7 @@ sequence's tokens do not depend on what else is in its batch.
 """
 from __future__ import annotations
 
+import threading
 from dataclasses import dataclass
 
 import numpy as np
@@ -84,6 +85,7 @@ class DeviceSampler:
         self.device = device
         self._torch = torch
         self._work = None
+        self._lock = threading.Lock()      # (a call's parameters and probabilities lie in `_work` until the call has waited for its tokens)
 
     def __call__(self, logits, temperatures, top_ps, uniforms):
         """logits ``[R, V]`` float32 on the device -> list of R token ids."""
@@ -93,13 +95,14 @@ class DeviceSampler:
         if R == 0:
             return []
         n = K.sample_work_size(R, V) + 3 * R
-        if self._work is None or self._work.numel() < n:
-            self._work = torch.empty(n, dtype=torch.float32, device=self.device)
-        out = torch.empty(R, dtype=torch.int32, pin_memory=True)      # (a call's own: another thread's call may run beside this one)
+        out = torch.empty(R, dtype=torch.int32, pin_memory=True)
         parameters = None
         if not all(t == 0 for t in temperatures):       # (every row greedy: the rows are read by many blocks at once)
             parameters = [[float(x) for x in p] for p in (temperatures, top_ps, uniforms)]
             if len({len(p) for p in parameters}) != 1:
                 raise ValueError("as many temperatures as top-p and uniform numbers")
-        K.sample_host(logits, self._work, parameters, out)
+        with self._lock:                                # (the library lets go of the interpreter: another thread's call would run beside this one)
+            if self._work is None or self._work.numel() < n:
+                self._work = torch.empty(n, dtype=torch.float32, device=self.device)
+            K.sample_host(logits, self._work, parameters, out)
         return out.tolist()

@@ -41,3 +41,23 @@ def test_the_call_from_host_memory_refuses():
             lib.sample_host(*arguments)
     with pytest.raises(ValueError):
         DeviceSampler(torch.device("cuda:0"))(logits, [1.0, 1.0], [1.0], [0.5, 0.5])
+
+
+@pytest.mark.parametrize("own_streams", [False, True])
+def test_calls_of_two_threads(own_streams):
+    from concurrent.futures import ThreadPoolExecutor
+    rng = np.random.default_rng(7)
+    sampler = DeviceSampler(torch.device("cuda:0"))
+    calls = []
+    for rows, temperature in ((300, 0.7), (257, 1.3)):              # (two launches of parameters each; scratch of two sizes)
+        logits = torch.tensor(3 * rng.standard_normal((rows, 1031)), dtype=torch.float32, device="cuda:0")
+        par = ([temperature] * rows, [0.9] * rows, rng.random(rows).tolist())
+        calls.append((logits, par, DeviceSampler(torch.device("cuda:0"))(logits, *par)))
+    torch.cuda.synchronize()
+
+    def calls_of(thread):
+        logits, par, want = calls[thread]
+        with torch.cuda.stream(torch.cuda.Stream() if own_streams else torch.cuda.default_stream()):
+            return sum(sampler(logits, *par) != want for _ in range(100))
+    with ThreadPoolExecutor(2) as threads:
+        assert list(threads.map(calls_of, range(2))) == [0, 0]

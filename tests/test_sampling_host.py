@@ -38,3 +38,31 @@ def test_validation_as_the_reference_options():
     with pytest.raises(ValueError):
         SamplingParams(0.5, 1.5)
     assert select_sampler(100, 0.7, 0.9, 42) == SamplingParams(0.7, 0.9, 42)
+
+
+def test_one_sampler_s_calls_of_several_threads_take_turns(monkeypatch):
+    """A call's parameters and probabilities lie in scratch that the sampler's calls share, while the library runs without the
+    interpreter's lock: the next call waits until this one has its tokens."""
+    import time
+    from concurrent.futures import ThreadPoolExecutor
+    from types import SimpleNamespace
+
+    import torch
+
+    from gpullama3_java_amd.csrc import lib
+    from gpullama3_java_amd.sampling import DeviceSampler
+    monkeypatch.setattr(lib, "sample_work_size", lambda rows, vocab: rows * vocab)
+
+    def sample_host(logits, work, parameters, out):
+        work[:len(out)] = torch.tensor(parameters[2])
+        time.sleep(0.002)
+        out.copy_(work[:len(out)])
+    monkeypatch.setattr(lib, "sample_host", sample_host)
+    sampler = DeviceSampler(torch.device("cpu"))
+    sampler._torch = SimpleNamespace(float32=torch.float32, int32=torch.int32,
+                                     empty=lambda n, dtype, device=None, pin_memory=False: torch.empty(n, dtype=dtype))
+
+    def calls(k):
+        return all(sampler(torch.zeros(2 + k, 5), [1.0] * (2 + k), [0.9] * (2 + k), [k] * (2 + k)) == [k] * (2 + k) for _ in range(10))
+    with ThreadPoolExecutor(4) as threads:
+        assert all(threads.map(calls, range(4)))
