@@ -976,6 +976,14 @@ static bool turns_takes(int head_dim, int page_size, int group, int n_seqs, int 
 }
 static bool turns_wanted(int max_q_len) { return max_q_len >= 1024; }
 
+// The library's choice: 0: 64 queries a block, 1: 128, 2: the kernel of turns. plain: the plain rule (one score map, no window, chunked
+// mask, bias, sink, kept keys, cap, temperature or gate), no splits, caches at 16-byte addresses (its loads into shared memory bring
+// 16 bytes a lane and want them aligned, where the other kernels' ordinary loads do not).
+extern "C" int gl3_prefill_kernel(int head_dim, int page_size, int n_heads, int n_kv, int n_seqs, int max_q_len, int n_tokens, int plain) {
+  if (!prefill_wide(head_dim, n_heads, n_seqs, max_q_len)) return 0;
+  return plain && turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && turns_wanted(max_q_len) ? 2 : 1;
+}
+
 extern "C" int gl3_attention_prefill_supports(int head_dim, int page_size) {
   return (head_dim == 32 || head_dim == 64 || head_dim == 96 || head_dim == 128) && page_size % 32 == 0;
 }
@@ -1007,7 +1015,16 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
   GL3_REQUIRE(q_stride % 8 == 0 && (uintptr_t)q % 16 == 0 && out_stride % 4 == 0 && (uintptr_t)out % 8 == 0,
               "gl3_attention_prefill: queries must be 16-byte aligned, outputs 8-byte aligned");
   const int g = n_heads / n_kv;
-  const bool wide = splits > 1 ? true : wide_from > 0 ? max_q_len >= wide_from : prefill_wide(head_dim, n_heads, n_seqs, max_q_len);
+  const Gl3ScoreRule rule{softcap, temp_coef, temp_every, gate, gate_ld};
+  GL3_CHECK_RULE(rule, "gl3_attention_prefill");
+  const bool ruled = rule.any();
+  const bool biased = slopes != nullptr || has_sink || sinks != nullptr || keep_first > 0;    // (the kernels that know of kept first keys)
+  const bool plain = splits == 1 && !ruled && !biased && maps == 1 && window == 0 && mask_chunk == 0 && (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0;
+  GL3_REQUIRE(wide_from != PF_TURNS || (plain && turns_takes(head_dim, page_size, g, n_seqs, n_tokens)),
+              "gl3_attention_prefill: the kernel of turns takes heads of 128, pages of whole 64 keys, caches at 16-byte addresses, at most 64 sequences, no splits, the plain rule");
+  const int kernel = wide_from == PF_TURNS ? 2 : splits > 1 ? 1 : wide_from > 0 ? max_q_len >= wide_from
+                     : gl3_prefill_kernel(head_dim, page_size, n_heads, n_kv, n_seqs, max_q_len, n_tokens, plain);
+  const bool wide = kernel > 0;
   // query heads per wave: as many as the registers hold with two blocks on a CU; one with 32 queries a wave
   const int gh = wide ? 1 : head_dim <= 32 ? 4 : head_dim <= 64 ? 2 : 1;
   const long z = (long)n_kv * ((g + gh - 1) / gh);
@@ -1016,18 +1033,12 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
               n_seqs, q_blocks);
   dim3 grid((unsigned)z * (splits > 1 ? splits : 1), n_seqs, q_blocks), block(256);
   GL3_REQUIRE(keep_first >= 0 && (keep_first == 0 || window > 0), "gl3_attention_prefill: %d kept first keys without a window", keep_first);
-  const Gl3ScoreRule rule{softcap, temp_coef, temp_every, gate, gate_ld};
-  GL3_CHECK_RULE(rule, "gl3_attention_prefill");
   GL3_REQUIRE(!gate || (gate_ld % 4 == 0 && (uintptr_t)gate % 8 == 0), "gl3_attention_prefill: gate rows must be 8-byte aligned");
-  const bool ruled = rule.any();
-  const bool biased = slopes != nullptr || has_sink || sinks != nullptr || keep_first > 0;    // (the kernels that know of kept first keys)
   const PfSplit sp{splits, n_tokens, part_o, part_ml};
   GL3_REQUIRE(splits >= 1 && splits <= PF_SPLITS, "gl3_attention_prefill: %d splits (1 to %d)", splits, PF_SPLITS);
   GL3_REQUIRE(splits == 1 || (part_o && part_ml && n_tokens > 0 && !ruled && !biased && maps == 1 && (uintptr_t)part_o % 16 == 0),
               "gl3_attention_prefill: splits need buffers for their sums and the plain rule (one score map, no bias, sink, kept keys, cap, temperature or gate)");
-  const bool turns_can = turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && splits == 1 && !ruled && !biased && maps == 1 && window == 0 && mask_chunk == 0;
-  GL3_REQUIRE(wide_from != PF_TURNS || turns_can, "gl3_attention_prefill: the kernel of turns takes heads of 128, pages of whole 64 keys, at most 64 sequences, no splits, the plain rule");
-  if (wide_from == PF_TURNS || (wide_from <= 0 && wide && turns_can && turns_wanted(max_q_len))) {
+  if (kernel == 2) {
     const int heads = g % 2 == 0 ? 2 : 1, queries = 256 / heads, qbs = (max_q_len + queries - 1) / queries;
     dim3 tgrid((unsigned)(n_heads / heads), n_seqs == 1 ? qbs : n_tokens / queries + n_seqs);
 #define GOT(HEADS)                                                                                                    \

@@ -7,6 +7,24 @@ import torch
 from gpullama3_java_amd.csrc import lib
 
 
+def test_the_kernel_of_turns_asks_for_caches_at_16_byte_addresses():
+    """Its loads into shared memory bring 16 bytes a lane. (A call that names it is refused before anything is launched; the library's own
+    choice is another kernel.)"""
+    import ctypes
+    L = lib.library()
+    memory = ctypes.create_string_buffer(4096)
+    at = -(-ctypes.addressof(memory) // 16) * 16
+
+    def call(k, v):
+        p = ctypes.c_void_p
+        return L.gl3_attention_prefill(p(at), 256, p(at + k), p(at + v), p(at), p(at), p(at), None, 1, p(at), 256, 1, 1, 2, 1, 128, 64, 0, 0.1,
+                                       lib.PREFILL_TURNS, None, 0, 0.0, 0, 0, 1, None, 0.0, 0.0, 0, None, 0, 1, 1, None, None, None)
+    for k, v in ((2, 0), (0, 8)):
+        assert call(k, v) != 0 and b"16-byte addresses" in L.gl3_last_error()
+    choice = L.gl3_prefill_kernel
+    assert choice(128, 64, 24, 8, 8, 1752, 5886, 1) == 2 and choice(128, 64, 24, 8, 8, 1752, 5886, 0) == 1          # (0: not plain)
+
+
 def fn(before, new, wide_from):
     from test_gpu_kernels import dev
 
