@@ -967,21 +967,27 @@ static bool prefill_wide(int head_dim, int n_heads, int n_seqs, int max_q_len) {
 }
 
 // The kernel of turns: what it is built for, and where it is taken instead of the kernel of 128 queries a block (whose bits it gives),
-// unless the caller says otherwise: from 1,024 tokens of the longest sequence on. Its blocks are longer to start (128 KB of shared memory
-// are filled first) and a CU holds one. 32 heads of 128: two sequences of 1,024 tokens 43 -> 36 us, eight of 96 to 1,752 99 -> 89; 24 heads: 317, 1,203 and
-// 701 tokens 46 -> 37, the eight 84 -> 73; but eight of 512 33 -> 39, 32 of 100 21 -> 27.
+// unless the caller says otherwise: from 1,024 tokens of the longest sequence on, where those are a fifth of the step's tokens at least
+// or the sequences are long on average. Its blocks are longer to start (128 KB of shared memory are filled first) and a CU holds one: a
+// long sequence is done sooner, many short ones later. Time against the kernel of 128 queries, 24 and 32 heads of 128, one sequence of 1,024 to 8,000 tokens
+// beside 1 to 60 of 20 to 1,000 and random batches (profiles/prefill_turns_rule.txt): from a fifth on 0.59 to 1.03 (330
+// sizes, 0.80 on average); below 0.98 to 1.25 (60 sizes, 1.08 on average; 1,300 tokens and sixty of 100 58 -> 68 us with 24 heads), but six or eight
+// of 1,280 to 2,000 0.92 to 1.01. (What the sequences hold already is not known here: with sixty of 1 to 30 tokens behind 500 beside 1,300
+// or 2,048 24 heads take 1.13 to 1.23 times as long, 32 heads 0.82 to 0.87; behind 4,000 0.89 to 0.99 and 0.58 to 0.64.)
 #define PF_TURNS -1
 static bool turns_takes(int head_dim, int page_size, int group, int n_seqs, int n_tokens) {
   return head_dim == 128 && page_size % 64 == 0 && (n_seqs == 1 || (n_seqs <= 64 && n_tokens > 0 && n_tokens / (group % 2 ? 256 : 128) + n_seqs <= 65535));
 }
-static bool turns_wanted(int max_q_len) { return max_q_len >= 1024; }
+static bool turns_wanted(int n_seqs, int max_q_len, int n_tokens) {
+  return max_q_len >= 1024 && (n_tokens <= 5L * max_q_len || n_tokens >= 1280L * n_seqs);
+}
 
 // The library's choice: 0: 64 queries a block, 1: 128, 2: the kernel of turns. plain: the plain rule (one score map, no window, chunked
 // mask, bias, sink, kept keys, cap, temperature or gate), no splits, caches at 16-byte addresses (its loads into shared memory bring
 // 16 bytes a lane and want them aligned, where the other kernels' ordinary loads do not).
 extern "C" int gl3_prefill_kernel(int head_dim, int page_size, int n_heads, int n_kv, int n_seqs, int max_q_len, int n_tokens, int plain) {
   if (!prefill_wide(head_dim, n_heads, n_seqs, max_q_len)) return 0;
-  return plain && turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && turns_wanted(max_q_len) ? 2 : 1;
+  return plain && turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && turns_wanted(n_seqs, max_q_len, n_tokens) ? 2 : 1;
 }
 
 extern "C" int gl3_attention_prefill_supports(int head_dim, int page_size) {

@@ -25,6 +25,16 @@ def test_the_kernel_of_turns_asks_for_caches_at_16_byte_addresses():
     assert choice(128, 64, 24, 8, 8, 1752, 5886, 1) == 2 and choice(128, 64, 24, 8, 8, 1752, 5886, 0) == 1          # (0: not plain)
 
 
+def test_many_short_sequences_beside_a_long_one_take_the_kernel_of_128_queries():
+    def choice(lengths, heads=24):
+        return lib.library().gl3_prefill_kernel(128, 64, heads, 8, len(lengths), max(lengths), sum(lengths), 1)
+    assert choice([1300] + [100] * 60) == 1 and choice([1300] + [100] * 60, 32) == 1 and choice([2048] + [300] * 31) == 1
+    assert choice([8192], 32) == 2 and choice([4096]) == 2 and choice([8000] + [100] * 60) == 2 and choice([2048] + [20] * 60) == 2
+    assert choice([1752, 96, 1390, 211, 803, 1101, 377, 156]) == 2 and choice([317, 1203, 701]) == 2 and choice([1024] * 2, 32) == 2
+    assert choice([2000] * 8) == 2 and choice([1024] * 8) == 1 and choice([512] * 8) == 1
+    assert choice([2048]) == 0 and choice([1024] * 2) == 0 and choice([100]) == 0           # (too few blocks for either)
+
+
 def fn(before, new, wide_from):
     from test_gpu_kernels import dev
 
