@@ -87,8 +87,10 @@ __global__ __launch_bounds__(64 * AF_WAVES, AHEAD || HB > 4 ? 2 : 4) void attent
         }
         // AHEAD (at most one block a CU): all of a step's keys are asked for before the first is waited for, its values in front of the
         // scores or, where the registers do not hold both, of the softmax. Otherwise the compiler waits for one load after
-        // the other, 32 trips to memory a step, which the other block of a CU hides.
-        constexpr int EARLY = HB > 6 ? HB / 2 : HB;
+        // the other, 32 trips to memory a step, which the other block of a CU hides. With heads of 128 the registers hold half of the keys or
+        // of the values (PART) beside the sums; the other half is asked for when the first is multiplied. (All of them at once went to
+        // scratch memory: 2,000 keys for each of four tokens 73 us, in halves 63, without AHEAD 87; 700 for each of two 30, 25 and 26.)
+        constexpr int PART = HB > 6 ? HB / 2 : HB;
         f32x4 vf[AHEAD ? HB : 1][2][2];
         auto load_values = [&](int d0, int d1) {
 #pragma unroll
@@ -99,20 +101,28 @@ __global__ __launch_bounds__(64 * AF_WAVES, AHEAD || HB > 4 ? 2 : 4) void attent
               for (int e = 0; e < 2; ++e) vf[AHEAD ? d : 0][b][e] = *(const f32x4*)(vp[b] + (((long)d * (page_size >> 3)) << 7) + e * 4);
         };
         f32x4 kf[AHEAD ? HB : 1][2][2];
-        if (AHEAD) {
+        auto load_keys = [&](int d0, int d1) {
 #pragma unroll
-          for (int d = 0; d < HB; ++d)
+          for (int d = d0; d < d1; ++d)
 #pragma unroll
             for (int b = 0; b < 2; ++b)
 #pragma unroll
               for (int e = 0; e < 2; ++e) kf[AHEAD ? d : 0][b][e] = *(const f32x4*)(kp[b] + ((e * (HS >> 3) + d * 2) << 7));
+        };
+        if (AHEAD) {
+          load_keys(0, PART);
           if (HB <= 4) load_values(0, HB);
         }
         if (AHEAD) look_up(min(first + 64 * AF_WAVES, p_max));
         if (AHEAD) __builtin_amdgcn_sched_barrier(0);
         f32x4 s[2][2] = {{zero, zero}, {zero, zero}};
 #pragma unroll
-        for (int d = 0; d < HB; ++d)
+        for (int d = 0; d < HB; ++d) {
+          if (AHEAD && PART < HB && d == PART) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_keys(PART, HB);
+            __builtin_amdgcn_sched_barrier(0);
+          }
 #pragma unroll
           for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -121,9 +131,10 @@ __global__ __launch_bounds__(64 * AF_WAVES, AHEAD || HB > 4 ? 2 : 4) void attent
 #pragma unroll
               for (int j = 0; j < 4; ++j) s[b][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j], qf[d][j], s[b][e], 0, 0, 0);
             }
+        }
         if (AHEAD && HB > 4) {
           __builtin_amdgcn_sched_barrier(0);
-          load_values(0, EARLY);
+          load_values(0, PART);
           __builtin_amdgcn_sched_barrier(0);
         }
         // a lane's scores: positions first + 32 b + 8 q + 4 e + v of row r
@@ -168,22 +179,27 @@ __global__ __launch_bounds__(64 * AF_WAVES, AHEAD || HB > 4 ? 2 : 4) void attent
           }
         };
         if (AHEAD) {
-          if (HB > EARLY) {
+          auto multiply = [&](int d0, int d1) {
+            if (edge) {
+#pragma unroll
+              for (int i = 4 * d0; i < 4 * d1; ++i) leave_out((&vf[0][0][0])[i]);
+            }
+#pragma unroll
+            for (int d = d0; d < d1; ++d) acc[d] *= alpha;
+            // (an output tile's products one after the other in the order of the keys; the tiles take turns)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+#pragma unroll
+              for (int d = d0; d < d1; ++d)
+                acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[AHEAD ? d : 0][i >> 3][(i >> 2) & 1][i & 3], s[i >> 3][(i >> 2) & 1][i & 3], acc[d], 0, 0, 0);
+          };
+          multiply(0, PART);
+          if (PART < HB) {
             __builtin_amdgcn_sched_barrier(0);
-            load_values(EARLY, HB);
+            load_values(PART, HB);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(PART, HB);
           }
-          if (edge) {
-#pragma unroll
-            for (int i = 0; i < 4 * HB; ++i) leave_out((&vf[0][0][0])[i]);
-          }
-#pragma unroll
-          for (int d = 0; d < HB; ++d) acc[d] *= alpha;
-          // (an output tile's products one after the other in the order of the keys; the tiles take turns)
-#pragma unroll
-          for (int i = 0; i < 16; ++i)
-#pragma unroll
-            for (int d = 0; d < HB; ++d)
-              acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[AHEAD ? d : 0][i >> 3][(i >> 2) & 1][i & 3], s[i >> 3][(i >> 2) & 1][i & 3], acc[d], 0, 0, 0);
         } else {
 #pragma unroll
           for (int d = 0; d < HB; ++d) {
@@ -275,7 +291,8 @@ int gl3_attention_f32(const float* q, long q_stride, const float* k_cache, const
   const int per_tile = (long)((n_tokens + most - 1) / most) * n_kv >= 512 ? most : 1;
   const dim3 grid((n_tokens + per_tile - 1) / per_tile, n_kv), block(64 * AF_WAVES);
   // (the loads of a step in registers at once take the room of the other block that a CU would hold: 333 and 180 tokens, 32 heads of
-  // 64, 34 us without and 40 with; 2,000 keys for each of four tokens 46 and 35)
+  // 64, 34 us without and 40 with; 2,000 keys for each of four tokens 49 and 34, heads of 32 20.0 and 19.9, of 96 59 and 52, of 128 87 and 63.
+  // Of 75 steps of 1 to 32 tokens with 0 to 8,000 keys, heads of 32 to 128, the greatest loss is 0.9 us of 14 (heads of 96, 350 keys))
   const bool ahead = (long)grid.x * grid.y <= 256;
 #define AF_GO(HB, AHEAD)                                                                                                        \
   attention_f32_kernel<HB, AHEAD><<<grid, block, 0, stream>>>(q, q_stride, k_cache, v_cache, positions, table_rows, block_table, \
