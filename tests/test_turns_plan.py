@@ -1,5 +1,6 @@
 """Rules that choose a prompt step's kernels (the plan of the tiled products into the residual rows, the splits of its attention):
 plain arithmetic on the host, at sizes they were measured at."""
+import pytest
 import torch
 
 from gpullama3_java_amd.csrc import lib
@@ -42,7 +43,8 @@ def test_splits_of_a_prompt_step_s_attention():
                 assert 1 <= n <= 8 and (n == 1 or n * n_seqs * T * heads <= lib.PREFILL_SPLIT_ROWS)
 
 
-def test_a_prompt_step_runs_without_splits_where_their_buffers_have_no_room(monkeypatch):
+@pytest.mark.parametrize("head_dim", [16, 128])
+def test_a_prompt_step_runs_without_splits_where_their_buffers_have_no_room(monkeypatch, head_dim):
     """A portion behind a long context asks for buffers that it can do without: on a full device it runs as it would without them."""
     from types import SimpleNamespace
 
@@ -61,15 +63,15 @@ def test_a_prompt_step_runs_without_splits_where_their_buffers_have_no_room(monk
         room[0] -= n
         return empty(n, **kw)
     monkeypatch.setattr(ops, "attention_kernel", lambda *a: "prefill")
-    monkeypatch.setattr(lib, "attention_prefill", lambda *a, **kw: calls.append(kw.get("splits", 1)))
-    q, cache = torch.zeros(300, 64), torch.zeros(1, 1, 64, 16)
+    monkeypatch.setattr(lib, "attention_prefill", lambda *a, **kw: calls.append(kw.get("splits", 1) if "wide_from" not in kw else None))
+    q, cache = torch.zeros(300, 64), torch.zeros(1, 1, 64, head_dim)
 
     def steps():
         with monkeypatch.context() as m:
             m.setattr(torch, "empty", small_device)
             for _ in range(2):
-                ops.attention(ctx, q, cache, cache, None, q, 32, 8, 16, None, 0.25)
-    small, large = lib.PREFILL_SPLIT_ROWS * 2, lib.PREFILL_SPLIT_ROWS * 16
+                ops.attention(ctx, q, cache, cache, None, q, 32, 8, head_dim, None, 0.25)
+    small, large = lib.PREFILL_SPLIT_ROWS * 2, lib.PREFILL_SPLIT_ROWS * head_dim
     for total, held in ((0, 0), (small, small), (large, small), (large + small - 1, small), (large + small, large + small)):
         room[0] = total
         engine.workspace = Workspace("cpu")
