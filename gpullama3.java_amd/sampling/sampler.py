@@ -95,7 +95,7 @@ class DeviceSampler:
         if R == 0:
             return []
         n = K.sample_work_size(R, V) + 3 * R
-        out = torch.empty(R, dtype=torch.int32, pin_memory=True)
+        out = torch.empty(R, dtype=torch.int32, device="cpu", pin_memory=True)      # (whatever the caller's default device is)
         parameters = None
         if not all(t == 0 for t in temperatures):       # (every row greedy: the rows are read by many blocks at once)
             parameters = [[float(x) for x in p] for p in (temperatures, top_ps, uniforms)]

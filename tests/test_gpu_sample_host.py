@@ -43,6 +43,13 @@ def test_the_call_from_host_memory_refuses():
         DeviceSampler(torch.device("cuda:0"))(logits, [1.0, 1.0], [1.0], [0.5, 0.5])
 
 
+def test_the_call_where_tensors_are_made_on_the_gpu_by_default():
+    logits = torch.zeros(2, 50, device="cuda:0")
+    logits[0, 7] = logits[1, 31] = 40.0
+    with torch.device("cuda:0"):
+        assert DeviceSampler(torch.device("cuda:0"))(logits, [0.5] * 2, [0.9] * 2, [0.3] * 2) == [7, 31]
+
+
 @pytest.mark.parametrize("own_streams", [False, True])
 def test_calls_of_two_threads(own_streams):
     from concurrent.futures import ThreadPoolExecutor

@@ -60,7 +60,7 @@ def test_one_sampler_s_calls_of_several_threads_take_turns(monkeypatch):
     monkeypatch.setattr(lib, "sample_host", sample_host)
     sampler = DeviceSampler(torch.device("cpu"))
     sampler._torch = SimpleNamespace(float32=torch.float32, int32=torch.int32,
-                                     empty=lambda n, dtype, device=None, pin_memory=False: torch.empty(n, dtype=dtype))
+                                     empty=lambda n, dtype, device, pin_memory=False: torch.empty(n, dtype=dtype, device=device))
 
     def calls(k):
         return all(sampler(torch.zeros(2 + k, 5), [1.0] * (2 + k), [0.9] * (2 + k), [k] * (2 + k)) == [k] * (2 + k) for _ in range(10))
