@@ -24,6 +24,7 @@
 // spreads the 16 rows that a quarter of the lanes reads over all banks.
 #include "common.h"
 #include "lds_loads.h"
+#include <climits>
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -974,7 +975,7 @@ static bool prefill_wide(int head_dim, int n_heads, int n_seqs, int max_q_len) {
 // sizes, 0.80 on average); below 0.98 to 1.25 (60 sizes, 1.08 on average; 1,300 tokens and sixty of 100 58 -> 68 us with 24 heads), but six or eight
 // of 1,280 to 2,000 0.92 to 1.01. (What the sequences hold already is not known here: with sixty of 1 to 30 tokens behind 500 beside 1,300
 // or 2,048 24 heads take 1.13 to 1.23 times as long, 32 heads 0.82 to 0.87; behind 4,000 0.89 to 0.99 and 0.58 to 0.64.)
-#define PF_TURNS -1
+#define PF_TURNS INT_MIN
 static bool turns_takes(int head_dim, int page_size, int group, int n_seqs, int n_tokens) {
   return head_dim == 128 && page_size % 64 == 0 && (n_seqs == 1 || (n_seqs <= 64 && n_tokens > 0 && n_tokens / (group % 2 ? 256 : 128) + n_seqs <= 65535));
 }
@@ -996,8 +997,8 @@ extern "C" int gl3_attention_prefill_supports(int head_dim, int page_size) {
 
 // max_q_len: the most tokens any sequence brings in this step (it sizes the grid).
 // seq_rows (may be null): the row of `block_table` that holds sequence b's pages; null: row b.
-// wide_from: the kernel with 128 queries a block is taken when max_q_len reaches it; 0: the library's choice; PF_TURNS: the kernel
-// of turns.
+// wide_from: the kernel with 128 queries a block is taken when max_q_len reaches it; <= 0: the library's choice, but for PF_TURNS: the
+// kernel of turns.
 extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k_cache, const void* v_cache,
                                      const int* cu_seqlens, const int* kv_before, const int* block_table,
                                      const int* seq_rows, int table_stride, void* out, long out_stride, int n_seqs,

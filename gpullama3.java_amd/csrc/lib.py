@@ -2047,7 +2047,7 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len):
     return max(1, min(8, -(-512 // blocks), max_kv_len // 256))
 
 
-PREFILL_TURNS = -1                    # ``attention_prefill``'s ``wide_from`` that names the kernel of turns
+PREFILL_TURNS = -2 ** 31              # ``attention_prefill``'s ``wide_from`` that names the kernel of turns
 
 
 def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, out, max_q_len, n_heads, n_kv,
@@ -2058,7 +2058,7 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
     of the packed ``q`` belong to which sequence and where they sit in it. ``seq_rows`` [B] (optional)
     names each sequence's row of ``block_table``; without it sequence b reads row b. ``wide_from``: from
     how many tokens of the step's longest sequence on the kernel with 128 queries a block runs
-    (0: the library's choice; ``PREFILL_TURNS``: the kernel of turns, which takes heads of 128 and the plain rule, gives the same bits
+    (0 and below: the library's choice; ``PREFILL_TURNS``: the kernel of turns, which takes heads of 128 and the plain rule, gives the same bits
     and has no splits; tests run all kernels on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
     128 queries are shared out over that many blocks of the same kernel, whose sums lie in ``part_o`` (float32, at least
     splits * T * H * hs) and ``part_ml`` (2 * splits * T * H) until a second kernel merges them; the plain rule only."""

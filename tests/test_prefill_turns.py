@@ -125,6 +125,16 @@ def test_attention_of_turns_with_one_key_that_counts_and_scores_that_are_not_num
 
 
 @pytest.mark.gpu
+def test_thresholds_of_zero_and_below_are_the_library_s_choice():
+    from test_gpu_kernels import attention_case, run_attention
+    for hs in (64, 128):
+        sk, sv, qs = attention_case(np.random.default_rng(hs), 4, 2, hs, [40], [70], "bfloat16")
+        got = [run_attention(fn([40], [70], w), sk, sv, qs, [40], [70], 4, 2, hs, "bfloat16", np.random.default_rng(1))[0] for w in (0, -1, -64)]
+        np.testing.assert_array_equal(got[1], got[0])
+        np.testing.assert_array_equal(got[2], got[0])
+
+
+@pytest.mark.gpu
 def test_attention_of_turns_refuses_what_it_is_not_built_for():
     from test_gpu_kernels import attention_case, run_attention
     for hs, page, before, new, window in ((64, 64, [0], [70], 0), (128, 96, [0], [70], 0), (128, 64, [0], [70], 20), (128, 64, [0] * 65, [2] * 65, 0)):
