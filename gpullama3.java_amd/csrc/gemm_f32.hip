@@ -15,10 +15,11 @@
 //   4.0 TB/s), the head 179 us (5.9 TB/s), against the kernel for any sizes, whose 64 x 64 tiles leave a
 //   product of 2,048 columns 32 blocks that walk K in steps of 16 behind two barriers each. Eight waves a block were 1.0
 //   to 1.3 times as long.
-// * more, K in no whole steps of 32 (for others see gemm_f32_stream_kernel): bound by the matrix cores (256 flops a clock and CU). Tiles through shared memory in steps of 32 k, two
-//   buffers, one barrier a step; rows in shared memory are 36 floats apart, so that the sixteen lanes that read 16 bytes of
-//   sixteen rows meet all 64 banks once. 4,096 x 4,096 x 4,096: 1.15 ms, 119 TFLOP/s (157 is the unit's peak); 513 rows of
-//   the 1B layers: 57 to 92 TFLOP/s against about 20.
+// * more: bound by the matrix cores (256 flops a clock and CU; 157 TFLOP/s at most). K in whole steps of 32, rows of A at and in whole
+//   16 bytes, offsets of 31 bits (f32_streams): gemm_f32_stream_kernel, with its figures. Everything else: tiles through registers into shared
+//   memory in steps of 32 k, two buffers, one barrier a step; rows in shared memory are 36 floats apart, so that the sixteen lanes that
+//   read 16 bytes of sixteen rows meet all 64 banks once. 4,096 x 4,096 x 4,096, rows of A at an odd float: 1.21 ms, 114 TFLOP/s; 513 rows of
+//   the 1B layers 57 to 90 TFLOP/s, against about 20 of the kernel for any sizes.
 #include "common.h"
 #include "lds_loads.h"
 #include <type_traits>
@@ -326,8 +327,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
 // The kernel above keeps one step of operands in registers on the way to shared memory; behind its barrier every wave then waits for
 // its reads with little else in flight. Here a block asks for steps ahead (STAGES - 1 of them), no wave writes shared memory, and what a
 // tile needs of it is small enough for several blocks a CU, of which one multiplies while another waits. The kernel above and this one at
-// 513 rows of the 1B layers: gate/up 393 -> 292 us (118 TFLOP/s), down 276 -> 212, output 76 -> 58, QKV 91 -> 72; at 4,096 rows gate/up
-// 2,280 -> 1,980 (139 TFLOP/s; the library's own product of 8,192 cubed reaches 153). What bounds the small ones: whole tiles of 32 rows
+// 513 rows of the 1B layers: gate/up 381 -> 293 us (118 TFLOP/s), down 276 -> 210, output 75 -> 60, QKV 89 -> 72; at 4,096 rows gate/up
+// 2,462 -> 1,974 (139 TFLOP/s; the library's own product of 8,192 cubed reaches 153; profiles/float32_tiles.txt). What bounds the small ones: whole tiles of 32 rows
 // and whole rounds of the chip's 256 CUs. Rows in shared memory are 128
 // bytes in eight pieces of 16, piece c of row r at place c ^ (r / 2 % 8): the sixteen rows that sixteen lanes read at one piece meet all
 // banks once. A step is asked for into the place of the step before, behind the barrier that every wave reaches with that step's
@@ -471,8 +472,8 @@ static bool f32_streams(const void* A, int N, int K, long lda, long ldw, bool ga
   return K % F3_BK == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 && 128 * lda * 4 < (1L << 31) && ((gated ? (long)N : 0) + 128) * ldw * 4 < (1L << 31);
 }
 // Its tile: 1 to 4: 128 rows of W x 128 tokens, 128 x 64, 64 x 64, 64 x 32; 5: 32 x 32 (not gated). As in gl3_f32_shape: one tile alone
-// on a CU takes `alone`, a CU with several `each` a tile (us for K = 2,048, both measured; of 108 products of 17 to 4,096 rows
-// one was more than 10% from the best of the five tiles).
+// on a CU takes `alone`, a CU with several `each` a tile (us for K = 2,048, both measured; of 85 products of 17 to 4,096 rows
+// one is more than 2% from the best of the tiles, 6%: profiles/float32_tiles.txt).
 extern "C" int gl3_f32_stream_shape(int M, int N, int gated) {
   static const int bn[5] = {128, 128, 64, 64, 32}, bm[5] = {128, 64, 64, 32, 32};
   static const float alone[5] = {144, 80, 45.5f, 28.6f, 20.5f}, each[5] = {124.4f, 62.5f, 33.4f, 17.7f, 11.f};
@@ -524,8 +525,8 @@ static int launch_f32(const float* A, const float* W, float* C, int M, int N, in
 // 1: the kernel for few rows; 2 to 5: tiles of 128 x 128, 128 x 64, 64 x 64 and 64 rows of W x 32 tokens. Of the tiles the
 // one that takes the least time: one tile alone on a CU takes `alone`, a CU with several of them `each` a tile (us for
 // K = 2,048, both measured; the sum of a CU's tiles was within 4% of the measured time at 513 to 4,096 rows). Few rows: 48
-// rows of the down projection of the 1B layers 136 us in the smallest tile; gated products of more than 32 rows fill the
-// chip with those (48 rows: 55 us) where the other kernel would hold 128 KB of sums a block.
+// rows of the down projection of the 1B layers 136 us in the smallest tile; gated products of more than 32 rows (of more than 16 where
+// gemm_f32_stream_kernel takes them) fill the chip with those (48 rows: 55 us, 43 there) where the other kernel would hold 128 KB of sums a block.
 extern "C" int gl3_f32_shape(int M, int N, int gated) {
   if (M <= (gated ? 32 : 64)) return 1;
   static const int bn[4] = {128, 128, 64, 64}, bm[4] = {128, 64, 64, 32}, alone[4] = {154, 89, 53, 34}, each[4] = {144, 76, 41, 23};
