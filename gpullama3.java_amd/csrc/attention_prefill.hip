@@ -607,7 +607,7 @@ __global__ __launch_bounds__(256, OCC) void attention_prefill_wide_kernel(
 // that maximum moved), weights are added up in the order of the keys, and a half that none of a wave's queries sees is left out. One maximum
 // for a whole chunk was 2 to 3% faster and its error against 64 bits up to 1.006 times as large.
 // Group 0 has matrix turn i in turn 2 i, group 1 in turn 2 i + 1. What bounds it now: the vector instructions of both waves together with
-// the matrix instructions. With heads of 64, whose matrix part is half as long, such a loop was no faster than the kernel above
+// the matrix instructions (16,384 tokens: vector units busy 61% of the time, matrix cores 58%). With heads of 64, whose matrix part is half as long, such a loop was no faster than the kernel above
 // (8,192 tokens 345 and 341 us) and is not built.
 // 32 heads, one sequence, the kernel above and this one: 2,048 tokens 75 -> 61 us, 4,096 172 -> 143, 8,192 608 -> 520, 16,384 2,325 -> 1,956
 // (1.12 PFLOP/s). Nor has it splits: one block a CU, so that as many splits as the kernel above has are two rounds of the chip (512 tokens
