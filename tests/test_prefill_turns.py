@@ -83,7 +83,7 @@ def test_attention_of_turns(H, Kh, page, before, new, sharp):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("at", [0, 31, 32, 63, 64, 95, 1000, 1037, 1038, 1055])
+@pytest.mark.parametrize("at", [0, 31, 32, 63, 64, 95, 1000, 1037, 1038, 1055, 1060])
 def test_values_that_are_not_finite_reach_as_far_as_in_the_kernel_beside_it(at):
     """A weight of zero does not make nothing of an infinite value: it spoils the queries in front of it whose keys share its 32, and
     what a page still holds behind the sequence's end (here from 1,038 on) likewise; no more than that on either kernel."""
