@@ -22,6 +22,9 @@
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -279,7 +282,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 // 4,096). What bounds it now is the power budget: the clock stands at 1.4 to 1.8 GHz of 2.4, the matrix cores are busy 74 to 79% of
 // a CU's cycles (gate/up and plain products of 8,192 rows, K = 4,096), and with the 32x32x16 instruction, whose accumulators pass
 // through the registers twice as often per flop, the same loop lost 11%.
-// (8,192 x 28,672 x 4,096: the kernel above 1,680 us, this one 1,312.)
+// (8,192 x 28,672 x 4,096: the kernel above 1,680 us, this one 1,283.)
 //
 // Halves of A and of W: AH = WH = 2 is the tile of 256 x 256. AH = 1: 128 rows x 256, two phases a step, a third step in shared
 // memory instead of registers read ahead (2,048 rows, 3,072 columns, K = 2,048: 42 -> 30 us; 512 rows of the 3B layers' gate/up
@@ -309,38 +312,6 @@ __device__ __forceinline__ unsigned mf_w_offset(int row, int k, long ldw, int w_
   return WT == 1   ? (unsigned)gl3_operand_offset(w_pos ? w_pos[row] : row, k, w_steps) * 2
          : WT == 2 ? (unsigned)gl3_packed_offset(row, k, w_steps) * 2
                    : (unsigned)((long)(row - n0) * ldw + k) * 2;
-}
-
-// Four consecutive columns n .. n + 3 of an output row (`vec`: they may go at once).
-template <int EPI, typename TC>
-__device__ __forceinline__ void mf_finish4(TC* c, f32x4 s, f32x4 up, int n, int N, bool vec, const float* bias, int act, const MfExtras& ex) {
-  typedef TC tc4 __attribute__((ext_vector_type(4)));
-  const int left = N - n;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int at = min(n + j, N - 1);
-    if (bias) {
-      s[j] += bias[at];
-      if (EPI == MF_GATED) up[j] += bias[N + at];
-    }
-    if (EPI == MF_GATED) s[j] = gl3_gated<true>(s[j], up[j], act, ex.act_limit, ex.act_shift);
-    else if (ex.col_scale) s[j] *= ex.col_scale[at];
-  }
-  if (vec && left >= 4) {
-    if (EPI == MF_ADD) {
-      const tc4 old = *(const tc4*)c;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] += to_f32<TC>(old[j]);
-    }
-    tc4 o;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = from_f32<TC>(s[j]);
-    *(tc4*)c = o;
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j < left) c[j] = from_f32<TC>(EPI == MF_ADD ? to_f32<TC>(c[j]) + s[j] : s[j]);
-  }
 }
 
 template <int EPI, typename TC, int WT, int AH, int WH>
@@ -537,37 +508,137 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   if (wm == 0) mf_barrier();
   mf_wait_loads<0>();                 // (what was asked for beyond the last step has landed)
 
-  // A lane holds four consecutive columns of a row (column 4 * (lane / 16), row lane % 16 of a 16 x 16 tile). The sums
-  // go through shared memory, half the tile's rows at a time, so that a wave then works on whole rows: 1 KB of a row of
-  // floats an instruction. Row r's sixteen bytes c lie at place c ^ (r % 16): no two lanes of a write meet in a bank.
-  const bool vec = slice ? ldp % 4 == 0 && p_stride % 4 == 0 && (uintptr_t)P % 16 == 0
-                         : ldc % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;
-  constexpr int LPR = NCOLS / 4, RPW = 64 / LPR, ROW = 512 * WH;      // lanes of an output row, such rows a wave, bytes of a row of sums
-#pragma unroll
-  for (int ah = 0; ah < AH; ++ah) {
-    mf_barrier();                     // (both groups have read what lay here)
-#pragma unroll
-    for (int tm = 0; tm < 4; ++tm)
-#pragma unroll
-      for (int wh = 0; wh < WH; ++wh)
-#pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
-          *(f32x4*)(lds + (wm * 64 + tm * 16 + lr) * ROW + (((wh * 32 + wn * 8 + tn * 4 + lq) ^ lr) << 4)) = acc[ah][tm][wh][tn];
-    mf_wait_reads<0>();
-    mf_barrier();
-    const int rows = min(128, M - m0 - ah * 128), c4 = lane % LPR, n = n0 + c4 * 4;
-    const int gate = EPI == MF_GATED && WH == 1 ? (c4 >> 2) * 8 + (c4 & 3) : c4, up = WH == 1 ? gate + 4 : gate + 32;
-#pragma unroll 4
-    for (int r = wave * RPW + lane / LPR; r < rows; r += 8 * RPW) {
-      const f32x4 v = *(const f32x4*)(lds + r * ROW + ((gate ^ (r & 15)) << 4));
+  // The sums go to memory straight from the registers: a lane holds four consecutive columns of a row (4 * (lane / 16) of the 16
+  // of a 16 x 16 tile, row lane % 16). Gate and up value of a column are the same lane's, so the gated rule needs nobody else's.
+  // 16-bit outputs: two tiles' lanes hand each other half of their columns and store 16 bytes of eight (64 consecutive bytes of
+  // sixteen rows an instruction, 32 where a wave has 16 columns); 32-bit ones are 16 bytes a lane as they are. The rule of an
+  // epilogue's extras is looked at once, not per element: most products have none, and then the code is short. Against the sums
+  // through shared memory, a wave on whole rows: gate/up of 2,048 rows of the 1B layers 123 -> 104 us (93 without any epilogue), of
+  // 16,384 910 -> 790, of 8,192 of the 8B layers 1,379 -> 1,283; QKV of 2,048 rows 30.1 -> 27.8, of 512 rows of the 3B layers
+  // 26.1 -> 24.7; the output projection of 5,886 rows of the 3B layers, which reads the rows it adds to, 137 -> 132 (110 without);
+  // a head's 2,221 x 128,256 floats, bound by their way to memory, 1,048 to 1,090 on both.
+  const int col0 = n0 + (EPI == MF_GATED && WH == 1 ? wn * 16 : wn * 32), row0 = m0 + wm * 64 + lr;
+  auto finish = [&](auto plain_t) {
+    constexpr bool PLAIN = decltype(plain_t)::value;
+    // columns n .. n + 3, ready to be stored (an add's old values aside)
+    auto sums = [&](int ah, int tm, int wh, int tn, int n) {
+      f32x4 v = acc[ah][tm][wh][tn];
       f32x4 u = v;
-      if (EPI == MF_GATED) u = *(const f32x4*)(lds + r * ROW + ((up ^ (r & 15)) << 4));
-      if (n >= N) continue;
-      const long m = m0 + ah * 128 + r;
-      if (EPI != MF_GATED && slice > 0) mf_finish4<MF_STORE, float>(P + (long)(slice - 1) * p_stride + m * ldp + n, v, u, n, N, vec, nullptr, act, ex);
-      else mf_finish4<EPI, TC>(C + m * ldc + n, v, u, n, N, vec, bias, act, ex);
+      if constexpr (EPI == MF_GATED) u = WH == 2 ? acc[ah][tm][WH - 1][tn] : acc[ah][tm][0][1];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (PLAIN) {
+          if (EPI == MF_GATED) v[j] = gl3_activation<true>(v[j], GL3_ACT_SILU) * u[j];
+        } else {
+          const int at = min(n + j, N - 1);
+          if (bias) {
+            v[j] += bias[at];
+            if (EPI == MF_GATED) u[j] += bias[N + at];
+          }
+          if (EPI == MF_GATED) v[j] = gl3_gated<true>(v[j], u[j], act, ex.act_limit, ex.act_shift);
+          else if (ex.col_scale) v[j] *= ex.col_scale[at];
+        }
+      }
+      return v;
+    };
+    constexpr int HALVES = EPI == MF_GATED ? 1 : WH, TILES = EPI == MF_GATED && WH == 1 ? 1 : 2;      // of output columns
+    if constexpr (sizeof(TC) == 2) {
+      if (ldc % 8 == 0 && N % 8 == 0 && (uintptr_t)C % 16 == 0) {
+        auto pack = [&](int ah, int tm, int wh, int tn) {
+          const f32x4 v = sums(ah, tm, wh, tn, col0 + wh * 128 + tn * 16 + lq * 4);
+          return __builtin_bit_cast(u32x2, bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]});
+        };
+        // (lanes of odd lq get the columns of tile b, of even ones those of a: eight from column 8 * (lq / 2))
+        auto put = [&](u32x2 a, u32x2 b, int row, int n) {
+          const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+          const auto hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+          if (row < M && n < N) *(u32x4*)(C + (long)row * ldc + n) = u32x4{lo[0], hi[0], lo[1], hi[1]};
+        };
+#pragma unroll
+        for (int ah = 0; ah < AH; ++ah) {
+          if constexpr (TILES == 1) {
+#pragma unroll
+            for (int tm = 0; tm < 4; tm += 2)
+              put(pack(ah, tm, 0, 0), pack(ah, tm + 1, 0, 0), row0 + ah * 128 + (tm + (lq & 1)) * 16, col0 + (lq >> 1) * 8);
+          } else {
+#pragma unroll
+            for (int tm = 0; tm < 4; ++tm)
+#pragma unroll
+              for (int wh = 0; wh < HALVES; ++wh)
+                put(pack(ah, tm, wh, 0), pack(ah, tm, wh, 1), row0 + ah * 128 + tm * 16, col0 + wh * 128 + (lq & 1) * 16 + (lq >> 1) * 8);
+          }
+        }
+        return;
+      }
     }
+    const bool vec = ldc % 4 == 0 && N % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;
+    typedef TC tc4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int ah = 0; ah < AH; ++ah) {
+      tc4 old[4][WH][2];
+      if (EPI == MF_ADD && vec) {       // (all asked for before the first is needed; beyond the matrix: its last row and columns again)
+#pragma unroll
+        for (int tm = 0; tm < 4; ++tm)
+#pragma unroll
+          for (int wh = 0; wh < HALVES; ++wh)
+#pragma unroll
+            for (int tn = 0; tn < TILES; ++tn)
+              old[tm][wh][tn] = *(const tc4*)(C + (long)min(row0 + ah * 128 + tm * 16, M - 1) * ldc + min(col0 + wh * 128 + tn * 16 + lq * 4, N - 4));
+      }
+#pragma unroll
+      for (int tm = 0; tm < 4; ++tm)
+#pragma unroll
+        for (int wh = 0; wh < HALVES; ++wh)
+#pragma unroll
+          for (int tn = 0; tn < TILES; ++tn) {
+            const int n = col0 + wh * 128 + tn * 16 + lq * 4, row = row0 + ah * 128 + tm * 16;
+            const f32x4 v = sums(ah, tm, wh, tn, n);
+            if (row >= M || n >= N) continue;
+            TC* c = C + (long)row * ldc + n;
+            if (vec) {
+              tc4 o;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) o[j] = from_f32<TC>(EPI == MF_ADD ? to_f32<TC>(old[tm][wh][tn][j]) + v[j] : v[j]);
+              *(tc4*)c = o;
+            } else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                if (n + j < N) c[j] = from_f32<TC>(EPI == MF_ADD ? to_f32<TC>(c[j]) + v[j] : v[j]);
+            }
+          }
+    }
+  };
+  if (EPI != MF_GATED && slice > 0) {
+    float* const p = P + (long)(slice - 1) * p_stride;
+    const bool vec = ldp % 4 == 0 && N % 4 == 0 && (uintptr_t)p % 16 == 0;
+#pragma unroll
+    for (int ah = 0; ah < AH; ++ah)
+#pragma unroll
+      for (int tm = 0; tm < 4; ++tm)
+#pragma unroll
+        for (int wh = 0; wh < WH; ++wh)
+#pragma unroll
+          for (int tn = 0; tn < 2; ++tn) {
+            const int n = col0 + wh * 128 + tn * 16 + lq * 4, row = row0 + ah * 128 + tm * 16;
+            f32x4 v = acc[ah][tm][wh][tn];
+            if (row >= M || n >= N) continue;
+            if (ex.col_scale) {
+#pragma unroll
+              for (int j = 0; j < 4; ++j) v[j] *= ex.col_scale[min(n + j, N - 1)];
+            }
+            float* c = p + (long)row * ldp + n;
+            if (vec) *(f32x4*)c = v;
+            else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                if (n + j < N) c[j] = v[j];
+            }
+          }
+    return;
   }
+  const bool plain = !bias && !ex.col_scale && (EPI != MF_GATED || (act == GL3_ACT_SILU && ex.act_limit <= 0.f && ex.act_shift == 0.f));
+  if (plain) finish(std::true_type{});
+  else finish(std::false_type{});
 }
 
 // What gemm_mfma_turns_kernel is built for: whole steps of 64 k, and byte offsets of 31 bits inside a tile's rows of A and
@@ -613,7 +684,7 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
 // The tile the library takes where the caller names none. Where gemm_mfma_turns_kernel takes the product: the tile whose rounds on
 // the chip take the least time, a round (a block on every CU: 32 of an XCD, which has an eighth of the tiles of every slice) being
 // 0.42 us a step of 64 k and 0.9 us beside them for 128 x 128, 0.60 and 4.0 for 128 rows x 256, 1.0 and 4.5 for 256 x 256. The
-// constants rank the tiles and are no times of their own (at 8,192 rows of 28,672 x 4,096 they say 959 us and it is 1,312).
+// constants rank the tiles and are no times of their own (at 8,192 rows of 28,672 x 4,096 they say 959 us and it is 1,283).
 // Measured with the norm behind, 143 products into the residual rows (70 to 5,886 rows, 512 to 4,096 columns, K of 1,024 to 14,336 in
 // mfma_plan's slices): the tile chosen is the fastest of the three or within 5% but at 512 rows of 1,280 x 5,120 (29.2 against
 // 27.0 us) and 1,024 rows of 1,024 x 4,096 (34.2 against 31.8). With rounds of 256 blocks, whatever their XCD, 300 rows of 3,072 x

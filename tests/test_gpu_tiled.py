@@ -121,3 +121,49 @@ def test_unknown_tiles_are_refused(shape):
     a, w, x = (torch.zeros(128, 128, device=DEV, dtype=d) for d in (torch.bfloat16, torch.bfloat16, torch.float32))
     with pytest.raises(lib.KernelError, match="unknown tile shape"):
         lib.gemm_mfma(a, w, x, shape=shape)
+
+
+# (columns in whole eights, in fours and in neither; one row, whole tiles, one row more than a tile)
+@pytest.mark.parametrize("shape", [1, 2, 5])
+@pytest.mark.parametrize("M, N", [(1, 8), (129, 136), (256, 256), (257, 260), (300, 523)])
+def test_epilogues_of_the_tiled_products(shape, M, N):
+    """An output that may be stored sixteen bytes at a time against one that begins at an odd place and is stored element by element:
+    the same bits, whatever the epilogue applies, and nothing beside the output is written."""
+    lib = K()
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    Kd = 192
+    A, W = (torch.randn(n, Kd, generator=gen, device="cuda").to(torch.bfloat16) for n in (M, 2 * N))
+    bias, factor = torch.randn(2 * N, generator=gen, device="cuda"), torch.randn(N, generator=gen, device="cuda")
+    res = torch.randn(M, N, generator=gen, device="cuda")
+
+    def both(dtype, epilogue, add=False, **kw):
+        w = W if epilogue == lib.EPI_GATED else W[:N]
+        outs = []
+        for pad, first in ((8 - N % 8, 0), (3, 1)):
+            whole = torch.full((M, N + pad + first), -7.0, device=DEV, dtype=dtype)
+            out = whole[:, first:first + N]
+            if add:
+                out.copy_(res)
+            lib.gemm_mfma(A, w, out, epilogue, shape=shape, **kw)
+            assert torch.all(whole[:, :first] == -7.0) and torch.all(whole[:, first + N:] == -7.0)
+            outs.append(out.clone())
+        assert torch.equal(outs[0], outs[1]), (dtype, epilogue, kw)
+        return outs[0].double()
+    sums = A.double() @ W.double().T
+    size = A.double().abs() @ W.double().abs().T                                      # (a sum of 192 products: 192 roundings of it at most)
+    for dtype, bits in ((torch.bfloat16, 8), (torch.float32, 23)):
+        for kw, want in (({}, sums[:, :N]), ({"bias": bias[:N].contiguous()}, sums[:, :N] + bias[:N].double()),
+                         ({"col_scale": factor}, sums[:, :N] * factor.double())):
+            off = (both(dtype, lib.EPI_STORE, **kw) - want).abs()
+            assert (off <= 2.0 ** -bits * want.abs() + Kd * 2.0 ** -23 * size[:, :N] * max(1.0, factor.abs().max().item())).all()
+        for kw in ({}, {"bias": bias}, {"act": "gelu_tanh"}, {"act_limit": 3.0, "act_shift": 1.0}):
+            gate, up = (sums + (bias.double() if "bias" in kw else 0.0)).split(N, 1)
+            if "act_limit" in kw:
+                gate, up = gate.clamp(max=3.0), up.clamp(-3.0, 3.0) + 1.0
+            want = (torch.nn.functional.gelu(gate, approximate="tanh") if "act" in kw else gate / (1.0 + torch.exp(-gate))) * up
+            off = (both(dtype, lib.EPI_GATED, **kw) - want).abs()
+            # (a sum's error goes through a rule whose slope is at most 1.1 times the other factor; the exponential: 2^-20)
+            slack = 1.2 * Kd * 2.0 ** -23 * (size[:, :N] * (up.abs() + 1.0) + size[:, N:] * (gate.abs() + 1.0))
+            assert (off <= (2.0 ** -bits + 2.0 ** -17) * want.abs() + slack + 1e-6).all(), (dtype, kw)
+    want = sums[:, :N] + res.double()
+    assert ((both(torch.float32, lib.EPI_ADD, add=True) - want).abs() <= 2.0 ** -23 * want.abs() + Kd * 2.0 ** -23 * size[:, :N]).all()
