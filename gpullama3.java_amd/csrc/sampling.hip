@@ -20,7 +20,7 @@
 // At most 2^13 probabilities are 2^-13 or more. They are gathered while the row is normalised; when
 // their mass alone exceeds top_p, the threshold and the drawn token lie among them and both searches
 // walk that short list, in shared memory, instead of the row. A flat distribution, whose nucleus
-// reaches further down, takes eight passes over the whole row.
+// reaches further down, takes three passes over the whole row (nine if a factor of 1.05 holds more than 8,192 values).
 #include "common.h"
 #include "gl3_noalloc.h"
 #include <mutex>
@@ -31,6 +31,8 @@
 #define QSCALE 4611686018427387904.0   // 2^62: probabilities as 64-bit integers, sums exact and in any order
 #define CAND_MAX 8192  // candidates kept in shared memory: the probabilities of at least CAND_CUT
 #define CAND_CUT 0.0001220703125f      // 2^-13
+#define BIN_SHIFT 19   // a flat row's bins: exponent and four bits of the mantissa, of a probability of at most 1 below 2,048
+#define BINS 2048
 
 // A probability (0 <= p <= 1) as an integer: floor(p * 2^62), exact for p >= 2^-38, truncated below;
 // taken from the float's bits: mantissa shifted by its exponent.
@@ -157,10 +159,38 @@ __device__ Found radix_search(Src p, int V, unsigned long long thr,
   return Found{};
 }
 
-// A row's softmax is made by many blocks, ST_SLICES slices a row, in three kernels (the maximum, the
-// sum, the probabilities), before the row's one block picks the token: a single CU draws too few
+// How many of the values that equal the threshold are kept: the smallest k with above + k * each > tq.
+__device__ __forceinline__ long kept_ties(const Found& f1, unsigned long long tq) {
+  long k1 = 1;
+  if (f1.each > 0 && tq >= f1.above) k1 = (long)((tq - f1.above) / f1.each) + 1;
+  if (k1 > f1.ties) k1 = f1.ties;
+  return k1 < 1 ? 1 : k1;
+}
+// Which of the values that equal the drawn one is drawn, from 0 in ascending order of index.
+__device__ __forceinline__ long drawn_tie(const Found& f1, long k1, const Found& f2, unsigned long long target) {
+  const long j = (f2.each > 0 && target >= f2.above) ? (long)((target - f2.above) / f2.each) : 0;
+  const long limit = (f2.bits == f1.bits) ? k1 : (long)f2.ties;
+  return max(0L, min(j, limit - 1));
+}
+// The same from a list in shared memory that holds all of them (in any order): the one with that many equal ones of smaller index.
+__device__ __forceinline__ void pick_equal(const float* list_p, const int* list_i, int n, const Found& f1, long k1, const Found& f2,
+                                           unsigned long long target, int* winner) {
+  const long j = drawn_tie(f1, k1, f2, target);
+  const float want = __uint_as_float(f2.bits);
+  for (int a = threadIdx.x; a < n; a += SB) {
+    if (list_p[a] != want) continue;
+    const int ia = list_i[a];
+    long rank = 0;
+    if (f2.ties > 1)
+      for (int b = 0; b < n; ++b) rank += (list_p[b] == want && list_i[b] < ia) ? 1 : 0;
+    if (rank == j) *winner = ia;
+  }
+}
+
+// A row's softmax is made by many blocks, ST_SLICES slices a row, in two kernels (the slices' maxima and
+// sums, the probabilities), before the row's one block picks the token: a single CU draws too few
 // bytes a second, and has too little arithmetic, for a row of a hundred thousand logits. Rows with
-// temperature 0 are left alone by the three.
+// temperature 0 are left alone by both.
 #define ST_SLICES 64
 
 // Scratch of a call, for every row: the probabilities; per slice the maximum, the sum of the
@@ -191,43 +221,69 @@ static SampleWork carve_sample_work(float* work, int n_rows, int V) {
   return w;
 }
 
-__device__ __forceinline__ float row_max_of_slices(const float* slice_max, int row) {
-  float m = slice_max[row * ST_SLICES + (threadIdx.x & (ST_SLICES - 1))];   // every wave holds all 64 slices
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  return m;
-}
+// A call's parameters in host memory travel inside the first kernel's launch, which leaves them in the scratch for the kernels behind it
+// (`to`: temperatures, top-p, uniform numbers, n_rows each); with `to` null they are in device memory already.
+#define SAMPLE_STAGED 256
+struct SampleArgs { float v[3][SAMPLE_STAGED]; };
+struct SampleNoArgs {};
 
-__global__ __launch_bounds__(256) void softmax_max_kernel(const float* __restrict__ logits, long ld,
-                                                          const float* __restrict__ temperature, SampleWork w, int V) {
+// Every slice's maximum and the sum of its exponentials around that maximum: the logits are read once for both. A slice of at most 2,048
+// logits (a vocabulary of 131,072) is one stretch, held in registers between the two. Two kernels, the sum around the row's maximum,
+// took 4.3 and 4.6 us (8 rows of 128,256) and the parameters a third of 1.6.
+template <typename Args>
+__global__ __launch_bounds__(256) void softmax_slices_kernel(const float* __restrict__ logits, long ld,
+                                                             const float* __restrict__ temperature, Args args, float* __restrict__ to,
+                                                             int n_rows, SampleWork w, int V) {
   __shared__ float fs[16];
-  const int row = blockIdx.x, slice = blockIdx.y, tid = threadIdx.x;
-  const float T = temperature[row];
-  if (T == 0.f) return;
-  if (slice == 0 && tid == 0) { w.cand_count[row] = 0; w.cand_mass[row] = 0ull; }   // for the third kernel
-  const int per = (V + ST_SLICES - 1) / ST_SLICES;
-  const int lo = min(V, slice * per), hi = min(V, lo + per);
-  const float* lg = logits + (long)row * ld;
-  float m = -INFINITY;
-  for (int i = lo + tid; i < hi; i += 256) m = fmaxf(m, lg[i] / T);   // the division of the reference, per element
-  m = block_max(m, fs);
-  if (tid == 0) w.slice_max[row * ST_SLICES + slice] = m;
-}
-
-__global__ __launch_bounds__(256) void softmax_sum_kernel(const float* __restrict__ logits, long ld,
-                                                          const float* __restrict__ temperature, SampleWork w, int V) {
   __shared__ double ds[16];
   const int row = blockIdx.x, slice = blockIdx.y, tid = threadIdx.x;
-  const float T = temperature[row];
-  if (T == 0.f) return;
-  const float m = row_max_of_slices(w.slice_max, row);
   const int per = (V + ST_SLICES - 1) / ST_SLICES;
   const int lo = min(V, slice * per), hi = min(V, lo + per);
   const float* lg = logits + (long)row * ld;
+  float v[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) { const int i = lo + u * 256 + tid; v[u] = lg[min(i, V - 1)]; }      // (asked for before the temperature is known)
+  float T;
+  if constexpr (sizeof(Args) > 4) {
+    T = args.v[0][row];
+    if (slice == 0 && tid < 3) to[(long)tid * n_rows + row] = tid == 0 ? T : tid == 1 ? args.v[1][row] : args.v[2][row];
+  } else {
+    T = temperature[row];
+  }
+  if (T == 0.f) return;
+  if (slice == 0 && tid == 0) { w.cand_count[row] = 0; w.cand_mass[row] = 0ull; }   // for the next kernel
+  float m = -INFINITY;
   double z = 0.0;
-  for (int i = lo + tid; i < hi; i += 256) z += (double)expf(lg[i] / T - m);
+  for (int base = lo; base < hi; base += 8 * 256) {
+    if (base != lo) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = lg[min(base + u * 256 + tid, V - 1)];
+    }
+    float here = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      v[u] = base + u * 256 + tid < hi ? v[u] / T : -INFINITY;      // the division of the reference, per element
+      here = fmaxf(here, v[u]);
+    }
+    here = fmaxf(m, block_max(here, fs));
+    if (base != lo && m > -INFINITY) z *= exp((double)m - (double)here);
+    m = here;
+    const float around = m > -INFINITY ? m : 0.f;                   // (nothing but -inf so far: no term; NaN stays NaN)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) z += base + u * 256 + tid < hi ? (double)expf(v[u] - around) : 0.0;
+  }
   z = block_sum_f64(z, ds);
-  if (tid == 0) w.slice_sum[row * ST_SLICES + slice] = z;
+  if (tid == 0) { w.slice_max[row * ST_SLICES + slice] = m; w.slice_sum[row * ST_SLICES + slice] = z; }
+}
+
+// The row's maximum and sum from its slices', the same bits in every lane: lane k has slice k's.
+__device__ __forceinline__ void row_of_slices(float slice_max, double slice_sum, float& m, double& z) {
+  m = slice_max;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  z = slice_max > -INFINITY ? slice_sum * exp((double)slice_max - (double)m) : slice_sum;      // (a slice of -inf alone: 0, or NaN)
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) z += __shfl_xor(z, o, 64);
 }
 
 // p = softmax(logits / T) into the scratch, each slice's mass as an integer, and the candidates.
@@ -239,17 +295,22 @@ __global__ __launch_bounds__(256) void softmax_prob_kernel(const float* __restri
   __shared__ int bc_i[8 * 256];
   __shared__ int bc_n, bc_base;
   const int row = blockIdx.x, slice = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
-  const float T = temperature[row];
-  if (T == 0.f) return;
-  const float m = row_max_of_slices(w.slice_max, row);
-  double z = 0.0;
-  for (int k = 0; k < ST_SLICES; ++k) z += w.slice_sum[row * ST_SLICES + k];   // one order for every thread
-  const float zf = (float)z;
-  const float tp = top_p[row];
-  const bool nucleus = tp > 0.f && tp < 1.f;
+  // everything that the block reads is asked for before anything is looked at: one trip to memory, not five (8 rows of 128,256: 9.6 -> 8.7 us)
   const int per = (V + ST_SLICES - 1) / ST_SLICES;
   const int lo = min(V, slice * per), hi = min(V, lo + per);
   const float* lg = logits + (long)row * ld;
+  float v[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) v[u] = lg[min(lo + u * 256 + tid, V - 1)];
+  const float slice_max = w.slice_max[row * ST_SLICES + lane];
+  const double slice_sum = w.slice_sum[row * ST_SLICES + lane];
+  const float T = temperature[row], tp = top_p[row];
+  if (T == 0.f) return;
+  float m;
+  double z;
+  row_of_slices(slice_max, slice_sum, m, z);
+  const float zf = (float)z;
+  const bool nucleus = tp > 0.f && tp < 1.f;
   float* p = w.p + (long)row * V;
   unsigned long long mass = 0, cmass = 0;
   for (int base = lo; base < hi; base += 8 * 256) {
@@ -257,9 +318,10 @@ __global__ __launch_bounds__(256) void softmax_prob_kernel(const float* __restri
       if (tid == 0) bc_n = 0;
       __syncthreads();
     }
-    float v[8];
+    if (base != lo) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) { const int i = base + u * 256 + tid; v[u] = i < hi ? lg[i] : 0.f; }
+      for (int u = 0; u < 8; ++u) v[u] = lg[min(base + u * 256 + tid, V - 1)];
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int i = base + u * 256 + tid;
@@ -319,10 +381,21 @@ __global__ __launch_bounds__(SB) void sample_kernel(const float* __restrict__ lo
   __shared__ int winner;
   __shared__ float cand_p[CAND_MAX];
   __shared__ int cand_i[CAND_MAX];
-  __shared__ unsigned long long t_q[SB];
+  __shared__ unsigned long long t_q[SB + 8];
+  __shared__ unsigned long long bin_mass[BINS];
+  __shared__ int bin_cnt[BINS];
+  __shared__ int fill;
   const int row = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const float* lg = logits + (long)row * ld;
-  const float T = temperature[row];
+  // what the row's choice reads is asked for at once, the first candidates too, which are there or not
+  // (8 rows, some 20 candidates each: 9.5 -> 6.4 us, with the walk over the candidates eight at a time below)
+  const float T = temperature[row], tp = top_p[row];
+  const int n_cand = w.cand_count[row];
+  const unsigned long long c_mass = w.cand_mass[row];
+  const float first_p = w.cand_p[(long)row * CAND_MAX + tid];
+  const int first_i = w.cand_i[(long)row * CAND_MAX + tid];
+  // in a run of steps replayed from a graph the step's number is read from memory
+  const float uf = uniform[(step ? (long)step[0] * uniform_stride : 0) + row];
 
   if (T == 0.f) {
     float best = -INFINITY;
@@ -348,9 +421,7 @@ __global__ __launch_bounds__(SB) void sample_kernel(const float* __restrict__ lo
   }
 
   const float* p = w.p + (long)row * V;
-  const float tp = top_p[row];
-  // in a run of steps replayed from a graph the step's number is read from memory
-  const double u = (double)uniform[(step ? (long)step[0] * uniform_stride : 0) + row];
+  const double u = (double)uf;
   if (tid == 0) winner = -1;
   __syncthreads();
 
@@ -415,11 +486,11 @@ __global__ __launch_bounds__(SB) void sample_kernel(const float* __restrict__ lo
 
   // nucleus: the threshold value, the mass above it, and how many of the equal ones are kept
   const unsigned long long tq = (unsigned long long)((double)tp * QSCALE);
-  const int n_cand = w.cand_count[row];
-  if (n_cand <= CAND_MAX && w.cand_mass[row] > tq) {
+  if (n_cand <= CAND_MAX && c_mass > tq) {
     // the candidates alone exceed top_p: every probability from the threshold upwards is among them
     const int n = n_cand;
-    for (int a = tid; a < n; a += SB) {
+    if (tid < n) { cand_p[tid] = first_p; cand_i[tid] = first_i; }
+    for (int a = tid + SB; a < n; a += SB) {
       cand_p[a] = w.cand_p[(long)row * CAND_MAX + a];
       cand_i[a] = w.cand_i[(long)row * CAND_MAX + a];
     }
@@ -431,15 +502,21 @@ __global__ __launch_bounds__(SB) void sample_kernel(const float* __restrict__ lo
       float pa = 0.f;
       int ia = 0;
       unsigned long long qa = 0;
-      if (tid < n) { pa = cand_p[tid]; ia = cand_i[tid]; qa = to_q(pa); }
-      if (tid < n) t_q[tid] = qa;
-      if (tid == 0) res[0] = w.cand_mass[row];
+      if (tid < n) { pa = first_p; ia = first_i; qa = to_q(pa); }
+      t_q[tid] = qa;
+      if (tid >= n && tid < n + 8) cand_p[tid] = -1.f;      // (n is at most SB: up to eight entries behind the last, that count for nothing)
+      if (tid == 0) res[0] = c_mass;
       __syncthreads();
       unsigned long long excl = 0;
       if (tid < n)
-        for (int b = 0; b < n; ++b) {
-          const float pb = cand_p[b];
-          excl += (pb > pa || (pb == pa && cand_i[b] < ia)) ? t_q[b] : 0ull;
+        for (int b0 = 0; b0 < n; b0 += 8) {      // (eight at a time: a trip to shared memory for eight, not for each)
+          float pb[8];
+          int ib[8];
+          unsigned long long qb[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) { pb[k] = cand_p[b0 + k]; ib[k] = cand_i[b0 + k]; qb[k] = t_q[b0 + k]; }
+#pragma unroll
+          for (int k = 0; k < 8; ++k) excl += (pb[k] > pa || (pb[k] == pa && ib[k] < ia)) ? qb[k] : 0ull;
         }
       if (tid < n && excl <= tq && tq < excl + qa) res[0] = excl + qa;   // the last kept one: the kept mass
       __syncthreads();
@@ -450,45 +527,121 @@ __global__ __launch_bounds__(SB) void sample_kernel(const float* __restrict__ lo
       return;
     }
     const Found f1 = radix_search(cand_p, n, tq, h_mass, h_cnt, t_mass, t_cnt, res);
-    long k1 = 1;
-    if (f1.each > 0 && tq >= f1.above) k1 = (long)((tq - f1.above) / f1.each) + 1;
-    if (k1 > f1.ties) k1 = f1.ties;
-    if (k1 < 1) k1 = 1;
+    const long k1 = kept_ties(f1, tq);
     const unsigned long long mass = f1.above + (unsigned long long)k1 * f1.each;
     const unsigned long long target = (unsigned long long)(u * (double)mass);
     const Found f2 = radix_search(cand_p, n, target, h_mass, h_cnt, t_mass, t_cnt, res);
-    long j = (f2.each > 0 && target >= f2.above) ? (long)((target - f2.above) / f2.each) : 0;
-    const long limit = (f2.bits == f1.bits) ? k1 : (long)f2.ties;
-    if (j > limit - 1) j = limit - 1;
-    if (j < 0) j = 0;
-    const float want = __uint_as_float(f2.bits);
-    // the candidate with this probability that has exactly j equal ones of smaller index before it
-    for (int a = tid; a < n; a += SB) {
-      if (cand_p[a] != want) continue;
-      const int ia = cand_i[a];
-      long rank = 0;
-      for (int b = 0; b < n; ++b) rank += (cand_p[b] == want && cand_i[b] < ia) ? 1 : 0;
-      if (rank == j) winner = ia;
-    }
+    pick_equal(cand_p, cand_i, n, f1, k1, f2, target, &winner);
     __syncthreads();
     if (tid == 0) out[row] = winner >= 0 ? winner : V - 1;
     return;
   }
+
+  // A flat row, whose nucleus reaches below the candidates. One pass sorts the row's mass into bins of an eighth and less of a factor of two
+  // (exponent and four bits of the mantissa); the bin in which the mass exceeds top_p, and then the one that the drawn token lies in,
+  // are gathered from the row, and the searches walk those lists in shared memory: three passes over the row in place of nine
+  // whose first two put all of a row into a dozen bins (8 rows of 128,256, temperature 1.2, top-p 0.95: a call 324 -> 125 us; one row 312 -> 120, 64 rows 377 -> 163). A bin with more than CAND_MAX
+  // values (a distribution with hardly any) is left to the searches over the row below.
+  for (int i = tid; i < BINS; i += SB) { bin_mass[i] = 0; bin_cnt[i] = 0; }
+  __syncthreads();
+  for (int base = tid; base < V; base += UN * SB) {
+    float v[UN];
+#pragma unroll
+    for (int k = 0; k < UN; ++k) v[k] = base + k * SB < V ? p[base + k * SB] : -1.f;
+#pragma unroll
+    for (int k = 0; k < UN; ++k)
+      if (v[k] >= 0.f) {
+        const uint32_t b = __float_as_uint(v[k]) >> BIN_SHIFT;
+        atomicAdd(&bin_mass[b], to_q(v[k]));
+        atomicAdd(&bin_cnt[b], 1);
+      }
+  }
+  __syncthreads();
+  int n = 0, n_bin = -1;
+  // the values of the bin where the mass from the top exceeds thr (the lowest bin with any if none does), and the mass above that bin
+  auto gather = [&](unsigned long long thr, unsigned long long& above) {
+    if (wave == 0) {
+      // lane l owns bins BINS - 1 - 32 l downwards
+      unsigned long long mine = 0;
+      int cnt_mine = 0;
+      for (int k = 0; k < BINS / 64; ++k) { mine += bin_mass[BINS - 1 - lane * (BINS / 64) - k]; cnt_mine += bin_cnt[BINS - 1 - lane * (BINS / 64) - k]; }
+      unsigned long long incl = mine;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+      }
+      const unsigned long long hit = __ballot(incl > thr), some = __ballot(cnt_mine > 0);
+      const int who = hit ? __ffsll((long long)hit) - 1 : some ? 63 - __builtin_clzll(some) : 0;
+      if (lane == who) {
+        unsigned long long cum = incl - mine, at = cum;
+        int bin = -1;
+        for (int k = 0; k < BINS / 64; ++k) {
+          const int b = BINS - 1 - lane * (BINS / 64) - k;
+          if (bin_cnt[b] > 0) { bin = b; at = cum; }
+          if (hit && cum + bin_mass[b] > thr) break;
+          cum += bin_mass[b];
+        }
+        res[0] = (unsigned long long)(long long)bin;
+        res[1] = at;
+      }
+    }
+    __syncthreads();
+    const int bin = (int)(long long)res[0];
+    above = res[1];
+    const int found = bin < 0 ? -1 : bin_cnt[bin];
+    if (found < 0 || found > CAND_MAX) return found;
+    if (bin != n_bin) {
+      n_bin = bin;
+      n = found;
+      if (tid == 0) fill = 0;
+      __syncthreads();
+      for (int base = tid; base < V; base += UN * SB) {
+        float v[UN];
+#pragma unroll
+        for (int k = 0; k < UN; ++k) v[k] = base + k * SB < V ? p[base + k * SB] : -1.f;
+#pragma unroll
+        for (int k = 0; k < UN; ++k)
+          if (v[k] >= 0.f && (int)(__float_as_uint(v[k]) >> BIN_SHIFT) == bin) {
+            const int slot = atomicAdd(&fill, 1);
+            cand_p[slot] = v[k];
+            cand_i[slot] = base + k * SB;
+          }
+      }
+    }
+    __syncthreads();
+    return found;
+  };
+  unsigned long long over1 = 0, over2 = 0;
+  const int found1 = gather(tq, over1);
+  if (found1 < 0) {                 // (not a number in the row: the last index)
+    if (tid == 0) out[row] = V - 1;
+    return;
+  }
+  if (found1 <= CAND_MAX) {
+    Found f1 = radix_search(cand_p, n, tq - over1, h_mass, h_cnt, t_mass, t_cnt, res);
+    f1.above += over1;
+    const long k1 = kept_ties(f1, tq);
+    const unsigned long long mass = f1.above + (unsigned long long)k1 * f1.each;
+    const unsigned long long target = (unsigned long long)(u * (double)mass);
+    const int found2 = gather(target, over2);
+    if (found2 >= 0 && found2 <= CAND_MAX) {
+      Found f2 = radix_search(cand_p, n, target > over2 ? target - over2 : 0ull, h_mass, h_cnt, t_mass, t_cnt, res);
+      f2.above += over2;
+      pick_equal(cand_p, cand_i, n, f1, k1, f2, target, &winner);
+      __syncthreads();
+      if (tid == 0) out[row] = winner >= 0 ? winner : V - 1;
+      return;
+    }
+  }
   const Found f1 = radix_search(p, V, tq, h_mass, h_cnt, t_mass, t_cnt, res);
-  long k1 = 1;
-  if (f1.each > 0 && tq >= f1.above) k1 = (long)((tq - f1.above) / f1.each) + 1;   // smallest k with above + k*each > tq
-  if (k1 > f1.ties) k1 = f1.ties;
-  if (k1 < 1) k1 = 1;
+  const long k1 = kept_ties(f1, tq);
   const unsigned long long mass = f1.above + (unsigned long long)k1 * f1.each;
   // the drawn token: first in the kept order whose running sum exceeds u * mass
   const unsigned long long target = (unsigned long long)(u * (double)mass);
   const Found f2 = radix_search(p, V, target, h_mass, h_cnt, t_mass, t_cnt, res);
-  long j = (f2.each > 0 && target >= f2.above) ? (long)((target - f2.above) / f2.each) : 0;
-  const long limit = (f2.bits == f1.bits) ? k1 : (long)f2.ties;
-  if (j > limit - 1) j = limit - 1;
-  if (j < 0) j = 0;
   const float want_value = __uint_as_float(f2.bits);   // the drawn token is the `want_index`-th (from 0) with this
-  const long want_index = j;                           // probability, in ascending order of index
+  const long want_index = drawn_tie(f1, k1, f2, target);   // probability, in ascending order of index
 
   // every wave owns a contiguous range of the row, a multiple of 64 long
   const int per = ((V + SW - 1) / SW + 63) / 64 * 64;
@@ -682,6 +835,15 @@ extern "C" long gl3_sample_work_floats(int n_rows, int V) {
   return (((long)n_rows * V + 1) & ~1L) + (long)n_rows * SAMPLE_ROW_FLOATS;
 }
 
+static int launch_choice(const float* logits, long ld, const SampleWork& w, const float* temperature, const float* top_p,
+                         const float* uniform, int* out, int n_rows, int V, const int* step, int uniform_stride, hipStream_t stream) {
+  softmax_prob_kernel<<<dim3(n_rows, ST_SLICES), dim3(256), 0, stream>>>(logits, ld, temperature, top_p, w, V);
+  GL3_LAUNCH_CHECK();
+  sample_kernel<<<dim3(n_rows), dim3(SB), 0, stream>>>(logits, ld, w, temperature, top_p, uniform, out, V, step, uniform_stride);
+  GL3_LAUNCH_CHECK();
+  return 0;
+}
+
 // work: gl3_sample_work_floats(n_rows, V) floats of scratch, 8-byte aligned.
 // step (may be null): a counter in device memory; row r then takes uniform[step[0] * uniform_stride + r].
 extern "C" int gl3_sample(const float* logits, long ld, float* work, const float* temperature, const float* top_p,
@@ -693,35 +855,17 @@ extern "C" int gl3_sample(const float* logits, long ld, float* work, const float
               ld);
   GL3_REQUIRE((uintptr_t)work % 8 == 0, "gl3_sample: the scratch must be 8-byte aligned");
   const SampleWork w = carve_sample_work(work, n_rows, V);
-  const dim3 slices(n_rows, ST_SLICES);
-  softmax_max_kernel<<<slices, dim3(256), 0, stream>>>(logits, ld, temperature, w, V);
+  softmax_slices_kernel<<<dim3(n_rows, ST_SLICES), dim3(256), 0, stream>>>(logits, ld, temperature, SampleNoArgs{}, nullptr, n_rows, w, V);
   GL3_LAUNCH_CHECK();
-  softmax_sum_kernel<<<slices, dim3(256), 0, stream>>>(logits, ld, temperature, w, V);
-  GL3_LAUNCH_CHECK();
-  softmax_prob_kernel<<<slices, dim3(256), 0, stream>>>(logits, ld, temperature, top_p, w, V);
-  GL3_LAUNCH_CHECK();
-  sample_kernel<<<dim3(n_rows), dim3(SB), 0, stream>>>(logits, ld, w, temperature, top_p, uniform, out, V, step,
-                                                       uniform_stride);
-  GL3_LAUNCH_CHECK();
-  return 0;
+  return launch_choice(logits, ld, w, temperature, top_p, uniform, out, n_rows, V, step, uniform_stride, stream);
 }
 
 // A whole call of a sampler whose caller waits for the tokens: parameters in host memory, tokens into host memory. The parameters
-// travel inside a small kernel's launch and the tokens are written by the last kernel into pinned memory (`out`: hipHostMalloc's, which
+// travel inside the first kernel's launch and the tokens are written by the last kernel into pinned memory (`out`: hipHostMalloc's, which
 // the GPU reaches under the host's address), so a call has no copy to wait for on either side, only the stream's end: 8 rows of
-// 128,256 logits 62 -> 48 us a call, of which the four kernels take 28 and this one 2.
+// 128,256 logits 39 us a call, of which the three kernels take 20 (48 with a kernel for the parameters and one more for the softmax).
 // work: gl3_sample_work_floats(n_rows, V) floats and 3 * n_rows for the parameters. temperature null: every row greedy (work as
 // gl3_argmax's). The stream must not be capturing.
-#define SAMPLE_STAGED 256
-struct SampleArgs { float v[3][SAMPLE_STAGED]; };
-
-__global__ __launch_bounds__(SAMPLE_STAGED) void stage_sample_kernel(float* __restrict__ dst, int first, int n_rows, SampleArgs a) {
-  const int i = threadIdx.x, row = first + i;
-  if (row >= n_rows) return;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) dst[(long)k * n_rows + row] = a.v[k][i];
-}
-
 extern "C" int gl3_sample_host(const float* logits, long ld, float* work, const float* temperature, const float* top_p,
                                const float* uniform, int* out, int n_rows, int V, hipStream_t stream) {
   if (n_rows == 0) return 0;
@@ -729,17 +873,24 @@ extern "C" int gl3_sample_host(const float* logits, long ld, float* work, const 
   int rc;
   if (temperature) {
     GL3_REQUIRE(top_p && uniform, "gl3_sample_host: null argument");
+    GL3_REQUIRE(n_rows <= 65535 && ld >= V && (uintptr_t)work % 8 == 0, "gl3_sample_host: bad sizes (rows=%d V=%d ld=%ld) or scratch", n_rows, V, ld);
+    const SampleWork w = carve_sample_work(work, n_rows, V);
     float* par = work + gl3_sample_work_floats(n_rows, V);
-    const float* from[3] = {temperature, top_p, uniform};
+    // (SAMPLE_STAGED rows at a time: their parameters are 3 KB of a launch's arguments)
     for (int first = 0; first < n_rows; first += SAMPLE_STAGED) {
       SampleArgs a;
       const int count = n_rows - first < SAMPLE_STAGED ? n_rows - first : SAMPLE_STAGED;
-      for (int k = 0; k < 3; ++k)
-        for (int i = 0; i < SAMPLE_STAGED; ++i) a.v[k][i] = i < count ? from[k][first + i] : 0.f;
-      stage_sample_kernel<<<dim3(1), dim3(SAMPLE_STAGED), 0, stream>>>(par, first, n_rows, a);
+      for (int i = 0; i < count; ++i) { a.v[0][i] = temperature[first + i]; a.v[1][i] = top_p[first + i]; a.v[2][i] = uniform[first + i]; }
+      for (int i = count; i < SAMPLE_STAGED; ++i) a.v[0][i] = a.v[1][i] = a.v[2][i] = 0.f;
+      SampleWork part = w;      // (what the slices' kernel writes, from row `first` on)
+      part.slice_sum += (long)first * ST_SLICES;
+      part.slice_max += (long)first * ST_SLICES;
+      part.cand_mass += first;
+      part.cand_count += first;
+      softmax_slices_kernel<<<dim3(count, ST_SLICES), dim3(256), 0, stream>>>(logits + (long)first * ld, ld, nullptr, a, par + first, n_rows, part, V);
       GL3_LAUNCH_CHECK();
     }
-    rc = gl3_sample(logits, ld, work, par, par + n_rows, par + 2L * n_rows, out, n_rows, V, nullptr, 0, stream);
+    rc = launch_choice(logits, ld, w, par, par + n_rows, par + 2L * n_rows, out, n_rows, V, nullptr, 0, stream);
   } else {
     rc = gl3_argmax(logits, ld, work, out, n_rows, V, stream);
   }

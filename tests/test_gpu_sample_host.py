@@ -68,3 +68,50 @@ def test_calls_of_two_threads(own_streams):
             return sum(sampler(logits, *par) != want for _ in range(100))
     with ThreadPoolExecutor(2) as threads:
         assert list(threads.map(calls_of, range(2))) == [0, 0]
+
+
+def _flat(kind, rows, V, rng):
+    if kind == "normal":                    # a nucleus of thousands, in many bins
+        return rng.standard_normal((rows, V)) * 1.5
+    if kind == "ties":                      # hundreds of equal values at every place
+        return rng.integers(0, 40, (rows, V)) / 8.0
+    if kind == "two values":                # the threshold and the drawn token in a bin with more values than the lists hold, or in the other
+        return np.where(rng.random((rows, V)) < 0.5, 0.0, -0.5)
+    if kind == "equal":                     # one value: no bin is short enough
+        return np.zeros((rows, V))
+    x = rng.standard_normal((rows, V))      # most of the row without any probability
+    x[:, V // 2:] = -np.inf
+    return x
+
+
+# (short rows, the last slices empty; a vocabulary whose slices are two stretches; lists at, below and beyond their length)
+@pytest.mark.parametrize("kind", ["normal", "ties", "two values", "equal", "half"])
+@pytest.mark.parametrize("V", [70, 8192, 16500, 128256, 140001])
+def test_flat_rows(kind, V):
+    """Rows whose nucleus reaches below the gathered candidates take the bins; the tokens are the definition's."""
+    rng = np.random.default_rng(V)
+    rows = 24
+    x = _flat(kind, rows, V, rng).astype(np.float32)
+    par = [[1.0] * rows, rng.choice([0.3, 0.7, 0.95, 0.999], rows).tolist(), rng.random(rows).astype(np.float32).tolist()]
+    got = DeviceSampler(torch.device("cuda:0"))(torch.from_numpy(x).cuda(), *par)
+    want = [sample_host(x[r], *(p[r] for p in par)) for r in range(rows)]
+    order = [np.lexsort((np.arange(V), -x[r].astype(np.float64))) for r in range(rows)]
+    place = [np.argsort(o) for o in order]
+    # p is off by a few 2^-24 of itself, the running sum of the nucleus by as much of its mass, so a drawn token stands at most as many places
+    # from the definition's as such an error spans: 2^-20 of the row's mass over the token's own probability, and one (where all values
+    # are equal a third of the tokens are the neighbour)
+    p = [np.exp(r.astype(np.float64) - r.max()) for r in x]
+    for r in range(rows):
+        span = 2.0 ** -20 * p[r].sum() / p[r][want[r]] + 1.0
+        assert abs(int(place[r][got[r]]) - int(place[r][want[r]])) <= span, (r, got[r], want[r])
+
+
+def test_a_row_without_a_number():
+    """Nothing to choose from (no finite maximum): a token of the vocabulary all the same, and the rows beside it are as alone."""
+    x = torch.randn(3, 5000, generator=torch.Generator().manual_seed(2))
+    alone = DeviceSampler(torch.device("cuda:0"))(x.cuda(), [0.9] * 3, [0.9] * 3, [0.3] * 3)
+    for bad in (float("nan"), float("-inf")):
+        y = x.clone()
+        y[1] = bad
+        got = DeviceSampler(torch.device("cuda:0"))(y.cuda(), [0.9] * 3, [0.9] * 3, [0.3] * 3)
+        assert [got[0], got[2]] == [alone[0], alone[2]] and 0 <= got[1] < 5000
