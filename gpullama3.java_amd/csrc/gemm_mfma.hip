@@ -399,6 +399,23 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
           acc[ah][tm][wh][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[wh][tn][ks], af[ah][tm][ks], acc[ah][tm][wh][tn], 0, 0, 0);
   };
 
+  // The rows that an add reads. With one half of A there are registers for all of them beside the sums: they are asked for in the
+  // last three steps in the place of loads beyond the last step (as many, so that the counts hold), and come while those are
+  // multiplied (beyond the matrix: its last row and columns again). In the slices of their plans, 2,048 rows of the 1B layers: output projection
+  // 25.5 -> 23.0 us, down 61.9 -> 60.0; 512 rows of the 3B layers 20.7 -> 19.1 and 32.2 -> 31.4; 4,096 rows x 2,048 x 2,048 38.3 -> 35.5. The tile of
+  // 256 x 256 has no registers left and reads them behind the last step.
+  const int col0 = n0 + (EPI == MF_GATED && WH == 1 ? wn * 16 : wn * 32), row0 = m0 + wm * 64 + lr;
+  const bool vec = ldc % 4 == 0 && N % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;
+  typedef TC tc4 __attribute__((ext_vector_type(4)));
+  constexpr bool ADDS = EPI == MF_ADD;
+  tc4 old[ADDS ? 8 * WH : 1];
+  auto ask_old = [&](int ah, int i) {
+    const int tm = i / (2 * WH), wh = i / 2 % WH, tn = i % 2;
+    old[ADDS ? i : 0] = *(const tc4*)(C + (long)min(row0 + ah * 128 + tm * 16, M - 1) * ldc + min(col0 + wh * 128 + tn * 16 + lq * 4, N - 4));
+  };
+  const bool early = ADDS && AH == 1 && vec && slice == 0 && steps >= 3;
+  const int plain_steps = early ? steps - 3 : steps;
+
   if constexpr (AH == 2) {
     load_a(0, 0, 0);
     load_w(1, 0, 0);
@@ -458,19 +475,30 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
     mf_wait_loads<12>();
     mf_barrier();
     if (wm == 1) mf_barrier();
-    for (int t = 0, here = 0, before = 2 * STAGE; t < steps; ++t) {
+    int here = 0, before = 2 * STAGE;
+    auto step = [&](int t, auto tail) {       // tail: 0, or the step is the first, second or third of the last three and asks for rows
+      constexpr int TAIL = decltype(tail)::value;
       read_a(0, here, 0);
       read_a(0, here, 1);
       read_w(0, here);
-      load_w(1, t + 2, before);
+      if constexpr (TAIL < 2) load_w(1, t + 2, before);
+      else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) ask_old(0, (TAIL == 2 ? 4 : 10) + i);
+      }
       mf_wait_loads<12>();              // this step's W1 has come
       mf_wait_reads<0>();
       mf_barrier();
       products(0, 0);
       mf_barrier();
       read_w(1, here);
-      load_a(0, t + 3, here);
-      load_w(0, t + 3, here);
+      if constexpr (TAIL == 0) {
+        load_a(0, t + 3, here);
+        load_w(0, t + 3, here);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ask_old(0, (TAIL - 1) * 6 + i);
+      }
       mf_wait_loads<12>();              // the next step's A and W0 have
       mf_wait_reads<0>();
       mf_barrier();
@@ -478,6 +506,14 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
       mf_barrier();
       before = here;
       here = here == 2 * STAGE ? 0 : here + STAGE;
+    };
+    for (int t = 0; t < plain_steps; ++t) step(t, std::integral_constant<int, 0>{});
+    if constexpr (ADDS) {
+      if (early) {
+        step(steps - 3, std::integral_constant<int, 1>{});
+        step(steps - 2, std::integral_constant<int, 2>{});
+        step(steps - 1, std::integral_constant<int, 3>{});
+      }
     }
   } else {
     // 128 x 128: one phase a step, four steps in shared memory.
@@ -490,12 +526,19 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
     mf_wait_loads<8>();
     mf_barrier();
     if (wm == 1) mf_barrier();
-    for (int t = 0, here = 0, before = 3 * STAGE; t < steps; ++t) {
+    int here = 0, before = 3 * STAGE;
+    auto step = [&](int t, auto tail) {       // (tail as above; the third asks for nothing but repeats the last step)
+      constexpr int TAIL = decltype(tail)::value;
       read_a(0, here, 0);
       read_w(0, here);
       read_a(0, here, 1);
-      load_a(0, t + 3, before);         // (where the step before lay, which both groups have read)
-      load_w(0, t + 3, before);
+      if constexpr (TAIL == 1 || TAIL == 2) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ask_old(0, (TAIL - 1) * 4 + i);
+      } else {
+        load_a(0, t + 3, before);       // (where the step before lay, which both groups have read)
+        load_w(0, t + 3, before);
+      }
       mf_wait_loads<8>();               // the next step has come
       mf_wait_reads<0>();
       mf_barrier();
@@ -503,6 +546,14 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
       mf_barrier();
       before = here;
       here = here == 3 * STAGE ? 0 : here + STAGE;
+    };
+    for (int t = 0; t < plain_steps; ++t) step(t, std::integral_constant<int, 0>{});
+    if constexpr (ADDS) {
+      if (early) {
+        step(steps - 3, std::integral_constant<int, 1>{});
+        step(steps - 2, std::integral_constant<int, 2>{});
+        step(steps - 1, std::integral_constant<int, 3>{});
+      }
     }
   }
   if (wm == 0) mf_barrier();
@@ -517,7 +568,6 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   // 16,384 910 -> 790, of 8,192 of the 8B layers 1,379 -> 1,283; QKV of 2,048 rows 30.1 -> 27.8, of 512 rows of the 3B layers
   // 26.1 -> 24.7; the output projection of 5,886 rows of the 3B layers, which reads the rows it adds to, 137 -> 132 (110 without);
   // a head's 2,221 x 128,256 floats, bound by their way to memory, 1,048 to 1,090 on both.
-  const int col0 = n0 + (EPI == MF_GATED && WH == 1 ? wn * 16 : wn * 32), row0 = m0 + wm * 64 + lr;
   auto finish = [&](auto plain_t) {
     constexpr bool PLAIN = decltype(plain_t)::value;
     // columns n .. n + 3, ready to be stored (an add's old values aside)
@@ -571,19 +621,11 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
         return;
       }
     }
-    const bool vec = ldc % 4 == 0 && N % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;
-    typedef TC tc4 __attribute__((ext_vector_type(4)));
 #pragma unroll
     for (int ah = 0; ah < AH; ++ah) {
-      tc4 old[4][WH][2];
-      if (EPI == MF_ADD && vec) {       // (all asked for before the first is needed; beyond the matrix: its last row and columns again)
+      if (ADDS && vec && !early) {      // (all asked for before the first is needed)
 #pragma unroll
-        for (int tm = 0; tm < 4; ++tm)
-#pragma unroll
-          for (int wh = 0; wh < HALVES; ++wh)
-#pragma unroll
-            for (int tn = 0; tn < TILES; ++tn)
-              old[tm][wh][tn] = *(const tc4*)(C + (long)min(row0 + ah * 128 + tm * 16, M - 1) * ldc + min(col0 + wh * 128 + tn * 16 + lq * 4, N - 4));
+        for (int i = 0; i < 8 * WH; ++i) ask_old(ah, i);
       }
 #pragma unroll
       for (int tm = 0; tm < 4; ++tm)
@@ -598,7 +640,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
             if (vec) {
               tc4 o;
 #pragma unroll
-              for (int j = 0; j < 4; ++j) o[j] = from_f32<TC>(EPI == MF_ADD ? to_f32<TC>(old[tm][wh][tn][j]) + v[j] : v[j]);
+              for (int j = 0; j < 4; ++j) o[j] = from_f32<TC>(ADDS ? to_f32<TC>(old[ADDS ? (tm * WH + wh) * 2 + tn : 0][j]) + v[j] : v[j]);
               *(tc4*)c = o;
             } else {
 #pragma unroll
@@ -610,7 +652,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   };
   if (EPI != MF_GATED && slice > 0) {
     float* const p = P + (long)(slice - 1) * p_stride;
-    const bool vec = ldp % 4 == 0 && N % 4 == 0 && (uintptr_t)p % 16 == 0;
+    const bool whole = ldp % 4 == 0 && N % 4 == 0 && (uintptr_t)p % 16 == 0;
 #pragma unroll
     for (int ah = 0; ah < AH; ++ah)
 #pragma unroll
@@ -627,7 +669,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
               for (int j = 0; j < 4; ++j) v[j] *= ex.col_scale[min(n + j, N - 1)];
             }
             float* c = p + (long)row * ldp + n;
-            if (vec) *(f32x4*)c = v;
+            if (whole) *(f32x4*)c = v;
             else {
 #pragma unroll
               for (int j = 0; j < 4; ++j)
