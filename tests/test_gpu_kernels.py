@@ -1476,3 +1476,31 @@ def test_rows_handed_over_in_the_packed_order(M, d, F):
         assert torch.equal(got, plain)
     with pytest.raises(lib.KernelError):
         lib.gemm_skinny(packed, w2, dev(res0), lib.EPI_ADD, strip_rows=16, a_packed=True)
+
+
+# (a thread's piece: none beside the first, the last one alone, one each, and the widths where the number of threads changes)
+@pytest.mark.parametrize("d", [4, 8, 252, 1024, 1028, 2044, 2048, 3072, 4092, 4096, 4100])
+@pytest.mark.parametrize("S", [0, 1, 2, 3, 4, 5, 8, 9])
+def test_norms_of_rows_held_at_once(d, S):
+    """Rows that a block holds at once against the kernels for any rows, which a weight at an odd place asks for: the same bits."""
+    lib = K()
+    gen = torch.Generator(device="cuda").manual_seed(d + S)
+    n = 5
+    x = torch.randn(n, d, generator=gen, device="cuda")
+    parts = torch.randn(S, n, d, generator=gen, device="cuda") if S else None
+    rows = torch.tensor([3, 0, 3], dtype=torch.int32, device="cuda")
+    for wdtype in (torch.float32, torch.bfloat16):
+        odd = torch.empty(d + 1, device="cuda", dtype=wdtype)[1:]
+        odd.copy_(1.0 + 0.1 * torch.randn(d, generator=gen, device="cuda"))
+        whole = odd.clone()
+        for odtype in (torch.float32, torch.bfloat16):
+            for r in (None, rows):
+                got = []
+                for w in (whole, odd):
+                    X, out = x.clone(), torch.full((n if r is None else 3, d), -7.0, device="cuda", dtype=odtype)
+                    if S:
+                        lib.add_slices_rmsnorm(X, parts, w, out, 1e-5, r)
+                    else:
+                        lib.rmsnorm(X, w, out, 1e-5, r)
+                    got.append((X, out))
+                assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (wdtype, odtype, r is None)
