@@ -103,14 +103,14 @@ extern "C" int gl3_embed(const void* table, int table_dtype, const int* ids, flo
 }
 
 // ----------------------------------------------------------------- rmsnorm of rows that a block holds at once
-// What rmsnorm_kernel and add_slices_rmsnorm_kernel (below) do, the same bits, for rows of whole 16-byte pieces of which a thread has one
-// at most (up to 4,096 floats: the launchers' threads are as many there) and NS slices (0: none; 8: five to eight, the ones that
+// What rmsnorm_kernel and add_slices_rmsnorm_kernel (below) do, the same bits, for rows of whole 16-byte pieces of which a thread has PIECES
+// at most (one up to 2,048 floats and at 4,096, two up to 8,192: the launchers' threads are as many there) and NS slices (0: none; 8: five to eight, the ones that
 // do not exist read the last again and are not added). These norms of few rows are bound by trips to memory one after the other: there
 // it was the row, then its slices (a branch for each, in front of which the compiler waits), then, behind the sum of squares, the weight; here
 // all of them are asked for at once, and the waves' sums are read at once as well. In a replayed graph, 64 rows of 2,048 with four slices 3.85 ->
-// 3.16 us, 150 of 4,096 with seven 7.8 -> 7.2; 2,048 rows of 2,048 with one slice 15.3 -> 12.7, 8,192 of 4,096 without 47 -> 39 (bound by
-// memory: 5.2 TB/s).
-template <typename TW, typename TO, int NS>
+// 3.13 us, 150 of 4,096 with seven 7.6 -> 7.2; 2,048 rows of 2,048 with one slice 15.4 -> 12.5, 8,192 of 4,096 without 47 -> 39, 5,886 of 3,072 with
+// two 52 -> 48 (bound by memory: 5 to 6.8 TB/s).
+template <typename TW, typename TO, int NS, int PIECES>
 __global__ __launch_bounds__(1024) void norm_rows_kernel(float* __restrict__ x, const int* __restrict__ rows, const float* __restrict__ P,
                                                          int n_slices, long slice_stride, long ldp, const TW* __restrict__ w,
                                                          TO* __restrict__ out, int d, float eps) {
@@ -118,24 +118,34 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(float* __restrict__ x, 
   typedef TW w4 __attribute__((ext_vector_type(4)));
   typedef TO o4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) float sums[16];
-  const int tid = threadIdx.x, i = tid * 4, at = min(i, d - 4);      // (threads beyond the row read its end again)
+  const int tid = threadIdx.x, first = tid * 4, stride = blockDim.x * 4;
   const long r = blockIdx.x, src = rows ? rows[r] : r;
   float* const xr = x + src * d;
-  f4 v = *(const f4*)(xr + at), p[NS > 0 ? NS : 1];
+  f4 v[PIECES], p[PIECES][NS > 0 ? NS : 1];
+  w4 wv[PIECES];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) p[s] = *(const f4*)(P + (long)(NS == 8 ? min(s, n_slices - 1) : s) * slice_stride + src * ldp + at);
-  const w4 wv = *(const w4*)(w + at);
+  for (int k = 0; k < PIECES; ++k) {
+    const int at = min(first + k * stride, d - 4);      // (what is beyond the row reads its end again)
+    v[k] = *(const f4*)(xr + at);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) p[k][s] = *(const f4*)(P + (long)(NS == 8 ? min(s, n_slices - 1) : s) * slice_stride + src * ldp + at);
+    wv[k] = *(const w4*)(w + at);
+  }
   __builtin_amdgcn_sched_barrier(0);
+  float ss = 0.f;
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    if (NS < 8 || s < n_slices) v += p[s];
-  const bool mine = i < d;
-  if (NS > 0 && !rows && mine) *(f4*)(xr + i) = v;
-  float ss = v[0] * v[0];              // (fused by hand: which product of a sum of two the compiler fuses is its own choice)
+  for (int k = 0; k < PIECES; ++k) {
 #pragma unroll
-  for (int e = 1; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
-  ss = wave_sum(mine ? ss : 0.f);
-  if (tid < 16) sums[tid] = 0.f;       // (wave 0's, in front of its own sum: no barrier between them)
+    for (int s = 0; s < NS; ++s)
+      if (NS < 8 || s < n_slices) v[k] += p[k][s];
+    const int i = first + k * stride;
+    if (i >= d) continue;
+    if (NS > 0 && !rows) *(f4*)(xr + i) = v[k];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = fmaf(v[k][e], v[k][e], ss);      // (fused by hand: which of two products the compiler fuses is its own choice)
+  }
+  ss = wave_sum(ss);
+  if (tid < 16) sums[tid] = 0.f;
   __syncthreads();
   if (tid % 64 == 0) sums[tid >> 6] = ss;
   __syncthreads();
@@ -149,23 +159,32 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(float* __restrict__ x, 
   total = total / (float)d;
   total = total + eps;
   total = 1.0f / sqrtf(total);
-  if (!mine) return;
-  o4 res;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) res[e] = from_f32<TO>(to_f32<TW>(wv[e]) * (total * v[e]));
-  *(o4*)(out + r * d + i) = res;
+  for (int k = 0; k < PIECES; ++k) {
+    const int i = first + k * stride;
+    if (i >= d) continue;
+    o4 res;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) res[e] = from_f32<TO>(to_f32<TW>(wv[k][e]) * (total * v[k][e]));
+    *(o4*)(out + r * d + i) = res;
+  }
 }
 
 // Whether norm_rows_kernel takes these rows (with `threads` threads a row); the launch. P null: no slices.
 static bool norm_rows_takes(const void* x, const void* P, int n_slices, long slice_stride, long ldp, const void* w, int w_dtype, const void* out,
                             int d, int threads) {
-  return d % 4 == 0 && d <= 4 * threads && n_slices <= 8 && ldp % 4 == 0 && slice_stride % 4 == 0 && (uintptr_t)x % 16 == 0 &&
+  return d % 4 == 0 && d <= 8 * threads && n_slices <= 8 && ldp % 4 == 0 && slice_stride % 4 == 0 && (uintptr_t)x % 16 == 0 &&
          (uintptr_t)P % 16 == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)w % (w_dtype == GL3_F32 ? 16 : 8) == 0;
 }
 template <typename TW, typename TO>
 static void launch_norm_rows(float* x, const int* rows, const float* P, int n_slices, long slice_stride, long ldp, const void* w, void* out,
                              int n_rows, int d, float eps, int threads, hipStream_t stream) {
-#define GO(NS) norm_rows_kernel<TW, TO, NS><<<dim3(n_rows), dim3(threads), 0, stream>>>(x, rows, P, n_slices, slice_stride, ldp, (const TW*)w, (TO*)out, d, eps)
+#define ARGS <<<dim3(n_rows), dim3(threads), 0, stream>>>(x, rows, P, n_slices, slice_stride, ldp, (const TW*)w, (TO*)out, d, eps)
+#define GO(NS)                                                \
+  do {                                                        \
+    if (d <= 4 * threads) norm_rows_kernel<TW, TO, NS, 1> ARGS; \
+    else norm_rows_kernel<TW, TO, NS, 2> ARGS;                  \
+  } while (0)
   switch (P ? n_slices : 0) {
     case 0: GO(0); break;
     case 1: GO(1); break;
@@ -175,6 +194,7 @@ static void launch_norm_rows(float* x, const int* rows, const float* P, int n_sl
     default: GO(8);
   }
 #undef GO
+#undef ARGS
 }
 
 // ----------------------------------------------------------------- rmsnorm
@@ -412,8 +432,8 @@ __global__ void rope_cache_kernel(T* __restrict__ qkv, const int* __restrict__ p
     const int i1 = adjacent ? 2 * j + 1 : j + half;
     const float c = cos_tab[(long)pos * half + j], s = sin_tab[(long)pos * half + j];
     const float v0 = to_f32<T>(src[i0]), v1 = to_f32<T>(src[i1]);
-    put(i0, from_f32<T>(v0 * c - v1 * s));
-    put(i1, from_f32<T>(v0 * s + v1 * c));
+    put(i0, from_f32<T>(fmaf(v0, c, -(v1 * s))));      // (fused by hand, as the product that turns its own sums does: gemm_f32.hip)
+    put(i1, from_f32<T>(fmaf(v0, s, v1 * c)));
   }
   if (kpage)
     for (int i = rot_dim + threadIdx.x; i < head_dim; i += blockDim.x) put(i, src[i]);

@@ -1478,8 +1478,9 @@ def test_rows_handed_over_in_the_packed_order(M, d, F):
         lib.gemm_skinny(packed, w2, dev(res0), lib.EPI_ADD, strip_rows=16, a_packed=True)
 
 
-# (a thread's piece: none beside the first, the last one alone, one each, and the widths where the number of threads changes)
-@pytest.mark.parametrize("d", [4, 8, 252, 1024, 1028, 2044, 2048, 3072, 4092, 4096, 4100])
+# (a thread's pieces: none beside the first, the last one alone, one each, two for some and for all, and the widths where the number of
+# threads changes)
+@pytest.mark.parametrize("d", [4, 8, 252, 1024, 1028, 2044, 2048, 2052, 3072, 4092, 4096, 4100, 8192, 8196])
 @pytest.mark.parametrize("S", [0, 1, 2, 3, 4, 5, 8, 9])
 def test_norms_of_rows_held_at_once(d, S):
     """Rows that a block holds at once against the kernels for any rows, which a weight at an odd place asks for: the same bits."""
