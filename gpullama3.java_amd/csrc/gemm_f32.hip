@@ -22,6 +22,7 @@
 //   the 1B layers 57 to 90 TFLOP/s, against about 20 of the kernel for any sizes.
 #include "common.h"
 #include "lds_loads.h"
+#include <algorithm>
 #include <type_traits>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -199,6 +200,165 @@ __global__ __launch_bounds__(64 * F3_WAVES) void gemm_f32_rows_kernel(const floa
     const int l = (e >> 2) & 63, m = (e >> 8) * 16 + (l & 15), n = n0 + 4 * (l >> 4) + (e & 3);
     if (e < 256 * TM && m < M && n < N) f3_finish<EPI>(C + (long)m * ldc + n, total[0][i], total[G - 1][i], n, N, o);
   }
+}
+
+// ---- at most four rows: norm, the product with the stacked q, k, v rows, rotation and cache write in one kernel
+//
+// A decode step of a few sequences is a chain of short kernels: norm, product and rotation took 4.8, 8.4 and 5.4 us of a layer's 89 under the
+// profiler (1B layers, two tokens), this one takes 11.9; without it a step of 16 layers 1.60 -> 1.56 ms, for a small kernel of a replayed graph
+// costs some 2 us there. Every block works out the norm of the rows itself (8 KB each, in the second-level cache) while its first weights
+// are on their way: the sums of squares by as many threads, in the same order, as gl3_rmsnorm's kernels have a row, so the normalised rows
+// are the same bits, and so is everything behind them. They lie in shared memory, where all waves read them: from memory, beside the norm's
+// weight, they were as many requests as W's rows (15.6 us). A block's sixteen rows of W are eight pairs that the rotation turns (or
+// sixteen rows of a value head), and its sums, turned as rope_cache_kernel turns them, go to the query rows and into the pages of the cache.
+// The gated product behind its norm the same way was slower (41 us against 29 and 4.8: its 512 blocks, two a CU, have 64
+// registers a lane, too few for the norm's operands beside the weights' loads) and keeps its norm in front.
+struct F3Norm {
+  const float* w;
+  float eps;
+  int threads;      // that gl3_rmsnorm's kernels give a row
+};
+struct F3Rope {
+  const int *positions, *table_rows, *block_table;
+  int table_stride;
+  const float *cos_tab, *sin_tab;      // null: no rotation
+  float *k_cache, *v_cache;
+  int n_heads, n_kv, head_dim, adjacent, page_size;
+};
+#define F3_NORM_ROWS 4
+#define F3_NORM_PAD 16
+
+__global__ __launch_bounds__(64 * F3_WAVES, 4) void qkv_f32_normed_kernel(
+    const float* __restrict__ X, F3Norm norm, const float* __restrict__ W, float* __restrict__ Q, int M, int K, long ldx, long ldw, long ldq,
+    F3Rope rope) {
+  constexpr int PART = 8;      // blocks of 16 k whose weights are on their way at a time
+  // the normalised rows, F3_NORM_PAD floats between two (four rows' sixteen bytes of four q meet all banks once), and later the chunks' sums
+  extern __shared__ __attribute__((aligned(16))) float shared_rows[];
+  f32x4(*const sums)[64] = (f32x4(*)[64])shared_rows;
+  __shared__ __attribute__((aligned(16))) float squares[F3_NORM_ROWS][16];
+  __shared__ float turned[16][F3_NORM_ROWS + 1];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int r = lane & 15, q = lane >> 4;
+  const int chunks = K / F3_CHUNK;                       // (whole ones, at most one a wave)
+  const int hs = rope.head_dim, half = hs / 2, per_head = hs / 16;
+  const int head = blockIdx.x / per_head, part = blockIdx.x % per_head, n0 = head * hs;
+  const bool turns = rope.cos_tab && head < rope.n_heads + rope.n_kv;
+  // the element of the head that column n of the block is
+  auto place = [&](int n) {
+    return turns && !rope.adjacent ? part * 8 + (n & 7) + (n & 8 ? half : 0) : part * 16 + n;
+  };
+  // element e = tid < 256 of the block's outputs: token lane' % 16, column 4 * (lane' / 16) + e % 4, lane' = e / 4
+  const int em = (tid >> 2) & 15, en = 4 * ((tid >> 6) & 3) + (tid & 3);
+  const bool ends = tid < 256 && em < M;
+  int pos = 0;
+  if (ends) pos = rope.positions[em];
+
+  // the rows, then the first weights: loads come back in order, and the sums of squares need not wait for the weights
+  // (a thread has one piece of a row, or, of a row of more than 2,048 with 512 threads, two; a wave four at most either way)
+  const int waves_a_row = norm.threads / 64, rows_at_once = F3_WAVES / waves_a_row, two = K > 4 * norm.threads;
+  const int group = wave / waves_a_row, piece = (tid & (norm.threads - 1)) * 4;
+  f32x4 xv[F3_NORM_ROWS];
+#pragma unroll
+  for (int i = 0; i < F3_NORM_ROWS; ++i) {
+    const int row = min((i >> two) * rows_at_once + group, M - 1), at = piece + (i & two) * 4 * norm.threads;
+    xv[i] = *(const f32x4*)(X + (long)row * ldx + min(at, K - 4));
+  }
+  f32x4 nw[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) nw[i] = *(const f32x4*)(norm.w + min(piece + (i & two) * 4 * norm.threads, K - 4));
+  __builtin_amdgcn_sched_barrier(0);
+  const int chunk = min(wave, chunks - 1), k0 = chunk * F3_CHUNK;      // (a wave without a chunk reads the last one and drops it)
+  const float* const wp = W + (long)(n0 + place(r)) * ldw + k0 + q * 4;
+  f32x4 w[PART];
+#pragma unroll
+  for (int b = 0; b < PART; ++b) w[b] = *(const f32x4*)(wp + b * 16);
+  __builtin_amdgcn_sched_barrier(0);
+  // what the end needs of the token: its page, its angle
+  int page = 0;
+  float cosine = 1.f, sine = 0.f;
+  const int angle = rope.adjacent ? (part * 16 + en) >> 1 : part * 8 + (en & 7);
+  if (ends) {
+    if (head >= rope.n_heads) page = rope.block_table[(long)rope.table_rows[em] * rope.table_stride + pos / rope.page_size];
+    if (turns) {
+      cosine = rope.cos_tab[(long)pos * half + angle];
+      sine = rope.sin_tab[(long)pos * half + angle];
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < F3_NORM_ROWS; ++i) {
+    const int row = (i >> two) * rows_at_once + group, at = piece + (i & two) * 4 * norm.threads;
+    if (row >= M) continue;
+    if (!(i & two)) ss = 0.f;
+    float more = ss;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) more = fmaf(xv[i][e], xv[i][e], more);
+    if (at < K) ss = more;
+    if (two && !(i & 1)) continue;
+    const float sum = wave_sum(ss);
+    if (lane == 0) squares[row][wave % waves_a_row] = sum;
+  }
+  __syncthreads();
+  const int pitch = K + F3_NORM_PAD;
+#pragma unroll
+  for (int i = 0; i < F3_NORM_ROWS; ++i) {
+    const int row = (i >> two) * rows_at_once + group, at = piece + (i & two) * 4 * norm.threads;
+    if (row >= M) continue;
+    float scale = 0.f;
+    for (int k = 0; k < waves_a_row; k += 4) {
+      const f32x4 four = *(const f32x4*)&squares[row][k];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) scale += four[e];
+    }
+    scale = scale / (float)K;
+    scale = scale + norm.eps;
+    scale = 1.0f / sqrtf(scale);
+    if (at < K) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (i & two ? nw[1] : nw[0])[e] * (scale * xv[i][e]);
+      *(f32x4*)(shared_rows + row * pitch + at) = v;
+    }
+  }
+  __syncthreads();
+  // (lanes without a row of their own work on the last one; their sums are dropped)
+  const float* const rows = shared_rows + min(r, M - 1) * pitch + k0 + q * 4;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  if (wave < chunks) {
+#pragma unroll
+    for (int p = 0; p < 16; p += PART) {
+#pragma unroll
+      for (int b = 0; b < PART; ++b) {
+        const f32x4 a = *(const f32x4*)(rows + (p + b) * 16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[b][j], a[j], acc, 0, 0, 0);
+        if (p + PART + b < 16) w[b] = *(const f32x4*)(wp + (p + PART + b) * 16);
+      }
+    }
+  }
+  __syncthreads();                     // (everybody has read the rows: the sums lie there now)
+  if (wave < chunks) sums[wave][lane] = acc;
+  __syncthreads();
+  float v = 0.f;
+  if (tid < 256)
+    for (int s = 0; s < chunks; ++s) v += ((const float*)&sums[s][0])[tid];
+  if (ends) turned[en][em] = v;
+  __syncthreads();
+  if (!ends) return;
+  if (turns) {
+    const int across = rope.adjacent ? 1 : 8;
+    const float other = turned[en ^ across][em];
+    v = en & across ? fmaf(other, sine, v * cosine) : fmaf(v, cosine, -(other * sine));      // (rounded as rope_cache_kernel's)
+  }
+  const int dim = place(en);
+  if (head < rope.n_heads) {
+    Q[(long)em * ldq + n0 + dim] = v;
+    return;
+  }
+  const int in_page = pos % rope.page_size, c = (head - rope.n_heads) % rope.n_kv;
+  const long at = ((long)page * rope.n_kv + c) * rope.page_size * hs;
+  if (head < rope.n_heads + rope.n_kv) rope.k_cache[at + gl3_k_offset(in_page, dim, hs)] = v;
+  else rope.v_cache[at + gl3_v_offset(dim, in_page, rope.page_size)] = v;
 }
 
 // A lane holds four consecutive columns (from n0) of one token (m0) per tile.
@@ -553,4 +713,29 @@ int gl3_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, lon
   if (epi == F3_ADD) return launch_f32<F3_ADD>(F3_ARGS);
   return launch_f32<F3_GATED>(F3_ARGS);
 #undef F3_ARGS
+}
+
+// gl3_rmsnorm (weight norm_w, K floats), gl3_gemm_generic with the stacked q, k, v rows W and gl3_rope_cache_write (whole heads rotated; cos_tab null: not)
+// of at most four rows, bit for bit: queries to q, keys and values into the cache. K in whole chunks of 256, at most 4,096 and 64 KB of rows; rows of x,
+// of W and norm_w at 16 bytes.
+extern "C" int gl3_qkv_f32_normed(const float* x, const float* norm_w, float eps, const float* W, float* q, int M, int K, long ldx, long ldw, long ldq,
+                                  const int* positions, const int* table_rows, const int* block_table, int table_stride, const float* cos_tab,
+                                  const float* sin_tab, float* k_cache, float* v_cache, int n_heads, int n_kv, int head_dim, int adjacent, int page_size,
+                                  hipStream_t stream) {
+  if (M == 0) return 0;
+  GL3_REQUIRE(n_heads > 0 && n_kv > 0 && head_dim > 0 && head_dim % 16 == 0 && page_size > 0 && page_size % 32 == 0 && table_stride > 0,
+              "gl3_qkv_f32_normed: %d and %d heads of %d, pages of %d", n_heads, n_kv, head_dim, page_size);
+  const int rows = M * (K + F3_NORM_PAD) * 4;      // (bytes of the rows that a block keeps)
+  GL3_REQUIRE(x && norm_w && W && M > 0 && M <= F3_NORM_ROWS && K > 0 && K % F3_CHUNK == 0 && K <= F3_CHUNK * F3_WAVES && rows <= 65536,
+              "gl3_qkv_f32_normed: %d rows of %d: up to four of whole 256, 4,096 at most, 64 KB together", M, K);
+  GL3_REQUIRE(ldx >= K && ldw >= K && ldx % 4 == 0 && ldw % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)norm_w % 16 == 0 && (uintptr_t)W % 16 == 0,
+              "gl3_qkv_f32_normed: rows at whole 16 bytes (ldx=%ld ldw=%ld)", ldx, ldw);
+  GL3_REQUIRE(q && ldq >= (long)n_heads * head_dim && positions && table_rows && block_table && k_cache && v_cache && (cos_tab == nullptr) == (sin_tab == nullptr),
+              "gl3_qkv_f32_normed: outputs, cache or tables missing (ldq=%ld)", ldq);
+  const F3Rope rope{positions, table_rows, block_table, table_stride, cos_tab, sin_tab, k_cache, v_cache, n_heads, n_kv, head_dim, adjacent, page_size};
+  const F3Norm norm{norm_w, eps, K / 4 >= 1024 ? 1024 : K / 4 > 256 ? 512 : 256};      // (gl3_rmsnorm's rule)
+  const int blocks = (n_heads + 2 * n_kv) * (head_dim / 16);
+  qkv_f32_normed_kernel<<<dim3(blocks), dim3(64 * F3_WAVES), std::max(rows, K / F3_CHUNK * 1024), stream>>>(x, norm, W, q, M, K, ldx, ldw, ldq, rope);
+  GL3_LAUNCH_CHECK();
+  return 0;
 }

@@ -57,6 +57,7 @@ def _declare(lib):
         "gl3_gather_rows": [P, P, P, I, I, I, P],
         "gl3_add_slices_rmsnorm": [P, P, P, I, L, L, P, I, P, I, I, I, F, P],
         "gl3_rope_cache_write": [P, I, P, P, P, I, P, P, P, P, I, I, I, I, I, I, I, I, P],
+        "gl3_qkv_f32_normed": [P, P, F, P, P, I, I, L, L, L, P, P, P, I, P, P, P, P, I, I, I, I, I, P],
         "gl3_gemm_generic": [P, I, P, I, P, I, I, I, I, L, L, L, I, P, I, I, P, F, F, P, P],
         "gl3_attention_generic": [P, L, P, P, I, P, P, P, I, P, L, I, I, I, I, I, I, F, I, P, I, F, I, I, I, I, P, I, F, F, I, P, L, P],
         "gl3_pair_rows": [P, P, P, P, P, P, L, L, L, L, P, I, P],
@@ -453,6 +454,37 @@ def gemm_generic(a, w, out, epilogue=EPI_STORE, bias=None, act="silu", act_limit
                                       _bias(bias, rows, "gemm_generic"), _act(act, "gemm_generic"), order, pos,
                                       float(act_limit), float(act_shift), _ptr(col_scale), _stream()),
            "gemm_generic")
+
+
+F32_NORMED_ROWS = 4
+
+
+def qkv_f32_normed_fits(x, weight, w, head_dim, rot_dim):
+    """Few rows ``x``, of whole chunks of 256 (one a wave) and 64 KB together; heads that are rotated as a whole or not at all."""
+    M, K = x.shape
+    return (M <= F32_NORMED_ROWS and K % 256 == 0 and 0 < K <= 4096 and M * (K + 16) * 4 <= 65536 and x.dtype == torch.float32 and weight.dtype == torch.float32
+            and w.dtype == torch.float32 and w.dim() == 2 and rot_dim in (0, head_dim) and head_dim % 16 == 0 and w.shape[1] == K and w.is_contiguous() and x.is_contiguous()
+            and weight.is_contiguous() and all(t.data_ptr() % 16 == 0 for t in (x, weight, w)) and _w_order(w)[0] == 0)
+
+
+def qkv_f32_normed(x, weight, eps, w, q, positions, table_rows, block_table, cos, sin, k_cache, v_cache, n_heads, n_kv, head_dim, adjacent, page_size):
+    """``rmsnorm``, the product with the stacked q, k, v rows and ``rope_cache_write`` (whole heads rotated, or none) in one kernel, bit for bit the same;
+    ``q`` [T, n_heads * head_dim] receives the queries (``qkv_f32_normed_fits``)."""
+    _dev(x, "x", torch.float32); _dev(weight, "weight", torch.float32); _dev(w, "w", torch.float32); _dev(q, "q", torch.float32)
+    _dev(positions, "positions", torch.int32); _dev(table_rows, "table_rows", torch.int32); _dev(block_table, "block_table", torch.int32)
+    _dev(k_cache, "k_cache", torch.float32); _dev(v_cache, "v_cache", torch.float32)
+    T, K = x.shape
+    if (weight.shape != (K,) or w.shape != ((n_heads + 2 * n_kv) * head_dim, K) or q.shape != (T, n_heads * head_dim) or positions.numel() != T
+            or table_rows.numel() != T or block_table.dim() != 2):
+        raise KernelError(f"qkv_f32_normed: x {tuple(x.shape)}, w {tuple(w.shape)}, q {tuple(q.shape)}, {n_heads} + 2 * {n_kv} heads of {head_dim}")
+    if cos is not None:
+        _dev(cos, "cos", torch.float32); _dev(sin, "sin", torch.float32)
+        if cos.shape != sin.shape or cos.dim() != 2 or cos.shape[1] != head_dim // 2:
+            raise KernelError(f"qkv_f32_normed: table {tuple(cos.shape)} for heads of {head_dim}")
+    _check_cache(k_cache, v_cache, n_kv, page_size, head_dim, "qkv_f32_normed")
+    _check(library().gl3_qkv_f32_normed(_ptr(x), _ptr(weight), float(eps), _ptr(w), _ptr(q), T, K, x.stride(0), w.stride(0), q.stride(0), _ptr(positions),
+                                        _ptr(table_rows), _ptr(block_table), block_table.shape[1], _ptr(cos), _ptr(sin), _ptr(k_cache), _ptr(v_cache),
+                                        n_heads, n_kv, head_dim, int(adjacent), page_size, _stream()), "qkv_f32_normed")
 
 
 def attention_generic(q, k_cache, v_cache, positions, seq_of_token, block_table, out, n_heads, n_kv, head_dim,

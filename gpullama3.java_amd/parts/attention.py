@@ -267,6 +267,11 @@ class GQAAttention:
     def state_need(self):
         return StateNeed(max(-(-self.channels * (self.conv_taps - 1) // 4) * 4, 4), torch.float32) if self.conv_taps else None
 
+    @property
+    def norms_rows(self):
+        """Whether ``forward`` takes rows whose norm is not computed yet (``ops.RowsToNorm``): where they go to ``ops.qkv_project`` alone."""
+        return not self.general and self.vd == self.hs
+
     def forward(self, ctx, h, x, run, epilogue=ops.EPI_ADD):
         """``epilogue``: EPI_ADD adds the output into the residual rows ``x``; EPI_STORE writes it to ``x``, a float32
         buffer of the caller's (a mixer that stands beside another)."""

@@ -40,7 +40,9 @@ class PreNormBlock:
     def forward(self, ctx, x, run, norm_after=None):
         """``norm_after``: the norm that reads the residual rows after this block, if known."""
         behind, norm_after = norm_after, (norm_after if self.side is None else None)
-        h = self._whole_rows_for(self.mixer_norm, "takes_slices", ctx, x)(ctx, x)
+        norm = self._whole_rows_for(self.mixer_norm, "takes_slices", ctx, x)
+        # (a mixer that may do the norm's work itself: what the norm has for such parts)
+        h = (norm.for_mixer if getattr(self.mixer, "norms_rows", False) and hasattr(norm, "for_mixer") else norm)(ctx, x)
         ctx.next_norm = self.ffn_norm if self.ffn is not None else norm_after
         self._whole_rows_for(self.mixer, "adds_only", ctx, x).forward(ctx, h, x, run)
         if self.ffn is not None:

@@ -11,7 +11,6 @@ from . import ops
 from .ops import Normed
 
 
-
 class RMSNorm:
     graph_safe = True      # kernel launches on the current stream only, sizes fixed by (T, B)
     folds = True           # a product can take over this norm's work (see ``ops.Normed``)
@@ -56,6 +55,16 @@ class RMSNorm:
             return out
         K.rmsnorm(x, self.weight, out, self.eps, rows)
         return out
+
+
+    def for_mixer(self, ctx, x, name="normed"):
+        """What a mixer reads whose first product may do the norm's work itself (``norms_rows``): the rows as they are in a 32-bit step of
+        few tokens (``ops.RowsToNorm``), else what calling the norm gives."""
+        made = getattr(ctx, "normed", None)
+        if (self.dtype != torch.float32 or x.dtype != torch.float32 or x.shape[0] > K.F32_NORMED_ROWS or "fused" in ops._off(ctx)
+                or getattr(ctx, "pending", None) is not None or (made is not None and made[0] == x.data_ptr())):
+            return self(ctx, x, name=name)
+        return ops.RowsToNorm(ctx, x, self.weight_f32, self.eps, name)
 
 
 class LayerNorm:

@@ -152,6 +152,21 @@ class Normed:
         return out
 
 
+class RowsToNorm:
+    """The RMSNorm of the residual rows of a 32-bit step of few tokens, not computed yet: ``qkv_project`` does the norm's work with its
+    product (``lib.qkv_f32_normed``) or calls ``materialize``, the same bits either way. For mixers that say ``norms_rows``: the rows are read
+    before anything is added to them."""
+
+    def __init__(self, ctx, x, weight, eps, name):
+        self.ctx, self.x, self.weight, self.eps, self.name = ctx, x, weight, eps, name
+        self.shape, self.dtype = x.shape, x.dtype
+
+    def materialize(self):
+        out = self.ctx.buffer(self.name, tuple(self.shape), self.dtype)
+        K.rmsnorm(self.x, self.weight, out, self.eps)
+        return out
+
+
 def settle_residual(ctx, x):
     """A product of 17 to 64 rows into the residual stream may have left its sums as slices that the
     next norm adds up. Whoever else wants to READ the rows (adding to them is always fine) calls
@@ -459,6 +474,13 @@ def qkv_project(ctx, h, w_qkv, w_q, rotary, k_cache, v_cache, block_table, n_hea
                          block_table, cos, sin, k_cache, v_cache, n_heads, n_kv, head_dim, adjacent, page,
                          token_pages=pages, token_rot=rows_of_rotation)
         return q
+    if isinstance(h, RowsToNorm):
+        if writes_kv and bias is None and K.qkv_f32_normed_fits(h.x, h.weight, w_qkv, head_dim, rot):
+            q = ctx.buffer("q", (T, n_heads * head_dim), dtype)
+            K.qkv_f32_normed(h.x, h.weight, h.eps, w_qkv, q, ctx.positions, _table_rows(ctx), block_table, cos, sin, k_cache, v_cache,
+                             n_heads, n_kv, head_dim, adjacent, page)
+            return q
+        h = h.materialize()
     if isinstance(h, Normed):
         h = h.materialize()
     chunks = row_chunks(T, ctx) if getattr(ctx, "fuse", False) and "wide" not in disabled else None

@@ -228,3 +228,42 @@ def test_float32_attention_is_the_same_with_a_step_s_loads_at_once(H, Kh, hs, pa
     fine = np.isfinite(ref)
     assert not fine.all() and np.array_equal(np.isfinite(got), fine)
     np.testing.assert_allclose(got[fine], ref[fine], atol=2e-5 * np.abs(ref[fine]).max())
+
+
+# (the widths at which the norm's threads and their pieces change, one chunk and sixteen)
+@pytest.mark.parametrize("hs, adjacent, rotated", [(16, False, True), (64, False, True), (64, True, True), (128, False, True), (96, True, True), (64, False, False)])
+@pytest.mark.parametrize("M, Kd", [(1, 256), (2, 1024), (4, 1280), (3, 2048), (4, 3072), (3, 4096)])
+def test_query_key_value_rows_with_norm_rotation_and_cache_in_one_kernel(hs, adjacent, rotated, M, Kd):
+    """Against norm, product and rotation one after the other: the same queries and the same cache, bit for bit, everywhere."""
+    lib = K()
+    H, G, page, pages = 6, 2, 32, 9
+    gen = torch.Generator(device="cuda").manual_seed(hs + M)
+    x = torch.randn(M, Kd, generator=gen, device="cuda") * torch.tensor([1.0, 1e-3, 30.0, 5.0], device="cuda")[:M, None]
+    nw = 1.0 + 0.1 * torch.randn(Kd, generator=gen, device="cuda")
+    w = torch.randn((H + 2 * G) * hs, Kd, generator=gen, device="cuda") * 0.05
+    cos = sin = None
+    if rotated:
+        cos, sin = (torch.randn(pages * page, hs // 2, generator=gen, device="cuda") for _ in range(2))
+    table = torch.tensor([[3, 1, 7], [0, 8, 2], [5, 4, 6]], dtype=torch.int32, device="cuda")
+    rows = torch.tensor([2, 0, 1, 0], dtype=torch.int32, device="cuda")[:M].contiguous()
+    positions = torch.tensor([70, 31, 32, 0], dtype=torch.int32, device="cuda")[:M].contiguous()
+    caches = [[torch.full((pages, G, page, hs), -7.0, device="cuda"), torch.full((pages, G, hs, page), -7.0, device="cuda")] for _ in range(2)]
+    normed, qkv, q = torch.empty_like(x), torch.empty(M, (H + 2 * G) * hs, device="cuda"), torch.empty(M, H * hs, device="cuda")
+    lib.rmsnorm(x, nw, normed, 1e-5)
+    lib.gemm_generic(normed, w, qkv)
+    lib.rope_cache_write(qkv, positions, rows, table, cos, sin, *caches[0], H, G, hs, hs if rotated else 0, adjacent, page)
+    lib.qkv_f32_normed(x, nw, 1e-5, w, q, positions, rows, table, cos, sin, *caches[1], H, G, hs, adjacent, page)
+    assert torch.equal(q, qkv[:, :H * hs])
+    assert torch.equal(caches[0][0], caches[1][0]) and torch.equal(caches[0][1], caches[1][1])
+
+
+@pytest.mark.parametrize("M, Kd", [(5, 256), (1, 320), (1, 4352), (4, 4096)])
+def test_rows_that_the_one_kernel_does_not_take(M, Kd):
+    """More rows, other widths, more than a block keeps: said so beforehand and refused."""
+    lib = K()
+    x, nw, w = torch.zeros(M, Kd, device="cuda"), torch.zeros(Kd, device="cuda"), torch.zeros(48, Kd, device="cuda")
+    k, v = torch.zeros(1, 1, 32, 16, device="cuda"), torch.zeros(1, 1, 16, 32, device="cuda")
+    zero = torch.zeros(M, dtype=torch.int32, device="cuda")
+    assert not lib.qkv_f32_normed_fits(x, nw, w, 16, 0)
+    with pytest.raises(lib.KernelError):
+        lib.qkv_f32_normed(x, nw, 1e-5, w, torch.empty(M, 16, device="cuda"), zero, zero, zero[:1, None].contiguous(), None, None, k, v, 1, 1, 16, False, 32)
