@@ -48,9 +48,9 @@ _current_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 class _DecodeGraph:
-    """A captured decode step for one batch bucket: its input buffer on the device and its logits;
-    for runs of steps also the sampling of the next tokens and their feeding back."""
-    graph = handle = logits = dev = step = fhost = fdev = None
+    """A captured decode step for one batch bucket: its input buffer on the device and what the head reads behind it;
+    for runs of steps also the head, the sampling of the next tokens and their feeding back."""
+    graph = handle = ctx = head_rows = dev = step = fhost = fdev = None
     B_pad = n_input = off_sampled = off_hist = 0
 
     def launch(self):
@@ -61,7 +61,7 @@ class _DecodeGraph:
             self.graph.replay()
 
 
-GRAPHS_KEPT = 24    # captured decode steps that an engine keeps (each owns its logits and the sampler's scratch)
+GRAPHS_KEPT = 24    # captured decode steps that an engine keeps (those of runs own their logits and the sampler's scratch)
 
 
 def _without(without, weight_copies):
@@ -338,7 +338,9 @@ class Engine:
             cache.flush_tables()
             K.stage_decode(dg.dev, dg.B_pad, tokens, starts, slots, cache.sink_slot)
             dg.launch()
-            logits = dg.logits[:B].clone()       # the graph's own buffer is overwritten by the next step
+            # (the head's product is not in the graph: it writes to a tensor of this step's own. As the graph's last node it was followed by a copy out of the
+            # graph's buffer: one sequence of the 1B layers 744 -> 737 us a step, 64 sequences 33 MB of copying less)
+            logits = self.model.head_logits(dg.ctx, dg.head_rows, dg.B_pad)[:B]
         cache.advance_one_each(slots)
         return logits
 
@@ -448,26 +450,32 @@ class Engine:
             us = dg.fdev[2 * B_pad:]
 
         def body():
-            logits = self.model.forward(ctx, rows)
+            read = self.model.rows_for_head(ctx, rows)
+            if not run:
+                return read
+            logits = self.model.head_logits(ctx, read, B_pad)
             if run == "greedy":
                 K.argmax_advance(logits, work, sampled, ctx.token_ids, ctx.positions, ctx.kv_before, hist, step)
             elif run:
                 K.sample(logits, work, temps, tops, us, sampled, step=step, uniform_stride=B_pad)
                 K.decode_advance(ctx.token_ids, ctx.positions, ctx.kv_before, sampled, hist, step)
-            return logits
+            return read
 
         # once outside a capture: scratch buffers get their sizes, the library is loaded
         side = torch.cuda.Stream(device=self.device)
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
-            body()
+            read = body()
+            if not run:
+                self.model.head_logits(ctx, read, B_pad)
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         self.workspace.frozen = True
         try:
             dg.graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(dg.graph):
-                dg.logits = body()
+                dg.head_rows = body()
+            dg.ctx = ctx
         finally:
             self.workspace.frozen = False
         try:

@@ -173,6 +173,22 @@ class DecoderModel:
 
     def forward(self, ctx, want_rows):
         """Logits ``[len(want_rows), vocab]`` float32 at the wanted packed rows."""
+        n = want_rows.numel()
+        return self.head_logits(ctx, self.rows_for_head(ctx, want_rows), n)
+
+    def head_logits(self, ctx, rows, n):
+        """The head's product over what ``rows_for_head`` gave for n wanted rows: a tensor of its own."""
+        logits = ctx.logits_buffer(n, self.spec.vocab_size)
+        if n:
+            ops.linear(rows, self.head, logits, ops.EPI_STORE, ctx, bias=self.head_bias)
+            if self.spec.logit_scale is not None:
+                K.scale_(logits, self.spec.logit_scale)
+            if self.spec.logit_softcap is not None:
+                K.softcap_(logits, self.spec.logit_softcap)
+        return logits
+
+    def rows_for_head(self, ctx, want_rows):
+        """Everything in front of the head: what its product reads of the wanted packed rows (None: no row is wanted)."""
         S = int(getattr(self.spec, "streams", 1) or 1)      # copies of the residual row per token
         x = ctx.buffer("residual", (ctx.n_tokens, self.spec.hidden), torch.float32)
         ctx.ssq = ctx.normed = ctx.pending = ctx.next_norm = None   # a context may run more than one forward pass: nothing is left over
@@ -251,28 +267,22 @@ class DecoderModel:
                 ops.settle_residual(ctx, x)
                 watch(i, x)
         n = want_rows.numel()
-        logits = ctx.logits_buffer(n, self.spec.vocab_size)
-        if n:
-            if S > 1:
-                # the copies' sum at the wanted rows is what the final norm and the head read
-                ops.settle_residual(ctx, x)
-                copies, x = x, ctx.buffer("residual_wanted", (n, self.spec.hidden), torch.float32)
-                K.streams_sum(copies, S, x, which=want_rows)
-                want_rows = None                       # (every row of x, in order)
-                ops.residual_written(ctx, x)
-            if self.final_norm is not None:
-                h = self.final_norm(ctx, x, rows=want_rows, name="final_normed")
-            else:
-                # a decoder without a final norm: the head reads the wanted rows as they are
-                ops.settle_residual(ctx, x)
-                h = ctx.buffer("head_rows", (n, self.spec.hidden), self.dtype)
-                if want_rows is None:
-                    K.cast_rows(x, h)
-                else:
-                    K.gather_rows(x, want_rows, h)
-            ops.linear(h, self.head, logits, ops.EPI_STORE, ctx, bias=self.head_bias)
-            if self.spec.logit_scale is not None:
-                K.scale_(logits, self.spec.logit_scale)
-            if self.spec.logit_softcap is not None:
-                K.softcap_(logits, self.spec.logit_softcap)
-        return logits
+        if not n:
+            return None
+        if S > 1:
+            # the copies' sum at the wanted rows is what the final norm and the head read
+            ops.settle_residual(ctx, x)
+            copies, x = x, ctx.buffer("residual_wanted", (n, self.spec.hidden), torch.float32)
+            K.streams_sum(copies, S, x, which=want_rows)
+            want_rows = None                       # (every row of x, in order)
+            ops.residual_written(ctx, x)
+        if self.final_norm is not None:
+            return self.final_norm(ctx, x, rows=want_rows, name="final_normed")
+        # a decoder without a final norm: the head reads the wanted rows as they are
+        ops.settle_residual(ctx, x)
+        h = ctx.buffer("head_rows", (n, self.spec.hidden), self.dtype)
+        if want_rows is None:
+            K.cast_rows(x, h)
+        else:
+            K.gather_rows(x, want_rows, h)
+        return h
