@@ -1505,3 +1505,27 @@ def test_norms_of_rows_held_at_once(d, S):
                         lib.rmsnorm(X, w, out, 1e-5, r)
                     got.append((X, out))
                 assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (wdtype, odtype, r is None)
+
+
+# (sequences that begin and end at every place of a group of 8 positions and of a block of 16 tokens; one token each; one long one)
+@pytest.mark.parametrize("starts, lens", [([0], [1]), ([7], [130]), ([0, 5, 8, 63], [16, 11, 21, 9]), ([3] * 20, [1] * 20), ([0, 1, 2, 3, 4, 5, 6, 7], [15, 14, 13, 12, 11, 10, 9, 8]),
+                                          ([60, 0, 31, 64], [33, 7, 40, 64])])
+@pytest.mark.parametrize("Kh, hs", [(1, 16), (8, 64), (3, 128)])
+def test_values_of_a_prompt_s_tokens_in_the_cache(starts, lens, Kh, hs):
+    """Every token's value is in its place, whatever tokens share its 8 positions, and nothing else in the cache has changed."""
+    rng = np.random.default_rng(sum(lens) + hs)
+    H, page = 2, 64
+    T = sum(lens)
+    positions = np.concatenate([np.arange(b, b + n) for b, n in zip(starts, lens)])
+    seq_of = np.concatenate([[i] * n for i, n in enumerate(lens)])
+    zk = [rng.standard_normal((b + n, Kh, hs)).astype(np.float32) for b, n in zip(starts, lens)]
+    kc, vc, table = paged(zk, zk, Kh, hs, page, "bfloat16", rng)
+    qkv = dev(rng.standard_normal((T, (H + 2 * Kh) * hs)).astype(np.float32), torch.bfloat16)
+    want = untile_values(vc).clone()
+    v = qkv[:, (H + Kh) * hs:].reshape(T, Kh, hs)
+    pages = table.cpu().numpy()[seq_of, positions // page]
+    for i in range(T):
+        want[int(pages[i]), :, :, int(positions[i]) % page] = v[i].to(want.device)
+    cos, sin = P.rope_table(256, hs, 10000.0)
+    K().rope_cache_write(qkv, dev(positions, torch.int32), dev(seq_of, torch.int32), table, dev(cos), dev(sin), kc, vc, H, Kh, hs, hs, False, page)
+    assert torch.equal(untile_values(vc), want)
