@@ -725,15 +725,15 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
 
 // The tile the library takes where the caller names none. Where gemm_mfma_turns_kernel takes the product: the tile whose rounds on
 // the chip take the least time, a round (a block on every CU: 32 of an XCD, which has an eighth of the tiles of every slice) being
-// 0.42 us a step of 64 k and 0.9 us beside them for 128 x 128, 0.60 and 4.0 for 128 rows x 256, 1.0 and 4.5 for 256 x 256. The
+// 0.40 us a step of 64 k and 0.9 us beside them for 128 x 128, 0.60 and 3.0 for 128 rows x 256, 1.0 and 4.5 for 256 x 256. The
 // constants rank the tiles and are no times of their own (at 8,192 rows of 28,672 x 4,096 they say 959 us and it is 1,283).
-// Measured with the norm behind, 143 products into the residual rows (70 to 5,886 rows, 512 to 4,096 columns, K of 1,024 to 14,336 in
-// mfma_plan's slices): the tile chosen is the fastest of the three or within 5% but at 512 rows of 1,280 x 5,120 (29.2 against
-// 27.0 us) and 1,024 rows of 1,024 x 4,096 (34.2 against 31.8). With rounds of 256 blocks, whatever their XCD, 300 rows of 3,072 x
-// 8,192 took 47.3 instead of 40.8 us. At 31 sizes of other products, 70 to 8,192 rows, it takes the fastest of the three every time.
+// Measured at 580 sizes (66 to 8,192 rows; QKV, output, gate/up and down products of five layers' sizes, widths of 1,536 to 4,096, those
+// into the residual rows in mfma_plan's slices; profiles/tiled_products_tiles.txt): the tile chosen is the fastest of the three or within 5% at
+// all but one (1.07). With 0.42 and 4.0 for the first two, which suited epilogues through shared memory, 17 were beyond 5%, 1,024 rows of
+// 2,048 x 2,048 20.3 instead of 17.2 us. With rounds of 256 blocks, whatever their XCD, 300 rows of 3,072 x 8,192 took 47.3 instead of 40.8 us.
 static int choose_turns_shape(int M, int N, int K, int slices, bool gated) {
   static const int rows[3] = {128, 128, 256}, cols[3] = {128, 256, 256}, shape[3] = {1, 5, 2};
-  static const double step_us[3] = {0.42, 0.60, 1.0}, round_us[3] = {0.9, 4.0, 4.5};
+  static const double step_us[3] = {0.40, 0.60, 1.0}, round_us[3] = {0.9, 3.0, 4.5};
   const int steps = (K / 64 + slices - 1) / slices;
   int best = 0;
   double least = 0;
