@@ -13,6 +13,7 @@ from __future__ import annotations
 import array
 import contextlib
 import tempfile
+import weakref
 from collections import OrderedDict
 
 import numpy as np
@@ -431,6 +432,9 @@ class Engine:
                           max_q_len=1, max_kv_len=kv_bucket)
         ctx.kv_len_hint = kv_bucket
         ctx.replayed = True
+        # The captured step keeps its context, the engine keeps the step: the engine is held weakly here. In a circle an engine whose last reference goes would wait
+        # for the garbage collector, with all its memory, and the collector may come in the middle of another engine's capture, where no graph may be destroyed.
+        ctx.engine = weakref.proxy(self)
         d = dg.dev
         ctx.token_ids, ctx.positions, ctx.kv_before = d[0:B_pad], d[B_pad:2 * B_pad], d[2 * B_pad:3 * B_pad]
         ctx.slot_ids = d[3 * B_pad:4 * B_pad]

@@ -371,6 +371,26 @@ def test_sizes_that_the_cache_cannot_hold_are_refused_before_the_weights_are_rea
         Engine.from_folder(model("A")[0], dtype="float32", max_tokens=256, page_size=48)
 
 
+@pytest.mark.parametrize("name, dtype", [("A", "float32"), ("C", "bfloat16")])
+def test_an_engine_and_its_captured_steps_go_with_the_last_reference(name, dtype):
+    """Without the garbage collector's help: it may come while another engine captures, and no graph may be destroyed then."""
+    import gc
+    import weakref
+    eng = engine(name, dtype, n_slots=2)
+    slot = eng.take_slot()
+    eng.step([(slot, rand_tokens(name, 900, 9))], want="none")
+    eng.step([(slot, [1])])
+    held = [weakref.ref(eng)] + [weakref.ref(g) for g in eng._graphs.values()]
+    assert len(held) > 1
+    torch.cuda.synchronize()
+    gc.disable()
+    try:
+        del eng
+        assert [r() for r in held] == [None] * len(held)
+    finally:
+        gc.enable()
+
+
 def test_captured_steps_are_bounded_in_number_and_memory():
     """Every batch bucket and context bucket has a captured step of its own, with its logits and the
     sampler's scratch; an engine keeps ``max_graphs`` of them and drops the least recently used, so a process
