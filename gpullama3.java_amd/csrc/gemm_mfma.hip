@@ -279,7 +279,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const bf16_t* _
 // tile of a later step from memory to shared memory) and sixteen 16x16x32 matrix instructions, with a barrier after each
 // part; the second group runs one part behind the first, so on every SIMD one wave's matrix instructions run while the
 // other wave's memory part does. Without that lag the same loop is 19% slower (1.24 against 1.50 PFLOP/s at 8,192 x 8,192 x
-// 4,096). What bounds it now is the power budget: the clock stands at 1.4 to 1.8 GHz of 2.4, the matrix cores are busy 74 to 79% of
+// 4,096). What bounds it now is the power budget: the clock stands at 1.2 to 1.65 GHz of 2.4, the matrix cores are busy 83 to 85% of
 // a CU's cycles (gate/up and plain products of 8,192 rows, K = 4,096), and with the 32x32x16 instruction, whose accumulators pass
 // through the registers twice as often per flop, the same loop lost 11%.
 // (8,192 x 28,672 x 4,096: the kernel above 1,680 us, this one 1,283.)
