@@ -50,8 +50,9 @@ _current_device = getattr(torch._C, "_cuda_getDevice", None)
 
 class _DecodeGraph:
     """A captured decode step for one batch bucket: its input buffer on the device and what the head reads behind it;
-    for runs of steps also the head, the sampling of the next tokens and their feeding back."""
-    graph = handle = ctx = head_rows = dev = step = fhost = fdev = None
+    for runs of steps also the head, the sampling of the next tokens and their feeding back. What was allocated in front of
+    the capture and is none of the workspace's is held here: the captured launches have its address."""
+    graph = handle = ctx = head_rows = dev = step = fhost = fdev = work = None
     B_pad = n_input = off_sampled = off_hist = 0
 
     def launch(self):
@@ -447,7 +448,7 @@ class Engine:
         if run:
             dg.fhost = torch.zeros((2 + RUN_LENGTH) * B_pad, dtype=torch.float32).pin_memory()
             dg.fdev = torch.zeros((2 + RUN_LENGTH) * B_pad, dtype=torch.float32, device=self.device)
-            work = torch.empty(K.sample_work_size(B_pad, self.spec.vocab_size), dtype=torch.float32, device=self.device)
+            work = dg.work = torch.empty(K.sample_work_size(B_pad, self.spec.vocab_size), dtype=torch.float32, device=self.device)
             sampled = d[dg.off_sampled:dg.off_sampled + B_pad]
             hist = d[dg.off_hist:dg.off_hist + RUN_LENGTH * B_pad].view(RUN_LENGTH, B_pad)
             temps, tops = dg.fdev[0:B_pad], dg.fdev[B_pad:2 * B_pad]

@@ -391,8 +391,31 @@ def test_an_engine_and_its_captured_steps_go_with_the_last_reference(name, dtype
         gc.enable()
 
 
+@pytest.mark.parametrize("temperature", [0.0, 0.9])
+@pytest.mark.parametrize("name, B", [("A", 1), ("C", 3)])
+def test_a_captured_run_writes_to_memory_of_its_own(name, B, temperature):
+    """The sampler's scratch of a captured run belongs to it as long as it is replayed: tensors of that size that are made
+    after the capture hold what was put into them, and the run gives the same tokens again."""
+    from gpullama3_java_amd.csrc import lib
+    eng = engine(name, "float32", n_slots=B)
+    prompt = rand_tokens(name, 950, 9)
+
+    def run():
+        slots = [eng.take_slot() for _ in range(B)]
+        eng.step([(s, prompt) for s in slots], want="none")
+        toks = eng.decode_run([(s, i + 1) for i, s in enumerate(slots)], 5, [temperature] * B, [0.9] * B, [[0.1 + 0.17 * k] * B for k in range(5)])
+        for s in slots:
+            eng.give_back_slot(s)
+        return toks
+    first = run()
+    size = lib.sample_work_size(B, eng.spec.vocab_size)
+    others = [torch.full((size,), -7.0, device=eng.device) for _ in range(64)]
+    assert run() == first and len(eng._graphs) == 1
+    assert all(bool((t == -7.0).all()) for t in others)
+
+
 def test_captured_steps_are_bounded_in_number_and_memory():
-    """Every batch bucket and context bucket has a captured step of its own, with its logits and the
+    """Every batch bucket and context bucket has a captured step of its own, those of runs with their logits and the
     sampler's scratch; an engine keeps ``max_graphs`` of them and drops the least recently used, so a process
     that walks many batch sizes and contexts levels off. Results stay right across the drops."""
     name, dtype = "C", "bfloat16"
