@@ -342,7 +342,7 @@ class Engine:
             dg.launch()
             # (the head's product is not in the graph: it writes to a tensor of this step's own. As the graph's last node it was followed by a copy out of the
             # graph's buffer: one sequence of the 1B layers 744 -> 737 us a step, 64 sequences 33 MB of copying less)
-            logits = self.model.head_logits(dg.ctx, dg.head_rows, dg.B_pad)[:B]
+            logits = self.model.head_logits(dg.ctx, dg.head_rows, B)          # (of the batch's rows: those that pad it have none)
         cache.advance_one_each(slots)
         return logits
 

@@ -177,9 +177,11 @@ class DecoderModel:
         return self.head_logits(ctx, self.rows_for_head(ctx, want_rows), n)
 
     def head_logits(self, ctx, rows, n):
-        """The head's product over what ``rows_for_head`` gave for n wanted rows: a tensor of its own."""
+        """The head's product over the first n of the rows that ``rows_for_head`` gave: a tensor of its own."""
         logits = ctx.logits_buffer(n, self.spec.vocab_size)
         if n:
+            if rows.shape[0] > n:
+                rows = rows.first(n) if isinstance(rows, ops.Normed) else rows[:n]
             ops.linear(rows, self.head, logits, ops.EPI_STORE, ctx, bias=self.head_bias)
             if self.spec.logit_scale is not None:
                 K.scale_(logits, self.spec.logit_scale)

@@ -146,6 +146,14 @@ class Normed:
         self.xg, self.ssq, self.n_partials, self.rows, self.name = xg, ssq, n_partials, rows, name
         self.shape = (x.shape[0] if rows is None else rows.numel(), x.shape[1])
 
+    def first(self, n):
+        """The first n of the rows."""
+        if self.rows is None:
+            x, xg, rows = self.x[:n], self.xg[:n], None
+        else:
+            x, xg, rows = self.x, self.xg, self.rows[:n]
+        return Normed(self.ctx, x, self.weight, self.eps, self.dtype, xg, self.ssq, self.n_partials, rows, self.name)
+
     def materialize(self):
         out = self.ctx.buffer(self.name, self.shape, self.dtype)
         K.rmsnorm(self.x, self.weight, out, self.eps, self.rows)

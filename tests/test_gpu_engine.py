@@ -414,6 +414,20 @@ def test_a_captured_run_writes_to_memory_of_its_own(name, B, temperature):
     assert all(bool((t == -7.0).all()) for t in others)
 
 
+@pytest.mark.parametrize("name, dtype", CASES)
+def test_a_decode_step_returns_the_batch_s_rows_alone(name, dtype):
+    """A batch is padded to whole eights; the logits that a caller keeps hold no padded rows, and are those of the padded product."""
+    eng = engine(name, dtype, n_slots=63, max_tokens=63 * 64)
+    V = eng.spec.vocab_size
+    slots = [eng.take_slot() for _ in range(63)]
+    eng.step([(s, rand_tokens(name, 960 + i, 1 + i % 5)) for i, s in enumerate(slots)], want="none")
+    for B in (1, 8, 9, 15, 16, 17, 31, 40, 57, 63):
+        got = eng.step([(s, [i + 1]) for i, s in enumerate(slots[:B])])
+        assert got.shape == (B, V) and got.untyped_storage().nbytes() == B * V * 4
+        dg = next(reversed(eng._graphs.values()))
+        assert torch.equal(got, eng.model.head_logits(dg.ctx, dg.head_rows, dg.B_pad)[:B]), B
+
+
 def test_captured_steps_are_bounded_in_number_and_memory():
     """Every batch bucket and context bucket has a captured step of its own, those of runs with their logits and the
     sampler's scratch; an engine keeps ``max_graphs`` of them and drops the least recently used, so a process
