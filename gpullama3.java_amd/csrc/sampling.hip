@@ -20,7 +20,8 @@
 // At most 2^13 probabilities are 2^-13 or more. They are gathered while the row is normalised; when
 // their mass alone exceeds top_p, the threshold and the drawn token lie among them and both searches
 // walk that short list, in shared memory, instead of the row. A flat distribution, whose nucleus
-// reaches further down, takes three passes over the whole row (nine if a factor of 1.05 holds more than 8,192 values).
+// reaches further down, takes three passes over the whole row, and up to nine where a factor of 1.03 to 1.06 in probability holds more
+// than 8,192 values.
 #include "common.h"
 #include "gl3_noalloc.h"
 #include <mutex>
@@ -56,17 +57,16 @@ struct Found {
 // (8, 8, 8 and 7 bits): per digit one pass builds a histogram of mass and count over the values that
 // share the digits found so far, in private per-wave tables (integer adds in shared memory), and
 // wave 0 walks the 256 bins from the top. If no prefix of the values exceeds thr (thr is not below
-// the total mass), the smallest value is returned.
+// the total mass), the smallest value is returned. `bits` (of 31): the digits below them are searched, the value's upper digits are
+// `prefix` and the mass above all values with that prefix is `above`.
 template <typename Src>
 __device__ Found radix_search(Src p, int V, unsigned long long thr,
                               unsigned long long (*h_mass)[256], int (*h_cnt)[256], unsigned long long* t_mass,
-                              int* t_cnt, unsigned long long* res) {
+                              int* t_cnt, unsigned long long* res, int bits = 31, uint32_t prefix = 0, unsigned long long above = 0) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  uint32_t prefix = 0;
-  unsigned long long above = 0;
-  const int shifts[4] = {23, 15, 7, 0}, widths[4] = {8, 8, 8, 7};
-  for (int level = 0; level < 4; ++level) {
-    const int shift = shifts[level], width = widths[level];
+  for (int shift = bits; shift > 0;) {
+    const int width = min(8, shift);
+    shift -= width;
     const uint32_t mask = (1u << width) - 1u;
     for (int i = tid; i < SW * 256; i += SB) { (&h_mass[0][0])[i] = 0; (&h_cnt[0][0])[i] = 0; }
     __syncthreads();
@@ -145,7 +145,7 @@ __device__ Found radix_search(Src p, int V, unsigned long long thr,
     const int bin = (int)res[0];
     above = res[1];
     prefix = (prefix << width) | (uint32_t)bin;
-    if (level == 3) {
+    if (shift == 0) {
       Found f;
       f.bits = prefix;
       f.above = above;
@@ -172,19 +172,39 @@ __device__ __forceinline__ long drawn_tie(const Found& f1, long k1, const Found&
   const long limit = (f2.bits == f1.bits) ? k1 : (long)f2.ties;
   return max(0L, min(j, limit - 1));
 }
-// The same from a list in shared memory that holds all of them (in any order): the one with that many equal ones of smaller index.
+// The same from a list in shared memory that holds all of them (in any order): the index found bit by bit, a count of the equal ones with
+// the bits so far for each, so that thousands of equal values cost no more than two. (Every entry against every other: 8,000 equal logits of
+// 128,256 5.72 ms a call; so 0.15.) `counts`: 32 integers of shared memory that nobody reads any more. All threads of the block come here.
 __device__ __forceinline__ void pick_equal(const float* list_p, const int* list_i, int n, const Found& f1, long k1, const Found& f2,
-                                           unsigned long long target, int* winner) {
-  const long j = drawn_tie(f1, k1, f2, target);
+                                           unsigned long long target, int V, int* counts, int* winner) {
+  const int tid = threadIdx.x;
   const float want = __uint_as_float(f2.bits);
-  for (int a = threadIdx.x; a < n; a += SB) {
-    if (list_p[a] != want) continue;
-    const int ia = list_i[a];
-    long rank = 0;
-    if (f2.ties > 1)
-      for (int b = 0; b < n; ++b) rank += (list_p[b] == want && list_i[b] < ia) ? 1 : 0;
-    if (rank == j) *winner = ia;
+  int at[CAND_MAX / SB];      // the indices of the thread's entries with that value; -1 otherwise
+#pragma unroll
+  for (int e = 0; e < CAND_MAX / SB; ++e) {
+    const int a = tid + e * SB;
+    at[e] = a < n && list_p[a] == want ? list_i[a] : -1;
   }
+  if (f2.ties <= 1) {
+#pragma unroll
+    for (int e = 0; e < CAND_MAX / SB; ++e)
+      if (at[e] >= 0) *winner = at[e];
+    return;
+  }
+  if (tid < 32) counts[tid] = 0;
+  __syncthreads();
+  long left = drawn_tie(f1, k1, f2, target);
+  int index = 0;
+  for (int bit = 31 - __clz(max(V - 1, 1)); bit >= 0; --bit) {
+    int c = 0;                // of the wave: those whose bits down to this one are the ones found and a zero
+#pragma unroll
+    for (int e = 0; e < CAND_MAX / SB; ++e) c += __popcll(__ballot(at[e] >> bit == index >> bit));
+    if ((tid & 63) == 0 && c) atomicAdd(&counts[bit], c);
+    __syncthreads();
+    const int below = counts[bit];
+    if (left >= below) { left -= below; index |= 1 << bit; }
+  }
+  if (tid == 0) *winner = index;
 }
 
 // A row's softmax is made by many blocks, ST_SLICES slices a row, in two kernels (the slices' maxima and
@@ -531,35 +551,55 @@ __global__ __launch_bounds__(SB) void sample_kernel(const float* __restrict__ lo
     const unsigned long long mass = f1.above + (unsigned long long)k1 * f1.each;
     const unsigned long long target = (unsigned long long)(u * (double)mass);
     const Found f2 = radix_search(cand_p, n, target, h_mass, h_cnt, t_mass, t_cnt, res);
-    pick_equal(cand_p, cand_i, n, f1, k1, f2, target, &winner);
+    pick_equal(cand_p, cand_i, n, f1, k1, f2, target, V, h_cnt[0], &winner);
     __syncthreads();
     if (tid == 0) out[row] = winner >= 0 ? winner : V - 1;
     return;
   }
 
-  // A flat row, whose nucleus reaches below the candidates. One pass sorts the row's mass into bins of an eighth and less of a factor of two
+  // A flat row, whose nucleus reaches below the candidates. One pass sorts the row's mass into bins of a factor of 1.03 to 1.06
   // (exponent and four bits of the mantissa); the bin in which the mass exceeds top_p, and then the one that the drawn token lies in,
   // are gathered from the row, and the searches walk those lists in shared memory: three passes over the row in place of nine
-  // whose first two put all of a row into a dozen bins (8 rows of 128,256, temperature 1.2, top-p 0.95: a call 324 -> 125 us; one row 312 -> 120, 64 rows 377 -> 163). A bin with more than CAND_MAX
-  // values (a distribution with hardly any) is left to the searches over the row below.
+  // whose first two put all of a row into a dozen bins (8 rows of 128,256, temperature 1.2, top-p 0.95: a call 324 -> 125 us; one row 312 -> 120,
+  // 64 rows 377 -> 163). A bin with more than CAND_MAX values (many equal ones, or a distribution with hardly any) stays in the row, and the
+  // search goes on over the row below the bin's digits.
   for (int i = tid; i < BINS; i += SB) { bin_mass[i] = 0; bin_cnt[i] = 0; }
   __syncthreads();
-  for (int base = tid; base < V; base += UN * SB) {
+  for (int base = 0; base < V; base += UN * SB) {      // every lane stays in the loop: the wave votes below
+    const int i0 = base + tid;
     float v[UN];
 #pragma unroll
-    for (int k = 0; k < UN; ++k) v[k] = base + k * SB < V ? p[base + k * SB] : -1.f;
+    for (int k = 0; k < UN; ++k) v[k] = i0 + k * SB < V ? p[i0 + k * SB] : -1.f;
 #pragma unroll
-    for (int k = 0; k < UN; ++k)
-      if (v[k] >= 0.f) {
-        const uint32_t b = __float_as_uint(v[k]) >> BIN_SHIFT;
+    for (int k = 0; k < UN; ++k) {
+      bool in = v[k] >= 0.f;
+      const int b = (int)(__float_as_uint(v[k]) >> BIN_SHIFT);
+      // a bin that a quarter of the wave's lanes and more share is added to once (twice at most: rows of few values); lane by lane
+      // on one counter, 128,256 equal logits took 0.95 ms a call; so 0.67
+#pragma unroll 1
+      for (int turn = 0; turn < 2; ++turn) {
+        const unsigned long long who = __ballot(in);
+        if (!who) break;
+        const int shared = __builtin_amdgcn_readlane(b, __ffsll((long long)who) - 1);
+        const bool same = in && b == shared;
+        const int count = __popcll(__ballot(same));
+        if (count < 16) break;
+        unsigned long long q = same ? to_q(v[k]) : 0ull;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
+        if (lane == 0) { atomicAdd(&bin_mass[shared], q); atomicAdd(&bin_cnt[shared], count); }
+        in = in && !same;
+      }
+      if (in) {
         atomicAdd(&bin_mass[b], to_q(v[k]));
         atomicAdd(&bin_cnt[b], 1);
       }
+    }
   }
   __syncthreads();
   int n = 0, n_bin = -1;
   // the values of the bin where the mass from the top exceeds thr (the lowest bin with any if none does), and the mass above that bin
-  auto gather = [&](unsigned long long thr, unsigned long long& above) {
+  auto gather = [&](unsigned long long thr, unsigned long long& above, int& bin) {
     if (wave == 0) {
       // lane l owns bins BINS - 1 - 32 l downwards
       unsigned long long mine = 0;
@@ -587,10 +627,13 @@ __global__ __launch_bounds__(SB) void sample_kernel(const float* __restrict__ lo
       }
     }
     __syncthreads();
-    const int bin = (int)(long long)res[0];
+    bin = (int)(long long)res[0];
     above = res[1];
     const int found = bin < 0 ? -1 : bin_cnt[bin];
-    if (found < 0 || found > CAND_MAX) return found;
+    if (found < 0 || found > CAND_MAX) {
+      __syncthreads();
+      return found;
+    }
     if (bin != n_bin) {
       n_bin = bin;
       n = found;
@@ -613,33 +656,27 @@ __global__ __launch_bounds__(SB) void sample_kernel(const float* __restrict__ lo
     return found;
   };
   unsigned long long over1 = 0, over2 = 0;
-  const int found1 = gather(tq, over1);
+  int bin1 = 0, bin2 = 0;
+  const int found1 = gather(tq, over1, bin1);
   if (found1 < 0) {                 // (not a number in the row: the last index)
     if (tid == 0) out[row] = V - 1;
     return;
   }
-  if (found1 <= CAND_MAX) {
-    Found f1 = radix_search(cand_p, n, tq - over1, h_mass, h_cnt, t_mass, t_cnt, res);
-    f1.above += over1;
-    const long k1 = kept_ties(f1, tq);
-    const unsigned long long mass = f1.above + (unsigned long long)k1 * f1.each;
-    const unsigned long long target = (unsigned long long)(u * (double)mass);
-    const int found2 = gather(target, over2);
-    if (found2 >= 0 && found2 <= CAND_MAX) {
-      Found f2 = radix_search(cand_p, n, target > over2 ? target - over2 : 0ull, h_mass, h_cnt, t_mass, t_cnt, res);
-      f2.above += over2;
-      pick_equal(cand_p, cand_i, n, f1, k1, f2, target, &winner);
-      __syncthreads();
-      if (tid == 0) out[row] = winner >= 0 ? winner : V - 1;
-      return;
-    }
-  }
-  const Found f1 = radix_search(p, V, tq, h_mass, h_cnt, t_mass, t_cnt, res);
+  Found f1;
+  if (found1 <= CAND_MAX) f1 = radix_search(cand_p, n, tq, h_mass, h_cnt, t_mass, t_cnt, res, BIN_SHIFT, (uint32_t)bin1, over1);
+  else f1 = radix_search(p, V, tq, h_mass, h_cnt, t_mass, t_cnt, res, BIN_SHIFT, (uint32_t)bin1, over1);
   const long k1 = kept_ties(f1, tq);
   const unsigned long long mass = f1.above + (unsigned long long)k1 * f1.each;
   // the drawn token: first in the kept order whose running sum exceeds u * mass
   const unsigned long long target = (unsigned long long)(u * (double)mass);
-  const Found f2 = radix_search(p, V, target, h_mass, h_cnt, t_mass, t_cnt, res);
+  if (gather(target, over2, bin2) <= CAND_MAX) {
+    const Found f2 = radix_search(cand_p, n, target, h_mass, h_cnt, t_mass, t_cnt, res, BIN_SHIFT, (uint32_t)bin2, over2);
+    pick_equal(cand_p, cand_i, n, f1, k1, f2, target, V, h_cnt[0], &winner);
+    __syncthreads();
+    if (tid == 0) out[row] = winner >= 0 ? winner : V - 1;
+    return;
+  }
+  const Found f2 = radix_search(p, V, target, h_mass, h_cnt, t_mass, t_cnt, res, BIN_SHIFT, (uint32_t)bin2, over2);
   const float want_value = __uint_as_float(f2.bits);   // the drawn token is the `want_index`-th (from 0) with this
   const long want_index = drawn_tie(f1, k1, f2, target);   // probability, in ascending order of index
 
