@@ -405,13 +405,15 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   // 25.5 -> 23.0 us, down 61.9 -> 60.0; 512 rows of the 3B layers 20.7 -> 19.1 and 32.2 -> 31.4; 4,096 rows x 2,048 x 2,048 38.3 -> 35.5. The tile of
   // 256 x 256 has no registers left and reads them behind the last step.
   const int col0 = n0 + (EPI == MF_GATED && WH == 1 ? wn * 16 : wn * 32), row0 = m0 + wm * 64 + lr;
-  const bool vec = ldc % 4 == 0 && N % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;
+  // (a row's last columns may be fewer than four; an add in the tile of 256 x 256 has no registers left for that)
+  constexpr bool ENDS = EPI != MF_ADD || AH == 1;
+  const bool vec = ldc % 4 == 0 && (ENDS ? N >= 4 : N % 4 == 0) && (uintptr_t)C % (4 * sizeof(TC)) == 0;
   typedef TC tc4 __attribute__((ext_vector_type(4)));
   constexpr bool ADDS = EPI == MF_ADD;
   tc4 old[ADDS ? 8 * WH : 1];
   auto ask_old = [&](int ah, int i) {
     const int tm = i / (2 * WH), wh = i / 2 % WH, tn = i % 2;
-    old[ADDS ? i : 0] = *(const tc4*)(C + (long)min(row0 + ah * 128 + tm * 16, M - 1) * ldc + min(col0 + wh * 128 + tn * 16 + lq * 4, N - 4));
+    old[ADDS ? i : 0] = *(const tc4*)(C + (long)min(row0 + ah * 128 + tm * 16, M - 1) * ldc + min(col0 + wh * 128 + tn * 16 + lq * 4, (N & ~3) - 4));
   };
   const bool early = ADDS && AH == 1 && vec && slice == 0 && steps >= 3;
   const int plain_steps = early ? steps - 3 : steps;
@@ -559,6 +561,12 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   if (wm == 0) mf_barrier();
   mf_wait_loads<0>();                 // (what was asked for beyond the last step has landed)
 
+  // the first `left` of a few columns
+  auto store_ends = [](auto* c, auto v, int left) {
+#pragma unroll
+    for (int j = 0; j + 1 < (int)(sizeof(v) / sizeof(v[0])); ++j)
+      if (j < left) c[j] = v[j];
+  };
   // The sums go to memory straight from the registers: a lane holds four consecutive columns of a row (4 * (lane / 16) of the 16
   // of a 16 x 16 tile, row lane % 16). Gate and up value of a column are the same lane's, so the gated rule needs nobody else's.
   // 16-bit outputs: two tiles' lanes hand each other half of their columns and store 16 bytes of eight (64 consecutive bytes of
@@ -593,7 +601,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
     };
     constexpr int HALVES = EPI == MF_GATED ? 1 : WH, TILES = EPI == MF_GATED && WH == 1 ? 1 : 2;      // of output columns
     if constexpr (sizeof(TC) == 2) {
-      if (ldc % 8 == 0 && N % 8 == 0 && (uintptr_t)C % 16 == 0) {
+      if (ldc % 8 == 0 && (uintptr_t)C % 16 == 0) {
         auto pack = [&](int ah, int tm, int wh, int tn) {
           const f32x4 v = sums(ah, tm, wh, tn, col0 + wh * 128 + tn * 16 + lq * 4);
           return __builtin_bit_cast(u32x2, bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]});
@@ -602,7 +610,11 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
         auto put = [&](u32x2 a, u32x2 b, int row, int n) {
           const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
           const auto hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
-          if (row < M && n < N) *(u32x4*)(C + (long)row * ldc + n) = u32x4{lo[0], hi[0], lo[1], hi[1]};
+          const u32x4 eight = {lo[0], hi[0], lo[1], hi[1]};
+          TC* c = C + (long)row * ldc + n;
+          if (row >= M || n >= N) return;
+          if (n + 8 <= N) *(u32x4*)c = eight;
+          else store_ends(c, __builtin_bit_cast(bf16x8, eight), N - n);
         };
 #pragma unroll
         for (int ah = 0; ah < AH; ++ah) {
@@ -623,7 +635,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
     }
 #pragma unroll
     for (int ah = 0; ah < AH; ++ah) {
-      if (ADDS && vec && !early) {      // (all asked for before the first is needed)
+      if (ADDS && !early) {             // (all asked for before the first is needed)
 #pragma unroll
         for (int i = 0; i < 8 * WH; ++i) ask_old(ah, i);
       }
@@ -636,23 +648,72 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
             const int n = col0 + wh * 128 + tn * 16 + lq * 4, row = row0 + ah * 128 + tm * 16;
             const f32x4 v = sums(ah, tm, wh, tn, n);
             if (row >= M || n >= N) continue;
+            tc4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = from_f32<TC>(ADDS ? to_f32<TC>(old[ADDS ? (tm * WH + wh) * 2 + tn : 0][j]) + v[j] : v[j]);
             TC* c = C + (long)row * ldc + n;
-            if (vec) {
-              tc4 o;
-#pragma unroll
-              for (int j = 0; j < 4; ++j) o[j] = from_f32<TC>(ADDS ? to_f32<TC>(old[ADDS ? (tm * WH + wh) * 2 + tn : 0][j]) + v[j] : v[j]);
+            if (!ENDS || n + 4 <= N) {
               *(tc4*)c = o;
-            } else {
+            } else {                    // (their old values are not among those asked for)
 #pragma unroll
-              for (int j = 0; j < 4; ++j)
-                if (n + j < N) c[j] = from_f32<TC>(EPI == MF_ADD ? to_f32<TC>(c[j]) + v[j] : v[j]);
+              for (int j = 0; j < 3; ++j)
+                if (n + j < N) c[j] = from_f32<TC>(ADDS ? to_f32<TC>(c[j]) + v[j] : v[j]);
             }
           }
     }
   };
+  // Outputs whose rows do not begin at whole fours of columns: single elements from the registers are sixteen rows an
+  // instruction, so the sums go through shared memory, half the tile's rows at a time, and a wave stores 64 consecutive columns. Row r's
+  // sixteen bytes c lie at place c ^ (r % 16): no two lanes of a write meet in a bank. Against element by element from the registers:
+  // 512 x 50,257 x 1,024 100 -> 66 us (58 where rows are whole eights), 2,048 x 32,001 x 2,048 316 -> 238 (239), the same in 16 bits
+  // 280 -> 223 (198), an add into 2,048 x 2,050 49 -> 36 (29). Rows of any width whose beginnings are whole fours need none of this: their
+  // last columns are stored one by one (2,048 x 32,001, rows 32,008 apart, 313 -> 231).
+  auto by_rows = [&](auto before, auto store) {
+    constexpr int ROW = 512 * WH, COLS = NCOLS / 64, RPT = 8 / COLS;      // bytes of a row of sums; a lane's columns of a row, rows at a time
+#pragma unroll
+    for (int ah = 0; ah < AH; ++ah) {
+      mf_barrier();                    // (everybody has read what lay here)
+#pragma unroll
+      for (int tm = 0; tm < 4; ++tm)
+#pragma unroll
+        for (int wh = 0; wh < WH; ++wh)
+#pragma unroll
+          for (int tn = 0; tn < 2; ++tn)
+            *(f32x4*)(lds + (wm * 64 + tm * 16 + lr) * ROW + (((wh * 32 + wn * 8 + tn * 4 + lq) ^ lr) << 4)) = acc[ah][tm][wh][tn];
+      mf_wait_reads<0>();
+      mf_barrier();
+      const int rows = min(128, M - m0 - ah * 128);
+      auto put = [&](int r, int c, float was) {
+        const int quad = c >> 2, gate = EPI == MF_GATED && WH == 1 ? (quad >> 2) * 8 + (quad & 3) : quad, up = WH == 1 ? gate + 4 : gate + 32;
+        const float v = *(const float*)(lds + r * ROW + ((gate ^ (r & 15)) << 4) + (c & 3) * 4);
+        float u = 0.f;
+        if constexpr (EPI == MF_GATED) u = *(const float*)(lds + r * ROW + ((up ^ (r & 15)) << 4) + (c & 3) * 4);
+        if (n0 + c < N) store(v, u, was, m0 + ah * 128 + r, n0 + c);
+      };
+      if constexpr (ADDS) {            // (eight old values asked for before the first is needed)
+        for (int r0 = wave; r0 < rows; r0 += 8 * RPT) {
+          float was[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) was[i] = before(m0 + ah * 128 + min(r0 + i / COLS * 8, rows - 1), min(n0 + lane + i % COLS * 64, N - 1));
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            if (r0 + i / COLS * 8 < rows) put(r0 + i / COLS * 8, lane + i % COLS * 64, was[i]);
+        }
+      } else {
+#pragma unroll 2
+        for (int r = wave; r < rows; r += 8)
+#pragma unroll
+          for (int c = lane; c < NCOLS; c += 64) put(r, c, 0.f);
+      }
+    }
+  };
+  const bool plain = !bias && !ex.col_scale && (EPI != MF_GATED || (act == GL3_ACT_SILU && ex.act_limit <= 0.f && ex.act_shift == 0.f));
   if (EPI != MF_GATED && slice > 0) {
     float* const p = P + (long)(slice - 1) * p_stride;
-    const bool whole = ldp % 4 == 0 && N % 4 == 0 && (uintptr_t)p % 16 == 0;
+    if (ldp % 4 != 0 || (uintptr_t)p % 16 != 0) {
+      by_rows([](int, int) { return 0.f; }, [&](float v, float, float, int m, int n) { p[(long)m * ldp + n] = ex.col_scale ? v * ex.col_scale[n] : v; });
+      return;
+    }
 #pragma unroll
     for (int ah = 0; ah < AH; ++ah)
 #pragma unroll
@@ -669,16 +730,25 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
               for (int j = 0; j < 4; ++j) v[j] *= ex.col_scale[min(n + j, N - 1)];
             }
             float* c = p + (long)row * ldp + n;
-            if (whole) *(f32x4*)c = v;
-            else {
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                if (n + j < N) c[j] = v[j];
-            }
+            if (n + 4 <= N) *(f32x4*)c = v;
+            else store_ends(c, v, N - n);
           }
     return;
   }
-  const bool plain = !bias && !ex.col_scale && (EPI != MF_GATED || (act == GL3_ACT_SILU && ex.act_limit <= 0.f && ex.act_shift == 0.f));
+  if (!vec) {
+    auto before = [&](int m, int n) { return ADDS ? to_f32<TC>(C[(long)m * ldc + n]) : 0.f; };
+    by_rows(before, [&](float v, float u, float was, int m, int n) {
+      if (bias) v += bias[n];
+      if constexpr (EPI == MF_GATED) {
+        if (bias) u += bias[N + n];
+        v = plain ? gl3_activation<true>(v, GL3_ACT_SILU) * u : gl3_gated<true>(v, u, act, ex.act_limit, ex.act_shift);
+      } else if (ex.col_scale) {
+        v *= ex.col_scale[n];
+      }
+      C[(long)m * ldc + n] = from_f32<TC>(ADDS ? was + v : v);
+    });
+    return;
+  }
   if (plain) finish(std::true_type{});
   else finish(std::false_type{});
 }

@@ -125,7 +125,7 @@ def test_unknown_tiles_are_refused(shape):
 
 # (columns in whole eights, in fours and in neither; one row, whole tiles, one row more than a tile)
 @pytest.mark.parametrize("shape", [1, 2, 5])
-@pytest.mark.parametrize("M, N", [(1, 8), (129, 136), (256, 256), (257, 260), (300, 523)])
+@pytest.mark.parametrize("M, N", [(1, 8), (2, 3), (129, 136), (256, 256), (257, 260), (300, 523)])
 def test_epilogues_of_the_tiled_products(shape, M, N):
     """An output that may be stored sixteen bytes at a time against one that begins at an odd place and is stored element by element:
     the same bits, whatever the epilogue applies, and nothing beside the output is written."""
@@ -167,3 +167,43 @@ def test_epilogues_of_the_tiled_products(shape, M, N):
             assert (off <= (2.0 ** -bits + 2.0 ** -17) * want.abs() + slack + 1e-6).all(), (dtype, kw)
     want = sums[:, :N] + res.double()
     assert ((both(torch.float32, lib.EPI_ADD, add=True) - want).abs() <= 2.0 ** -23 * want.abs() + Kd * 2.0 ** -23 * size[:, :N]).all()
+
+
+@pytest.mark.parametrize("shape", [1, 2, 5])
+@pytest.mark.parametrize("M, N", [(1, 3), (129, 130), (300, 523)])
+def test_slices_whose_columns_are_no_whole_fours(shape, M, N):
+    """The sums of later slices of K in rows of any width, at any place: those of rows of whole fours, and nothing beside them is written."""
+    lib = K()
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    wide = -(-N // 4) * 4
+    A, W, factor = (torch.randn(n, generator=gen, device="cuda") for n in ((M, 192), (wide, 192), (wide,)))
+    A, W = A.to(torch.bfloat16), W.to(torch.bfloat16)
+    for scale in (None, factor):
+        x, want = torch.zeros(M, wide, device=DEV), torch.empty(2, M, wide, device=DEV)
+        lib.gemm_mfma(A, W, x, lib.EPI_ADD, more_slices=want, shape=shape, col_scale=scale)
+        for first, ld in ((0, N), (0, wide + 4), (1, N + 1)):
+            y, whole = torch.zeros(M, N, device=DEV), torch.full((2, M, ld), -7.0, device=DEV)
+            part = whole[:, :, first:first + N]
+            lib.gemm_mfma(A, W[:N], y, lib.EPI_ADD, more_slices=part, shape=shape, col_scale=None if scale is None else factor[:N])
+            assert torch.equal(part, want[:, :, :N]) and torch.equal(y, x[:, :N])
+            assert torch.all(whole[:, :, :first] == -7.0) and torch.all(whole[:, :, first + N:] == -7.0)
+
+
+@pytest.mark.parametrize("M, N, Kd, dtype", [(512, 50257, 1024, torch.float32), (2048, 32001, 2048, torch.float32), (2048, 32001, 2048, torch.bfloat16)])
+def test_columns_that_are_no_whole_fours_take_little_longer(M, N, Kd, dtype):
+    """Rows of an odd number of columns against rows of whole eights: stored one element at a time from the registers they took 1.3 to 1.6 times as long."""
+    lib = K()
+    wide = -(-N // 8) * 8
+    A, W = (torch.randn(n, Kd, device=DEV).to(torch.bfloat16) for n in (M, wide))
+    outs = [torch.empty(M, n, device=DEV, dtype=dtype) for n in (N, wide)]
+    times = [[], []]
+    for _ in range(8):
+        for i, out in enumerate(outs):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                lib.gemm_mfma(A, W[:out.shape[1]], out)
+            b.record()
+            b.synchronize()
+            times[i].append(a.elapsed_time(b))
+    assert min(times[0]) < 1.25 * min(times[1])
