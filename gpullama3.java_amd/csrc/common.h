@@ -154,9 +154,10 @@ __host__ __device__ __forceinline__ long gl3_w_offset(int order, long n, int k, 
 enum { GL3_ACT_SILU = 0, GL3_ACT_GELU_TANH = 1, GL3_ACT_QUICK_GELU = 2 };
 #define GL3_ACT_KNOWN(act) ((act) >= GL3_ACT_SILU && (act) <= GL3_ACT_QUICK_GELU)
 
-// v / (1 + e^-v): the quotient by a reciprocal and one correction with its remainder, which leaves the rounding of a division (another
-// rounding once in some 2^22) in five instructions where the compiler's division takes ten. A quarter of both sides, so that the
-// reciprocal is a normal number up to the greatest 1 + e^-v; infinities, zeros and NaN by the instruction that ends a division.
+// v / (1 + e^-v): the quotient by a reciprocal and one correction with its remainder, in five instructions where the compiler's division
+// takes ten. A quarter of both sides, so that the reciprocal is a normal number up to the greatest 1 + e^-v; infinities, zeros and NaN by
+// the instruction that ends a division. Of all 2^32 floats those below 2^-124 in magnitude alone, a quarter of which is not exact, may get other
+// bits than from the division (the last one or two of a number without a leading one).
 __device__ __forceinline__ float gl3_silu_fast(float v) {
   const float d = fmaf(__builtin_amdgcn_exp2f(-1.4426950408889634f * v), 0.25f, 0.25f), w = 0.25f * v;
   const float r = __builtin_amdgcn_rcpf(d);

@@ -207,3 +207,32 @@ def test_columns_that_are_no_whole_fours_take_little_longer(M, N, Kd, dtype):
             b.synchronize()
             times[i].append(a.elapsed_time(b))
     assert min(times[0]) < 1.25 * min(times[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_the_gated_rule_over_the_range_of_its_gate(dtype):
+    """v / (1 + e^-v) for gates that a bias alone makes: every magnitude, the ends where e^-v leaves the floats, and what is no number."""
+    lib = K()
+    ends = [0.0, -0.0, 1e-30, -1e-30, 1e-38, -1e-38, -80.0, -87.0, -88.5, -88.7, -89.0, -100.0, -1e30, 1e30, 3e38, -3e38, float("inf"), float("-inf"), float("nan")]
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    N = 1 << 17
+    v = torch.empty(N, device=DEV).uniform_(-88.0, 88.0, generator=gen)
+    v[::2] = torch.exp2(torch.empty(N // 2, device=DEV).uniform_(-120.0, 6.4, generator=gen)) * torch.where(v[1::2] < 0, -1.0, 1.0)
+    v[:len(ends)] = torch.tensor(ends, device=DEV)
+    out = torch.empty(1, N, device=DEV, dtype=dtype)
+    zeros = [torch.zeros(n, 64, device=DEV, dtype=torch.bfloat16) for n in (1, 2 * N)]
+    lib.gemm_mfma(*zeros, out, lib.EPI_GATED, bias=torch.cat([v, torch.ones_like(v)]))
+    got, x = out[0].double(), v.double()
+    e = torch.exp(-x)
+    want = x / (1.0 + e)
+    # a rounding of the sum and one of the quotient; the exponential counts by its share e / (1 + e): its argument, |v| log2(e), is rounded and
+    # so is the factor (three halves of 2^-24 of |v|), its own result is a unit off; then the output's rounding (16 bits: 2^-9, or half of the smallest step, 2^-133, below 2^-126)
+    share = torch.where(torch.isinf(e), 1.0, e / (1.0 + e))
+    bound = want.abs() * (2.0 ** -24 * (2.0 + share * (1.5 * x.abs() + 2.0)) * 1.001 + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) + (2.0 ** -134 if dtype == torch.bfloat16 else 0.0) + 2.0 ** -147
+    inside = (x > -88.0) & (x < 1e31)
+    assert ((got - want).abs() <= bound)[inside].all()
+    below = (x <= -88.0) & torch.isfinite(x)              # (e^-v is an infinity from -88.73 down: minus nothing)
+    assert ((got <= 0) & (got >= want * 1.01 - 1e-45))[below].all()
+    by_end = dict(zip(map(str, ends), got[:len(ends)].tolist()))
+    assert by_end["inf"] == float("inf") and by_end["-inf"] != by_end["-inf"] and by_end["nan"] != by_end["nan"]
+    assert by_end["3e+38"] == pytest.approx(3e38, rel=2.0 ** -8) and by_end["0.0"] == by_end["-0.0"] == 0.0
