@@ -561,12 +561,6 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   if (wm == 0) mf_barrier();
   mf_wait_loads<0>();                 // (what was asked for beyond the last step has landed)
 
-  // the first `left` of a few columns
-  auto store_ends = [](auto* c, auto v, int left) {
-#pragma unroll
-    for (int j = 0; j + 1 < (int)(sizeof(v) / sizeof(v[0])); ++j)
-      if (j < left) c[j] = v[j];
-  };
   // The sums go to memory straight from the registers: a lane holds four consecutive columns of a row (4 * (lane / 16) of the 16
   // of a 16 x 16 tile, row lane % 16). Gate and up value of a column are the same lane's, so the gated rule needs nobody else's.
   // 16-bit outputs: two tiles' lanes hand each other half of their columns and store 16 bytes of eight (64 consecutive bytes of
@@ -576,8 +570,9 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   // 16,384 910 -> 790, of 8,192 of the 8B layers 1,379 -> 1,283; QKV of 2,048 rows 30.1 -> 27.8, of 512 rows of the 3B layers
   // 26.1 -> 24.7; the output projection of 5,886 rows of the 3B layers, which reads the rows it adds to, 137 -> 132 (110 without);
   // a head's 2,221 x 128,256 floats, bound by their way to memory, 1,048 to 1,090 on both.
-  auto finish = [&](auto plain_t) {
-    constexpr bool PLAIN = decltype(plain_t)::value;
+  // (plain_t: no extras; whole_t: rows of whole eights of columns, fours if 32 bits wide. Looked at a piece of a row at a time, gate/up took 0.9% longer.)
+  auto finish = [&](auto plain_t, auto whole_t) {
+    constexpr bool PLAIN = decltype(plain_t)::value, WHOLE = !ENDS || decltype(whole_t)::value;
     // columns n .. n + 3, ready to be stored (an add's old values aside)
     auto sums = [&](int ah, int tm, int wh, int tn, int n) {
       f32x4 v = acc[ah][tm][wh][tn];
@@ -613,8 +608,13 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
           const u32x4 eight = {lo[0], hi[0], lo[1], hi[1]};
           TC* c = C + (long)row * ldc + n;
           if (row >= M || n >= N) return;
-          if (n + 8 <= N) *(u32x4*)c = eight;
-          else store_ends(c, __builtin_bit_cast(bf16x8, eight), N - n);
+          if (WHOLE || n + 8 <= N) *(u32x4*)c = eight;
+          else {
+            const bf16x8 each = __builtin_bit_cast(bf16x8, eight);
+#pragma unroll
+            for (int j = 0; j < 7; ++j)
+              if (n + j < N) c[j] = each[j];
+          }
         };
 #pragma unroll
         for (int ah = 0; ah < AH; ++ah) {
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
 #pragma unroll
             for (int j = 0; j < 4; ++j) o[j] = from_f32<TC>(ADDS ? to_f32<TC>(old[ADDS ? (tm * WH + wh) * 2 + tn : 0][j]) + v[j] : v[j]);
             TC* c = C + (long)row * ldc + n;
-            if (!ENDS || n + 4 <= N) {
+            if (WHOLE || n + 4 <= N) {
               *(tc4*)c = o;
             } else {                    // (their old values are not among those asked for)
 #pragma unroll
@@ -710,7 +710,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   const bool plain = !bias && !ex.col_scale && (EPI != MF_GATED || (act == GL3_ACT_SILU && ex.act_limit <= 0.f && ex.act_shift == 0.f));
   if (EPI != MF_GATED && slice > 0) {
     float* const p = P + (long)(slice - 1) * p_stride;
-    if (ldp % 4 != 0 || (uintptr_t)p % 16 != 0) {
+    if (ldp % 4 != 0 || N % 4 != 0 || (uintptr_t)p % 16 != 0) {
       by_rows([](int, int) { return 0.f; }, [&](float v, float, float, int m, int n) { p[(long)m * ldp + n] = ex.col_scale ? v * ex.col_scale[n] : v; });
       return;
     }
@@ -729,9 +729,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
 #pragma unroll
               for (int j = 0; j < 4; ++j) v[j] *= ex.col_scale[min(n + j, N - 1)];
             }
-            float* c = p + (long)row * ldp + n;
-            if (n + 4 <= N) *(f32x4*)c = v;
-            else store_ends(c, v, N - n);
+            *(f32x4*)(p + (long)row * ldp + n) = v;
           }
     return;
   }
@@ -749,8 +747,9 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
     });
     return;
   }
-  if (plain) finish(std::true_type{});
-  else finish(std::false_type{});
+  if (ENDS && N % (sizeof(TC) == 2 ? 8 : 4) != 0) finish(std::false_type{}, std::false_type{});
+  else if (plain) finish(std::true_type{}, std::true_type{});
+  else finish(std::false_type{}, std::true_type{});
 }
 
 // What gemm_mfma_turns_kernel is built for: whole steps of 64 k, and byte offsets of 31 bits inside a tile's rows of A and
