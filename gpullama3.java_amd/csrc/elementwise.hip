@@ -441,92 +441,92 @@ __global__ void rope_cache_kernel(T* __restrict__ qkv, const int* __restrict__ p
 
 // The same for bfloat16 rows in units of 8 elements (16 bytes): one block per token, a thread
 // takes a unit of 8 pairs (half pairing: 8 elements and the 8 half a head further; adjacent
-// pairing: 16 consecutive elements) or of 8 elements that pass through; values have blocks of their own. head_dim and rot_dim / 2
-// are multiples of 8.
+// pairing: 16 consecutive elements), of 8 elements that pass through, or of 8 elements of a value head; the values of whole groups
+// of 8 positions have blocks of their own. head_dim and rot_dim / 2 are multiples of 8.
 typedef __bf16 rc_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float rc_f32x4 __attribute__((ext_vector_type(4)));
-#define RC_TOKENS 16     // tokens whose values a block writes (32: 2,048 tokens 8.5 against 8.0 us, 512 4.9 against 4.0)
+#define RC_TOKENS 16     // tokens whose whole groups a block writes (32: 2,048 tokens 8.5 against 8.0 us, 512 4.9 against 4.0)
+#define RC_TWO_BLOCKS 256     // tokens up to which values have blocks of their own: a batch of that many 5.4 us instead of 5.7, of 64 3.4 instead of
+                              // 4.2 (24 + 2 x 8 heads of 128); beyond it they are as many blocks as the chip holds at once, most with nothing to do
 
 __global__ __launch_bounds__(256) void rope_cache_vec_kernel(
     bf16_t* __restrict__ qkv, const int* __restrict__ positions, const int* __restrict__ seq_of_token,
     const int* __restrict__ block_table, int table_stride, const float* __restrict__ cos_tab,
     const float* __restrict__ sin_tab, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache, int n_heads, int n_kv,
-    int head_dim, int rot_dim, int adjacent, int page_size, int write_kv, long row_stride, int n_tokens, unsigned v_blocks) {
-  // The values of 8 consecutive positions of a sequence share 16 bytes of a transposed page. The first of the step's tokens in such a group
-  // of 8 positions stands for all of them that the step brings (they follow it in the packed order): 16 bytes a dim where the group is whole,
-  // single elements at the ends of a sequence's tokens. The first `v_blocks` blocks do that, RC_TOKENS tokens each, beside those of the
-  // queries and keys: which tokens are firsts and how many follow comes from one look at all of them. (Done by the block of the first
-  // token, behind its queries and keys, with a look at one token after the other: 512 tokens of 32 + 2 x 8 heads of 64 5.4 -> 4.0 us, 2,048
-  // 11.4 -> 8.0; of 24 + 2 x 8 heads of 128 7.0 -> 5.7 and 15.7 -> 10.4, 8,192 56 -> 40, of which the values are a third.)
+    int head_dim, int rot_dim, int adjacent, int page_size, int write_kv, long row_stride, int n_tokens, unsigned v_blocks, int v_parts) {
+  // The values of 8 consecutive positions of a sequence share 16 bytes of a transposed page. Where the step brings all 8 (in the packed
+  // order), one of the first `v_blocks` blocks writes them, 16 bytes a dim: RC_TOKENS tokens a block, in `v_parts` blocks where two groups are more
+  // than 256 units; which groups are whole comes from one look at all of the tokens. Any other token's values are written single
+  // elements by a block of the token's own, or, in steps of many tokens, behind its queries and keys. All of it by the block of a group's first token,
+  // with a look at one token after the other: a prompt of 512 tokens of 32 + 2 x 8 heads of 64 5.6 us, of 24 + 2 x 8 heads of 128 7.1; so 4.3 and 5.5
+  // (2,048: 7.7 and 9.6, 8,192: 21 and 31). Short runs in the blocks of 16 tokens as well: 64 sequences with a token each, which are nothing
+  // else, 7.2 and 12.0 us, 41 with 32 + 2 x 32 heads of 128; so 3.2, 3.4 and 6.7.
   if (blockIdx.x < v_blocks) {
-    __shared__ int f_token[RC_TOKENS], f_run[RC_TOKENS], f_pos[RC_TOKENS], f_page[RC_TOKENS], n_first;
-    const int base = blockIdx.x * RC_TOKENS;
+    __shared__ int g_token[2], g_pos[2], g_page[2], n_whole;      // (sixteen tokens hold the beginnings of two groups at most)
+    const int base = blockIdx.x / v_parts * RC_TOKENS;
     if (base >= n_tokens) return;
     if (threadIdx.x < 64) {
-      // lane i: token base - 1 + i, one in front of the block's and seven behind them
-      const int i = threadIdx.x, t = base - 1 + i;
-      const bool is = t >= 0 && t < n_tokens;
-      const int pos = positions[min(max(t, 0), n_tokens - 1)], seq = seq_of_token[min(max(t, 0), n_tokens - 1)];
+      // lane i: token base + i, seven behind the block's among them
+      const int i = threadIdx.x, t = base + i;
+      const int pos = positions[min(t, n_tokens - 1)], seq = seq_of_token[min(t, n_tokens - 1)];
       const int pos0 = __shfl_up(pos, 1, 64), seq0 = __shfl_up(seq, 1, 64);
-      const bool follows = is && t > 0 && i > 0 && seq0 == seq && pos0 == pos - 1;
-      const unsigned long long after = __ballot(follows);
-      const bool first = is && i >= 1 && i <= RC_TOKENS && ((pos & 7) == 0 || !follows);
-      const unsigned long long firsts = __ballot(first);
-      if (first) {
-        const int k = __popcll(firsts & ((1ull << i) - 1));
-        f_token[k] = t;
-        f_pos[k] = pos;
-        f_run[k] = 1 + min(7 - (pos & 7), __builtin_ctzll(~(after >> (i + 1))));
-        f_page[k] = block_table[(long)seq * table_stride + pos / page_size];
+      const unsigned long long after = __ballot(i > 0 && t < n_tokens && seq0 == seq && pos0 == pos - 1);      // (follows the token in front)
+      const bool whole = i < RC_TOKENS && t < n_tokens && (pos & 7) == 0 && (after >> (i + 1) & 127) == 127;
+      const unsigned long long wholes = __ballot(whole);
+      if (whole) {
+        const int k = __popcll(wholes & ((1ull << i) - 1));
+        g_token[k] = t;
+        g_pos[k] = pos;
+        g_page[k] = block_table[(long)seq * table_stride + pos / page_size];
       }
-      if (i == 0) n_first = __popcll(firsts);
+      if (i == 0) n_whole = __popcll(wholes);
     }
     __syncthreads();
-    const int units = n_kv * (head_dim / 8), total = n_first * units;
-    for (int w = threadIdx.x; w < total; w += blockDim.x) {
-      const int k = w / units, u = w % units, in_page = f_pos[k] % page_size;
-      const int ch = u / (head_dim / 8), e0 = (u % (head_dim / 8)) * 8;
-      bf16_t* vpage = v_cache + ((long)f_page[k] * n_kv + ch) * page_size * head_dim;
-      const long at = gl3_v_offset(e0, in_page, page_size);   // dims e0 .. e0+7 lie in one tile, 8 elements apart
-      const bf16_t* from = qkv + (long)f_token[k] * row_stride + (long)(n_heads + n_kv + ch) * head_dim + e0;
-      if (f_run[k] == 8) {                         // a whole group of 8 positions (pos % 8 == 0): 16 bytes a dim
-        rc_bf16x8 v[8];
+    const int units = n_kv * (head_dim / 8), w = blockIdx.x % v_parts * 256 + threadIdx.x;
+    if (w >= n_whole * units) return;
+    const int k = w / units, u = w % units, in_page = g_pos[k] % page_size;
+    const int ch = u / (head_dim / 8), e0 = (u % (head_dim / 8)) * 8;
+    bf16_t* vpage = v_cache + ((long)g_page[k] * n_kv + ch) * page_size * head_dim;
+    const long at = gl3_v_offset(e0, in_page, page_size);   // dims e0 .. e0+7 lie in one tile, 8 elements apart
+    const bf16_t* from = qkv + (long)g_token[k] * row_stride + (long)(n_heads + n_kv + ch) * head_dim + e0;
+    rc_bf16x8 v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = *(const rc_bf16x8*)(from + (long)i * row_stride);
+    for (int i = 0; i < 8; ++i) v[i] = *(const rc_bf16x8*)(from + (long)i * row_stride);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          rc_bf16x8 o;
+    for (int e = 0; e < 8; ++e) {
+      rc_bf16x8 o;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) o[i] = v[i][e];
-          *(rc_bf16x8*)(vpage + at + 8 * e) = o;
-        }
-      } else {
-        for (int i = 0; i < f_run[k]; ++i) {
-          const rc_bf16x8 v = *(const rc_bf16x8*)(from + (long)i * row_stride);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) vpage[at + i + 8 * e] = v[e];
-        }
-      }
+      for (int i = 0; i < 8; ++i) o[i] = v[i][e];
+      *(rc_bf16x8*)(vpage + at + 8 * e) = o;
     }
     return;
   }
   // Blocks with consecutive numbers go to different XCDs, each with a second-level cache of its own; neighbouring
-  // tokens go to one XCD (v_blocks is a multiple of 8).
-  const int per_xcd = (n_tokens + 7) / 8, b = blockIdx.x - v_blocks;
-  const int t = (b % 8) * per_xcd + b / 8;
+  // tokens go to one XCD (v_blocks is a multiple of 8). A step of few tokens has two blocks a token, the second for its values alone.
+  const int per_xcd = (n_tokens + 7) / 8, b0 = blockIdx.x - v_blocks;
+  const bool two = gridDim.x - v_blocks > 8u * per_xcd, second = b0 >= 8 * per_xcd;
+  const int b = second ? b0 - 8 * per_xcd : b0, t = (b % 8) * per_xcd + b / 8;
   if (t >= n_tokens) return;
-  const int pos = positions[t];
   bf16_t* row = qkv + (long)t * row_stride;
   const int half = rot_dim / 2;
+  const int pos = positions[t];
+  const bool values = write_kv && second == two;
+  // lane i < 15: token t - 7 + i; lanes 7 - pos % 8 and the seven behind it are this token's group, if the step brings that
+  const int lane = threadIdx.x & 63, beside = lane < 15 ? t - 7 + lane : t, in = min(max(beside, 0), n_tokens - 1);
+  int p = 0, s = 0, seq = 0;
+  if (values) { p = positions[in]; s = seq_of_token[in]; }
   long page = 0;
-  if (write_kv) page = block_table[(long)seq_of_token[t] * table_stride + pos / page_size];
+  if (write_kv) {
+    seq = seq_of_token[t];
+    page = block_table[(long)seq * table_stride + pos / page_size];
+  }
   const int in_page = pos % page_size;
   const bool rotate = cos_tab != nullptr;
   const int rot_heads = write_kv ? n_heads + n_kv : n_heads;
   const int pair_units = rotate ? half / 8 : 0;              // per head
   const int plain_units = (head_dim - (rotate ? rot_dim : 0)) / 8;
   const int per_head = pair_units + plain_units;
-  const int total = rot_heads * per_head;
+  const int total = second ? 0 : rot_heads * per_head;
   for (int w = threadIdx.x; w < total; w += blockDim.x) {
     const int head = w / per_head, u = w % per_head;
     bf16_t* src = row + (long)head * head_dim;
@@ -570,6 +570,16 @@ __global__ __launch_bounds__(256) void rope_cache_vec_kernel(
     *(rc_bf16x8*)dst(ea) = oa;
     *(rc_bf16x8*)dst(eb) = ob;
   }
+  if (!values) return;
+  const unsigned long long group = 255ull << (7 - (pos & 7));
+  if ((__ballot(lane < 15 && beside == in && s == seq && p - pos == lane - 7) & group) == group) return;      // (a whole group: written above)
+  for (int w = threadIdx.x; w < n_kv * (head_dim / 8); w += blockDim.x) {
+    const int ch = w / (head_dim / 8), e0 = (w % (head_dim / 8)) * 8;
+    bf16_t* const to = v_cache + ((long)page * n_kv + ch) * page_size * head_dim + gl3_v_offset(e0, in_page, page_size);
+    const rc_bf16x8 v = *(const rc_bf16x8*)(row + (long)(n_heads + n_kv + ch) * head_dim + e0);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) to[8 * e] = v[e];
+  }
 }
 
 extern "C" int gl3_rope_cache_write(void* qkv, int dtype, const int* positions, const int* seq_of_token,
@@ -597,10 +607,12 @@ extern "C" int gl3_rope_cache_write(void* qkv, int dtype, const int* positions, 
                      (!cos_tab || ((uintptr_t)cos_tab % 16 == 0 && (uintptr_t)sin_tab % 16 == 0)) &&
                      (!write_kv || ((uintptr_t)k_cache % 16 == 0));
   if (units) {
-    const unsigned v_blocks = write_kv ? ((n_tokens + RC_TOKENS - 1) / RC_TOKENS + 7) / 8 * 8 : 0;
-    rope_cache_vec_kernel<<<dim3(v_blocks + (n_tokens + 7) / 8 * 8), dim3(256), 0, stream>>>(
+    const int v_parts = (2 * n_kv * (head_dim / 8) + 255) / 256;      // (two whole groups of 16 tokens at most, a unit a thread)
+    const unsigned v_blocks = write_kv && n_tokens >= 8 ? ((n_tokens + RC_TOKENS - 1) / RC_TOKENS * v_parts + 7) / 8 * 8 : 0;
+    const unsigned blocks_a_token = write_kv && n_tokens <= RC_TWO_BLOCKS ? 2 : 1;
+    rope_cache_vec_kernel<<<dim3(v_blocks + (n_tokens + 7) / 8 * 8 * blocks_a_token), dim3(256), 0, stream>>>(
         (bf16_t*)qkv, positions, seq_of_token, block_table, table_stride, cos_tab, sin_tab, (bf16_t*)k_cache,
-        (bf16_t*)v_cache, n_heads, n_kv, head_dim, cos_tab ? rot_dim : 0, adjacent, page_size, write_kv, row_stride, n_tokens, v_blocks);
+        (bf16_t*)v_cache, n_heads, n_kv, head_dim, cos_tab ? rot_dim : 0, adjacent, page_size, write_kv, row_stride, n_tokens, v_blocks, v_parts);
     GL3_LAUNCH_CHECK();
     return 0;
   }

@@ -1510,7 +1510,7 @@ def test_norms_of_rows_held_at_once(d, S):
 # (sequences that begin and end at every place of a group of 8 positions and of a block of 16 tokens; one token each; one long one)
 @pytest.mark.parametrize("starts, lens", [([0], [1]), ([7], [130]), ([0, 5, 8, 63], [16, 11, 21, 9]), ([3] * 20, [1] * 20), ([0, 1, 2, 3, 4, 5, 6, 7], [15, 14, 13, 12, 11, 10, 9, 8]),
                                           ([60, 0, 31, 64], [33, 7, 40, 64])])
-@pytest.mark.parametrize("Kh, hs", [(1, 16), (8, 64), (3, 128)])
+@pytest.mark.parametrize("Kh, hs", [(1, 16), (8, 64), (3, 128), (23, 96), (32, 128)])
 def test_values_of_a_prompt_s_tokens_in_the_cache(starts, lens, Kh, hs):
     """Every token's value is in its place, whatever tokens share its 8 positions, and nothing else in the cache has changed."""
     rng = np.random.default_rng(sum(lens) + hs)
@@ -1529,3 +1529,38 @@ def test_values_of_a_prompt_s_tokens_in_the_cache(starts, lens, Kh, hs):
     cos, sin = P.rope_table(256, hs, 10000.0)
     K().rope_cache_write(qkv, dev(positions, torch.int32), dev(seq_of, torch.int32), table, dev(cos), dev(sin), kc, vc, H, Kh, hs, hs, False, page)
     assert torch.equal(untile_values(vc), want)
+
+
+@pytest.mark.parametrize("H, Kh, hs, most", [(32, 8, 64, 1.7), (24, 8, 128, 1.7), (32, 32, 128, 2.5)])
+def test_rotation_of_a_batch_takes_little_longer_than_of_a_prompt(H, Kh, hs, most):
+    """One token of each of 64 sequences against 64 tokens of one: their values are written one element at a time, but by as many blocks as
+    there are tokens (by four blocks that took 2.2 to 4.9 times the prompt's time)."""
+    lib = K()
+    T, page = 64, 64
+    table = torch.arange(1, T + 1, dtype=torch.int32, device=DEV)
+    kc, vc = torch.zeros(T + 1, Kh, page, hs, dtype=torch.bfloat16, device=DEV), torch.zeros(T + 1, Kh, hs, page, dtype=torch.bfloat16, device=DEV)
+    cos, sin = (torch.rand(page, hs // 2, device=DEV) for _ in range(2))
+    places = torch.arange(T, dtype=torch.int32, device=DEV)
+    batch, prompt = (places, places, table.view(T, 1)), (places, torch.zeros_like(places), table.view(1, T))
+    graphs = []
+    for positions, seq_of, rows in (batch, prompt):
+        qkv = torch.randn(T, (H + 2 * Kh) * hs, device=DEV).to(torch.bfloat16)
+
+        def call():
+            lib.rope_cache_write(qkv, positions, seq_of, rows, cos, sin, kc, vc, H, Kh, hs, hs, False, page)
+        call()
+        torch.cuda.synchronize()
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            for _ in range(50):
+                call()
+    least = [float("inf")] * 2
+    for _ in range(10):
+        for i, graph in enumerate(graphs):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            least[i] = min(least[i], a.elapsed_time(b))
+    assert least[0] < most * least[1], least
