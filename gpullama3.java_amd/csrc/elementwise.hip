@@ -104,8 +104,7 @@ extern "C" int gl3_embed(const void* table, int table_dtype, const int* ids, flo
 
 // ----------------------------------------------------------------- rmsnorm of rows that a block holds at once
 // What rmsnorm_kernel and add_slices_rmsnorm_kernel (below) do, the same bits, for rows of whole 16-byte pieces of which a thread has PIECES
-// at most (one up to 2,048 floats and at 4,096, two up to 8,192: the launchers' threads are as many there) and NS slices (0: none; 8: five to eight, the ones that
-// do not exist read the last again and are not added). These norms of few rows are bound by trips to memory one after the other: there
+// at most (one up to 2,048 floats and at 4,096, two up to 8,192: the launchers' threads are as many there) and NS slices (0: none). These norms of few rows are bound by trips to memory one after the other: there
 // it was the row, then its slices (a branch for each, in front of which the compiler waits), then, behind the sum of squares, the weight; here
 // all of them are asked for at once, and the waves' sums are read at once as well. In a replayed graph, 64 rows of 2,048 with four slices 3.85 ->
 // 3.13 us, 150 of 4,096 with seven 7.6 -> 7.2; 2,048 rows of 2,048 with one slice 15.4 -> 12.5, 8,192 of 4,096 without 47 -> 39, 5,886 of 3,072 with
@@ -128,7 +127,7 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(float* __restrict__ x, 
     const int at = min(first + k * stride, d - 4);      // (what is beyond the row reads its end again)
     v[k] = *(const f4*)(xr + at);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) p[k][s] = *(const f4*)(P + (long)(NS == 8 ? min(s, n_slices - 1) : s) * slice_stride + src * ldp + at);
+    for (int s = 0; s < NS; ++s) p[k][s] = *(const f4*)(P + (long)s * slice_stride + src * ldp + at);
     wv[k] = *(const w4*)(w + at);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -136,8 +135,7 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(float* __restrict__ x, 
 #pragma unroll
   for (int k = 0; k < PIECES; ++k) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s)
-      if (NS < 8 || s < n_slices) v[k] += p[k][s];
+    for (int s = 0; s < NS; ++s) v[k] += p[k][s];
     const int i = first + k * stride;
     if (i >= d) continue;
     if (NS > 0 && !rows) *(f4*)(xr + i) = v[k];
@@ -170,10 +168,12 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(float* __restrict__ x, 
   }
 }
 
-// Whether norm_rows_kernel takes these rows (with `threads` threads a row); the launch. P null: no slices.
+// Whether norm_rows_kernel takes these rows (with `threads` threads a row); the launch. P null: no slices. Two pieces with more than four slices
+// are so many registers that a CU holds a row or two: 300 rows of 5,120 with five 11.3 us, the kernel for any rows 8.9 (with four 7.8 and 7.7, of 3,072
+// 5.3 and 5.7).
 static bool norm_rows_takes(const void* x, const void* P, int n_slices, long slice_stride, long ldp, const void* w, int w_dtype, const void* out,
                             int d, int threads) {
-  return d % 4 == 0 && d <= 8 * threads && n_slices <= 8 && ldp % 4 == 0 && slice_stride % 4 == 0 && (uintptr_t)x % 16 == 0 &&
+  return d % 4 == 0 && d <= (n_slices <= 4 ? 8 : 4) * threads && n_slices <= 8 && ldp % 4 == 0 && slice_stride % 4 == 0 && (uintptr_t)x % 16 == 0 &&
          (uintptr_t)P % 16 == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)w % (w_dtype == GL3_F32 ? 16 : 8) == 0;
 }
 template <typename TW, typename TO>
@@ -191,7 +191,10 @@ static void launch_norm_rows(float* x, const int* rows, const float* P, int n_sl
     case 2: GO(2); break;
     case 3: GO(3); break;
     case 4: GO(4); break;
-    default: GO(8);
+    case 5: norm_rows_kernel<TW, TO, 5, 1> ARGS; break;      // (these rows are one piece a thread)
+    case 6: norm_rows_kernel<TW, TO, 6, 1> ARGS; break;
+    case 7: norm_rows_kernel<TW, TO, 7, 1> ARGS; break;
+    case 8: norm_rows_kernel<TW, TO, 8, 1> ARGS; break;
   }
 #undef GO
 #undef ARGS

@@ -1507,6 +1507,34 @@ def test_norms_of_rows_held_at_once(d, S):
                 assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (wdtype, odtype, r is None)
 
 
+@pytest.mark.parametrize("d", [5120, 6144])
+def test_a_fifth_slice_costs_a_norm_its_reading(d):
+    """Rows of two pieces a thread with five slices against four: a sixth more to read (held at once, they took 1.4 times as long)."""
+    lib = K()
+    n = 300
+    x, w, out = torch.randn(n, d, device=DEV), torch.ones(d, device=DEV), torch.empty(n, d, device=DEV, dtype=torch.bfloat16)
+    graphs = []
+    for S in (4, 5):
+        parts = torch.randn(S, n, d, device=DEV) * 1e-3
+        lib.add_slices_rmsnorm(x, parts, w, out, 1e-5)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(50):
+                lib.add_slices_rmsnorm(x, parts, w, out, 1e-5)
+        graphs.append((graph, parts))
+    least = [float("inf")] * 2
+    for _ in range(10):
+        for i, (graph, _) in enumerate(graphs):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            least[i] = min(least[i], a.elapsed_time(b))
+    assert least[1] < 1.3 * least[0], least
+
+
 # (sequences that begin and end at every place of a group of 8 positions and of a block of 16 tokens; one token each; one long one)
 @pytest.mark.parametrize("starts, lens", [([0], [1]), ([7], [130]), ([0, 5, 8, 63], [16, 11, 21, 9]), ([3] * 20, [1] * 20), ([0, 1, 2, 3, 4, 5, 6, 7], [15, 14, 13, 12, 11, 10, 9, 8]),
                                           ([60, 0, 31, 64], [33, 7, 40, 64])])
