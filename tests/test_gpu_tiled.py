@@ -209,6 +209,48 @@ def test_columns_that_are_no_whole_fours_take_little_longer(M, N, Kd, dtype):
     assert min(times[0]) < 1.25 * min(times[1])
 
 
+@pytest.mark.parametrize("M, N, Kd", [(66, 1000, 1024), (400, 2048, 2048)])
+def test_a_bias_costs_little(M, N, Kd):
+    """32-bit sums with a bias against the same without: read behind the steps, between the stores, the bias took a fifth to a third of the product's time."""
+    lib = K()
+    A, W = (torch.randn(n, Kd, device=DEV).to(torch.bfloat16) for n in (M, N))
+    out, bias = torch.empty(M, N, device=DEV), torch.randn(N, device=DEV)
+    graphs = []
+    for b in (None, bias):
+        lib.gemm_mfma(A, W, out, bias=b)
+        torch.cuda.synchronize()
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            for _ in range(20):
+                lib.gemm_mfma(A, W, out, bias=b)
+    least = [float("inf")] * 2
+    for _ in range(10):
+        for i, graph in enumerate(graphs):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            least[i] = min(least[i], a.elapsed_time(b))
+    assert least[1] < 1.15 * least[0], least
+
+
+# (rows of whole fours, whose bias is read in front of the steps, and others; columns beyond the last tile's)
+@pytest.mark.parametrize("shape", [1, 2, 5])
+@pytest.mark.parametrize("M, N", [(3, 4), (130, 260), (66, 1000), (129, 131), (2, 3)])
+def test_every_column_gets_its_own_bias(shape, M, N):
+    """Products of nothing leave the bias alone, in every row."""
+    lib = K()
+    A, W = (torch.zeros(n, 192, device=DEV, dtype=torch.bfloat16) for n in (M, N))
+    bias = torch.arange(1, N + 1, device=DEV, dtype=torch.float32)
+    for first in (0, 1):                        # (at sixteen bytes and at an odd place)
+        whole = torch.full((M, N + 5), -7.0, device=DEV)
+        out = whole[:, first:first + N] if first else torch.full((M, N), -7.0, device=DEV)
+        lib.gemm_mfma(A, W, out, bias=torch.cat([bias[:1], bias])[1:] if first else bias, shape=shape)
+        assert torch.equal(out, bias.expand(M, N))
+        assert torch.all(whole[:, N + first:] == -7.0) and torch.all(whole[:, :first] == -7.0)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_the_gated_rule_over_the_range_of_its_gate(dtype):
     """v / (1 + e^-v) for gates that a bias alone makes: every magnitude, the ends where e^-v leaves the floats, and what is no number."""
