@@ -314,27 +314,45 @@ __device__ __forceinline__ unsigned mf_w_offset(int row, int k, long ldw, int w_
                    : (unsigned)((long)(row - n0) * ldw + k) * 2;
 }
 
+// bytes of shared memory of a tile: its steps in turn, each A's halves, then W's
+constexpr int mf_stages(int AH, int WH) { return AH == 2 ? 2 : WH == 2 ? 3 : 4; }
+constexpr int mf_lds(int AH, int WH) { return mf_stages(AH, WH) * (AH + WH) * 16384; }
+
+struct MfTurns {
+  const bf16_t* A;
+  const bf16_t* W;
+  void* C;
+  int M, N, K;
+  long lda, ldw, ldc;
+  int k_per_slice;
+  float* P;
+  long p_stride, ldp;
+  const float* bias;
+  int act, w_steps;
+  const int* w_pos;
+  MfExtras ex;
+};
+// Blocks of tiles_m x tiles_n tiles, the first at row m_first; `tile`: its number in their order (block -> tile as above).
 template <int EPI, typename TC, int WT, int AH, int WH>
-__global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
-                                                                  TC* __restrict__ C, int M, int N, int K, long lda, long ldw,
-                                                                  long ldc, int tiles_m, int tiles_n, int group_m,
-                                                                  int k_per_slice, float* __restrict__ P, long p_stride, long ldp,
-                                                                  const float* __restrict__ bias, int act, int w_steps,
-                                                                  const int* __restrict__ w_pos, MfExtras ex) {
+__device__ __forceinline__ void mf_turns_tile(char* lds, const MfTurns& a, int m_first, int tiles_m, int tiles_n, int group_m, int tile, int slice) {
+  const bf16_t* __restrict__ const A = a.A;
+  const bf16_t* __restrict__ const W = a.W;
+  TC* __restrict__ const C = (TC*)a.C;
+  float* __restrict__ const P = a.P;
+  const float* __restrict__ const bias = a.bias;
+  const int* __restrict__ const w_pos = a.w_pos;
+  const int M = a.M, N = a.N, K = a.K, k_per_slice = a.k_per_slice, act = a.act, w_steps = a.w_steps;
+  const long lda = a.lda, ldw = a.ldw, ldc = a.ldc, p_stride = a.p_stride, ldp = a.ldp;
+  const MfExtras ex = a.ex;
   constexpr int NCOLS = (EPI == MF_GATED ? 64 : 128) * WH;
-  constexpr int STAGES = AH == 2 ? 2 : WH == 2 ? 3 : 4, STAGE = (AH + WH) * 16384;      // a step: A's halves, then W's
-  __shared__ __attribute__((aligned(1024))) char lds[STAGES * STAGE];
+  constexpr int STAGE = (AH + WH) * 16384;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wm = wave >> 2, wn = wave & 3;
   const int lr = lane & 15, lq = lane >> 4;
-  const int n_tiles = tiles_m * tiles_n, per_xcd = (n_tiles + 7) / 8;
-  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;       // (block -> tile as above)
-  if (tile >= n_tiles) return;
   const int band = tile / (group_m * tiles_n), in_band = tile % (group_m * tiles_n);
   const int band_rows = min(group_m, tiles_m - band * group_m);
-  const int m0 = (band * group_m + in_band % band_rows) * (128 * AH);
+  const int m0 = m_first + (band * group_m + in_band % band_rows) * (128 * AH);
   const int n0 = (in_band / band_rows) * NCOLS;
-  const int slice = blockIdx.y;
   // (the last of many slices may have no step left: it stores zeros)
   const int k_begin = min(slice * k_per_slice, K - 64), steps = max(0, (min(K, (slice + 1) * k_per_slice) - slice * k_per_slice) >> 6);
 
@@ -764,12 +782,72 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   else finish(std::false_type{}, std::true_type{});
 }
 
+template <int EPI, typename TC, int WT, int AH, int WH>
+__global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                  TC* __restrict__ C, int M, int N, int K, long lda, long ldw,
+                                                                  long ldc, int tiles_m, int tiles_n, int group_m,
+                                                                  int k_per_slice, float* __restrict__ P, long p_stride, long ldp,
+                                                                  const float* __restrict__ bias, int act, int w_steps,
+                                                                  const int* __restrict__ w_pos, MfExtras ex) {
+  __shared__ __attribute__((aligned(1024))) char lds[mf_lds(AH, WH)];
+  const int n_tiles = tiles_m * tiles_n, per_xcd = (n_tiles + 7) / 8;
+  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;       // (block -> tile as above)
+  if (tile >= n_tiles) return;
+  const MfTurns a{A, W, C, M, N, K, lda, ldw, ldc, k_per_slice, P, p_stride, ldp, bias, act, w_steps, w_pos, ex};
+  mf_turns_tile<EPI, TC, WT, AH, WH>(lds, a, 0, tiles_m, tiles_n, group_m, tile, blockIdx.y);
+}
+
+// Tiles of 256 x 256 for the first 256 * big_m rows, smaller ones (128 rows x 256, or 128 x 128) for those behind them, the large
+// tiles of all slices first. What bounds a product of a few rounds of the chip is the last one: 2,221 rows of the 1B layers' gate/up product are
+// 2.25 rounds of 256 x 256 and took three. Here the small tiles fill the CUs that the last whole round of large ones leaves (one launch: they
+// start where a CU is done, not where all are), at a lower rate but for a tenth of the rows: 130.5 -> 112.5 us; 5,886 rows of the
+// 3B layers' output projection 126 -> 105, of their QKV product's 3,500 111 -> 89. The same sums, whatever the tile: bit for bit.
+template <int EPI, typename TC, int WT, int SWH>
+__global__ __launch_bounds__(512, 2) void gemm_mfma_two_tiles_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                      TC* __restrict__ C, int M, int N, int K, long lda, long ldw,
+                                                                      long ldc, int big_m, int big_n, int small_m, int small_n, int slices,
+                                                                      int k_per_slice, float* __restrict__ P, long p_stride, long ldp,
+                                                                      const float* __restrict__ bias, int act, int w_steps,
+                                                                      const int* __restrict__ w_pos, MfExtras ex) {
+  constexpr int BIG = mf_lds(2, 2), SMALL = mf_lds(1, SWH);
+  __shared__ __attribute__((aligned(1024))) char lds[BIG > SMALL ? BIG : SMALL];
+  const MfTurns a{A, W, C, M, N, K, lda, ldw, ldc, k_per_slice, P, p_stride, ldp, bias, act, w_steps, w_pos, ex};
+  const int big = big_m * big_n, small = small_m * small_n, big_xcd = (big + 7) / 8, small_xcd = (small + 7) / 8;
+  int at = blockIdx.x >> 3;                  // (an XCD's blocks: its large tiles slice by slice, then its small ones)
+  const int xcd = blockIdx.x & 7;
+  if (at < big_xcd * slices) {
+    const int slice = at / big_xcd, tile = xcd * big_xcd + at - slice * big_xcd;
+    if (tile < big) mf_turns_tile<EPI, TC, WT, 2, 2>(lds, a, 0, big_m, big_n, min(big_m, 4), tile, slice);
+  } else {
+    at -= big_xcd * slices;
+    const int slice = at / small_xcd, tile = xcd * small_xcd + at - slice * small_xcd;
+    if (tile < small) mf_turns_tile<EPI, TC, WT, 1, SWH>(lds, a, big_m * 256, small_m, small_n, min(small_m, 8), tile, slice);
+  }
+}
+
 // What gemm_mfma_turns_kernel is built for: whole steps of 64 k, and byte offsets of 31 bits inside a tile's rows of A and
 // inside W (or, as stored, from the tile's first row of W to its last).
 static bool turns_takes(int N, int K, long lda, long ldw, bool gated, int w_order) {
   const long rows = gated ? 2L * N : (long)N;
   return K % 64 == 0 && (255 * lda + K) * 2 < (1L << 31) &&
          (w_order ? rows * K * 2 : ((gated ? (long)N : 0) + 255) * ldw * 2 + 2L * K) < (1L << 31);
+}
+
+template <int EPI, typename TC, int SWH, int WT>
+static int launch_two_tiles(const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc,
+                            int slices, float* P, long p_stride, long ldp, const float* bias, int act, int w_steps,
+                            const int* w_pos, MfExtras ex, int big_m, hipStream_t stream) {
+  const int big_cols = EPI == MF_GATED ? 128 : 256, small_cols = big_cols * SWH / 2;
+  const int big_n = (N + big_cols - 1) / big_cols, small_n = (N + small_cols - 1) / small_cols;
+  const int small_m = (M - big_m * 256 + 127) / 128;
+  const long blocks = (((long)big_m * big_n + 7) / 8 + ((long)small_m * small_n + 7) / 8) * 8 * slices;
+  GL3_REQUIRE(big_m > 0 && small_m > 0 && blocks < (1L << 31), "gl3_gemm_mfma: %d rows of tiles of 256 x 256 for %d rows", big_m, M);
+  const int k_per_slice = ((K + MF_BK - 1) / MF_BK + slices - 1) / slices * MF_BK;
+  gemm_mfma_two_tiles_kernel<EPI, TC, WT, SWH><<<dim3((unsigned)blocks), dim3(512), 0, stream>>>(
+      (const bf16_t*)A, (const bf16_t*)W, (TC*)C, M, N, K, lda, ldw, ldc, big_m, big_n, small_m, small_n, slices, k_per_slice, P, p_stride,
+      ldp, bias, act, w_steps, w_pos, ex);
+  GL3_LAUNCH_CHECK();
+  return 0;
 }
 
 template <int EPI, typename TC, int TM, int WM, int WN, int WT = 0>
@@ -812,19 +890,54 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
 // into the residual rows in mfma_plan's slices; profiles/tiled_products_tiles.txt): the tile chosen is the fastest of the three or within 5% at
 // all but one (1.07). With 0.42 and 4.0 for the first two, which suited epilogues through shared memory, 17 were beyond 5%, 1,024 rows of
 // 2,048 x 2,048 20.3 instead of 17.2 us. With rounds of 256 blocks, whatever their XCD, 300 rows of 3,072 x 8,192 took 47.3 instead of 40.8 us.
-static int choose_turns_shape(int M, int N, int K, int slices, bool gated) {
+//
+// Where tiles of 256 x 256 end in a round that is mostly empty, two tiles (gemm_mfma_two_tiles_kernel): 8 * rows of large tiles + the small
+// tile. An XCD's small tiles go one after the other to the CUs that are done with their large ones; of all divisions with less than a round
+// and a half behind the large tiles the one that ends first, where it saves 4% or more. Small tiles that follow large ones take 0.48 us a step and 4.5
+// beside them, or 0.60 and 3.0. Measured at 216 sizes (600 to 13,000 rows, the products of three models, up to six divisions of each): the
+// choice is within 4% of the best at all but six (1.11). At 97 other sizes where the rule takes two tiles (300 to 16,000 rows, four models'
+// products; profiles/two_tiles.txt) they take 0.78 to 1.02 times as long as the single tile taken before, 0.90 on average.
+static int choose_turns_shape(int M, int N, int K, int slices, bool gated, bool two) {
   static const int rows[3] = {128, 128, 256}, cols[3] = {128, 256, 256}, shape[3] = {1, 5, 2};
   static const double step_us[3] = {0.40, 0.60, 1.0}, round_us[3] = {0.9, 3.0, 4.5};
+  static const double after_step_us[2] = {0.48, 0.60}, after_us[2] = {4.5, 3.0};
   const int steps = (K / 64 + slices - 1) / slices;
+  auto per_xcd = [&](int n_rows, int i) {            // blocks of an XCD
+    const int columns = gated ? cols[i] / 2 : cols[i];
+    return ((long)((n_rows + rows[i] - 1) / rows[i]) * ((N + columns - 1) / columns) + 7) / 8 * slices;
+  };
   int best = 0;
   double least = 0;
   for (int i = 0; i < 3; ++i) {
-    const int columns = gated ? cols[i] / 2 : cols[i];
-    const long tiles = (long)((M + rows[i] - 1) / rows[i]) * ((N + columns - 1) / columns);
-    const double time = ((tiles + 7) / 8 * slices + 31) / 32 * (steps * step_us[i] + round_us[i]);
+    const double time = (per_xcd(M, i) + 31) / 32 * (steps * step_us[i] + round_us[i]);
     if (!best || time < least) {
       best = shape[i];
       least = time;
+    }
+  }
+  if (!two) return best;
+  least *= 0.96;
+  const double large = steps * step_us[2] + round_us[2];
+  const int most = (M - 1) / 256;
+  for (int r = most; r > 0 && (most - r) * per_xcd(256, 2) <= 48; --r) {
+    const long big = per_xcd(r * 256, 2);
+    const double early = big / 32 * large, late = early + (big % 32 ? large : 0);      // when an XCD's CUs are done with the large tiles
+    if (early >= least) continue;
+    for (int i = 0; i < 2; ++i) {
+      const long small = per_xcd(M - r * 256, i), late_cus = big % 32;
+      const double each = steps * after_step_us[i] + after_us[i];
+      // the first end of a small tile by which all of them are done
+      double end = 0;
+      for (int k = 1; end == 0 && early + k * each < least; ++k)
+        for (const double t : {early + k * each, late + (k - 1) * each}) {
+          if (t < early || (end != 0 && t >= end)) continue;
+          const long done = (32 - late_cus) * (long)((t - early) / each + 1e-6) + (t >= late ? late_cus * (long)((t - late) / each + 1e-6) : 0);
+          if (done >= small) end = t < late ? late : t;
+        }
+      if (end != 0 && end < least) {
+        best = 8 * r + shape[i];
+        least = end;
+      }
     }
   }
   return best;
@@ -862,9 +975,23 @@ static int launch_mfma(const void* A, const void* W, void* C, int M, int N, int 
                        const int* w_pos, MfExtras ex, hipStream_t stream) {
   const int w_steps = w_order == 1 ? (K + 31) / 32 : w_order == 2 ? (K + 63) / 64 : 0;
   if (shape < 0) shape = turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order) ? 0 : -shape;
+  constexpr bool TWO = EPI != MF_GATED || sizeof(TC) == 2;
   if (shape == 0)
-    shape = turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order) ? choose_turns_shape(M, N, K, slices, EPI == MF_GATED)
+    shape = turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order) ? choose_turns_shape(M, N, K, slices, EPI == MF_GATED, TWO)
                                                                   : choose_shape(M, N, slices, EPI == MF_GATED);
+  if (shape > 8) {
+    GL3_REQUIRE(TWO && turns_takes(N, K, lda, ldw, EPI == MF_GATED, w_order),
+                "gl3_gemm_mfma: two tiles are for whole steps of 64 k (K=%d), and for gated values of 16 bits", K);
+#define MF_ARGS A, W, C, M, N, K, lda, ldw, ldc, slices, P, p_stride, ldp, bias, act, w_steps, w_pos, ex, shape / 8, stream
+#define MF_TWO(WT) (shape % 8 == 1 ? launch_two_tiles<EPI, TC, 1, WT>(MF_ARGS) : launch_two_tiles<EPI, TC, 2, WT>(MF_ARGS))
+    if constexpr (TWO) {
+      if (w_order == 0) return MF_TWO(0);
+      if (w_order == 1) return MF_TWO(1);
+      if constexpr (EPI != MF_GATED) return MF_TWO(2);
+    }
+#undef MF_TWO
+#undef MF_ARGS
+  }
 #define MF_ARGS A, W, C, M, N, K, lda, ldw, ldc, slices, P, p_stride, ldp, bias, act, w_steps, w_pos, ex, stream
   if (w_order) {
     // W is one of its copies in the matrix cores' order (a weight that is held once): the three tiles that the library
@@ -923,7 +1050,8 @@ extern "C" int gl3_gemm_mfma(const void* A, const void* W, void* C, int c_dtype,
   GL3_REQUIRE(GL3_ACT_KNOWN(act), "gl3_gemm_mfma: unknown activation %d", act);
   GL3_REQUIRE(!col_scale || epilogue != MF_GATED, "gl3_gemm_mfma: a factor per column goes with the store and add epilogues");
   const MfExtras ex{col_scale, act_limit, act_shift};
-  GL3_REQUIRE(shape >= -5 && shape <= 5 && shape != -3 && shape != -4, "gl3_gemm_mfma: unknown tile shape %d", shape);
+  GL3_REQUIRE((shape >= -5 && shape <= 5 && shape != -3 && shape != -4) || (shape > 8 && (shape % 8 == 1 || shape % 8 == 5) && shape / 8 <= (M - 1) / 256),
+              "gl3_gemm_mfma: unknown tile shape %d", shape);
   // w_order: 0: W holds the rows as stored. 1: W is the copy in the matrix operands' order (lib.tile_weight), w_pos (may be
   // null) naming each row's place in it. 2: the copy in packed strips of 8 rows (lib.tile_weight8).
   {

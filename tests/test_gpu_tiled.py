@@ -114,6 +114,49 @@ def test_a_tile_and_its_kernel_have_no_say_in_the_sums(M, N, Kd, slices):
         assert torch.equal(got[-1], got[0]), shape
 
 
+# (one row, a part of a small tile and more than one of them behind the large ones; rows of output apart and not; K in slices of which the last has no step)
+@pytest.mark.parametrize("order", ["stored", "strips of 16", "strips of 8"])
+@pytest.mark.parametrize("shape, M, N, Kd", [(9, 257, 272, 192), (13, 300, 2304, 320), (9, 513, 128, 1088), (17, 770, 528, 320), (13, 1100, 528, 192)])
+def test_two_tiles_of_a_product_give_the_sums_of_one(order, shape, M, N, Kd):
+    """256 x 256 for the first 256 * (shape / 8) rows, shape % 8 behind them: bit for bit what tiles of 128 x 128 alone give."""
+    lib = K()
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    A = torch.randn(M, Kd + 8, generator=gen, device="cuda").to(torch.bfloat16)[:, :Kd]
+    w = torch.randn(2 * N, Kd, generator=gen, device="cuda").to(torch.bfloat16)
+    W, G = held(lib, w[:N], order), None if order == "strips of 8" else held(lib, w, order)
+    bias, factor, res = (torch.randn(n, generator=gen, device="cuda") for n in ((N,), (N,), (M, N)))
+
+    def both(dtype, weight, epilogue, pad=0, slices=1, **kw):
+        got = []
+        for tile in (1, shape):
+            x = torch.full((M, N + pad), -7.0, device=DEV, dtype=dtype)
+            x[:, :N] = res
+            part = torch.full((slices - 1, M, N), -7.0, device=DEV) if slices > 1 else None
+            lib.gemm_mfma(A, weight, x[:, :N], epilogue, more_slices=part, shape=tile, **kw)
+            assert torch.all(x[:, N:] == -7.0)
+            got.append(torch.cat([x[None, :, :N], part]) if slices > 1 else x)
+        assert torch.equal(*got), (dtype, epilogue, pad, slices)
+    for pad in (0, 3):
+        both(torch.float32, W, lib.EPI_STORE, pad, bias=bias)
+        both(torch.bfloat16, W, lib.EPI_STORE, pad, bias=bias, col_scale=factor)
+        both(torch.float32, W, lib.EPI_ADD, pad)
+        if G is not None:
+            both(torch.bfloat16, G, lib.EPI_GATED, pad)
+    for slices in (2, 3) + ((4,) if Kd == 320 else ()):
+        both(torch.float32, W, lib.EPI_ADD, slices=slices, col_scale=factor)
+
+
+def test_two_tiles_are_refused_where_they_do_not_fit():
+    """No rows behind the large tiles, a K of no whole steps, gated values of 32 bits: nothing is launched."""
+    lib = K()
+    a, w = torch.zeros(512, 200, device=DEV, dtype=torch.bfloat16), torch.zeros(256, 200, device=DEV, dtype=torch.bfloat16)
+    x = torch.zeros(512, 256, device=DEV)
+    for rows, k, shape, epilogue in ((256, 128, 9, lib.EPI_STORE), (512, 128, 17, lib.EPI_STORE), (512, 200, 9, lib.EPI_STORE), (512, 128, 9, lib.EPI_GATED),
+                                     (512, 128, 10, lib.EPI_STORE)):
+        with pytest.raises(lib.KernelError, match="tile"):
+            lib.gemm_mfma(a[:rows, :k], w[:, :k].contiguous(), x[:rows, :128 if epilogue == lib.EPI_GATED else 256], epilogue, shape=shape)
+
+
 @pytest.mark.parametrize("shape", [-6, -4, -3, 6])
 def test_unknown_tiles_are_refused(shape):
     """A plan names one of the library's own tiles (1, 2, 5); nothing is launched for another."""
