@@ -921,6 +921,233 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
     }
 }
 
+// Every earlier key, heads of 64, pages of whole chunks of 64 keys: eight waves a block, two blocks a CU.
+//
+// The kernel of 128 queries above carries keys and values through registers into shared memory and has 157 of them a thread, so that two waves
+// share a SIMD. Here chunks go from memory straight into shared memory, as they lie in the cache (the operands' order, as in the kernel of
+// turns); with 115 registers four waves share a SIMD, and while some have its matrix cores others work out their softmax. (A SIMD has one
+// vector instruction of a wave about every eight cycles, measured; of four waves one every 4.2, an exponential 8.2, an addition 2.4.)
+// GROUPS = 2, for few blocks: 128 queries of one head, four waves of 32 on the even chunks of keys and four on the odd ones, whose sums are
+// brought together at the end: a block's way along the keys is half as long. GROUPS = 1: 128 queries of two heads of one kv head, which
+// share the chunks: the same sums in the same order as the kernel of 128 queries, bit for bit. Two groups' error against 64 bits is 0.993 times
+// that on average, 1.0001 at most (54 sizes of 37 to 3,001 tokens, contexts to 3,000, scores spread 0.3 to 3): their maxima are nearer to the weights.
+// What bounds it: one sequence of 16,384 tokens the power (vector and matrix units together; the clock falls below 1.9 GHz), a prompt of
+// 2,048 the unequal ways of its blocks. 32 heads over 8, one sequence, the kernel of 128 queries and this one: 1,024 tokens 22.2 -> 15.6 us,
+// 2,048 41.6 -> 29.5, 4,096 97.9 -> 89.1, 8,192 346 -> 308, 16,384 1,313 -> 1,177; 317 + 1,203 + 701 tokens 27.5 -> 19.8, 64 of 83 29.4 -> 19.3.
+// Two waves a SIMD with the softmax woven between the matrix instructions (241 registers) took 31.0 us for 2,048 tokens and 1,238 for 16,384, the same
+// with 32 queries of two heads a wave 37.7 and 1,223.
+//
+// A round is a chunk a group; a wave brings a share of its group's chunk (of all, GROUPS = 1). STAGES chunks lie in shared memory in turn: behind
+// the barrier of a round the place that was read in the round before is written for the round STAGES - 1 further on, and the wait in
+// front of it leaves out the requests for later rounds than its own. Chunks beyond the last repeat it, so that the counts hold; nothing is in
+// flight when the sums go through shared memory, or when a block ends.
+// SPLIT: as in the kernel of 128 queries.
+template <int GROUPS, bool SPLIT>
+__global__ __launch_bounds__(512, 4) void attention_prefill_eight_kernel(
+    const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
+    const int* __restrict__ cu_seqlens, const int* __restrict__ kv_before, const int* __restrict__ block_table,
+    const int* __restrict__ seq_rows, int table_stride, bf16_t* __restrict__ out, long out_stride, int n_heads, int n_kv, int page_size,
+    float scale, int q_blocks, int folded, PfSplit sp) {
+  static_assert(!SPLIT || GROUPS == 2, "splits are for few blocks");
+  constexpr int HS = 64, CK = 64, KS = HS / 16, DT = HS / 32, QB = 128, HEADS = GROUPS == 2 ? 1 : 2;
+  constexpr int KB = CK * HS * 2;                  // bytes of a chunk's keys (and of its values)
+  constexpr int STAGE = 2 * KB, STAGES = 4 / GROUPS;
+  constexpr int PW = GROUPS;                       // pieces of 1 KB of either that a wave brings
+  __shared__ __attribute__((aligned(1024))) char lds[GROUPS * STAGES * STAGE];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, group = wave >> 2;
+  // (as in the kernel of 128 queries the longest blocks first; where all blocks are on the chip at once the shortest second, beside them)
+  const int half = q_blocks / 2, z = blockIdx.z;
+  const int qb = folded && z >= q_blocks - half ? z - (q_blocks - half) : q_blocks - 1 - z;
+  const int b = blockIdx.y, g = n_heads / n_kv;
+  const int split = SPLIT ? blockIdx.x / n_heads : 0, at = blockIdx.x - split * n_heads;
+  const int c = at % n_kv;                         // (blocks of one kv head are n_kv apart: on one XCD where n_kv is 8)
+  const int head = c * g + at / n_kv * HEADS + (HEADS == 2 ? group : 0);
+  const int n = lane & 31, h = lane >> 5;
+  const int tok0 = __builtin_amdgcn_readfirstlane(cu_seqlens[b]);
+  const int q_len = __builtin_amdgcn_readfirstlane(cu_seqlens[b + 1]) - tok0;
+  if (qb * QB >= q_len) return;                    // the whole block: no barrier has been passed yet
+  const int before = __builtin_amdgcn_readfirstlane(kv_before[b]);
+  const int* bt = block_table + (long)(seq_rows ? __builtin_amdgcn_readfirstlane(seq_rows[b]) : b) * table_stride;
+  int ck0 = 0, ck1 = (before + min(qb * QB + QB - 1, q_len - 1)) / CK;
+  if (SPLIT) {                                     // (no chunk: the block leaves a weight of nothing)
+    const int chunks = ck1 + 1;
+    ck0 = chunks * split / sp.splits;
+    ck1 = chunks * (split + 1) / sp.splits - 1;
+  }
+  const int rounds = (ck1 - ck0 + GROUPS) / GROUPS;
+  const int qi0 = qb * QB + (wave & 3) * 32;
+  const bool q_ok = qi0 + n < q_len;
+  const int p_mine = before + qi0 + n, p_first = before + qi0;
+  const int my_last = qi0 < q_len ? (before + min(qi0 + 31, q_len - 1)) / CK : -1;      // the last chunk with a key that one of the wave's queries sees
+
+  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  bf16x8 qt[KS];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk)
+    qt[kk] = q_ok ? *(const bf16x8*)(q + (long)(tok0 + qi0 + n) * q_stride + (long)head * HS + kk * 16 + 8 * h) : zero8;
+  float m_run = -INFINITY, l_run = 0.f;
+  f32x16 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[dt][v] = 0.f;
+
+  // where the group's chunks lie, sixty-four of them in a register (a lane one): keys in units of a chunk, values of 1,024 elements
+  const int per_page = page_size / CK, v_units = per_page * (HS / 16);
+  const int first_ck = ck0 + (GROUPS == 2 ? group : 0);
+  auto places = [&](int first, int& k_at, int& v_at) {
+    const int ck = max(0, min((first + lane) * GROUPS + first_ck, ck1)), entry = ck / per_page, in_page = ck - entry * per_page;
+    const int row = bt[entry] * n_kv + c;
+    k_at = row * per_page + in_page;
+    v_at = row * v_units + in_page;
+  };
+  int k_at, v_at;
+  places(0, k_at, v_at);
+  const int piece0 = (GROUPS == 2 ? wave & 3 : wave) * PW;
+  const int base = GROUPS == 2 ? group * STAGES * STAGE : 0;
+  const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)lds + base + piece0 * 1024;
+  unsigned v_off[PW];
+#pragma unroll
+  for (int i = 0; i < PW; ++i) v_off[i] = ((piece0 + i) >> 1) * (page_size * 32) + ((piece0 + i) & 1) * 1024 + lane * 16;
+  auto ask = [&](int x) {                          // the group's x-th chunk, one after the other; beyond the last the last again
+    if (x && (x & 63) == 0) places(x, k_at, v_at);
+    const i32x4 k_buf = mf_rsrc(k_cache + (long)__builtin_amdgcn_readlane(k_at, x & 63) * (CK * HS));
+    const i32x4 v_buf = mf_rsrc(v_cache + (long)__builtin_amdgcn_readlane(v_at, x & 63) * 1024);
+    const unsigned to = lds0 + (x % STAGES) * STAGE;
+#pragma unroll
+    for (int i = 0; i < PW; ++i) mf_dma16(to + i * 1024, (piece0 + i) * 1024 + lane * 16, k_buf, 0);
+#pragma unroll
+    for (int i = 0; i < PW; ++i) mf_dma16(to + KB + i * 1024, v_off[i], v_buf, 0);
+  };
+
+  const float c2 = scale * 1.4426950408889634f;    // scores in units of log2
+  const char* k_lds = lds + base + (n >> 4) * (32 * HS) + h * 256 + (n & 15) * 16;
+  const char* v_lds = lds + base + KB + (n >> 4) * 2048 + h * 256 + (n & 15) * 16;
+  auto max3 = [](float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); };
+  // (register of the lane's e-th key of a tile, in the order of the keys: score tiles as in the kernel of turns)
+  auto reg = [](int e) { return (e & 3) + ((e >> 2) & 1) * 8 + (e >> 3) * 4; };
+  auto chunk = [&](int at, int key0, bool masked) {
+    f32x16 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) s[t][v] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(k_lds + at + t * (64 * HS) + kk * 512), qt[kk], s[t], 0, 0, 0);
+    if (masked) {                                  // (the same for the whole wave: a branch around the tests, one body)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[t][reg(e)] = key0 + 32 * t + 16 * (e >> 3) + 8 * h + (e & 7) <= p_mine ? s[t][reg(e)] : -INFINITY;
+    }
+    float top[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      top[t] = s[t][0];
+#pragma unroll
+      for (int e = 1; e < 15; e += 2) top[t] = max3(top[t], s[t][e], s[t][e + 1]);
+    }
+    float mx = max3(max3(top[0], top[1], s[0][15]), s[1][15], s[1][15]);
+    {   // the other half of the keys of this query sits 32 lanes away
+      auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    mx *= c2;                                      // c2 > 0: the greatest score stays the greatest
+    const float m_new = fmaxf(m_run, mx);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    float ps = 0.f;
+    bf16x8 pb[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[t][reg(e)], c2, -m_use));
+        ps += p;
+        pb[t][e >> 3][e & 7] = static_cast<bf16_t>(p);
+      }
+    l_run = l_run * alpha + ps;
+    m_run = m_new;
+    if (!__all(alpha == 1.0f)) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(v_lds + at + dt * 4096 + j * 512), pb[j >> 1][j & 1], o[dt], 0, 0, 0);
+  };
+
+#pragma unroll
+  for (int x = 0; x < STAGES - 1; ++x) ask(x);
+  for (int x = 0; x < rounds; ++x) {
+    mf_wait_loads<(STAGES - 2) * 2 * PW>();        // this wave's share of chunk x has come, behind the barrier everybody's
+    mf_barrier();
+    ask(x + STAGES - 1);                           // (into the place that was read last before the barrier)
+    const int ck = x * GROUPS + first_ck;
+    if (ck <= (SPLIT ? min(my_last, ck1) : my_last)) chunk((x % STAGES) * STAGE, ck * CK, ck * CK + CK - 1 > p_first);
+  }
+  mf_wait_loads<0>();
+
+  float l = l_run;
+  l += __shfl_xor(l, 32, 64);
+  if constexpr (GROUPS == 2) {
+    // the second group's sums go through shared memory to the first's waves, which bring both to the greater maximum
+    mf_barrier();
+    float* const theirs = (float*)lds + (wave & 3) * (34 * 64) + lane;
+    if (group == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) theirs[(dt * 16 + v) * 64] = o[dt][v];
+      theirs[32 * 64] = m_run;
+      theirs[33 * 64] = l;
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = theirs[32 * 64], l1 = theirs[33 * 64];
+    if (!(m1 == -INFINITY && l1 == 0.f)) {         // (a query that sees none of their keys; scores that are all NaN have a weight)
+      const float m = fmaxf(m_run, m1), f0 = __builtin_amdgcn_exp2f(m_run - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
+      l = l * f0 + l1 * f1;
+      m_run = m;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[dt][v] = o[dt][v] * f0 + theirs[(dt * 16 + v) * 64] * f1;
+    }
+  }
+  if (!q_ok) return;
+  if (SPLIT) {
+    const long row = ((long)split * sp.n_tokens + tok0 + qi0 + n) * n_heads + head;
+    float* po = sp.o + row * HS + 4 * h;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) *(f32x4*)(po + dt * 32 + 8 * a) = f32x4{o[dt][4 * a], o[dt][4 * a + 1], o[dt][4 * a + 2], o[dt][4 * a + 3]};
+    if (h == 0) {
+      sp.ml[row * 2] = m_run;
+      sp.ml[row * 2 + 1] = l;
+    }
+    return;
+  }
+  const float inv = 1.0f / l;
+  bf16_t* op = out + (long)(tok0 + qi0 + n) * out_stride + (long)head * HS + 4 * h;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      bf16x4 r;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) r[v] = static_cast<bf16_t>(o[dt][4 * a + v] * inv);
+      *(bf16x4*)(op + dt * 32 + 8 * a) = r;
+    }
+}
+
 // The splits' sums of a row (token, head) brought to the greatest of their maxima, added in the order of the splits, and divided
 // by the weight: a thread four dims of a row, its splits' loads all on their way at once.
 template <int HS>
@@ -983,11 +1210,25 @@ static bool turns_wanted(int n_seqs, int max_q_len, int n_tokens) {
   return max_q_len >= 1024 && (n_tokens <= 5L * max_q_len || n_tokens >= 1280L * n_seqs);
 }
 
-// The library's choice: 0: 64 queries a block, 1: 128, 2: the kernel of turns. plain: the plain rule (one score map, no window, chunked
+// The kernel of eight waves: two groups on the keys where its blocks of one head are at most 1,100 (two are on each CU at a time), else two heads a
+// block (32 heads: one sequence of 4,096 tokens, 1,040 blocks, 89.1 and 92.7 us, of 6,000 180 and 182; eight of 512, 1,152 blocks, 23.1 and 21.3, 32 of 256
+// 34.6 and 29.5). An odd number of heads a kv head has no pairs: two groups there too, but for many short sequences, where the kernel
+// of 128 queries is as fast or faster (24 heads over 8: sixteen of 146 to 336 tokens 14.7 against 13.4 us).
+#define PF_KEYS (INT_MIN + 1)
+#define PF_HEADS (INT_MIN + 2)
+static bool eight_takes(int head_dim, int page_size) { return head_dim == 64 && page_size % 64 == 0; }
+static int eight_choice(int n_heads, int group, int n_seqs, int n_tokens) {
+  const long blocks = (long)n_heads * (n_tokens / 128 + (n_seqs + 1) / 2);
+  if (group % 2 == 0) return blocks <= 1100 ? 3 : 4;
+  return blocks <= 512 || n_tokens >= 256L * n_seqs ? 3 : 1;
+}
+
+// The library's choice: 0: 64 queries a block, 1: 128, 2: the kernel of turns, 3: eight waves in two groups on the keys, 4: on two heads. plain: the plain rule (one score map, no window, chunked
 // mask, bias, sink, kept keys, cap, temperature or gate), no splits, caches at 16-byte addresses (its loads into shared memory bring
 // 16 bytes a lane and want them aligned, where the other kernels' ordinary loads do not).
 extern "C" int gl3_prefill_kernel(int head_dim, int page_size, int n_heads, int n_kv, int n_seqs, int max_q_len, int n_tokens, int plain) {
   if (!prefill_wide(head_dim, n_heads, n_seqs, max_q_len)) return 0;
+  if (plain && eight_takes(head_dim, page_size)) return eight_choice(n_heads, n_heads / n_kv, n_seqs, n_tokens);
   return plain && turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && turns_wanted(n_seqs, max_q_len, n_tokens) ? 2 : 1;
 }
 
@@ -998,7 +1239,7 @@ extern "C" int gl3_attention_prefill_supports(int head_dim, int page_size) {
 // max_q_len: the most tokens any sequence brings in this step (it sizes the grid).
 // seq_rows (may be null): the row of `block_table` that holds sequence b's pages; null: row b.
 // wide_from: the kernel with 128 queries a block is taken when max_q_len reaches it; <= 0: the library's choice, but for PF_TURNS: the
-// kernel of turns.
+// kernel of turns, and PF_KEYS, PF_HEADS: the kernel of eight waves in two groups on the keys, or on two heads.
 extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k_cache, const void* v_cache,
                                      const int* cu_seqlens, const int* kv_before, const int* block_table,
                                      const int* seq_rows, int table_stride, void* out, long out_stride, int n_seqs,
@@ -1026,10 +1267,14 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
   GL3_CHECK_RULE(rule, "gl3_attention_prefill");
   const bool ruled = rule.any();
   const bool biased = slopes != nullptr || has_sink || sinks != nullptr || keep_first > 0;    // (the kernels that know of kept first keys)
-  const bool plain = splits == 1 && !ruled && !biased && maps == 1 && window == 0 && mask_chunk == 0 && (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0;
+  const bool splits_plain = !ruled && !biased && maps == 1 && window == 0 && mask_chunk == 0 && (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0;
+  const bool plain = splits == 1 && splits_plain;
+  const bool eight = plain && eight_takes(head_dim, page_size);
+  GL3_REQUIRE((wide_from != PF_KEYS && wide_from != PF_HEADS) || (eight && (wide_from == PF_KEYS || g % 2 == 0)),
+              "gl3_attention_prefill: the kernels of eight waves take heads of 64, pages of whole 64 keys, caches at 16-byte addresses, no splits, the plain rule, and two heads a block an even number of heads a kv head");
   GL3_REQUIRE(wide_from != PF_TURNS || (plain && turns_takes(head_dim, page_size, g, n_seqs, n_tokens)),
               "gl3_attention_prefill: the kernel of turns takes heads of 128, pages of whole 64 keys, caches at 16-byte addresses, at most 64 sequences, no splits, the plain rule");
-  const int kernel = wide_from == PF_TURNS ? 2 : splits > 1 ? 1 : wide_from > 0 ? max_q_len >= wide_from
+  const int kernel = wide_from == PF_TURNS ? 2 : wide_from == PF_KEYS ? 3 : wide_from == PF_HEADS ? 4 : splits > 1 ? 1 : wide_from > 0 ? max_q_len >= wide_from
                      : gl3_prefill_kernel(head_dim, page_size, n_heads, n_kv, n_seqs, max_q_len, n_tokens, plain);
   const bool wide = kernel > 0;
   // query heads per wave: as many as the registers hold with two blocks on a CU; one with 32 queries a wave
@@ -1055,6 +1300,24 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
     if (heads == 2) GOT(2);
     else GOT(1);
 #undef GOT
+    GL3_LAUNCH_CHECK();
+    return 0;
+  }
+  if (kernel >= 3 || (kernel == 1 && splits > 1 && splits_plain && eight_takes(head_dim, page_size))) {
+    const int heads = kernel == 4 ? 2 : 1;
+    const bool folded = n_seqs == 1 && (long)n_heads / heads * q_blocks * splits <= 512;
+    dim3 egrid((unsigned)(n_heads / heads * splits), n_seqs, q_blocks);
+#define GOE(GROUPS, SPLIT)                                                                                            \
+  attention_prefill_eight_kernel<GROUPS, SPLIT><<<egrid, dim3(512), 0, stream>>>(                                            \
+      (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu_seqlens, kv_before, block_table, \
+      seq_rows, table_stride, (bf16_t*)out, out_stride, n_heads, n_kv, page_size, scale, q_blocks, (int)folded, sp)
+    if (splits > 1) {
+      GOE(2, true);
+      const long rows = (long)n_tokens * n_heads * (64 / 4);
+      attention_prefill_merge_kernel<64><<<dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream>>>(sp, (bf16_t*)out, out_stride, n_heads);
+    } else if (kernel == 3) GOE(2, false);
+    else GOE(1, false);
+#undef GOE
     GL3_LAUNCH_CHECK();
     return 0;
   }

@@ -2063,7 +2063,7 @@ PREFILL_SPLIT_KEYS = 1024            # keys that the longest sequence of a step 
 PREFILL_SPLIT_ROWS = 1024 * 128      # (token, head, split) rows that a step's splits never exceed
 
 
-def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len):
+def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=False):
     """Blocks of 128 queries that share their keys out (``attention_prefill``'s ``splits``): for steps that bring few tokens behind
     a long context (a prompt in portions, the next turn of a dialogue), whose blocks are fewer than two for every CU and walk
     the context one chunk after another. Only where every sequence held at least as many tokens as the longest one
@@ -2072,14 +2072,23 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len):
     24 heads of 128 692 -> 391. Prompts without a context lose: 1,024 tokens, 24 heads of 128 31 -> 36 us (their blocks' keys are
     few, and the merge costs 5 to 10 us). A split's sums are 32-bit as the unsplit kernel's and shorter; only the maximum around which
     weights are rounded is another: the error against 64 bits is 0.967 times that without splits on average, smaller at all of 90
-    sizes (contexts of 700 to 12,000, 37 to 1,100 tokens, heads of 32 to 128)."""
+    sizes (contexts of 700 to 12,000, 37 to 1,100 tokens, heads of 32 to 128).
+    ``eight`` (heads of 64 in pages of whole 64 positions: the kernel of eight waves): one of its blocks keeps a CU's units busy, 1.2 us for 128
+    keys, and two on a CU take twice as long, so the splits are those whose rounds of 256 blocks are done first, a merge being 6 us and a
+    split's sums 2.8 TB/s of it. 32 heads, 300 tokens behind 3,000 31.2 us in the six splits of the rule above and 27.1 in two; 512 behind 1,024
+    24.3 in four, 19.9 without; 700 behind 12,000 119 in three, 100 in four; 1,000 behind 1,000 32.9 in two, 25.3 without."""
     blocks = n_heads * n_seqs * -(-max_q_len // 128)
     if blocks >= 512 or max_kv_len < PREFILL_SPLIT_KEYS or not kv_before or min(kv_before) < max_q_len:
         return 1
+    if eight:
+        rows = n_heads * n_seqs * max_q_len
+        return min((s for s in range(1, 9) if s == 1 or (s * 256 <= max_kv_len and s * blocks <= 1024)),
+                   key=lambda s: -(-blocks * s // 256) / s * max_kv_len / 128 * 1.2 + (s > 1) * (6 + s * rows * 256 / 2.8e6))
     return max(1, min(8, -(-512 // blocks), max_kv_len // 256))
 
 
 PREFILL_TURNS = -2 ** 31              # ``attention_prefill``'s ``wide_from`` that names the kernel of turns
+PREFILL_KEYS, PREFILL_HEADS = PREFILL_TURNS + 1, PREFILL_TURNS + 2      # and the kernel of eight waves, in two groups on the keys or on two heads
 
 
 def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, out, max_q_len, n_heads, n_kv,
@@ -2091,7 +2100,8 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
     names each sequence's row of ``block_table``; without it sequence b reads row b. ``wide_from``: from
     how many tokens of the step's longest sequence on the kernel with 128 queries a block runs
     (0 and below: the library's choice; ``PREFILL_TURNS``: the kernel of turns, which takes heads of 128 and the plain rule, gives the same bits
-    and has no splits; tests run all kernels on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
+    and has no splits; ``PREFILL_KEYS``, ``PREFILL_HEADS``: the kernel of eight waves, which takes heads of 64 and the plain rule; tests run all
+    kernels on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
     128 queries are shared out over that many blocks of the same kernel, whose sums lie in ``part_o`` (float32, at least
     splits * T * H * hs) and ``part_ml`` (2 * splits * T * H) until a second kernel merges them; the plain rule only."""
     _dev(q, "q", torch.bfloat16, contiguous=False); _dev(out, "out", torch.bfloat16, contiguous=False)

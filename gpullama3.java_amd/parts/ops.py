@@ -556,7 +556,8 @@ def attention(ctx, q, k_cache, v_cache, block_table, out, n_heads, n_kv, head_di
     if kernel == "prefill":
         if (ctx.max_kv_len >= K.PREFILL_SPLIT_KEYS and not window and not chunk and slopes is None and sink is None
                 and n_v_heads is None and rule is None):
-            splits = K.prefill_splits(n_heads, ctx.n_seqs, ctx.max_q_len, getattr(ctx, "kv_before_host", None), ctx.max_kv_len)
+            splits = K.prefill_splits(n_heads, ctx.n_seqs, ctx.max_q_len, getattr(ctx, "kv_before_host", None), ctx.max_kv_len,
+                                      eight=head_dim == 64 and page % 64 == 0)
             if splits > 1:
                 # (of one size, whatever the step brings: a buffer that grew would take the captured decode steps with it. On a
                 # device without room for them the step runs without splits: it never needed this memory before. The small one
