@@ -921,20 +921,24 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
     }
 }
 
-// Every earlier key, heads of 64, pages of whole chunks of 64 keys: eight waves a block, two blocks a CU.
+// Every earlier key, heads of 64 or 128, pages of whole chunks of 64 keys: eight waves a block.
 //
-// The kernel of 128 queries above carries keys and values through registers into shared memory and has 157 of them a thread, so that two waves
-// share a SIMD. Here chunks go from memory straight into shared memory, as they lie in the cache (the operands' order, as in the kernel of
-// turns); with 115 registers four waves share a SIMD, and while some have its matrix cores others work out their softmax. (A SIMD has one
-// vector instruction of a wave about every eight cycles, measured; of four waves one every 4.2, an exponential 8.2, an addition 2.4.)
+// The kernel of 128 queries above carries keys and values through registers into shared memory, and a block walks its keys alone. Here chunks go
+// from memory straight into shared memory, as they lie in the cache (the operands' order, as in the kernel of turns).
 // GROUPS = 2, for few blocks: 128 queries of one head, four waves of 32 on the even chunks of keys and four on the odd ones, whose sums are
 // brought together at the end: a block's way along the keys is half as long. GROUPS = 1: 128 queries of two heads of one kv head, which
 // share the chunks: the same sums in the same order as the kernel of 128 queries, bit for bit. Two groups' error against 64 bits is 0.993 times
-// that on average, 1.0001 at most (54 sizes of 37 to 3,001 tokens, contexts to 3,000, scores spread 0.3 to 3): their maxima are nearer to the weights.
+// that on average, 1.0002 at most (54 sizes of 37 to 3,001 tokens, contexts to 3,000, scores spread 0.3 to 3; heads of 64, and of 128): their maxima are
+// nearer to the weights. (With one maximum for 64 keys heads of 128 took 8 to 15% less time, at up to 1.004 times the error.)
+// Heads of 64: 115 registers where the kernel of 128 queries has 157, so that four waves share a SIMD and while some have its matrix cores others
+// work out their softmax (a SIMD has one vector instruction of a wave about every eight cycles, of four waves one every 4.2, an
+// exponential 8.2, an addition 2.4); two blocks a CU. Heads of 128: 164, two waves a SIMD and a block a CU.
 // What bounds it: one sequence of 16,384 tokens the power (vector and matrix units together; the clock falls below 1.9 GHz), a prompt of
-// 2,048 the unequal ways of its blocks. 32 heads over 8, one sequence, the kernel of 128 queries and this one: 1,024 tokens 22.2 -> 15.6 us,
-// 2,048 41.6 -> 29.5, 4,096 97.9 -> 89.1, 8,192 346 -> 308, 16,384 1,313 -> 1,177; 317 + 1,203 + 701 tokens 27.5 -> 19.8, 64 of 83 29.4 -> 19.3.
-// Two waves a SIMD with the softmax woven between the matrix instructions (241 registers) took 31.0 us for 2,048 tokens and 1,238 for 16,384, the same
+// 2,048 the unequal ways of its blocks, few blocks a wave's chain of scores, softmax and values. Time of the kernel taken before and of this one:
+//   32 heads of 64 over 8, one sequence: 1,024 tokens 22.2 -> 15.6 us, 2,048 41.6 -> 29.5, 4,096 97.9 -> 89.1, 8,192 346 -> 308, 16,384 1,313 -> 1,177;
+//     317 + 1,203 + 701 tokens 27.5 -> 19.8, 64 of 83 29.4 -> 19.3
+//   24 heads of 128 over 8: 512 tokens 17.5 -> 16.1, 1,024 31.1 -> 24.6, 2,048 62.0 -> 52.0; 512 behind 512 29.2 -> 24.3, 512 behind 4,096, unsplit, 112 -> 80
+// Heads of 64 with two waves a SIMD and the softmax woven between the matrix instructions (241 registers) took 31.0 us for 2,048 tokens and 1,238 for 16,384, the same
 // with 32 queries of two heads a wave 37.7 and 1,223.
 //
 // A round is a chunk a group; a wave brings a share of its group's chunk (of all, GROUPS = 1). STAGES chunks lie in shared memory in turn: behind
@@ -942,17 +946,17 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
 // front of it leaves out the requests for later rounds than its own. Chunks beyond the last repeat it, so that the counts hold; nothing is in
 // flight when the sums go through shared memory, or when a block ends.
 // SPLIT: as in the kernel of 128 queries.
-template <int GROUPS, bool SPLIT>
-__global__ __launch_bounds__(512, 4) void attention_prefill_eight_kernel(
+template <int HS, int GROUPS, bool SPLIT>
+__global__ __launch_bounds__(512, HS == 64 ? 4 : 2) void attention_prefill_eight_kernel(
     const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ cu_seqlens, const int* __restrict__ kv_before, const int* __restrict__ block_table,
     const int* __restrict__ seq_rows, int table_stride, bf16_t* __restrict__ out, long out_stride, int n_heads, int n_kv, int page_size,
     float scale, int q_blocks, int folded, PfSplit sp) {
   static_assert(!SPLIT || GROUPS == 2, "splits are for few blocks");
-  constexpr int HS = 64, CK = 64, KS = HS / 16, DT = HS / 32, QB = 128, HEADS = GROUPS == 2 ? 1 : 2;
+  constexpr int CK = 64, KS = HS / 16, DT = HS / 32, QB = 128, HEADS = GROUPS == 2 ? 1 : 2;
   constexpr int KB = CK * HS * 2;                  // bytes of a chunk's keys (and of its values)
   constexpr int STAGE = 2 * KB, STAGES = 4 / GROUPS;
-  constexpr int PW = GROUPS;                       // pieces of 1 KB of either that a wave brings
+  constexpr int PW = KB / 8192 * GROUPS;           // pieces of 1 KB of either that a wave brings
   __shared__ __attribute__((aligned(1024))) char lds[GROUPS * STAGES * STAGE];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, group = wave >> 2;
@@ -978,8 +982,8 @@ __global__ __launch_bounds__(512, 4) void attention_prefill_eight_kernel(
   const int rounds = (ck1 - ck0 + GROUPS) / GROUPS;
   const int qi0 = qb * QB + (wave & 3) * 32;
   const bool q_ok = qi0 + n < q_len;
-  const int p_mine = before + qi0 + n, p_first = before + qi0;
-  const int my_last = qi0 < q_len ? (before + min(qi0 + 31, q_len - 1)) / CK : -1;      // the last chunk with a key that one of the wave's queries sees
+  const int p_mine = before + qi0 + n, p_first = before + qi0, p_last = before + min(qi0 + 31, q_len - 1);
+  const int my_last = qi0 < q_len ? p_last / CK : -1;      // the last chunk with a key that one of the wave's queries sees
 
   const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
   bf16x8 qt[KS];
@@ -1027,31 +1031,36 @@ __global__ __launch_bounds__(512, 4) void attention_prefill_eight_kernel(
   auto max3 = [](float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); };
   // (register of the lane's e-th key of a tile, in the order of the keys: score tiles as in the kernel of turns)
   auto reg = [](int e) { return (e & 3) + ((e >> 2) & 1) * 8 + (e >> 3) * 4; };
-  auto chunk = [&](int at, int key0, bool masked) {
-    f32x16 s[2];
+  // The keys of a chunk around whose maximum weights are rounded together: those of a chunk of the kernel of 128 queries.
+  constexpr int SUB = HS == 64 ? 64 : 32, NT = SUB / 32;
+  auto part = [&](int at, int first, int key0, bool masked) {      // (`first`: the part's first tile of 32 keys)
+    f32x16 s[NT];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int v = 0; v < 16; ++v) s[t][v] = 0.f;
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
-        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(k_lds + at + t * (64 * HS) + kk * 512), qt[kk], s[t], 0, 0, 0);
+      for (int t = 0; t < NT; ++t)
+        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(k_lds + at + (first + t) * (64 * HS) + kk * 512), qt[kk], s[t], 0, 0, 0);
     if (masked) {                                  // (the same for the whole wave: a branch around the tests, one body)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) s[t][reg(e)] = key0 + 32 * t + 16 * (e >> 3) + 8 * h + (e & 7) <= p_mine ? s[t][reg(e)] : -INFINITY;
     }
-    float top[2];
+    // (v_maximum3, which keeps NaNs: fmaxf of a matrix instruction's results costs one more for each pair to quieten them. A row with a NaN
+    // is NaN by its weights either way)
+    float top[2 * NT];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      top[t] = s[t][0];
-#pragma unroll
-      for (int e = 1; e < 15; e += 2) top[t] = max3(top[t], s[t][e], s[t][e + 1]);
+    for (int k = 0; k < 2 * NT; ++k) {
+      const f32x16& v = s[k >> 1];
+      const int r = (k & 1) * 8;
+      top[k] = max3(max3(max3(v[r], v[r + 1], v[r + 2]), v[r + 3], v[r + 4]), v[r + 5], v[r + 6]);
     }
-    float mx = max3(max3(top[0], top[1], s[0][15]), s[1][15], s[1][15]);
+    float mx = max3(max3(top[0], top[1], s[0][7]), s[0][15], s[0][15]);
+    if constexpr (NT == 2) mx = max3(mx, max3(top[2], top[3], s[1][7]), s[1][15]);
     {   // the other half of the keys of this query sits 32 lanes away
       auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
       mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
@@ -1061,9 +1070,9 @@ __global__ __launch_bounds__(512, 4) void attention_prefill_eight_kernel(
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
     float ps = 0.f;
-    bf16x8 pb[2][2];
+    bf16x8 pb[NT][2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const float p = __builtin_amdgcn_exp2f(fmaf(s[t][reg(e)], c2, -m_use));
@@ -1077,10 +1086,14 @@ __global__ __launch_bounds__(512, 4) void attention_prefill_eight_kernel(
       for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 2 * NT; ++j)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(v_lds + at + dt * 4096 + j * 512), pb[j >> 1][j & 1], o[dt], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(v_lds + at + dt * 4096 + (2 * first + j) * 512), pb[j >> 1][j & 1], o[dt], 0, 0, 0);
+  };
+  auto chunk = [&](int at, int key0) {
+    part(at, 0, key0, key0 + SUB - 1 > p_first);
+    if (SUB < CK && key0 + SUB <= p_last) part(at, 1, key0 + SUB, key0 + CK - 1 > p_first);      // (a half that none of the wave's queries sees is left out)
   };
 
 #pragma unroll
@@ -1090,7 +1103,7 @@ __global__ __launch_bounds__(512, 4) void attention_prefill_eight_kernel(
     mf_barrier();
     ask(x + STAGES - 1);                           // (into the place that was read last before the barrier)
     const int ck = x * GROUPS + first_ck;
-    if (ck <= (SPLIT ? min(my_last, ck1) : my_last)) chunk((x % STAGES) * STAGE, ck * CK, ck * CK + CK - 1 > p_first);
+    if (ck <= (SPLIT ? min(my_last, ck1) : my_last)) chunk((x % STAGES) * STAGE, ck * CK);
   }
   mf_wait_loads<0>();
 
@@ -1099,18 +1112,18 @@ __global__ __launch_bounds__(512, 4) void attention_prefill_eight_kernel(
   if constexpr (GROUPS == 2) {
     // the second group's sums go through shared memory to the first's waves, which bring both to the greater maximum
     mf_barrier();
-    float* const theirs = (float*)lds + (wave & 3) * (34 * 64) + lane;
+    float* const theirs = (float*)lds + (wave & 3) * ((DT * 16 + 2) * 64) + lane;
     if (group == 1) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) theirs[(dt * 16 + v) * 64] = o[dt][v];
-      theirs[32 * 64] = m_run;
-      theirs[33 * 64] = l;
+      theirs[DT * 16 * 64] = m_run;
+      theirs[(DT * 16 + 1) * 64] = l;
     }
     __syncthreads();
     if (group == 1) return;
-    const float m1 = theirs[32 * 64], l1 = theirs[33 * 64];
+    const float m1 = theirs[DT * 16 * 64], l1 = theirs[(DT * 16 + 1) * 64];
     if (!(m1 == -INFINITY && l1 == 0.f)) {         // (a query that sees none of their keys; scores that are all NaN have a weight)
       const float m = fmaxf(m_run, m1), f0 = __builtin_amdgcn_exp2f(m_run - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
       l = l * f0 + l1 * f1;
@@ -1210,25 +1223,37 @@ static bool turns_wanted(int n_seqs, int max_q_len, int n_tokens) {
   return max_q_len >= 1024 && (n_tokens <= 5L * max_q_len || n_tokens >= 1280L * n_seqs);
 }
 
-// The kernel of eight waves: two groups on the keys where its blocks of one head are at most 1,100 (two are on each CU at a time), else two heads a
+// Whether the library takes the kernel of eight waves. 3: with two groups on the keys, 4: with two heads a block, 0: another kernel (`plain` as below).
+// Heads of 64: two groups where its blocks of one head are at most 1,100 (two are on each CU at a time), else two heads a
 // block (32 heads: one sequence of 4,096 tokens, 1,040 blocks, 89.1 and 92.7 us, of 6,000 180 and 182; eight of 512, 1,152 blocks, 23.1 and 21.3, 32 of 256
 // 34.6 and 29.5). An odd number of heads a kv head has no pairs: two groups there too, but for many short sequences, where the kernel
 // of 128 queries is as fast or faster (24 heads over 8: sixteen of 146 to 336 tokens 14.7 against 13.4 us).
+// Heads of 128, one block on a CU at a time: two groups from 300 tokens of the longest sequence on (256 tokens 11.6 us, 10.9 with 64 queries a block;
+// 333 11.9 and 12.5) to 512 blocks of one sequence, or of a longest one with half of the tokens, to 256 of others (24 heads: 2,048 tokens, 408 blocks, 52 us
+// where turns take 57 and 64 queries a block 62, 3,000, 576 blocks, 84 and 80; 32 heads: three of 300 behind 1,000, 288 equal blocks, 51 and 46). Two heads a
+// block where the kernel of 128 queries would have them, for sequences of 384 tokens on average and more (32 heads: eight of 512 45.2 -> 38.5 us,
+// four of 1,000 58.8 -> 51.6, 32 of 256 59.6 and 67.6).
 #define PF_KEYS (INT_MIN + 1)
 #define PF_HEADS (INT_MIN + 2)
-static bool eight_takes(int head_dim, int page_size) { return head_dim == 64 && page_size % 64 == 0; }
-static int eight_choice(int n_heads, int group, int n_seqs, int n_tokens) {
+static bool eight_takes(int head_dim, int page_size) { return (head_dim == 64 || head_dim == 128) && page_size % 64 == 0; }
+extern "C" int gl3_prefill_eight(int head_dim, int page_size, int n_heads, int n_kv, int n_seqs, int max_q_len, int n_tokens, int plain) {
+  if (!plain || !eight_takes(head_dim, page_size)) return 0;
+  const int group = n_heads / n_kv;
   const long blocks = (long)n_heads * (n_tokens / 128 + (n_seqs + 1) / 2);
-  if (group % 2 == 0) return blocks <= 1100 ? 3 : 4;
-  return blocks <= 512 || n_tokens >= 256L * n_seqs ? 3 : 1;
+  if (head_dim == 64) {
+    if (max_q_len <= 32) return 0;
+    if (group % 2 == 0) return blocks <= 1100 ? 3 : 4;
+    return blocks <= 512 || n_tokens >= 256L * n_seqs ? 3 : 0;
+  }
+  if (max_q_len >= 300 && blocks <= (n_seqs == 1 || n_tokens <= 2L * max_q_len ? 512 : 256)) return 3;
+  return group % 2 == 0 && n_tokens >= 384L * n_seqs && prefill_wide(head_dim, n_heads, n_seqs, max_q_len) && !turns_wanted(n_seqs, max_q_len, n_tokens) ? 4 : 0;
 }
 
-// The library's choice: 0: 64 queries a block, 1: 128, 2: the kernel of turns, 3: eight waves in two groups on the keys, 4: on two heads. plain: the plain rule (one score map, no window, chunked
+// The library's choice where that is not it: 0: 64 queries a block, 1: 128, 2: the kernel of turns. plain: the plain rule (one score map, no window, chunked
 // mask, bias, sink, kept keys, cap, temperature or gate), no splits, caches at 16-byte addresses (its loads into shared memory bring
 // 16 bytes a lane and want them aligned, where the other kernels' ordinary loads do not).
 extern "C" int gl3_prefill_kernel(int head_dim, int page_size, int n_heads, int n_kv, int n_seqs, int max_q_len, int n_tokens, int plain) {
   if (!prefill_wide(head_dim, n_heads, n_seqs, max_q_len)) return 0;
-  if (plain && eight_takes(head_dim, page_size)) return eight_choice(n_heads, n_heads / n_kv, n_seqs, n_tokens);
   return plain && turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && turns_wanted(n_seqs, max_q_len, n_tokens) ? 2 : 1;
 }
 
@@ -1271,11 +1296,12 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
   const bool plain = splits == 1 && splits_plain;
   const bool eight = plain && eight_takes(head_dim, page_size);
   GL3_REQUIRE((wide_from != PF_KEYS && wide_from != PF_HEADS) || (eight && (wide_from == PF_KEYS || g % 2 == 0)),
-              "gl3_attention_prefill: the kernels of eight waves take heads of 64, pages of whole 64 keys, caches at 16-byte addresses, no splits, the plain rule, and two heads a block an even number of heads a kv head");
+              "gl3_attention_prefill: the kernels of eight waves take heads of 64 or 128, pages of whole 64 keys, caches at 16-byte addresses, no splits, the plain rule, and two heads a block an even number of heads a kv head");
   GL3_REQUIRE(wide_from != PF_TURNS || (plain && turns_takes(head_dim, page_size, g, n_seqs, n_tokens)),
               "gl3_attention_prefill: the kernel of turns takes heads of 128, pages of whole 64 keys, caches at 16-byte addresses, at most 64 sequences, no splits, the plain rule");
+  const int eights = gl3_prefill_eight(head_dim, page_size, n_heads, n_kv, n_seqs, max_q_len, n_tokens, plain);
   const int kernel = wide_from == PF_TURNS ? 2 : wide_from == PF_KEYS ? 3 : wide_from == PF_HEADS ? 4 : splits > 1 ? 1 : wide_from > 0 ? max_q_len >= wide_from
-                     : gl3_prefill_kernel(head_dim, page_size, n_heads, n_kv, n_seqs, max_q_len, n_tokens, plain);
+                     : eights ? eights : gl3_prefill_kernel(head_dim, page_size, n_heads, n_kv, n_seqs, max_q_len, n_tokens, plain);
   const bool wide = kernel > 0;
   // query heads per wave: as many as the registers hold with two blocks on a CU; one with 32 queries a wave
   const int gh = wide ? 1 : head_dim <= 32 ? 4 : head_dim <= 64 ? 2 : 1;
@@ -1307,16 +1333,22 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
     const int heads = kernel == 4 ? 2 : 1;
     const bool folded = n_seqs == 1 && (long)n_heads / heads * q_blocks * splits <= 512;
     dim3 egrid((unsigned)(n_heads / heads * splits), n_seqs, q_blocks);
-#define GOE(GROUPS, SPLIT)                                                                                            \
-  attention_prefill_eight_kernel<GROUPS, SPLIT><<<egrid, dim3(512), 0, stream>>>(                                            \
+#define GOE(HS, GROUPS, SPLIT)                                                                                        \
+  attention_prefill_eight_kernel<HS, GROUPS, SPLIT><<<egrid, dim3(512), 0, stream>>>(                                            \
       (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu_seqlens, kv_before, block_table, \
       seq_rows, table_stride, (bf16_t*)out, out_stride, n_heads, n_kv, page_size, scale, q_blocks, (int)folded, sp)
-    if (splits > 1) {
-      GOE(2, true);
-      const long rows = (long)n_tokens * n_heads * (64 / 4);
-      attention_prefill_merge_kernel<64><<<dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream>>>(sp, (bf16_t*)out, out_stride, n_heads);
-    } else if (kernel == 3) GOE(2, false);
-    else GOE(1, false);
+#define GOEH(HS)                                                                                                      \
+  do {                                                                                                                \
+    if (splits > 1) {                                                                                                 \
+      GOE(HS, 2, true);                                                                                               \
+      const long rows = (long)n_tokens * n_heads * (HS / 4);                                                          \
+      attention_prefill_merge_kernel<HS><<<dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream>>>(sp, (bf16_t*)out, out_stride, n_heads); \
+    } else if (kernel == 3) GOE(HS, 2, false);                                                                        \
+    else GOE(HS, 1, false);                                                                                           \
+  } while (0)
+    if (head_dim == 64) GOEH(64);
+    else GOEH(128);
+#undef GOEH
 #undef GOE
     GL3_LAUNCH_CHECK();
     return 0;

@@ -114,6 +114,7 @@ def _declare(lib):
         "gl3_attention_decode_supports": [I, I],
         "gl3_attention_prefill_supports": [I, I],
         "gl3_prefill_kernel": [I, I, I, I, I, I, I, I],
+        "gl3_prefill_eight": [I, I, I, I, I, I, I, I],
         "gl3_attention_prefill": [P, L, P, P, P, P, P, P, I, P, L, I, I, I, I, I, I, I, F, I, P, I, F, I, I, I, P, F, F, I, P, L, I, I, P, P, P],
         "gl3_scatter_i32": [P, L, P, P, I, P],
         "gl3_upload": [P, P, L, P],
@@ -2063,7 +2064,7 @@ PREFILL_SPLIT_KEYS = 1024            # keys that the longest sequence of a step 
 PREFILL_SPLIT_ROWS = 1024 * 128      # (token, head, split) rows that a step's splits never exceed
 
 
-def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=False):
+def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=0):
     """Blocks of 128 queries that share their keys out (``attention_prefill``'s ``splits``): for steps that bring few tokens behind
     a long context (a prompt in portions, the next turn of a dialogue), whose blocks are fewer than two for every CU and walk
     the context one chunk after another. Only where every sequence held at least as many tokens as the longest one
@@ -2073,17 +2074,18 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=Fals
     few, and the merge costs 5 to 10 us). A split's sums are 32-bit as the unsplit kernel's and shorter; only the maximum around which
     weights are rounded is another: the error against 64 bits is 0.967 times that without splits on average, smaller at all of 90
     sizes (contexts of 700 to 12,000, 37 to 1,100 tokens, heads of 32 to 128).
-    ``eight`` (heads of 64 in pages of whole 64 positions: the kernel of eight waves): one of its blocks keeps a CU's units busy, 1.2 us for 128
-    keys, and two on a CU take twice as long, so the splits are those whose rounds of 256 blocks are done first, a merge being 6 us and a
-    split's sums 2.8 TB/s of it. 32 heads, 300 tokens behind 3,000 31.2 us in the six splits of the rule above and 27.1 in two; 512 behind 1,024
-    24.3 in four, 19.9 without; 700 behind 12,000 119 in three, 100 in four; 1,000 behind 1,000 32.9 in two, 25.3 without."""
+    ``eight``: the head size where it is 64 or 128 in pages of whole 64 positions, the kernel of eight waves. One of its blocks keeps a CU's
+    units busy, 1.2 or 2.1 us for 128 keys, and two on a CU take twice as long, so the splits are those whose rounds of 256 blocks are done
+    first, a merge being 6 us and a split's sums 2.8 TB/s of it. 32 heads of 64: 300 tokens behind 3,000 31.2 us in the six splits of the rule
+    above and 27.1 in two; 512 behind 1,024 24.3 in four, 19.9 without; 700 behind 12,000 119 in three, 100 in four; 1,000 behind 1,000
+    32.9 in two, 25.3 without."""
     blocks = n_heads * n_seqs * -(-max_q_len // 128)
     if blocks >= 512 or max_kv_len < PREFILL_SPLIT_KEYS or not kv_before or min(kv_before) < max_q_len:
         return 1
     if eight:
         rows = n_heads * n_seqs * max_q_len
         return min((s for s in range(1, 9) if s == 1 or (s * 256 <= max_kv_len and s * blocks <= 1024)),
-                   key=lambda s: -(-blocks * s // 256) / s * max_kv_len / 128 * 1.2 + (s > 1) * (6 + s * rows * 256 / 2.8e6))
+                   key=lambda s: -(-blocks * s // 256) / s * max_kv_len / 128 * (1.2 if eight == 64 else 2.1) + (s > 1) * (6 + s * rows * eight * 4 / 2.8e6))
     return max(1, min(8, -(-512 // blocks), max_kv_len // 256))
 
 
@@ -2093,17 +2095,18 @@ PREFILL_KEYS, PREFILL_HEADS = PREFILL_TURNS + 1, PREFILL_TURNS + 2      # and th
 
 def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, out, max_q_len, n_heads, n_kv,
                       head_dim, page_size, window, scale, seq_rows=None, wide_from=0, slopes=None, sink=None, keep_first=0,
-                      chunk=0, n_v_heads=None, rule=None, splits=1, part_o=None, part_ml=None):
+                      chunk=0, n_v_heads=None, rule=None, splits=1, part_o=None, part_ml=None, eight_splits=None):
     """``rule``: a ``ScoreRule``; ``slopes`` (float32 [H]): score - slopes[h] * distance; ``sink``: the score of a key without a value that every
     query sees (None: none); ``chunk`` and ``n_v_heads`` as in ``attention_generic``. Any number of tokens per sequence; ``cu_seqlens`` [B+1] and ``kv_before`` [B] say which tokens
     of the packed ``q`` belong to which sequence and where they sit in it. ``seq_rows`` [B] (optional)
     names each sequence's row of ``block_table``; without it sequence b reads row b. ``wide_from``: from
     how many tokens of the step's longest sequence on the kernel with 128 queries a block runs
     (0 and below: the library's choice; ``PREFILL_TURNS``: the kernel of turns, which takes heads of 128 and the plain rule, gives the same bits
-    and has no splits; ``PREFILL_KEYS``, ``PREFILL_HEADS``: the kernel of eight waves, which takes heads of 64 and the plain rule; tests run all
+    and has no splits; ``PREFILL_KEYS``, ``PREFILL_HEADS``: the kernel of eight waves, which takes heads of 64 and 128 and the plain rule; tests run all
     kernels on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
     128 queries are shared out over that many blocks of the same kernel, whose sums lie in ``part_o`` (float32, at least
-    splits * T * H * hs) and ``part_ml`` (2 * splits * T * H) until a second kernel merges them; the plain rule only."""
+    splits * T * H * hs) and ``part_ml`` (2 * splits * T * H) until a second kernel merges them; the plain rule only.
+    ``eight_splits``: as many instead, where the splits run on the kernel of eight waves (1: none)."""
     _dev(q, "q", torch.bfloat16, contiguous=False); _dev(out, "out", torch.bfloat16, contiguous=False)
     _dev(k_cache, "k_cache", torch.bfloat16); _dev(v_cache, "v_cache", torch.bfloat16)
     _dev(cu_seqlens, "cu_seqlens", torch.int32); _dev(kv_before, "kv_before", torch.int32)
@@ -2127,6 +2130,8 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
     elif block_table.shape[0] < B:
         raise KernelError("attention: the block table has fewer rows than there are sequences")
     has_sink, sink_value, sinks = _sink(sink, n_heads, "attention_prefill")
+    if splits > 1 and eight_splits is not None:
+        splits = int(eight_splits)
     if splits > 1:
         _dev(part_o, "part_o", torch.float32); _dev(part_ml, "part_ml", torch.float32)
         if part_o.numel() < splits * T * n_heads * head_dim or part_ml.numel() < 2 * splits * T * n_heads:

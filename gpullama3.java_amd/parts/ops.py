@@ -556,8 +556,7 @@ def attention(ctx, q, k_cache, v_cache, block_table, out, n_heads, n_kv, head_di
     if kernel == "prefill":
         if (ctx.max_kv_len >= K.PREFILL_SPLIT_KEYS and not window and not chunk and slopes is None and sink is None
                 and n_v_heads is None and rule is None):
-            splits = K.prefill_splits(n_heads, ctx.n_seqs, ctx.max_q_len, getattr(ctx, "kv_before_host", None), ctx.max_kv_len,
-                                      eight=head_dim == 64 and page % 64 == 0)
+            splits = K.prefill_splits(n_heads, ctx.n_seqs, ctx.max_q_len, getattr(ctx, "kv_before_host", None), ctx.max_kv_len)
             if splits > 1:
                 # (of one size, whatever the step brings: a buffer that grew would take the captured decode steps with it. On a
                 # device without room for them the step runs without splits: it never needed this memory before. The small one
@@ -566,6 +565,8 @@ def attention(ctx, q, k_cache, v_cache, block_table, out, n_heads, n_kv, head_di
                 part_o = ctx.buffer_if_room("prefill_part_o", (K.PREFILL_SPLIT_ROWS * head_dim,), torch.float32) if part_ml is not None else None
                 if part_o is not None:
                     extras.update(splits=splits, part_o=part_o, part_ml=part_ml)
+                    if head_dim in (64, 128) and page % 64 == 0:
+                        extras["eight_splits"] = K.prefill_splits(n_heads, ctx.n_seqs, ctx.max_q_len, ctx.kv_before_host, ctx.max_kv_len, eight=head_dim)
         return K.attention_prefill(q, k_cache, v_cache, ctx.cu_seqlens, ctx.kv_before, block_table, out,
                                    ctx.max_q_len, n_heads, n_kv, head_dim, page, window, scale,
                                    seq_rows=getattr(ctx, "seq_rows", None), **extras)

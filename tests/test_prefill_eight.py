@@ -1,4 +1,4 @@
-"""The prefill attention of eight waves (heads of 64): its results against the plain reference and the kernel of 128 queries a block."""
+"""The prefill attention of eight waves (heads of 64 and 128): its results against the plain reference and the kernel of 128 queries a block."""
 import numpy as np
 import pytest
 
@@ -7,23 +7,29 @@ from test_prefill_turns import fn, rounding
 
 
 def test_which_calls_take_it():
-    def choice(lengths, heads=32, n_kv=8, page=64, plain=1):
-        return lib.library().gl3_prefill_kernel(64, page, heads, n_kv, len(lengths), max(lengths), sum(lengths), plain)
+    def choice(lengths, heads=32, n_kv=8, hs=64, page=64, plain=1):
+        return lib.library().gl3_prefill_eight(hs, page, heads, n_kv, len(lengths), max(lengths), sum(lengths), plain)
     assert choice([2048]) == 3 and choice([37]) == 3 and choice([317, 1203, 701]) == 3 and choice([4096]) == 3 and choice([8192]) == 4
-    assert choice([512] * 8) == 4 and choice([83] * 64) == 4 and choice([8192], 16, 16) == 3 and choice([200] * 16, 24) == 1
-    assert choice([32]) == 0 and choice([2048], page=96) == 1 and choice([2048], plain=0) == 1
+    assert choice([512] * 8) == 4 and choice([83] * 64) == 4 and choice([8192], 16, 16) == 3 and choice([200] * 16, 24) == 0
+    assert choice([32]) == 0 and choice([2048], page=96) == 0 and choice([2048], plain=0) == 0 and choice([2048], hs=96) == 0
+    large = dict(heads=24, hs=128)
+    assert choice([2048], **large) == 3 and choice([333], **large) == 3 and choice([256], **large) == 0 and choice([3000], **large) == 0
+    assert choice([1203, 317, 701], **large) == 3 and choice([512] * 8, **large) == 0 and choice([2048], hs=128) == 0
+    assert choice([512] * 8, hs=128) == 4 and choice([1000] * 4, hs=128) == 4 and choice([256] * 32, hs=128) == 0 and choice([8192], hs=128) == 0
 
 
 def test_splits_of_its_blocks():
-    def s(heads, n_seqs, T, before):
-        return lib.prefill_splits(heads, n_seqs, T, [before] * n_seqs, T + before, eight=True)
+    def s(heads, n_seqs, T, before, hs=64):
+        return lib.prefill_splits(heads, n_seqs, T, [before] * n_seqs, T + before, eight=hs)
     assert s(32, 1, 64, 4000) == 8 and s(32, 1, 150, 3000) == 4 and s(32, 1, 512, 1024) == 1 and s(32, 1, 512, 4096) == 2
     assert s(32, 1, 1000, 6000) == 1 and s(32, 3, 300, 1000) == 1 and s(32, 1, 512, 500) == 1 and s(16, 4, 100, 2000) == 4
+    assert s(24, 1, 512, 2048, 128) == 2 and s(24, 1, 512, 512, 128) == 1
     for heads in (1, 2, 24, 32, 128, 511):
         for n_seqs in (1, 2, 7):
             for T in (1, 128, 129, 1000, 5000):
-                n = s(heads, n_seqs, T, 100000)
-                assert 1 <= n <= 8 and (n == 1 or n * n_seqs * T * heads <= lib.PREFILL_SPLIT_ROWS)
+                for hs in (64, 128):
+                    n = s(heads, n_seqs, T, 100000, hs)
+                    assert 1 <= n <= 8 and (n == 1 or n * n_seqs * T * heads <= lib.PREFILL_SPLIT_ROWS)
 
 
 # one, two, three and four heads a kv head; waves, blocks and chunks with one row and all but one, one chunk (none for the second group); sequences that start no
@@ -34,12 +40,13 @@ CASES = [(4, 2, 64, [0, 70, 0, 130, 5], [33, 1, 200, 17, 64]), (3, 1, 64, [0, 0,
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("sharp", [1, 8])
+@pytest.mark.parametrize("hs", [64, 128])
 @pytest.mark.parametrize("H, Kh, page, before, new", CASES)
-def test_attention_of_eight_waves(H, Kh, page, before, new, sharp):
+def test_attention_of_eight_waves(H, Kh, page, before, new, hs, sharp):
     from test_gpu_kernels import attention_case, run_attention
-    sk, sv, qs = attention_case(np.random.default_rng(H * page + sharp), H, Kh, 64, before, new, "bfloat16")
+    sk, sv, qs = attention_case(np.random.default_rng(H * page + sharp), H, Kh, hs, before, new, "bfloat16")
     qs = [q * sharp for q in qs]                     # (8: a few keys have all the weight, and maxima move in all chunks)
-    run = lambda f: run_attention(f, sk, sv, qs, before, new, H, Kh, 64, "bfloat16", np.random.default_rng(1), page=page)
+    run = lambda f: run_attention(f, sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1), page=page)
     got, ref = run(fn(before, new, lib.PREFILL_KEYS))
     assert float((np.abs(got - ref) / rounding(qs, sk, sv, ref, before, new)).max()) <= 1
     np.testing.assert_array_equal(got, run(fn(before, new, lib.PREFILL_KEYS, shuffled_rows=True))[0])
@@ -50,12 +57,13 @@ def test_attention_of_eight_waves(H, Kh, page, before, new, sharp):
 
 
 @pytest.mark.gpu
-def test_scores_that_are_not_numbers_are_in_the_rows_that_see_them():
+@pytest.mark.parametrize("hs", [64, 128])
+def test_scores_that_are_not_numbers_are_in_the_rows_that_see_them(hs):
     from test_gpu_kernels import attention_case, run_attention
     H, Kh, before, new = 4, 2, [700], [300]
-    sk, sv, qs = attention_case(np.random.default_rng(3), H, Kh, 64, before, new, "bfloat16")
+    sk, sv, qs = attention_case(np.random.default_rng(3), H, Kh, hs, before, new, "bfloat16")
     for mode in (lib.PREFILL_KEYS, lib.PREFILL_HEADS):
-        run = lambda k: run_attention(fn(before, new, mode), k, sv, qs, before, new, H, Kh, 64, "bfloat16", np.random.default_rng(1))[0]
+        run = lambda k: run_attention(fn(before, new, mode), k, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1))[0]
         clean = run(sk)
         for lo, hi in ((900, 930), (768, 832), (0, 64)):      # (a part of a chunk, all of an even one, all of the first)
             k = [s.copy() for s in sk]
