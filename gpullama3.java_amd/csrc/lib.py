@@ -7,6 +7,7 @@ fallback: without a GPU, or without the library, the call raises.
 """
 from __future__ import annotations
 
+import array
 import ctypes
 from ctypes import c_float, c_int, c_long, c_uint32, c_void_p
 from typing import NamedTuple, Optional
@@ -1500,8 +1501,8 @@ def sample(logits, work, temperature, top_p, uniform, out, step=None, uniform_st
 
 
 def sample_host(logits, work, parameters, out):
-    """``sample`` (or, with ``parameters`` None, ``argmax``) of every row, waited for: ``parameters``: three lists of one number a row
-    (temperatures, top-p, uniforms) in host memory; ``out``: int32 in pinned host memory, written when the call returns.
+    """``sample`` (or, with ``parameters`` None, ``argmax``) of every row, waited for: ``parameters``: three lists (or arrays of 32-bit
+    floats) of one number a row (temperatures, top-p, uniforms) in host memory; ``out``: int32 in pinned host memory, written when the call returns.
     ``work``: ``sample_work_size`` floats and three a row."""
     _dev(logits, "logits", torch.float32, contiguous=False); _dev(work, "work", torch.float32)
     R, V = logits.shape
@@ -1513,7 +1514,7 @@ def sample_host(logits, work, parameters, out):
     if parameters is not None:
         if any(len(p) < R for p in parameters):
             raise KernelError("sample: argument sizes")
-        par = [(ctypes.c_float * R)(*p[:R]) for p in parameters]
+        par = [(ctypes.c_float * R).from_buffer(p) if isinstance(p, array.array) else (ctypes.c_float * R)(*p[:R]) for p in parameters]
     _check(library().gl3_sample_host(_ptr(logits), logits.stride(0), _ptr(work), *par, _ptr(out), R, V, _stream()), "sample")
 
 

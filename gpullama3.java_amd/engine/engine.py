@@ -491,6 +491,8 @@ class Engine:
 
     # ------------------------------------------------------------------ generation
     def sample(self, logits, temperatures, top_ps, uniforms):
+        if self.device.index == torch.cuda.current_device():      # (entering the device it is takes as long as a launch)
+            return self.sampler(logits, temperatures, top_ps, uniforms)
         with torch.cuda.device(self.device):
             return self.sampler(logits, temperatures, top_ps, uniforms)
 

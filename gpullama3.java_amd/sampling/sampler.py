@@ -10,6 +10,7 @@ sequence's tokens do not depend on what else is in its batch.
 from __future__ import annotations
 
 import threading
+from array import array
 from dataclasses import dataclass
 
 import numpy as np
@@ -98,7 +99,7 @@ class DeviceSampler:
         out = torch.empty(R, dtype=torch.int32, device="cpu", pin_memory=True)      # (whatever the caller's default device is)
         parameters = None
         if not all(t == 0 for t in temperatures):       # (every row greedy: the rows are read by many blocks at once)
-            parameters = [[float(x) for x in p] for p in (temperatures, top_ps, uniforms)]
+            parameters = [array("f", map(float, p)) for p in (temperatures, top_ps, uniforms)]
             if len({len(p) for p in parameters}) != 1:
                 raise ValueError("as many temperatures as top-p and uniform numbers")
         with self._lock:                                # (the library lets go of the interpreter: another thread's call would run beside this one)
