@@ -494,21 +494,16 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
 // banks once. A step is asked for into the place of the step before, behind the barrier that every wave reaches with that step's
 // products issued (its reads have returned); the wait in front of the barrier leaves out the later steps. Steps beyond the last repeat it,
 // so that the counts hold; nothing is in flight when a block ends. Sums as above: the same bits.
+constexpr int f3_stage(int TW, int TT) { return 32 * (TW + TT) * 128; }      // bytes of a step: rows of W, then rows of A
 template <int EPI, int TW, int TT, int STAGES>
-__global__ __launch_bounds__(256, 2) void gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                                                                 float* __restrict__ C, int M, int N, int K, long lda,
-                                                                 long ldw, long ldc, int tiles_m, int tiles_n, F3Out o) {
+__device__ __forceinline__ void f3_stream_tile(char* lds, const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
+                                               int K, long lda, long ldw, long ldc, int m0, int n0, const F3Out& o) {
   constexpr int BN = 32 * TW, BM = 32 * TT, PW = (BN + BM) / 32;       // PW: pieces of 1 KB (8 rows) of a step that a wave brings
-  constexpr int NCOLS = EPI == F3_GATED ? BN / 2 : BN, STAGE = (BN + BM) * 128;
+  constexpr int STAGE = f3_stage(TW, TT);
   static_assert(EPI != F3_GATED || TW % 2 == 0, "a wave's tiles are gate rows and their up rows");
-  __shared__ __attribute__((aligned(1024))) char lds[STAGES * STAGE];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r = lane & 15, q = lane >> 4;
   const int ww = wave & 1, wt = wave >> 1;
-  const int n_tiles = tiles_m * tiles_n, per_xcd = (n_tiles + 7) / 8;          // (block -> tile as above)
-  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-  if (tile >= n_tiles) return;
-  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * NCOLS;
   const int steps = K / F3_BK;
 
   const i32x4 a_buf = mf_rsrc(A + (long)m0 * lda), w_buf = mf_rsrc(W + (long)n0 * ldw);
@@ -583,6 +578,38 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_stream_kernel(const float* __
   mf_wait_loads<0>();
   f3_finish_tile<EPI, TW, TT>(C, total, m0 + wt * 16 * TT + r, n0 + ww * (EPI == F3_GATED ? 8 : 16) * TW + q * 4, M, N, ldc, o);
 }
+template <int EPI, int TW, int TT, int STAGES>
+__global__ __launch_bounds__(256, 2) void gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                 float* __restrict__ C, int M, int N, int K, long lda,
+                                                                 long ldw, long ldc, int tiles_m, int tiles_n, F3Out o) {
+  __shared__ __attribute__((aligned(1024))) char lds[STAGES * f3_stage(TW, TT)];
+  const int n_tiles = tiles_m * tiles_n, per_xcd = (n_tiles + 7) / 8;          // (block -> tile as above)
+  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (tile >= n_tiles) return;
+  f3_stream_tile<EPI, TW, TT, STAGES>(lds, A, W, C, M, N, K, lda, ldw, ldc, tile % tiles_m * (32 * TT), tile / tiles_m * ((EPI == F3_GATED ? 16 : 32) * TW), o);
+}
+
+// Two tiles: the first `big_m` rows of tiles are TW x TT, those behind them SW x ST, smaller ones, which the CUs take that are done with the
+// large ones, one launch. Whole rounds of the chip are what bounds a product of few tiles: 513 rows of the 1B layers' down projection are 544 tiles of
+// 64 x 32, three rounds for the work of 2.1, or one round of 64 x 64 and a row: 223 -> 189 us; their output projection 62 -> 53, gate/up 336 -> 302.
+// The same bits: a sum does not know its tile.
+template <int EPI, int TW, int TT, int STAGES, int SW, int ST, int SSTAGES>
+__global__ __launch_bounds__(256, 2) void gemm_f32_two_tiles_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                    float* __restrict__ C, int M, int N, int K, long lda, long ldw,
+                                                                    long ldc, int big_m, int big_n, int small_m, int small_n, F3Out o) {
+  constexpr int BIG = STAGES * f3_stage(TW, TT), SMALL = SSTAGES * f3_stage(SW, ST), COLS = EPI == F3_GATED ? 16 : 32;
+  __shared__ __attribute__((aligned(1024))) char lds[BIG > SMALL ? BIG : SMALL];
+  const int big = big_m * big_n, small = small_m * small_n, big_xcd = (big + 7) / 8, small_xcd = (small + 7) / 8;
+  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  if (at < big_xcd) {
+    const int tile = xcd * big_xcd + at;
+    if (tile < big) f3_stream_tile<EPI, TW, TT, STAGES>(lds, A, W, C, M, N, K, lda, ldw, ldc, tile % big_m * (32 * TT), tile / big_m * (COLS * TW), o);
+  } else {
+    const int tile = xcd * small_xcd + at - big_xcd;
+    if (tile < small)
+      f3_stream_tile<EPI, SW, ST, SSTAGES>(lds, A, W, C, M, N, K, lda, ldw, ldc, big_m * (32 * TT) + tile % small_m * (32 * ST), tile / small_m * (COLS * SW), o);
+  }
+}
 
 template <int EPI, int TM, bool PAIRS = false>
 static int launch_rows(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
@@ -604,6 +631,20 @@ static int launch_stream(const float* A, const float* W, float* C, int M, int N,
   GL3_REQUIRE(blocks < (1L << 31), "gl3_gemm_generic: too many tiles");
   gemm_f32_stream_kernel<EPI, TW, TT, STAGES><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, tiles_m,
                                                                                                tiles_n, o);
+  GL3_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int EPI, int TW, int TT, int STAGES, int SW, int ST, int SSTAGES>
+static int launch_two_tiles(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc,
+                            const F3Out& o, int big_m, hipStream_t stream) {
+  constexpr int COLS = EPI == F3_GATED ? 16 : 32;
+  const int big_n = (N + COLS * TW - 1) / (COLS * TW), small_n = (N + COLS * SW - 1) / (COLS * SW);
+  const int small_m = (M - big_m * 32 * TT + 32 * ST - 1) / (32 * ST);
+  const long blocks = (((long)big_m * big_n + 7) / 8 + ((long)small_m * small_n + 7) / 8) * 8;
+  GL3_REQUIRE(big_m > 0 && small_m > 0 && blocks < (1L << 31), "gl3_gemm_generic: too many tiles");
+  gemm_f32_two_tiles_kernel<EPI, TW, TT, STAGES, SW, ST, SSTAGES><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(
+      A, W, C, M, N, K, lda, ldw, ldc, big_m, big_n, small_m, small_n, o);
   GL3_LAUNCH_CHECK();
   return 0;
 }
@@ -634,17 +675,51 @@ static bool f32_streams(const void* A, int N, int K, long lda, long ldw, bool ga
 // Its tile: 1 to 4: 128 rows of W x 128 tokens, 128 x 64, 64 x 64, 64 x 32; 5: 32 x 32 (not gated). As in gl3_f32_shape: one tile alone
 // on a CU takes `alone`, a CU with several `each` a tile (us for K = 2,048, both measured; of 85 products of 17 to 4,096 rows
 // one is more than 2% from the best of the tiles, 6%: profiles/float32_tiles.txt).
-extern "C" int gl3_f32_stream_shape(int M, int N, int gated) {
-  static const int bn[5] = {128, 128, 64, 64, 32}, bm[5] = {128, 64, 64, 32, 32};
-  static const float alone[5] = {144, 80, 45.5f, 28.6f, 20.5f}, each[5] = {124.4f, 62.5f, 33.4f, 17.7f, 11.f};
+struct F3Cost { int bn, bm; float alone, each; };
+static const F3Cost f3_cost[5] = {{128, 128, 144, 124.4f}, {128, 64, 80, 62.5f}, {64, 64, 45.5f, 33.4f}, {64, 32, 28.6f, 17.7f}, {32, 32, 20.5f, 11.f}};
+static int f3_best_tile(int M, int N, int gated, float& least) {
   int best = 4;
-  float least = 0.f;
+  least = 0.f;
   for (int i = 0; i < (gated ? 4 : 5); ++i) {
-    const long tiles = (long)((M + bm[i] - 1) / bm[i]) * (((gated ? 2L : 1L) * N + bn[i] - 1) / bn[i]);
-    const float cu = (float)((tiles + 255) / 256) * each[i], cost = cu < alone[i] ? alone[i] : cu;
+    const F3Cost& t = f3_cost[i];
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * (((gated ? 2L : 1L) * N + t.bn - 1) / t.bn);
+    const float cu = (float)((tiles + 255) / 256) * t.each, cost = cu < t.alone ? t.alone : cu;
     if (i == 0 || cost < least) {
       least = cost;
       best = i + 1;
+    }
+  }
+  return best;
+}
+extern "C" int gl3_f32_stream_shape(int M, int N, int gated) {
+  float least;
+  return f3_best_tile(M, N, gated, least);
+}
+// Whether two tiles (gemm_f32_two_tiles_kernel) are expected to take less than 0.95 of the best single tile's time, and which: 64 * rows of large
+// tiles + 8 * the large tile + the small one; 0: one tile. The blocks are all handed out at once, about as many of either kind to every CU, so a CU's
+// time is taken as that of its large tiles and then its small ones. (As if the small ones went to the CUs that have no large tile: of 42 sizes
+// seven took 1.03 to 1.08 times as long as one tile, those this rule leaves out.) A small tile beside others takes 1.05 of its time. Measured at 72 sizes
+// (100 to 2,500 rows, the 1B layers' products and the 3B layers' QKV) that a margin of 0.96 without the 1.05 takes: 0.82 to 1.02 times as long as one tile
+// and 0.91 on average, but for two (1.03, 1.11), which this rule leaves out.
+extern "C" int gl3_f32_stream_two(int M, int N, int gated) {
+  float least;
+  f3_best_tile(M, N, gated, least);
+  least *= 0.95f;
+  const long rows = (gated ? 2L : 1L) * N;
+  int best = 0;
+  for (int i = 0; i < 3; ++i) {
+    const F3Cost& t = f3_cost[i];
+    for (int r = (M - 1) / t.bm, first = r - 3; r > 0 && r >= first; --r) {
+      const float big = (float)((r * ((rows + t.bn - 1) / t.bn) + 255) / 256) * t.each;
+      for (int j = i < 2 ? 3 : 4; j < (gated ? 4 : 5); ++j) {      // (64 x 32 behind 64 x 64 never is the best)
+        const F3Cost& u = f3_cost[j];
+        const long small = (long)((M - r * t.bm + u.bm - 1) / u.bm) * ((rows + u.bn - 1) / u.bn);
+        const float cu = big + (float)((small + 255) / 256) * 1.05f * u.each, cost = cu < t.alone ? t.alone : cu;
+        if (cost < least) {
+          best = r * 64 + (i + 1) * 8 + j + 1;
+          least = cost;
+        }
+      }
     }
   }
   return best;
@@ -657,6 +732,17 @@ static int launch_f32(const float* A, const float* W, float* C, int M, int N, in
   int shape = gl3_f32_shape(M, N, EPI == F3_GATED);
   // (gated products of 17 to 32 rows too: 1B layers' gate/up 35 us with the kernel for few rows, 29 in tiles of 64 x 32)
   if ((shape != 1 || (EPI == F3_GATED && M > 16)) && f32_streams(A, N, K, lda, ldw, EPI == F3_GATED)) {
+    const int two = gl3_f32_stream_two(M, N, EPI == F3_GATED);
+#define F3_TWO_ARGS A, W, C, M, N, K, lda, ldw, ldc, o, two / 64, stream
+    switch (two % 64) {
+      case 014: return launch_two_tiles<EPI, 4, 4, 2, 2, 1, 3>(F3_TWO_ARGS);
+      case 024: return launch_two_tiles<EPI, 4, 2, 2, 2, 1, 3>(F3_TWO_ARGS);
+      case 015: if constexpr (EPI != F3_GATED) return launch_two_tiles<EPI, 4, 4, 2, 1, 1, 4>(F3_TWO_ARGS); break;
+      case 025: if constexpr (EPI != F3_GATED) return launch_two_tiles<EPI, 4, 2, 2, 1, 1, 4>(F3_TWO_ARGS); break;
+      case 035: if constexpr (EPI != F3_GATED) return launch_two_tiles<EPI, 2, 2, 3, 1, 1, 4>(F3_TWO_ARGS); break;
+      default: break;
+    }
+#undef F3_TWO_ARGS
     switch (gl3_f32_stream_shape(M, N, EPI == F3_GATED)) {
       case 1: return launch_stream<EPI, 4, 4, 2>(F3_ARGS);
       case 2: return launch_stream<EPI, 4, 2, 2>(F3_ARGS);

@@ -112,6 +112,7 @@ def _declare(lib):
         "gl3_gemm_mfma": [P, P, P, I, I, I, I, L, L, L, I, I, P, L, L, P, I, I, I, P, F, F, P, P],
         "gl3_f32_shape": [I, I, I],
         "gl3_f32_stream_shape": [I, I, I],
+        "gl3_f32_stream_two": [I, I, I],
         "gl3_attention_decode_supports": [I, I],
         "gl3_attention_prefill_supports": [I, I],
         "gl3_prefill_kernel": [I, I, I, I, I, I, I, I],

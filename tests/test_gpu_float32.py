@@ -129,6 +129,32 @@ def test_float32_products_in_every_tile_of_whole_steps(tile, gated, M, N, Kd):
         assert torch.equal(one[0], out[r, :N])
 
 
+# (large and small tile, rows of large tiles) each pair of tiles that there is: one row, all but one and several tiles of them behind the large ones,
+# columns beyond whole tiles; one step of K, a chunk and a step
+@pytest.mark.parametrize("Kd", [32, 288])
+@pytest.mark.parametrize("large, small, rows, gated, M, N", [(1, 4, 19, False, 2478, 5120), (1, 5, 19, False, 2440, 5120), (2, 4, 12, False, 816, 5120), (2, 5, 21, False, 1406, 3070),
+                                                             (3, 5, 8, False, 513, 2048), (3, 5, 5, False, 333, 3071),
+                                                             (1, 4, 18, True, 2305, 3584), (2, 4, 2, True, 130, 8190), (2, 4, 10, True, 671, 8192), (2, 4, 10, True, 705, 1490)])
+def test_float32_products_in_two_tiles(large, small, rows, gated, M, N, Kd):
+    """The same bits as the rows in smaller companies, which go by one tile each, or by none."""
+    lib = K()
+    code = lib.library().gl3_f32_stream_two(M, N, int(gated))
+    assert (code // 8 % 8, code % 8, code // 64) == (large, small, rows)
+    gen = torch.Generator(device="cuda").manual_seed(M + Kd)
+    A, W = torch.randn(M, Kd + 4, generator=gen, device="cuda")[:, :Kd], torch.randn(2 * N if gated else N, Kd, generator=gen, device="cuda")
+    bias = torch.randn(W.shape[0], generator=gen, device="cuda")
+    for epilogue in (lib.EPI_GATED,) if gated else (lib.EPI_STORE, lib.EPI_ADD):
+        out = torch.full((M, N + 1), -7.0, device="cuda")
+        was = out[:, :N].clone()
+        lib.gemm_generic(A, W, out[:, :N], epilogue, bias=bias)
+        assert torch.all(out[:, N] == -7.0)
+        for lo in range(0, M, 60):                       # (60 rows: no two tiles)
+            assert lib.library().gl3_f32_stream_two(min(60, M - lo), N, int(gated)) == 0
+            part = was[lo:lo + 60].clone()
+            lib.gemm_generic(A[lo:lo + 60], W, part, epilogue, bias=bias)
+            assert torch.equal(part, out[lo:lo + 60, :N]), (epilogue, lo)
+
+
 def test_float32_products_keep_small_numbers_and_infinities():
     lib = K()
     a, w = np.zeros((20, 64), np.float32), np.zeros((32, 64), np.float32)
