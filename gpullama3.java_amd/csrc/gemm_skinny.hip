@@ -38,6 +38,7 @@
 // nothing else, which is what limits the streaming kernel when the same A is read for every
 // strip. The wide one, for 17 to 64 rows, takes several strips at once (see there).
 #include "common.h"
+#include "lds_loads.h"
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -978,7 +979,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_decode_kernel(
 //
 // XNORM (one slice of K): the product is that of an RMSNorm, as in the other kernels: A holds
 // bfloat16(weight * x) and the rows' 1/rms, from the partial sums of squares, is applied to the sums.
-template <int MT, int NS, int NW, int EPI, typename TC, bool XNORM, int WL>
+//
+// DMA (W in one of its copies' orders, K in whole pairs of k-steps): a wave's lines of A go from memory straight to their places in its piece of
+// shared memory, which holds two pairs, so that no registers carry them, and two pairs of k-steps are on their way instead of one. With four token
+// tiles and one strip or a plain epilogue the trip to memory behind each of a wave's few pairs is what bounds the product: 64 rows of 3,072 x 2,048
+// 9.64 -> 8.11 us in a graph, 2,048 x 2,048 in four slices 6.29 -> 6.02, 2,048 x 8,192 12.32 -> 12.00, 3,072 x 3,072 8.96 -> 8.52, 4,096 x 14,336 31.4 -> 31.0.
+// Fewer tiles have less of A to carry (17 rows of 3,072 x 3,072 6.29 -> 6.55, 48 7.32 -> 7.60), gated ones ask for enough of W as it is
+// (64 rows of 8,192 x 2,048 18.7 -> 19.2): those go as before. The same sums in the same order.
+template <int MT, int NS, int NW, int EPI, typename TC, bool XNORM, int WL, bool DMA>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_wide_kernel(const bf16_t* __restrict__ A,
                                                                    const bf16_t* __restrict__ W, TC* __restrict__ C,
                                                                    int M, int N, int K, long lda, long ldw, long ldc,
@@ -996,8 +1004,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_wide_kernel(const bf16_t*
   constexpr int NT = NWT + MT;        // tiles a wave stages for a pair of k-steps: 16 rows x 128 bytes each
   SK_STAMP(0); SK_STAMP(1);
   constexpr int NTILES = NS * NG * MT;   // the partial tiles of a wave: all of the block's strips end together
-  constexpr int STAGE = NW * NT * 2048, RED = NW * NTILES * 1024;
-  __shared__ __attribute__((aligned(16))) char smem[STAGE > RED ? STAGE : RED];
+  constexpr int WAVE_STAGE = (DMA ? 2 * MT : NT) * 2048, STAGE = NW * WAVE_STAGE, RED = NW * NTILES * 1024;
+  static_assert(!DMA || WL != 0, "rows of W as they are stored pass through shared memory");
+  __shared__ __attribute__((aligned(1024))) char smem[STAGE > RED ? STAGE : RED];
   __shared__ float sm_ssq[XNORM ? NW : 1][64];
   f32x4 (*red)[NTILES][64] = (f32x4 (*)[NTILES][64])smem;   // the partial tiles, once the staging is over
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -1006,7 +1015,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_wide_kernel(const bf16_t*
   const int n_strips = (N + 15) / 16;
   const int strip0 = blockIdx.x * NS;
   SK_STAMP(10);
-  char* stage = smem + wave * (NT * 2048);
+  char* stage = smem + wave * WAVE_STAGE;
   // where this lane's loads go inside a tile (rows l8 and 8 + l8) and where its operands lie (k-steps 0, 1)
   const int put0 = l8 * 128 + ((c8 ^ l8) * 16);
   const int put1 = (8 + ((l8 + 1) & 7)) * 128 + ((c8 ^ l8) * 16);
@@ -1049,6 +1058,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_wide_kernel(const bf16_t*
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
+      if (DMA) {   // (lane l's 16 bytes land at 16 l: it brings what belongs there; a row beyond A's end is its last, and nobody's result)
+        const int i = j ? (l8 + 7) & 7 : l8, m = min(mt * 16 + 8 * j + i, M - 1);
+        xo[mt][j] = ((unsigned)m * (unsigned)lda + (unsigned)(c8 ^ i) * 8u) * 2u;
+        continue;
+      }
       const int m = mt * 16 + 8 * j + l8;
       xo[mt][j] = m < M ? ((unsigned)m * (unsigned)lda + (unsigned)c8 * 8u) * 2u : NOWHERE;
     }
@@ -1119,8 +1133,32 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_wide_kernel(const bf16_t*
       for (int j = 0; j < 2; ++j)
         held[NWT + mt][j] = sk_ld_b128(a_buf, ((xo[mt][j] | k2) & NOWHERE) ? NOWHERE : xo[mt][j] + k2);
   };
+  // DMA: pair i of the wave's into place `slot` of its two, the lines of A first; a pair beyond the last asks for nothing (of W for zeros)
+  bf16x8 two[DMA ? 2 : 1][NWT][2];
+  const i32x4 a_at = mf_rsrc(A);
+  const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)stage;
+  auto ask_ahead = [&](int i, auto slot) {
+    constexpr int S = decltype(slot)::value;
+    const int p = pair_at(i);
+    if (p < p_end) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) mf_dma16(lds0 + (S * MT + mt) * 2048 + j * 1024, xo[mt][j], a_at, (unsigned)p * 128u);
+    }
+    const unsigned kw = p < p_end ? (unsigned)p * w_pair : NOWHERE;
+#pragma unroll
+    for (int t = 0; t < NWT; ++t)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) two[S][t][j] = sk_ld_b128(w_buf, wo[t][j] + kw);
+  };
   SK_STAMP(12);
-  ask(pair_at(0));
+  if constexpr (DMA) {
+    ask_ahead(0, std::integral_constant<int, 0>{});
+    ask_ahead(1, std::integral_constant<int, 1>{});
+  } else {
+    ask(pair_at(0));
+  }
   SK_STAMP(2);
   SkPre pre[ENDS];
   int end_hd[ENDS], end_sub[ENDS];
@@ -1139,7 +1177,35 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_wide_kernel(const bf16_t*
     }
   }
   if (XNORM) sk_ssq_ask<NW, MT>(sq, M, nrm, sq_row);
-  for (int i = 0; i < n_it; ++i) {
+  if constexpr (DMA) {
+    auto pair = [&](int i, auto slot) {
+      constexpr int S = decltype(slot)::value;
+      mf_wait_loads<2 * NWT>();                    // all but the next pair's W has come
+      if (pair_at(i) < p_end) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          bf16x8 xf[MT];
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) xf[mt] = *(const bf16x8*)(stage + (S * MT + mt) * 2048 + (s ? get1 : get0));
+#pragma unroll
+          for (int g = 0; g < NS; ++g)
+#pragma unroll
+            for (int h = 0; h < NG; ++h)
+#pragma unroll
+              for (int mt = 0; mt < MT; ++mt)
+                acc[g][h][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(two[S][g * NG + h][s], xf[mt], acc[g][h][mt], 0, 0, 0);
+        }
+      }
+      mf_wait_reads<0>();                          // (the place may be written again)
+      ask_ahead(i + 2, slot);
+    };
+    for (int i = 0; i < n_it; i += 2) {
+      pair(i, std::integral_constant<int, 0>{});
+      pair(i + 1, std::integral_constant<int, 1>{});
+    }
+    mf_wait_loads<0>();
+  }
+  for (int i = 0; i < (DMA ? 0 : n_it); ++i) {
     bf16x8 wnow[NWT][2];   // (wl 1, 2) this pair's operands of W, which the next pair's loads are about to replace
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -1446,17 +1512,22 @@ static int launch_wide(const SkCall& a, int slices, long slice_stride) {
   const int n_strips = (a.N + 15) / 16;
   const int pairs = (a.K + 63) / 64;   // pairs of k-steps
   const int per_slice = (pairs + slices - 1) / slices;
-#define SK_WIDE(WL)                                                                                               \
-  gemm_skinny_wide_kernel<MT, NS, NW, EPI, TC, XNORM, WL>                                                         \
+#define SK_WIDE(WL, DMA)                                                                                          \
+  gemm_skinny_wide_kernel<MT, NS, NW, EPI, TC, XNORM, WL, DMA>                                                    \
       <<<dim3((n_strips + NS - 1) / NS, slices), dim3(NW * 64), 0, a.stream>>>(                                   \
           (const bf16_t*)a.A, (const bf16_t*)a.W, (TC*)a.C, a.M, a.N, a.K, a.lda, a.ldw, a.ldc, slice_stride, per_slice, \
           a.rp, a.nx, a.nrm)
-  if (a.wl == 0) SK_WIDE(0);
-  else if (a.wl == 1) SK_WIDE(1);
+  constexpr bool DMA = MT == 4 && EPI != SK_GATED && !XNORM;
+  const bool dma = DMA && a.K % 64 == 0;
+  if (a.wl == 0) SK_WIDE(0, false);
+  else if (a.wl == 1 && dma) SK_WIDE(1, DMA);
+  else if (a.wl == 1) SK_WIDE(1, false);
   else {
     // the packed strips of 8 rows: the copies of the output and down projections
-    if constexpr ((EPI == SK_STORE || EPI == SK_ADD) && !XNORM) SK_WIDE(2);
-    else GL3_REQUIRE(false, "gl3_gemm_skinny_wide: W in packed strips of 8 is read by the store and add epilogues (epilogue %d)", EPI);
+    if constexpr ((EPI == SK_STORE || EPI == SK_ADD) && !XNORM) {
+      if (dma) SK_WIDE(2, DMA);
+      else SK_WIDE(2, false);
+    } else GL3_REQUIRE(false, "gl3_gemm_skinny_wide: W in packed strips of 8 is read by the store and add epilogues (epilogue %d)", EPI);
   }
 #undef SK_WIDE
   GL3_LAUNCH_CHECK();
