@@ -2078,17 +2078,20 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=0):
     sizes (contexts of 700 to 12,000, 37 to 1,100 tokens, heads of 32 to 128).
     ``eight``: the head size where it is 64 or 128 in pages of whole 64 positions, the kernel of eight waves. One of its blocks keeps a CU's
     units busy, 1.2 or 2.1 us for 128 keys, and two on a CU take twice as long, so the splits are those whose rounds of 256 blocks are done
-    first, a merge being 6 us and a split's sums 2.8 TB/s of it. 32 heads of 64: 300 tokens behind 3,000 31.2 us in the six splits of the rule
-    above and 27.1 in two; 512 behind 1,024 24.3 in four, 19.9 without; 700 behind 12,000 119 in three, 100 in four; 1,000 behind 1,000
-    32.9 in two, 25.3 without."""
+    first, a merge being 6 us and a split's sums 2.8 TB/s of it, but at least half as many as the rule above has: a block's two groups have a maximum
+    each, and the more maxima the more weights are one, which rounding leaves alone (with half as many maxima the error against 64 bits was 1.002 to 1.019
+    times that of the rule above; so 0.976 to 1.001 at 72 sizes, spreads of the scores among them). 32 heads of 64: 300 tokens behind 3,000 31.2 us in the six splits
+    of the rule above, 512 behind 512 17.5 in two, 14.9 without, 512 behind 3,584 32.6 in two, 35.6 in four; 24 heads of 128: 512 behind 3,584 64 in six on
+    the kernel of 128 queries, 51.9 in five, 64.1 in three, 50.9 in two."""
     blocks = n_heads * n_seqs * -(-max_q_len // 128)
     if blocks >= 512 or max_kv_len < PREFILL_SPLIT_KEYS or not kv_before or min(kv_before) < max_q_len:
         return 1
+    shared = max(1, min(8, -(-512 // blocks), max_kv_len // 256))
     if eight:
         rows = n_heads * n_seqs * max_q_len
-        return min((s for s in range(1, 9) if s == 1 or (s * 256 <= max_kv_len and s * blocks <= 1024)),
+        return min((s for s in range(-(-shared // 2), 9) if s == 1 or (s * 256 <= max_kv_len and s * blocks <= 1024)),
                    key=lambda s: -(-blocks * s // 256) / s * max_kv_len / 128 * (1.2 if eight == 64 else 2.1) + (s > 1) * (6 + s * rows * eight * 4 / 2.8e6))
-    return max(1, min(8, -(-512 // blocks), max_kv_len // 256))
+    return shared
 
 
 PREFILL_TURNS = -2 ** 31              # ``attention_prefill``'s ``wide_from`` that names the kernel of turns
