@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import array
 import ctypes
+import functools
 from ctypes import c_float, c_int, c_long, c_uint32, c_void_p
 from typing import NamedTuple, Optional
 
@@ -2066,6 +2067,12 @@ PREFILL_SPLIT_KEYS = 1024            # keys that the longest sequence of a step 
 PREFILL_SPLIT_ROWS = 1024 * 128      # (token, head, split) rows that a step's splits never exceed
 
 
+@functools.lru_cache(maxsize=256)      # (all layers of a step ask the same: 8 us a layer of the host's time where portions of 250 tokens wait for it)
+def _eight_splits(blocks, rows, max_kv_len, head_dim, shared):
+    return min((s for s in range(-(-shared // 2), 9) if s == 1 or (s * 256 <= max_kv_len and s * blocks <= 1024)),
+               key=lambda s: -(-blocks * s // 256) / s * max_kv_len / 128 * (1.2 if head_dim == 64 else 2.1) + (s > 1) * (6 + s * rows * head_dim * 4 / 2.8e6))
+
+
 def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=0):
     """Blocks of 128 queries that share their keys out (``attention_prefill``'s ``splits``): for steps that bring few tokens behind
     a long context (a prompt in portions, the next turn of a dialogue), whose blocks are fewer than two for every CU and walk
@@ -2088,9 +2095,7 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=0):
         return 1
     shared = max(1, min(8, -(-512 // blocks), max_kv_len // 256))
     if eight:
-        rows = n_heads * n_seqs * max_q_len
-        return min((s for s in range(-(-shared // 2), 9) if s == 1 or (s * 256 <= max_kv_len and s * blocks <= 1024)),
-                   key=lambda s: -(-blocks * s // 256) / s * max_kv_len / 128 * (1.2 if eight == 64 else 2.1) + (s > 1) * (6 + s * rows * eight * 4 / 2.8e6))
+        return _eight_splits(blocks, n_heads * n_seqs * max_q_len, max_kv_len, eight, shared)
     return shared
 
 
