@@ -1503,8 +1503,8 @@ def sample(logits, work, temperature, top_p, uniform, out, step=None, uniform_st
 
 
 def sample_host(logits, work, parameters, out):
-    """``sample`` (or, with ``parameters`` None, ``argmax``) of every row, waited for: ``parameters``: three lists (or arrays of 32-bit
-    floats) of one number a row (temperatures, top-p, uniforms) in host memory; ``out``: int32 in pinned host memory, written when the call returns.
+    """``sample`` (or, with ``parameters`` None, ``argmax``) of every row, waited for: ``parameters``: three lists (or arrays; those of
+    32-bit floats are read where they lie) of one number a row (temperatures, top-p, uniforms) in host memory; ``out``: int32 in pinned host memory, written when the call returns.
     ``work``: ``sample_work_size`` floats and three a row."""
     _dev(logits, "logits", torch.float32, contiguous=False); _dev(work, "work", torch.float32)
     R, V = logits.shape
@@ -1516,7 +1516,9 @@ def sample_host(logits, work, parameters, out):
     if parameters is not None:
         if any(len(p) < R for p in parameters):
             raise KernelError("sample: argument sizes")
-        par = [(ctypes.c_float * R).from_buffer(p) if isinstance(p, array.array) else (ctypes.c_float * R)(*p[:R]) for p in parameters]
+        # (an array's own bytes where they are 32-bit floats; any other one's numbers are converted as a list's are)
+        par = [(ctypes.c_float * R).from_buffer(p) if isinstance(p, array.array) and p.typecode == "f" else (ctypes.c_float * R)(*p[:R])
+               for p in parameters]
     _check(library().gl3_sample_host(_ptr(logits), logits.stride(0), _ptr(work), *par, _ptr(out), R, V, _stream()), "sample")
 
 

@@ -66,3 +66,25 @@ def test_one_sampler_s_calls_of_several_threads_take_turns(monkeypatch):
         return all(sampler(torch.zeros(2 + k, 5), [1.0] * (2 + k), [0.9] * (2 + k), [k] * (2 + k)) == [k] * (2 + k) for _ in range(10))
     with ThreadPoolExecutor(4) as threads:
         assert all(threads.map(calls, range(4)))
+
+
+# (arrays of other numbers than 32-bit floats are converted as lists are, not read as if they were)
+@pytest.mark.parametrize("kinds", ["fff", "ddd", "fdl", "idd"])
+def test_a_call_s_numbers_come_in_arrays_of_any_kind(monkeypatch, kinds):
+    from array import array
+    from types import SimpleNamespace
+
+    import torch
+
+    from gpullama3_java_amd.csrc import lib
+    numbers = [[1] * 3 if kinds[0] == "i" else [0.8, 0.0, 1.3], [0.9, 1.0, 0.5], [0] * 3 if kinds[2] == "l" else [0.25, 0.1, 0.7]]
+    given = []
+    calls = SimpleNamespace(gl3_sample_work_floats=lambda rows, vocab: 0,
+                            gl3_sample_host=lambda logits, ld, work, t, p, u, *rest: given.append([list(t), list(p), list(u)]) or 0)
+    for name, stand_in in (("_dev", lambda *a, **kw: None), ("_ptr", lambda t: None), ("_stream", lambda: None), ("library", lambda: calls)):
+        monkeypatch.setattr(lib, name, stand_in)
+    out = SimpleNamespace(numel=lambda: 2, dtype=torch.int32, is_contiguous=lambda: True, is_pinned=lambda: True)
+    for par in (numbers, [array(k, n) for k, n in zip(kinds, numbers)]):
+        lib.sample_host(torch.zeros(2, 9), torch.zeros(300), par, out)
+    want = [np.float32(n[:2]).tolist() for n in numbers]               # (a call of two rows takes two numbers each)
+    assert given == [want, want]
