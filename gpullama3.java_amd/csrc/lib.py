@@ -2142,7 +2142,9 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
     elif block_table.shape[0] < B:
         raise KernelError("attention: the block table has fewer rows than there are sequences")
     has_sink, sink_value, sinks = _sink(sink, n_heads, "attention_prefill")
-    if splits > 1 and eight_splits is not None:
+    # (the kernel of eight waves takes a step in splits where it is built for its sizes, no mask but the causal one, and caches at 16-byte addresses)
+    if (splits > 1 and eight_splits is not None and head_dim in (64, 128) and page_size % 64 == 0 and not window and not chunk
+            and n_v == n_kv and slopes is None and sink is None and rule is None and (k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0):
         splits = int(eight_splits)
     if splits > 1:
         _dev(part_o, "part_o", torch.float32); _dev(part_ml, "part_ml", torch.float32)

@@ -33,6 +33,30 @@ def test_splits_of_its_blocks():
                     assert 2 * n >= lib.prefill_splits(heads, n_seqs, T, [100000] * n_seqs, T + 100000)      # (a maximum a group: no fewer than on the other kernel)
 
 
+@pytest.mark.parametrize("more, taken", [({}, True), (dict(head_dim=64), True), (dict(page_size=192), True), (dict(page_size=96), False), (dict(head_dim=96), False),
+                                         (dict(window=100), False), (dict(chunk=64), False), (dict(sink=0.5), False), (dict(n_v_heads=1), False), (dict(at=4), False)])
+def test_its_splits_are_for_its_calls_alone(monkeypatch, more, taken):
+    """``eight_splits`` stands in for ``splits`` where the kernel of eight waves runs: not with another mask, other sizes, or caches between 16-byte addresses."""
+    from types import SimpleNamespace
+
+    import torch
+    given = []
+    calls = SimpleNamespace(gl3_attention_prefill=lambda *a: given.append(a[-5]) or 0)
+    for name, stand_in in (("_dev", lambda *a, **kw: None), ("_ptr", lambda t: None), ("_stream", lambda: None), ("library", lambda: calls)):
+        monkeypatch.setattr(lib, name, stand_in)
+    kw = dict(head_dim=128, page_size=64, window=None, at=0) | more
+    hs, page, window, at = (kw.pop(name) for name in ("head_dim", "page_size", "window", "at"))
+
+    def cache(heads, *tile):
+        return torch.empty(heads * hs * page + 8, dtype=torch.bfloat16)[at:at + heads * hs * page].view(1, heads, *tile)
+    q, out = torch.zeros(3, 2 * hs), torch.zeros(3, 2 * hs)
+    i32 = torch.zeros(2, dtype=torch.int32)
+    for n in (1, 2):
+        lib.attention_prefill(q, cache(2, page, hs), cache(kw.get("n_v_heads", 2), hs, page), i32, i32[:1], i32.view(2, 1), out, 3, 2, 2, hs, page, window, 0.1,
+                              splits=3, part_o=torch.zeros(18 * hs), part_ml=torch.zeros(36), eight_splits=n, **kw)
+        assert given.pop() == (n if taken else 3)
+
+
 # one, two, three and four heads a kv head; waves, blocks and chunks with one row and all but one, one chunk (none for the second group); sequences that start no
 # block of the longest one's kind; more chunks than a register holds places of (64), twice as many
 CASES = [(4, 2, 64, [0, 70, 0, 130, 5], [33, 1, 200, 17, 64]), (3, 1, 64, [0, 0, 0], [256, 257, 31]), (8, 2, 128, [63, 64, 65], [129, 128, 127]),
