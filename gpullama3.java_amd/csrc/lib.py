@@ -2096,9 +2096,13 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=0):
     if blocks >= 512 or max_kv_len < PREFILL_SPLIT_KEYS or not kv_before or min(kv_before) < max_q_len:
         return 1
     shared = max(1, min(8, -(-512 // blocks), max_kv_len // 256))
-    if eight:
-        return _eight_splits(blocks, n_heads * n_seqs * max_q_len, max_kv_len, eight, shared)
-    return shared
+    return eight_splits(shared, n_heads, n_seqs, max_q_len, max_kv_len, eight) if eight else shared
+
+
+def eight_splits(shared, n_heads, n_seqs, max_q_len, max_kv_len, head_dim):
+    """``prefill_splits`` on the kernel of eight waves, where ``shared`` is what it says for the other one (a layer asks for both, and goes over the
+    sequences' contexts once)."""
+    return _eight_splits(n_heads * n_seqs * -(-max_q_len // 128), n_heads * n_seqs * max_q_len, max_kv_len, head_dim, shared)
 
 
 PREFILL_TURNS = -2 ** 31              # ``attention_prefill``'s ``wide_from`` that names the kernel of turns

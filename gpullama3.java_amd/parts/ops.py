@@ -566,7 +566,7 @@ def attention(ctx, q, k_cache, v_cache, block_table, out, n_heads, n_kv, head_di
                 if part_o is not None:
                     extras.update(splits=splits, part_o=part_o, part_ml=part_ml)
                     if head_dim in (64, 128) and page % 64 == 0:
-                        extras["eight_splits"] = K.prefill_splits(n_heads, ctx.n_seqs, ctx.max_q_len, ctx.kv_before_host, ctx.max_kv_len, eight=head_dim)
+                        extras["eight_splits"] = K.eight_splits(splits, n_heads, ctx.n_seqs, ctx.max_q_len, ctx.max_kv_len, head_dim)
         return K.attention_prefill(q, k_cache, v_cache, ctx.cu_seqlens, ctx.kv_before, block_table, out,
                                    ctx.max_q_len, n_heads, n_kv, head_dim, page, window, scale,
                                    seq_rows=getattr(ctx, "seq_rows", None), **extras)

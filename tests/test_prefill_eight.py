@@ -57,6 +57,31 @@ def test_its_splits_are_for_its_calls_alone(monkeypatch, more, taken):
         assert given.pop() == (n if taken else 3)
 
 
+# (no splits at all, where the other kernel has two; fewer; not its sizes: none of its own)
+@pytest.mark.parametrize("heads, hs, page, T, before, eight", [(32, 64, 64, 1000, 6000, 1), (24, 128, 128, 512, 3584, 5), (32, 64, 64, 150, 3000, 4), (32, 64, 96, 512, 512, None),
+                                                               (32, 96, 64, 512, 512, None)])
+def test_a_layer_asks_for_its_splits(monkeypatch, heads, hs, page, T, before, eight):
+    from types import SimpleNamespace
+
+    import torch
+
+    from gpullama3_java_amd.parts import ops
+    walks = []
+
+    class Contexts(list):
+        def __iter__(self):
+            walks.append(1)
+            return super().__iter__()
+    ctx = SimpleNamespace(n_seqs=1, max_q_len=T, max_kv_len=T + before, kv_before_host=Contexts([before]), cu_seqlens=None, kv_before=None,
+                          buffer_if_room=lambda name, shape, dtype: torch.empty(shape, dtype=dtype, device="meta"))
+    calls = []
+    monkeypatch.setattr(ops, "attention_kernel", lambda *a: "prefill")
+    monkeypatch.setattr(lib, "attention_prefill", lambda *a, **kw: calls.append((kw["splits"], kw.get("eight_splits"))))
+    ops.attention(ctx, torch.zeros(1), torch.zeros(1, 8, page, hs), None, None, None, heads, 8, hs, None, 0.1)
+    assert calls == [(lib.prefill_splits(heads, 1, T, [before], T + before), eight)] and len(walks) == 1
+    assert eight in (None, lib.prefill_splits(heads, 1, T, [before], T + before, eight=hs))
+
+
 # one, two, three and four heads a kv head; waves, blocks and chunks with one row and all but one, one chunk (none for the second group); sequences that start no
 # block of the longest one's kind; more chunks than a register holds places of (64), twice as many
 CASES = [(4, 2, 64, [0, 70, 0, 130, 5], [33, 1, 200, 17, 64]), (3, 1, 64, [0, 0, 0], [256, 257, 31]), (8, 2, 128, [63, 64, 65], [129, 128, 127]),
