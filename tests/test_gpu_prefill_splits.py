@@ -22,7 +22,8 @@ def fn(lens_before, new, splits):
 
 # contexts of fewer chunks than splits, of one page, long ones; last blocks of one query and of 128
 @pytest.mark.parametrize("splits", [2, 3, 8])
-@pytest.mark.parametrize("H, Kh, hs, page", [(4, 2, 32, 64), (6, 2, 64, 64), (2, 1, 64, 96), (5, 5, 96, 32), (3, 1, 128, 64)])
+@pytest.mark.parametrize("H, Kh, hs, page", [(4, 2, 32, 64), (6, 2, 64, 64), (2, 1, 64, 96), (5, 5, 96, 32), (3, 1, 128, 64),
+                                             (3, 1, 128, 32), (4, 2, 128, 96)])
 def test_split_prefill_attention(H, Kh, hs, page, splits):
     rng = np.random.default_rng(H * hs + splits)
     before, new = [700, 0, 129, 1300, 31], [40, 3, 129, 1, 256]
@@ -31,6 +32,26 @@ def test_split_prefill_attention(H, Kh, hs, page, splits):
     np.testing.assert_allclose(got, ref, atol=1e-2 * np.abs(ref).max())
     whole, _ = run_attention(fn(before, new, 1), sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1), page=page)
     np.testing.assert_allclose(got, whole, atol=2.0 ** -7 * np.abs(ref).max())       # (weights are rounded to 16 bits around another maximum)
+
+
+# pages of 64: as many splits as the second number says, none for 1; of 96, and caches between 16-byte addresses: as the first says
+@pytest.mark.parametrize("hs, page, shift, taken", [(64, 64, 0, True), (128, 64, 0, True), (128, 96, 0, False), (64, 64, 4, False)])
+@pytest.mark.parametrize("eight", [1, 2, 5])
+def test_a_number_of_splits_for_the_kernel_of_eight_waves(hs, page, shift, taken, eight):
+    H, Kh, before, new = 4, 2, [1300], [200]
+    sk, sv, qs = attention_case(np.random.default_rng(hs + eight), H, Kh, hs, before, new, "bfloat16")
+
+    def run(**kw):
+        def call(q, kc, vc, positions, seq_of, table, out, *rest):
+            moved = [torch.empty(c.numel() + 8, dtype=c.dtype, device=DEV)[shift:shift + c.numel()].view(c.shape).copy_(c) for c in (kc, vc)]
+            n = 5 * 200 * H
+            part_o, part_ml = torch.full((n * hs,), float("nan"), device=DEV), torch.full((2 * n,), float("nan"), device=DEV)
+            K().attention_prefill(q, *moved, dev([0, 200], torch.int32), dev(before, torch.int32), table, out, 200, *rest, part_o=part_o, part_ml=part_ml, **kw)
+        return run_attention(call, sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1), page=page)
+    got, ref = run(splits=4, eight_splits=eight)
+    np.testing.assert_allclose(got, ref, atol=1e-2 * np.abs(ref).max())
+    np.testing.assert_array_equal(got, run(splits=eight if taken else 4)[0])
+    assert not np.array_equal(got, run(splits=4 if taken and eight != 4 else 3)[0])
 
 
 def test_split_prefill_attention_with_one_key_that_counts_and_a_window():

@@ -30,6 +30,45 @@ def test_the_call_from_host_memory(rows):
     assert sampler(logits, [0.0] * rows, par[1], par[2]) == host.argmax(1).tolist()
 
 
+@pytest.mark.parametrize("temperature", [0.8, 0.0])
+def test_a_call_behind_longer_work_than_it_looks_for(temperature):
+    """Some 10 ms of products are in front of it on the stream, where it looks for its tokens for half a millisecond and then waits for the stream."""
+    rng = np.random.default_rng(4)
+    logits = torch.tensor(3 * rng.standard_normal((8, 1031)), dtype=torch.float32, device="cuda:0")
+    par = ([temperature] * 8, [0.9] * 8, rng.random(8).tolist())
+    sampler = DeviceSampler(torch.device("cuda:0"))
+    want = sampler(logits, *par)
+    other = torch.randn(8192, 8192, device="cuda:0")
+    torch.cuda.synchronize()
+    for _ in range(3):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        late = torch.zeros_like(logits)
+        begin.record()
+        product = other @ other
+        late.copy_(logits)                                              # (the logits themselves come late)
+        end.record()
+        got = sampler(late, *par)
+        assert end.query() and begin.elapsed_time(end) > 1.0            # (all in front of it is done; it took longer than the look)
+        assert got == want
+        del product
+
+
+@pytest.mark.parametrize("greedy", [False, True])
+def test_tokens_of_an_earlier_call_are_not_taken_for_this_one_s(greedy):
+    logits = torch.zeros(2, 3, 1031, device="cuda:0")
+    places = torch.tensor([[5, 700, 1030], [6, 0, 44]])
+    for call in range(2):
+        logits[call, torch.arange(3), places[call]] = 60.0
+    work = torch.empty(lib.sample_work_size(3, 1031) + 9, device="cuda:0")
+    pinned = torch.empty(3, dtype=torch.int32, pin_memory=True)
+    other = torch.randn(2048, 2048, device="cuda:0")
+    for call in (0, 1, 0, 1):
+        for _ in range(2):
+            other @ other                                               # (so that the tokens are not there at the first look)
+        lib.sample_host(logits[call], work, None if greedy else [[0.7] * 3, [0.9] * 3, [0.5] * 3], pinned)
+        assert pinned.tolist() == places[call].tolist()
+
+
 def test_the_call_from_host_memory_refuses():
     logits = torch.zeros(2, 50, device="cuda:0")
     work = torch.empty(lib.sample_work_size(2, 50) + 6, device="cuda:0")

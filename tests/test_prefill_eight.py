@@ -126,6 +126,28 @@ def test_scores_that_are_not_numbers_are_in_the_rows_that_see_them(hs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hs", [64, 128])
+@pytest.mark.parametrize("at", [0, 31, 32, 63, 64, 95, 127, 1000, 1023, 1024, 1037, 1038, 1055, 1060])
+def test_values_that_are_not_finite_reach_as_far_as_in_the_kernel_of_128_queries(at, hs):
+    """An infinite value or a NaN spoils the queries that share their 64 keys with it (heads of 64; of 128: 32 keys), in front of it or behind the sequence's end
+    (here from 1,038 on), and no others; on two groups of keys both that hold it and that do not."""
+    from test_gpu_kernels import attention_case, run_attention
+    H, Kh, before, new = 4, 2, [700], [338]
+    sk, sv, qs = attention_case(np.random.default_rng(at), H, Kh, hs, before, [400], "bfloat16")
+    keys = 64 if hs == 64 else 32
+    positions = np.arange(700, 1038)
+    last = np.minimum((positions - 700 >> 5) * 32 + 731, 1037)       # (32 queries walk their keys together)
+    for value in (np.inf, np.nan):
+        sv[0][at, 0, 57] = value
+        run = lambda f: run_attention(f, sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1))[0]
+        by_heads, by_keys = run(fn(before, new, lib.PREFILL_HEADS)), run(fn(before, new, lib.PREFILL_KEYS))
+        np.testing.assert_array_equal(by_heads, run(fn(before, new, 1)))
+        for got in (by_heads, by_keys):
+            assert np.isfinite(got[last // keys < at // keys]).all() and np.isfinite(got[:, :, :57]).all() and np.isfinite(got[:, 2:]).all()
+            assert not np.isfinite(got[positions >= at, :2, 57]).any()
+
+
+@pytest.mark.gpu
 def test_it_refuses_what_it_is_not_built_for():
     from test_gpu_kernels import K, attention_case, run_attention
     before, new = [0], [40]
