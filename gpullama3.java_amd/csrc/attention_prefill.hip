@@ -951,7 +951,7 @@ __global__ __launch_bounds__(512, HS == 64 ? 4 : 2) void attention_prefill_eight
     const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ cu_seqlens, const int* __restrict__ kv_before, const int* __restrict__ block_table,
     const int* __restrict__ seq_rows, int table_stride, bf16_t* __restrict__ out, long out_stride, int n_heads, int n_kv, int page_size,
-    float scale, int q_blocks, int folded, PfSplit sp) {
+    float scale, int q_blocks, int folded, int n_seqs, PfSplit sp) {
   static_assert(!SPLIT || GROUPS == 2, "splits are for few blocks");
   constexpr int CK = 64, KS = HS / 16, DT = HS / 32, QB = 128, HEADS = GROUPS == 2 ? 1 : 2;
   constexpr int KB = CK * HS * 2;                  // bytes of a chunk's keys (and of its values)
@@ -968,6 +968,7 @@ __global__ __launch_bounds__(512, HS == 64 ? 4 : 2) void attention_prefill_eight
   const int c = at % n_kv;                         // (blocks of one kv head are n_kv apart: on one XCD where n_kv is 8)
   const int head = c * g + at / n_kv * HEADS + (HEADS == 2 ? group : 0);
   const int n = lane & 31, h = lane >> 5;
+  if (b >= n_seqs) return;                         // (a row of the grid that is no sequence's)
   const int tok0 = __builtin_amdgcn_readfirstlane(cu_seqlens[b]);
   const int q_len = __builtin_amdgcn_readfirstlane(cu_seqlens[b + 1]) - tok0;
   if (qb * QB >= q_len) return;                    // the whole block: no barrier has been passed yet
@@ -1332,11 +1333,15 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
   if (kernel >= 3 || (kernel == 1 && splits > 1 && splits_plain && eight_takes(head_dim, page_size))) {
     const int heads = kernel == 4 ? 2 : 1;
     const bool folded = n_seqs == 1 && (long)n_heads / heads * q_blocks * splits <= 512;
-    dim3 egrid((unsigned)(n_heads / heads * splits), n_seqs, q_blocks);
+    // Blocks beyond their sequence's end leave at once. The blocks of an XCD go to its four engines in turn, so where an even number of sequences has one
+    // that is far longer than the others, its blocks would meet the same engines again and again: one row more of blocks that leave (16 heads of 128: 3,502 tokens beside
+    // three of 17 127 us, so 73; two heads a block 213 and 107).
+    const bool uneven = n_seqs % 2 == 0 && 10L * n_tokens < 7L * n_seqs * max_q_len;
+    dim3 egrid((unsigned)(n_heads / heads * splits), n_seqs + uneven, q_blocks);
 #define GOE(HS, GROUPS, SPLIT)                                                                                        \
   attention_prefill_eight_kernel<HS, GROUPS, SPLIT><<<egrid, dim3(512), 0, stream>>>(                                            \
       (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu_seqlens, kv_before, block_table, \
-      seq_rows, table_stride, (bf16_t*)out, out_stride, n_heads, n_kv, page_size, scale, q_blocks, (int)folded, sp)
+      seq_rows, table_stride, (bf16_t*)out, out_stride, n_heads, n_kv, page_size, scale, q_blocks, (int)folded, n_seqs, sp)
 #define GOEH(HS)                                                                                                      \
   do {                                                                                                                \
     if (splits > 1) {                                                                                                 \

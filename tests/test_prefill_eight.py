@@ -148,6 +148,37 @@ def test_values_that_are_not_finite_reach_as_far_as_in_the_kernel_of_128_queries
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode", [lib.PREFILL_KEYS, lib.PREFILL_HEADS])
+@pytest.mark.parametrize("beside", [1, 3])
+def test_short_sequences_beside_a_long_one_do_not_make_it_longer(beside, mode):
+    """Blocks that leave at once, of sequences that are over, do not send the others to half of the chip (with three short ones that was 1.5 and 2.0 times the
+    time of the long one alone, whose blocks are paired otherwise: 1.0 and less since)."""
+    import torch
+    H, Kh, hs, long = 16, 8, 128, 3502
+
+    def least(new):
+        T, pages = sum(new), [-(-n // 64) for n in new]
+        q, out = torch.randn(T, H * hs, device="cuda").bfloat16(), torch.empty(T, H * hs, dtype=torch.bfloat16, device="cuda")
+        kc, vc = (torch.randn(sum(pages), Kh, *size, device="cuda").bfloat16() for size in ((64, hs), (hs, 64)))
+        table = torch.zeros(len(new), max(pages), dtype=torch.int32)
+        for b, n in enumerate(pages):
+            table[b, :n] = torch.arange(n) + sum(pages[:b])
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+        cu, held, table = i32([sum(new[:b]) for b in range(len(new) + 1)]), i32([0] * len(new)), table.cuda()
+        times = []
+        for _ in range(12):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(8):
+                lib.attention_prefill(q, kc, vc, cu, held, table, out, max(new), H, Kh, hs, 64, None, 0.1, wide_from=mode)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+    assert least([long] + [17] * beside) < 1.25 * least([long])
+
+
+@pytest.mark.gpu
 def test_it_refuses_what_it_is_not_built_for():
     from test_gpu_kernels import K, attention_case, run_attention
     before, new = [0], [40]
