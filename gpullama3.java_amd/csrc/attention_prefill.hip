@@ -1224,38 +1224,54 @@ static bool turns_wanted(int n_seqs, int max_q_len, int n_tokens) {
   return max_q_len >= 1024 && (n_tokens <= 5L * max_q_len || n_tokens >= 1280L * n_seqs);
 }
 
-// Whether the library takes the kernel of eight waves. 3: with two groups on the keys, 4: with two heads a block, 0: another kernel (`plain` as below).
-// Heads of 64: two groups where its blocks of one head are at most 1,100 (two are on each CU at a time), else two heads a
-// block (32 heads: one sequence of 4,096 tokens, 1,040 blocks, 89.1 and 92.7 us, of 6,000 180 and 182; eight of 512, 1,152 blocks, 23.1 and 21.3, 32 of 256
-// 34.6 and 29.5). An odd number of heads a kv head has no pairs: two groups there too, but for many short sequences, where the kernel
-// of 128 queries is as fast or faster (24 heads over 8: sixteen of 146 to 336 tokens 14.7 against 13.4 us).
-// Heads of 128, one block on a CU at a time: two groups from 300 tokens of the longest sequence on (256 tokens 11.6 us, 10.9 with 64 queries a block;
-// 333 11.9 and 12.5) to 512 blocks of one sequence, or of a longest one with half of the tokens, to 256 of others (24 heads: 2,048 tokens, 408 blocks, 52 us
-// where turns take 57 and 64 queries a block 62, 3,000, 576 blocks, 84 and 80; 32 heads: three of 300 behind 1,000, 288 equal blocks, 51 and 46). Two heads a
-// block where the kernel of 128 queries would have them, for sequences of 384 tokens on average and more (32 heads: eight of 512 45.2 -> 38.5 us,
-// four of 1,000 58.8 -> 51.6, 32 of 256 59.6 and 67.6).
+// The library's choice where it is not the kernel of eight waves (below): 0: 64 queries a block, 1: 128, 2: the kernel of turns. plain: the plain rule (one score map, no window, chunked
+// mask, bias, sink, kept keys, cap, temperature or gate), no splits, caches at 16-byte addresses (its loads into shared memory bring
+// 16 bytes a lane and want them aligned, where the other kernels' ordinary loads do not).
+extern "C" int gl3_prefill_kernel(int head_dim, int page_size, int n_heads, int n_kv, int n_seqs, int max_q_len, int n_tokens, int plain) {
+  if (!prefill_wide(head_dim, n_heads, n_seqs, max_q_len)) return 0;
+  return plain && turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && turns_wanted(n_seqs, max_q_len, n_tokens) ? 2 : 1;
+}
+
+// Whether the library takes the kernel of eight waves. 3: with two groups on the keys, 4: with two heads a block, 0: another kernel (`plain` as above).
+// All that is known here are the sequences, the longest and the tokens together. Two groups halve a block's way along its keys, which is what a step waits
+// for where its blocks are few or one sequence is far longer than the others; two heads a block read half as many keys and values, which pays where many blocks are
+// left behind the longest. Measured in every form and on the kernels beside it: 5,843 batches (one sequence, equal and unequal ones, one or two long ones beside
+// short ones; 33 to 20,000 tokens) with 16 to 64 heads over 8, 16 over 16 and 32 over 32, of which the limits are, and 3,600 others
+// (`profiles/prefill_eight_rule.txt`): at the others, time against the kernel that would be taken without this one, heads of 64 0.846 on average (0.840 with the best
+// form everywhere), of 128 0.962 (0.942); above 1.05 of it 3 of them, and 12 of sequences of at most 64 tokens.
+// Heads of 64, two blocks a CU at a time. Even numbers of heads a kv head: two heads a block for more than 1,100 blocks of one head, or 400 where the step holds
+// five and a half times its longest sequence (32 heads: 4,096 tokens, 1,056 blocks, 86.2 us in two groups and 90.7, 8,192 304 and 293; six of 300 15.5
+// and 13.1, 14.3 with 128 queries a block); for sequences of unequal lengths more (1,300 tokens beside twenty of 100 25.0 and 37.9, 34.5). Odd numbers
+// have no pairs: two groups but for many short sequences (24 heads: eight of 300 15.7, with 128 queries a block 14.0; six of 1,000 36.5 and 41.9).
+// Heads of 128, one block on a CU at a time: two groups from 300 tokens of the longest sequence on (280 tokens 12.9 us, 11.9 with 64 queries a block; 320
+// 12.9 and 13.5) to 511 blocks of one sequence, 320 of a short one (24 heads: 2,600 tokens 76 us, with 64 queries a block 101; 32 heads: 2,000 tokens 63.3, with
+// turns 58.3; 64 heads: 646 tokens 29.5, with 64 queries 27.7), 512 where the longest has half of the tokens, 256 of others (24 heads: 1,203 beside 317 and
+// 701 35.8, with turns 38.7). Two heads a block where the kernel of 128 queries would have them, for 384 tokens a sequence on average and more, of equal length with little of
+// their last block empty (a block that is partly empty has its CU for as long; 32 heads: eight of 512 45.9 -> 40.3, ten of 450 43.3 and 46.3), or few (32 heads: 822 tokens
+// beside 1,102 of three others 40.4 -> 34.6); with eight heads a kv head unequal ones too (64 heads: 24 of 14,348 tokens, the longest 1,641, 0.90 of the time).
 #define PF_KEYS (INT_MIN + 1)
 #define PF_HEADS (INT_MIN + 2)
 static bool eight_takes(int head_dim, int page_size) { return (head_dim == 64 || head_dim == 128) && page_size % 64 == 0; }
 extern "C" int gl3_prefill_eight(int head_dim, int page_size, int n_heads, int n_kv, int n_seqs, int max_q_len, int n_tokens, int plain) {
   if (!plain || !eight_takes(head_dim, page_size)) return 0;
   const int group = n_heads / n_kv;
-  const long blocks = (long)n_heads * (n_tokens / 128 + (n_seqs + 1) / 2);
+  const bool pairs = group % 2 == 0;
+  const long blocks = (long)n_heads * (n_tokens / 128 + (n_seqs + 1) / 2);      // of one head: about as many as there are
+  const long most = max_q_len, tokens = n_tokens, padded = most * n_seqs;
   if (head_dim == 64) {
     if (max_q_len <= 32) return 0;
-    if (group % 2 == 0) return blocks <= 1100 ? 3 : 4;
-    return blocks <= 512 || n_tokens >= 256L * n_seqs ? 3 : 0;
+    if (!pairs) return blocks <= 400 || tokens <= 6 * most || (tokens >= 330L * n_seqs && blocks >= 1080) ? 3 : 0;
+    if (10 * tokens >= 7 * padded) return blocks > 1100 || (2 * tokens >= 11 * most && blocks > 400) ? 4 : 3;
+    if (tokens >= 9 * most) return blocks > 1100 ? 4 : blocks <= 400 ? 3 : 0;
+    return blocks > 1800 && tokens >= 5 * most ? 4 : 3;
   }
-  if (max_q_len >= 300 && blocks <= (n_seqs == 1 || n_tokens <= 2L * max_q_len ? 512 : 256)) return 3;
-  return group % 2 == 0 && n_tokens >= 384L * n_seqs && prefill_wide(head_dim, n_heads, n_seqs, max_q_len) && !turns_wanted(n_seqs, max_q_len, n_tokens) ? 4 : 0;
-}
-
-// The library's choice where that is not it: 0: 64 queries a block, 1: 128, 2: the kernel of turns. plain: the plain rule (one score map, no window, chunked
-// mask, bias, sink, kept keys, cap, temperature or gate), no splits, caches at 16-byte addresses (its loads into shared memory bring
-// 16 bytes a lane and want them aligned, where the other kernels' ordinary loads do not).
-extern "C" int gl3_prefill_kernel(int head_dim, int page_size, int n_heads, int n_kv, int n_seqs, int max_q_len, int n_tokens, int plain) {
-  if (!prefill_wide(head_dim, n_heads, n_seqs, max_q_len)) return 0;
-  return plain && turns_takes(head_dim, page_size, n_heads / n_kv, n_seqs, n_tokens) && turns_wanted(n_seqs, max_q_len, n_tokens) ? 2 : 1;
+  if (max_q_len >= 300) {
+    const long longest = n_heads * ((most + 127) / 128);
+    if (n_seqs == 1 ? longest <= (most >= 700 ? 511 : 320) : blocks <= (tokens <= 2 * most ? 512 : 256)) return 3;
+  }
+  if (!pairs || tokens < 384L * n_seqs || gl3_prefill_kernel(head_dim, page_size, n_heads, n_kv, n_seqs, max_q_len, n_tokens, plain) != 1) return 0;
+  const bool filled = 10 * tokens >= 9 * padded && (most % 128 == 0 || most % 128 >= 96);
+  return group % 8 == 0 || (5 * tokens <= 16 * most && blocks <= 700) || (filled && blocks <= 2200) ? 4 : 0;
 }
 
 extern "C" int gl3_attention_prefill_supports(int head_dim, int page_size) {

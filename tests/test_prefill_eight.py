@@ -18,6 +18,23 @@ def test_which_calls_take_it():
     assert choice([512] * 8, hs=128) == 4 and choice([1000] * 4, hs=128) == 4 and choice([256] * 32, hs=128) == 0 and choice([8192], hs=128) == 0
 
 
+def test_sequences_of_unequal_lengths_and_last_blocks_that_are_partly_empty():
+    """Not the form that takes longer than the kernel beside it: two heads a block where one sequence's way is what the step waits for, rounds of few blocks."""
+    def choice(lengths, heads=32, n_kv=8, hs=64):
+        return lib.library().gl3_prefill_eight(hs, 64, heads, n_kv, len(lengths), max(lengths), sum(lengths), 1)
+    # two heads a block where the step is several times its longest sequence
+    assert choice([1300] + [100] * 20) == 3 and choice([2000] + [800] * 5) == 3 and choice([1000] * 8) == 4 and choice([300] * 6) == 4 and choice([40] * 32) == 4
+    assert choice([1000] * 4) == 3 and choice([600] + [200] * 40) == 4 and choice([300] * 10 + [80] * 10, 16) == 0
+    # no pairs of heads
+    assert choice([300] * 8, 24) == 0 and choice([300] * 12, 16, 16) == 0 and choice([384] * 12, 24) == 0 and choice([1000] * 6, 24) == 3
+    assert choice([1300] + [100] * 20, 24) == 3 and choice([1469] * 8, 24) == 3
+    large = dict(hs=128)
+    assert choice([2000], **large) == choice([2048], **large) == 0 and choice([1900], **large) == 3 and choice([650], 64, **large) == 0 and choice([640], 64, **large) == 3
+    assert choice([3502, 20, 20, 20], 16, **large) == 3 and choice([700, 200, 200, 200], **large) == 3 and choice([512] * 16, **large) == 0
+    assert choice([840, 808, 583, 140, 802, 45, 398, 400], **large) == 0 and choice([1641] + [500] * 23, **large) == 0
+    assert choice([427] * 8, **large) == 0 and choice([822, 600, 300, 202], **large) == 4 and choice([427] * 8, 64, **large) == 4
+
+
 def test_splits_of_its_blocks():
     def s(heads, n_seqs, T, before, hs=64):
         return lib.prefill_splits(heads, n_seqs, T, [before] * n_seqs, T + before, eight=hs)
