@@ -1241,14 +1241,14 @@ extern "C" int gl3_prefill_kernel(int head_dim, int page_size, int n_heads, int 
 // form everywhere), of 128 0.962 (0.942); above 1.05 of it 3 of them, and 12 of sequences of at most 64 tokens.
 // Heads of 64, two blocks a CU at a time. Even numbers of heads a kv head: two heads a block for more than 1,100 blocks of one head, or 400 where the step holds
 // five and a half times its longest sequence (32 heads: 4,096 tokens, 1,056 blocks, 86.2 us in two groups and 90.7, 8,192 304 and 293; six of 300 15.5
-// and 13.1, 14.3 with 128 queries a block); for sequences of unequal lengths more (1,300 tokens beside twenty of 100 25.0 and 37.9, 34.5). Odd numbers
+// and 13.1, 14.3 with 128 queries a block); for sequences of unequal lengths more (1,300 tokens beside twenty of 100 28.2 and 43.4, 34.3). Odd numbers
 // have no pairs: two groups but for many short sequences (24 heads: eight of 300 15.7, with 128 queries a block 14.0; six of 1,000 36.5 and 41.9).
 // Heads of 128, one block on a CU at a time: two groups from 300 tokens of the longest sequence on (280 tokens 12.9 us, 11.9 with 64 queries a block; 320
 // 12.9 and 13.5) to 511 blocks of one sequence, 320 of a short one (24 heads: 2,600 tokens 76 us, with 64 queries a block 101; 32 heads: 2,000 tokens 63.3, with
 // turns 58.3; 64 heads: 646 tokens 29.5, with 64 queries 27.7), 512 where the longest has half of the tokens, 256 of others (24 heads: 1,203 beside 317 and
 // 701 35.8, with turns 38.7). Two heads a block where the kernel of 128 queries would have them, for 384 tokens a sequence on average and more, of equal length with little of
 // their last block empty (a block that is partly empty has its CU for as long; 32 heads: eight of 512 45.9 -> 40.3, ten of 450 43.3 and 46.3), or few (32 heads: 822 tokens
-// beside 1,102 of three others 40.4 -> 34.6); with eight heads a kv head unequal ones too (64 heads: 24 of 14,348 tokens, the longest 1,641, 0.90 of the time).
+// beside 1,102 of three others 40.7 -> 35.1); with eight heads a kv head unequal ones too (64 heads: 24 of 14,348 tokens, the longest 1,641, 430 -> 392).
 #define PF_KEYS (INT_MIN + 1)
 #define PF_HEADS (INT_MIN + 2)
 static bool eight_takes(int head_dim, int page_size) { return (head_dim == 64 || head_dim == 128) && page_size % 64 == 0; }
@@ -1281,7 +1281,8 @@ extern "C" int gl3_attention_prefill_supports(int head_dim, int page_size) {
 // max_q_len: the most tokens any sequence brings in this step (it sizes the grid).
 // seq_rows (may be null): the row of `block_table` that holds sequence b's pages; null: row b.
 // wide_from: the kernel with 128 queries a block is taken when max_q_len reaches it; <= 0: the library's choice, but for PF_TURNS: the
-// kernel of turns, and PF_KEYS, PF_HEADS: the kernel of eight waves in two groups on the keys, or on two heads.
+// kernel of turns, and PF_KEYS, PF_HEADS: the kernel of eight waves in two groups on the keys, or on two heads. Splits: above 0 the kernel of 128 queries,
+// else that of eight waves where it is built for the call.
 extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k_cache, const void* v_cache,
                                      const int* cu_seqlens, const int* kv_before, const int* block_table,
                                      const int* seq_rows, int table_stride, void* out, long out_stride, int n_seqs,
@@ -1346,7 +1347,7 @@ extern "C" int gl3_attention_prefill(const void* q, long q_stride, const void* k
     GL3_LAUNCH_CHECK();
     return 0;
   }
-  if (kernel >= 3 || (kernel == 1 && splits > 1 && splits_plain && eight_takes(head_dim, page_size))) {
+  if (kernel >= 3 || (splits > 1 && wide_from <= 0 && splits_plain && eight_takes(head_dim, page_size))) {
     const int heads = kernel == 4 ? 2 : 1;
     const bool folded = n_seqs == 1 && (long)n_heads / heads * q_blocks * splits <= 512;
     // Blocks beyond their sequence's end leave at once. The blocks of an XCD go to its four engines in turn, so where an even number of sequences has one

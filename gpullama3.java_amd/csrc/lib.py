@@ -2096,13 +2096,26 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=0):
     if blocks >= 512 or max_kv_len < PREFILL_SPLIT_KEYS or not kv_before or min(kv_before) < max_q_len:
         return 1
     shared = max(1, min(8, -(-512 // blocks), max_kv_len // 256))
-    return eight_splits(shared, n_heads, n_seqs, max_q_len, max_kv_len, eight) if eight else shared
+    return _eight_splits(blocks, n_heads * n_seqs * max_q_len, max_kv_len, eight, shared) if eight else shared
 
 
+@functools.lru_cache(maxsize=256)
 def eight_splits(shared, n_heads, n_seqs, max_q_len, max_kv_len, head_dim):
-    """``prefill_splits`` on the kernel of eight waves, where ``shared`` is what it says for the other one (a layer asks for both, and goes over the
-    sequences' contexts once)."""
-    return _eight_splits(n_heads * n_seqs * -(-max_q_len // 128), n_heads * n_seqs * max_q_len, max_kv_len, head_dim, shared)
+    """``prefill_splits`` on the kernel of eight waves, where ``shared`` is what it says for the kernel of 128 queries; 0: that one in ``shared`` splits takes
+    no longer. (A layer asks for both, and goes over the sequences' contexts once.) Heads of 128 have one block on a CU where the other kernel has two, so that
+    a last round of few blocks costs twice as much: 24 heads, 300 tokens behind 1,500 35.0 us in seven splits, on the other kernel 30.2 in seven, 1,300 behind 1,500 86.6 in three and 70.2
+    in two; but 512 behind 3,584 53.9 in five and 58.3 in six. The times are fitted to 333 sizes (16, 24 and 32 heads; the other kernel's 4% off the measured
+    ones in the root mean square, this one's 5%): at 270 others 0.90 of the other kernel's time on average where this kernel alone has 0.91, and 9 more than
+    1.02 of it instead of 40 (`profiles/prefill_eight_splits.txt`). Heads of 64 have two blocks on a CU on both: at one of 603 sizes more than 1.02."""
+    blocks, rows = n_heads * n_seqs * -(-max_q_len // 128), n_heads * n_seqs * max_q_len
+    splits = _eight_splits(blocks, rows, max_kv_len, head_dim, shared)
+    if head_dim != 128:
+        return splits
+    keys, mb = (max_kv_len - max_q_len / 2) / 128, rows * head_dim * 4 / 1e6      # of a block on average (128 at a time); a split's sums
+    these = 10.3 + 2.0 * -(-blocks * splits // 256) * keys / splits + (0.4 + 0.69 * splits * mb if splits > 1 else 0.0)
+    n = blocks * shared
+    other = 10.0 + (3.8 if n <= 256 else 4.7 if n <= 512 else 5.6 + 2.8 * (n - 512) / 512) * keys / shared + 0.43 * shared * mb
+    return splits if these <= 1.02 * other else 0
 
 
 PREFILL_TURNS = -2 ** 31              # ``attention_prefill``'s ``wide_from`` that names the kernel of turns
@@ -2122,7 +2135,8 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
     kernels on the same inputs). ``splits`` > 1 (``prefill_splits``): the keys of
     128 queries are shared out over that many blocks of the same kernel, whose sums lie in ``part_o`` (float32, at least
     splits * T * H * hs) and ``part_ml`` (2 * splits * T * H) until a second kernel merges them; the plain rule only.
-    ``eight_splits``: as many instead, where the splits run on the kernel of eight waves (1: none)."""
+    Above 0 ``wide_from`` names the kernel of 128 queries for them too; else they run on the kernel of eight waves where it is built for the call, in
+    ``eight_splits`` instead, if given (``eight_splits()``; 1: not split, two groups on the keys; 0: on the kernel of 128 queries, in ``splits``)."""
     _dev(q, "q", torch.bfloat16, contiguous=False); _dev(out, "out", torch.bfloat16, contiguous=False)
     _dev(k_cache, "k_cache", torch.bfloat16); _dev(v_cache, "v_cache", torch.bfloat16)
     _dev(cu_seqlens, "cu_seqlens", torch.int32); _dev(kv_before, "kv_before", torch.int32)
@@ -2147,9 +2161,9 @@ def attention_prefill(q, k_cache, v_cache, cu_seqlens, kv_before, block_table, o
         raise KernelError("attention: the block table has fewer rows than there are sequences")
     has_sink, sink_value, sinks = _sink(sink, n_heads, "attention_prefill")
     # (the kernel of eight waves takes a step in splits where it is built for its sizes, no mask but the causal one, and caches at 16-byte addresses)
-    if (splits > 1 and eight_splits is not None and head_dim in (64, 128) and page_size % 64 == 0 and not window and not chunk
+    if (splits > 1 and eight_splits is not None and PREFILL_HEADS < wide_from <= 0 and head_dim in (64, 128) and page_size % 64 == 0 and not window and not chunk
             and n_v == n_kv and slopes is None and sink is None and rule is None and (k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0):
-        splits = int(eight_splits)
+        splits, wide_from = int(eight_splits) or splits, (1, PREFILL_KEYS, 0)[min(int(eight_splits), 2)]
     if splits > 1:
         _dev(part_o, "part_o", torch.float32); _dev(part_ml, "part_ml", torch.float32)
         if part_o.numel() < splits * T * n_heads * head_dim or part_ml.numel() < 2 * splits * T * n_heads:

@@ -34,9 +34,9 @@ def test_split_prefill_attention(H, Kh, hs, page, splits):
     np.testing.assert_allclose(got, whole, atol=2.0 ** -7 * np.abs(ref).max())       # (weights are rounded to 16 bits around another maximum)
 
 
-# pages of 64: as many splits as the second number says, none for 1; of 96, and caches between 16-byte addresses: as the first says
+# pages of 64: as many splits as the second number says, two groups on the keys for 1, the kernel of 128 queries for 0; of 96, and caches between 16-byte addresses: as the first says
 @pytest.mark.parametrize("hs, page, shift, taken", [(64, 64, 0, True), (128, 64, 0, True), (128, 96, 0, False), (64, 64, 4, False)])
-@pytest.mark.parametrize("eight", [1, 2, 5])
+@pytest.mark.parametrize("eight", [0, 1, 2, 5])
 def test_a_number_of_splits_for_the_kernel_of_eight_waves(hs, page, shift, taken, eight):
     H, Kh, before, new = 4, 2, [1300], [200]
     sk, sv, qs = attention_case(np.random.default_rng(hs + eight), H, Kh, hs, before, new, "bfloat16")
@@ -50,8 +50,9 @@ def test_a_number_of_splits_for_the_kernel_of_eight_waves(hs, page, shift, taken
         return run_attention(call, sk, sv, qs, before, new, H, Kh, hs, "bfloat16", np.random.default_rng(1), page=page)
     got, ref = run(splits=4, eight_splits=eight)
     np.testing.assert_allclose(got, ref, atol=1e-2 * np.abs(ref).max())
-    np.testing.assert_array_equal(got, run(splits=eight if taken else 4)[0])
-    assert not np.array_equal(got, run(splits=4 if taken and eight != 4 else 3)[0])
+    alone = dict(splits=1, wide_from=K().PREFILL_KEYS) if eight == 1 else dict(splits=4, wide_from=1) if eight == 0 else dict(splits=eight)
+    np.testing.assert_array_equal(got, run(**alone)[0] if taken else run(splits=4)[0])
+    assert not np.array_equal(got, run(splits=4 if taken else 3)[0])
 
 
 def test_split_prefill_attention_with_one_key_that_counts_and_a_window():

@@ -35,6 +35,14 @@ def test_sequences_of_unequal_lengths_and_last_blocks_that_are_partly_empty():
     assert choice([427] * 8, **large) == 0 and choice([822, 600, 300, 202], **large) == 4 and choice([427] * 8, 64, **large) == 4
 
 
+def test_splits_on_the_faster_of_two_kernels():
+    def s(heads, n_seqs, T, before, hs=128):
+        return lib.eight_splits(lib.prefill_splits(heads, n_seqs, T, [before] * n_seqs, T + before), heads, n_seqs, T, T + before, hs)
+    assert s(24, 1, 1300, 1500) == 0 and s(24, 1, 900, 1024) == 0 and s(24, 1, 300, 1500) == 0 and s(24, 1, 1300, 12000) == 3
+    assert s(24, 1, 512, 512) == 2 and s(24, 1, 512, 3584) == 5 and s(24, 1, 447, 4096) == 5 and s(32, 1, 64, 4000) == 8 and s(32, 1, 1000, 3000) == 1
+    assert s(24, 1, 1300, 1500, 64) == lib.prefill_splits(24, 1, 1300, [1500], 2800, eight=64) > 0
+
+
 def test_splits_of_its_blocks():
     def s(heads, n_seqs, T, before, hs=64):
         return lib.prefill_splits(heads, n_seqs, T, [before] * n_seqs, T + before, eight=hs)
@@ -53,12 +61,12 @@ def test_splits_of_its_blocks():
 @pytest.mark.parametrize("more, taken", [({}, True), (dict(head_dim=64), True), (dict(page_size=192), True), (dict(page_size=96), False), (dict(head_dim=96), False),
                                          (dict(window=100), False), (dict(chunk=64), False), (dict(sink=0.5), False), (dict(n_v_heads=1), False), (dict(at=4), False)])
 def test_its_splits_are_for_its_calls_alone(monkeypatch, more, taken):
-    """``eight_splits`` stands in for ``splits`` where the kernel of eight waves runs: not with another mask, other sizes, or caches between 16-byte addresses."""
+    """``eight_splits`` stands in for ``splits`` where the kernel of eight waves can run: not with another mask, other sizes, or caches between 16-byte addresses."""
     from types import SimpleNamespace
 
     import torch
     given = []
-    calls = SimpleNamespace(gl3_attention_prefill=lambda *a: given.append(a[-5]) or 0)
+    calls = SimpleNamespace(gl3_attention_prefill=lambda *a: given.append((a[-5], a[19])) or 0)
     for name, stand_in in (("_dev", lambda *a, **kw: None), ("_ptr", lambda t: None), ("_stream", lambda: None), ("library", lambda: calls)):
         monkeypatch.setattr(lib, name, stand_in)
     kw = dict(head_dim=128, page_size=64, window=None, at=0) | more
@@ -68,14 +76,14 @@ def test_its_splits_are_for_its_calls_alone(monkeypatch, more, taken):
         return torch.empty(heads * hs * page + 8, dtype=torch.bfloat16)[at:at + heads * hs * page].view(1, heads, *tile)
     q, out = torch.zeros(3, 2 * hs), torch.zeros(3, 2 * hs)
     i32 = torch.zeros(2, dtype=torch.int32)
-    for n in (1, 2):
+    for n, call in ((0, (3, 1)), (1, (1, lib.PREFILL_KEYS)), (2, (2, 0))):
         lib.attention_prefill(q, cache(2, page, hs), cache(kw.get("n_v_heads", 2), hs, page), i32, i32[:1], i32.view(2, 1), out, 3, 2, 2, hs, page, window, 0.1,
                               splits=3, part_o=torch.zeros(18 * hs), part_ml=torch.zeros(36), eight_splits=n, **kw)
-        assert given.pop() == (n if taken else 3)
+        assert given.pop() == (call if taken else (3, 0))
 
 
-# (no splits at all, where the other kernel has two; fewer; not its sizes: none of its own)
-@pytest.mark.parametrize("heads, hs, page, T, before, eight", [(32, 64, 64, 1000, 6000, 1), (24, 128, 128, 512, 3584, 5), (32, 64, 64, 150, 3000, 4), (32, 64, 96, 512, 512, None),
+# (no splits at all, where the other kernel has two; fewer; the other kernel's; not its sizes: none of its own)
+@pytest.mark.parametrize("heads, hs, page, T, before, eight", [(32, 64, 64, 1000, 6000, 1), (24, 128, 128, 512, 3584, 5), (32, 64, 64, 150, 3000, 4), (24, 128, 64, 1300, 1500, 0), (32, 64, 96, 512, 512, None),
                                                                (32, 96, 64, 512, 512, None)])
 def test_a_layer_asks_for_its_splits(monkeypatch, heads, hs, page, T, before, eight):
     from types import SimpleNamespace
@@ -96,7 +104,7 @@ def test_a_layer_asks_for_its_splits(monkeypatch, heads, hs, page, T, before, ei
     monkeypatch.setattr(lib, "attention_prefill", lambda *a, **kw: calls.append((kw["splits"], kw.get("eight_splits"))))
     ops.attention(ctx, torch.zeros(1), torch.zeros(1, 8, page, hs), None, None, None, heads, 8, hs, None, 0.1)
     assert calls == [(lib.prefill_splits(heads, 1, T, [before], T + before), eight)] and len(walks) == 1
-    assert eight in (None, lib.prefill_splits(heads, 1, T, [before], T + before, eight=hs))
+    assert eight in (0, None, lib.prefill_splits(heads, 1, T, [before], T + before, eight=hs))
 
 
 # one, two, three and four heads a kv head; waves, blocks and chunks with one row and all but one, one chunk (none for the second group); sequences that start no
