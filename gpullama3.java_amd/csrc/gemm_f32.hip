@@ -698,9 +698,11 @@ extern "C" int gl3_f32_stream_shape(int M, int N, int gated) {
 // Whether two tiles (gemm_f32_two_tiles_kernel) are expected to take less than 0.95 of the best single tile's time, and which: 64 * rows of large
 // tiles + 8 * the large tile + the small one; 0: one tile. The blocks are all handed out at once, about as many of either kind to every CU, so a CU's
 // time is taken as that of its large tiles and then its small ones. (As if the small ones went to the CUs that have no large tile: of 42 sizes
-// seven took 1.03 to 1.08 times as long as one tile, those this rule leaves out.) A small tile beside others takes 1.05 of its time. Measured at 72 sizes
-// (100 to 2,500 rows, the 1B layers' products and the 3B layers' QKV) that a margin of 0.96 without the 1.05 takes: 0.82 to 1.02 times as long as one tile
-// and 0.91 on average, but for two (1.03, 1.11), which this rule leaves out.
+// seven took 1.03 to 1.08 times as long as one tile, those this rule leaves out.) A small tile beside others takes 1.05 of its time. A single row of large tiles of 64
+// rows of A over more than 40,000 rows of W is left out: one tile reads each of them once, for all rows of A, two kinds twice (128,256 rows of W,
+// K = 2,048, 96 rows: 1.84 times the bytes from memory, 446 -> 490 us; 70 rows 423 and 461; 210 in three rows of large tiles 931 and 928). Measured at 179 sizes (66
+// to 4,096 rows, K of 768 to 14,336, 1,024 to 128,256 rows of W) 0.83 to 1.04 times as long as one tile, 0.920 on average; at 9 with that row 1.04 to 1.10
+// (profiles/float32_two_tiles.txt).
 extern "C" int gl3_f32_stream_two(int M, int N, int gated) {
   float least;
   f3_best_tile(M, N, gated, least);
@@ -709,7 +711,7 @@ extern "C" int gl3_f32_stream_two(int M, int N, int gated) {
   int best = 0;
   for (int i = 0; i < 3; ++i) {
     const F3Cost& t = f3_cost[i];
-    for (int r = (M - 1) / t.bm, first = r - 3; r > 0 && r >= first; --r) {
+    for (int r = (M - 1) / t.bm, first = r - 3; r > (i > 0 && rows > 40000 ? 1 : 0) && r >= first; --r) {
       const float big = (float)((r * ((rows + t.bn - 1) / t.bn) + 255) / 256) * t.each;
       for (int j = i < 2 ? 3 : 4; j < (gated ? 4 : 5); ++j) {      // (64 x 32 behind 64 x 64 never is the best)
         const F3Cost& u = f3_cost[j];

@@ -81,3 +81,12 @@ def test_a_prompt_step_runs_without_splits_where_their_buffers_have_no_room(monk
         assert calls == [splits] * 2 and (splits > 1) == (held > small)
         assert len(asked) == len(set(asked))                                                   # (each buffer asked for once)
         assert sum(t.numel() for t in engine.workspace._flat.values()) == held                 # (what is of no use is not kept)
+
+
+def test_two_tiles_of_a_32_bit_product_over_very_many_rows_of_weights():
+    """No single row of large tiles there: the weights are read twice, and the smaller tile alone takes less time."""
+    def rows_of_large_tiles(M, N, gated=0):
+        return lib.library().gl3_f32_stream_two(M, N, gated) // 64
+    assert [rows_of_large_tiles(M, 128256) for M in (70, 82, 96)] == [0] * 3 and rows_of_large_tiles(73, 65536) == rows_of_large_tiles(77, 65536, 1) == 0
+    assert rows_of_large_tiles(210, 128256) == 3 and rows_of_large_tiles(288, 65536) == 2
+    assert rows_of_large_tiles(67, 32768) == 1 and rows_of_large_tiles(77, 14336, 1) == 1 and rows_of_large_tiles(513, 2048) == 8
