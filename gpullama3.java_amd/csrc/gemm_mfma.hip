@@ -320,7 +320,9 @@ static int launch_shape(const void* A, const void* W, void* C, int M, int N, int
 // and a half behind the large tiles the one that ends first, where it saves 4% or more. Small tiles that follow large ones take 0.48 us a step and 4.5
 // beside them, or 0.60 and 3.0. Measured at 216 sizes (600 to 13,000 rows, the products of three models, up to six divisions of each): the
 // choice is within 4% of the best at all but six (1.11). At 97 other sizes where the rule takes two tiles (300 to 16,000 rows, four models'
-// products; profiles/two_tiles.txt) they take 0.78 to 1.02 times as long as the single tile taken before, 0.90 on average.
+// products; profiles/two_tiles.txt) they take 0.78 to 1.02 times as long as the single tile taken before, 0.90 on average. Not for up to 1,024 rows over more than
+// 40,000 rows of W: the large tiles and the small ones each read them from memory, which one tile's blocks of the same columns share (65,536 rows of W, K = 2,048: 262
+// rows 120 us in one tile and 158 in two, 640 182 and 195; 128,256, K = 4,096, 262 387 and 456; 1,030 to 2,221 rows 0.95 to 1.04 in two, 0.99 on average).
 static int choose_turns_shape(int M, int N, int K, int slices, bool gated, bool two) {
   static const int rows[3] = {128, 128, 256}, cols[3] = {128, 256, 256}, shape[3] = {1, 5, 2};
   static const double step_us[3] = {0.40, 0.60, 1.0}, round_us[3] = {0.9, 3.0, 4.5};
@@ -339,10 +341,10 @@ static int choose_turns_shape(int M, int N, int K, int slices, bool gated, bool 
       least = time;
     }
   }
-  if (!two) return best;
+  const int most = (M - 1) / 256;
+  if (!two || (most < 4 && (gated ? 2L : 1L) * N > 40000)) return best;
   least *= 0.96;
   const double large = steps * step_us[2] + round_us[2];
-  const int most = (M - 1) / 256;
   for (int r = most; r > 0 && (most - r) * per_xcd(256, 2) <= 48; --r) {
     const long big = per_xcd(r * 256, 2);
     const double early = big / 32 * large, late = early + (big % 32 ? large : 0);      // when an XCD's CUs are done with the large tiles
@@ -366,6 +368,9 @@ static int choose_turns_shape(int M, int N, int K, int slices, bool gated, bool 
   }
   return best;
 }
+
+// (for tests: the library's choice where gemm_mfma_turns_kernel takes the product)
+extern "C" int gl3_turns_shape(int M, int N, int K, int slices, int gated) { return choose_turns_shape(M, N, K, slices, gated, true); }
 
 // The same where it does not (K in no whole steps of 64, or offsets beyond its 31 bits), on the kernel without turns: 1 (128 x 128),
 // 2 (256 x 256) or 5 (128 rows x 256).

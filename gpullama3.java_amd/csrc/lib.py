@@ -111,6 +111,7 @@ def _declare(lib):
         "gl3_qkv_rope_cache": [P, P, I, F, P, P, L, I, I, L, L, P, P, P, I, P, P, P, P, I, I, I, I, I, I, P, P, P, I, P],
         "gl3_token_facts": [P, P, P, I, I, P, P, I, P, P, P, I, P],
         "gl3_gemm_mfma": [P, P, P, I, I, I, I, L, L, L, I, I, P, L, L, P, I, I, I, P, F, F, P, P],
+        "gl3_turns_shape": [I, I, I, I, I],
         "gl3_f32_shape": [I, I, I],
         "gl3_f32_stream_shape": [I, I, I],
         "gl3_f32_stream_two": [I, I, I],

@@ -90,3 +90,12 @@ def test_two_tiles_of_a_32_bit_product_over_very_many_rows_of_weights():
     assert [rows_of_large_tiles(M, 128256) for M in (70, 82, 96)] == [0] * 3 and rows_of_large_tiles(73, 65536) == rows_of_large_tiles(77, 65536, 1) == 0
     assert rows_of_large_tiles(210, 128256) == 3 and rows_of_large_tiles(288, 65536) == 2
     assert rows_of_large_tiles(67, 32768) == 1 and rows_of_large_tiles(77, 14336, 1) == 1 and rows_of_large_tiles(513, 2048) == 8
+
+
+def test_two_tiles_of_a_product_over_very_many_rows_of_weights():
+    """Few rows of the operand: one tile, whose blocks read the weights once; many, or fewer rows of weights: two where the last round is mostly empty."""
+    def two(M, N, K, gated=0):
+        return lib.library().gl3_turns_shape(M, N, K, 1, gated) > 8
+    for N, K, gated in ((128256, 2048, 0), (128256, 4096, 0), (65536, 2048, 0), (32768, 4096, 1), (256000, 1024, 0)):
+        assert not any(two(M, N, K, gated) for M in range(66, 1025))
+    assert two(1030, 151936, 1024) and two(600, 32768, 4096) and two(2221, 8192, 2048, 1) and two(5886, 3072, 3072)
