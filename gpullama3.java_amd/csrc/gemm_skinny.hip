@@ -981,8 +981,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_decode_kernel(
 // bfloat16(weight * x) and the rows' 1/rms, from the partial sums of squares, is applied to the sums.
 //
 // DMA (W in one of its copies' orders, K in whole pairs of k-steps): a wave's lines of A go from memory straight to their places in its piece of
-// shared memory, which holds two pairs, so that no registers carry them, and two pairs of k-steps are on their way instead of one. With four token
-// tiles and one strip or a plain epilogue the trip to memory behind each of a wave's few pairs is what bounds the product: 64 rows of 3,072 x 2,048
+// shared memory, which holds two pairs, so that no registers carry them. W's loads are two pairs of k-steps ahead. The lines of A are asked for as far ahead, but in front
+// of W's loads of the same pair, and the wait for a pair leaves out as many loads as W's of the next: it is over when the next pair's lines have come too, so
+// that their trip lies beside nothing but the other waves' work. With four token
+// tiles and one strip or a plain epilogue the trips to memory behind each of a wave's few pairs are what bounds the product: 64 rows of 3,072 x 2,048
 // 9.64 -> 8.11 us in a graph, 2,048 x 2,048 in four slices 6.29 -> 6.02, 2,048 x 8,192 12.32 -> 12.00, 3,072 x 3,072 8.96 -> 8.52, 4,096 x 14,336 31.4 -> 31.0.
 // Fewer tiles have less of A to carry (17 rows of 3,072 x 3,072 6.29 -> 6.55, 48 7.32 -> 7.60), gated ones ask for enough of W as it is
 // (64 rows of 8,192 x 2,048 18.7 -> 19.2): those go as before. The same sums in the same order.
@@ -1180,7 +1182,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_wide_kernel(const bf16_t*
   if constexpr (DMA) {
     auto pair = [&](int i, auto slot) {
       constexpr int S = decltype(slot)::value;
-      mf_wait_loads<2 * NWT>();                    // all but the next pair's W has come
+      mf_wait_loads<2 * NWT>();                    // all but the next pair's W has come (its lines of A have)
       if (pair_at(i) < p_end) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -1697,8 +1699,9 @@ extern "C" int gl3_qkv_rope_cache(const void* a_rows, const float* ssq, int n_pa
   if (w_once) { a.W = w_tiled; a.wl = 1; }
   if (!ssq && waves == 0 && M > 16 && wide_addressable(M, N, K, lda, ldw)) {
     // many rows, read in whole lines: two strips a block, so that the rows are read half as often, where one
-    // strip a block would be more blocks than CUs (N = 3,072, K = 2,048, 64 rows: 10.0 us with two, 8.9 us with
-    // one; N = 5,120, K = 3,072: 16.3 against 20.7 us)
+    // strip a block would be more blocks than CUs (64 rows, rows straight into shared memory: N = 3,072, K = 2,048 9.6 us with one
+    // and 11.4 with two, N = 4,096 10.0 and 11.6, N = 4,352 15.8 and 11.8, N = 5,120, K = 3,072 21.6 and 15.4; 32 rows, through registers: 7.6 and
+    // 9.2, 8.6 and 9.5, 11.5 and 9.6, 16.7 and 13.7)
     const int tiles = (M + 15) / 16;
     if ((N + 15) / 16 <= 256)
       return tiles <= 2   ? launch_wide<2, 1, SK_QKV, bf16_t>(a, 1, 0)

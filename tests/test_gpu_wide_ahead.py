@@ -1,4 +1,4 @@
-"""Products of 49 to 64 rows over a weight in one of its copies' orders, whose rows of ``a`` go from memory straight into shared memory two pairs of
+"""Products of 49 to 64 rows over a weight in one of its copies' orders, whose rows of ``a`` go from memory straight into shared memory, the weight's two pairs of
 k-steps ahead: the sums of the kernel for stored rows, and nothing but the call's own rows and columns read."""
 import numpy as np
 import pytest
