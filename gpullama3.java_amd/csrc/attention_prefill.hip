@@ -927,9 +927,10 @@ __global__ __launch_bounds__(512, 2) void attention_prefill_turns_kernel(
 // from memory straight into shared memory, as they lie in the cache (the operands' order, as in the kernel of turns).
 // GROUPS = 2, for few blocks: 128 queries of one head, four waves of 32 on the even chunks of keys and four on the odd ones, whose sums are
 // brought together at the end: a block's way along the keys is half as long. GROUPS = 1: 128 queries of two heads of one kv head, which
-// share the chunks: the same sums in the same order as the kernel of 128 queries, bit for bit. Two groups' error against 64 bits is 0.993 times
-// that on average, 1.0002 at most (54 sizes of 37 to 3,001 tokens, contexts to 3,000, scores spread 0.3 to 3; heads of 64, and of 128): their maxima are
-// nearer to the weights. (With one maximum for 64 keys heads of 128 took 8 to 15% less time, at up to 1.004 times the error.)
+// share the chunks: the same sums in the same order as the kernel of 128 queries, bit for bit. Two groups' error against 64 bits is 0.983 to 0.998 times
+// that of the kernels beside it at 9 sizes of 333 to 2,048 tokens with scores spread 0.3 to 3, heads of 64 and of 128, the average of 16 sets of inputs each, none of which
+// is larger (`profiles/prefill_eight_error.txt`): their maxima are nearer to the weights. (With one maximum for 64 keys heads of 128 took 8 to 15% less time, at up to
+// 1.004 times the error.) A value that is not finite spoils the queries that share its 64 keys (heads of 128: 32), as in that kernel.
 // Heads of 64: 115 registers where the kernel of 128 queries has 157, so that four waves share a SIMD and while some have its matrix cores others
 // work out their softmax (a SIMD has one vector instruction of a wave about every eight cycles, of four waves one every 4.2, an
 // exponential 8.2, an addition 2.4); two blocks a CU. Heads of 128: 164, two waves a SIMD and a block a CU.

@@ -2090,9 +2090,9 @@ def prefill_splits(n_heads, n_seqs, max_q_len, kv_before, max_kv_len, eight=0):
     units busy, 1.2 or 2.1 us for 128 keys, and two on a CU take twice as long, so the splits are those whose rounds of 256 blocks are done
     first, a merge being 6 us and a split's sums 2.8 TB/s of it, but at least half as many as the rule above has: a block's two groups have a maximum
     each, and the more maxima the more weights are one, which rounding leaves alone (with half as many maxima the error against 64 bits was 1.002 to 1.019
-    times that of the rule above; so 0.976 to 1.001 at 72 sizes, spreads of the scores among them). 32 heads of 64: 300 tokens behind 3,000 31.2 us in the six splits
-    of the rule above, 512 behind 512 17.5 in two, 14.9 without, 512 behind 3,584 32.6 in two, 35.6 in four; 24 heads of 128: 512 behind 3,584 64 in six on
-    the kernel of 128 queries, 51.9 in five, 64.1 in three, 50.9 in two."""
+    times that of the rule above; so 0.981 to 1.0003 at 10 sizes, three spreads of the scores each, averages of 16 or 48 sets of inputs: `profiles/prefill_eight_error.txt`). 32 heads of 64: 300 tokens behind 3,000 32.4 us in the
+    six splits of the rule above, 28.1 in five, 512 behind 512 18.4 in two, 15.7 without, 512 behind 3,584 34.7 in two, 37.0 in four; 24 heads of 128: 512 behind
+    3,584 58.3 in six on the kernel of 128 queries, 53.9 in five, 65.9 in three, 52.6 in two (`profiles/prefill_eight_splits.txt`)."""
     blocks = n_heads * n_seqs * -(-max_q_len // 128)
     if blocks >= 512 or max_kv_len < PREFILL_SPLIT_KEYS or not kv_before or min(kv_before) < max_q_len:
         return 1

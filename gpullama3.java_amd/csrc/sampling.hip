@@ -916,7 +916,9 @@ extern "C" int gl3_sample(const float* logits, long ld, float* work, const float
 // A whole call of a sampler whose caller waits for the tokens: parameters in host memory, tokens into host memory. The parameters
 // travel inside the first kernel's launch and the tokens are written by the last kernel into pinned memory (`out`: hipHostMalloc's, which
 // the GPU reaches under the host's address), where the call looks for them: nothing to copy on either side, and no wait for the stream's end,
-// which came 5 us behind the tokens. 8 rows of 128,256 logits 36.8 -> 31.6 us a call (greedy 22.7 -> 18.0), 64 rows 66.7 -> 62.4.
+// which came 5 us behind the tokens. 8 rows of 128,256 logits 36.8 -> 31.6 us a call, 64 rows 66.7 -> 62.4; greedy 8 rows 22.3 -> 17.5, other logits each
+// time 24.4 -> 19.2, after 3 ms without work 31.6 -> 25.4. Behind a decode step, which takes longer than the look, the call waits for the stream as ever and is no shorter
+// (both ways of waiting keep the calling thread's core busy: 2,582 us of its time behind 2.6 ms of products).
 // work: gl3_sample_work_floats(n_rows, V) floats and 3 * n_rows for the parameters. temperature null: every row greedy (work as
 // gl3_argmax's). The stream must not be capturing.
 extern "C" int gl3_sample_host(const float* logits, long ld, float* work, const float* temperature, const float* top_p,
